@@ -69,7 +69,7 @@ def check_blocks(Sq, Sk, block_q=None, block_k_major=None, block_k=None, block_q
         if not isinstance(blk, (int, np.integer)) or blk <= 0:
             raise ValueError(f"{name}={blk!r} must be a positive int")
         if n % SEQ_ALIGN:
-            return  # ragged length: the tensors are padded to the tile; the reference floors silently here (flex_attention_kernel.py:91)
+            return  # ragged length: the kernels' last tile starts early; the reference floors silently here (flex_attention_kernel.py:91)
         if n % blk:
             raise ValueError(f"{name}={blk} does not divide sequence length {n}")
     _div("block_q", block_q, Sq)
@@ -242,7 +242,16 @@ SEQ_ALIGN = 128   # every kernel's tiles divide it
 
 
 def padded_len(n: int) -> int:
-    return (n + SEQ_ALIGN - 1) // SEQ_ALIGN * SEQ_ALIGN
+    """Length the tensors of a call of sequence length n are padded to: the kernels take every length from one tile
+    on (their last tile starts early where the length is no multiple of it); shorter ones are padded to the tile."""
+    return n if n >= SEQ_ALIGN else SEQ_ALIGN
+
+
+def tile_lengths(bm: BlockMap):
+    """(Sq, Sk, pad) of the C parameter blocks: the lengths in whole tiles of the block map and, packed, the rows by
+    which these exceed the tensors (FLEXATTN_PAD)."""
+    Sq, Sk = bm.nq * bm.block_q, bm.nk * bm.block_k
+    return Sq, Sk, (Sq - bm.Sq) | (Sk - bm.Sk) << 16
 
 
 def kernel_head_dim(D: int, dtype) -> int:
@@ -310,9 +319,7 @@ def score_spec_c(score_fn: Optional[Callable], Hq: int, device, mod_q: int, mod_
 
 def kernel_block_map(pass_id: int, spec: MaskSpec, q: torch.Tensor, Sq: int, Sk: int, D: int, score_fn=None) -> BlockMap:
     bq, bk = _lib.tile_shape(pass_id, dtype_code(q), D)
-    if Sq % bq or Sk % bk:
-        raise ValueError(f"sequence lengths ({Sq}, {Sk}) must be multiples of the kernel tile ({bq}, {bk})")
-    return build_block_map(spec, Sq, Sk, bq, bk, q.device, score_code=score_code_of(score_fn))
+    return build_block_map(spec, Sq, Sk, bq, bk, q.device, score_code=score_code_of(score_fn), ragged=True)
 
 
 def mostly_partial_custom_mask(spec: MaskSpec, bm: BlockMap) -> bool:

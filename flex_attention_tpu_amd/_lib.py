@@ -106,7 +106,7 @@ class FwdParamsC(C.Structure):
         ("dtype", C.c_int32),
         ("sm_scale", C.c_float),
         ("flags", C.c_int32),
-        ("reserved", C.c_int32),
+        ("pad", C.c_int32),
         ("score", ScoreSpecC),
         ("mask", MaskSpecC),
         ("map", BlockMapC),
@@ -125,7 +125,7 @@ class BwdParamsC(C.Structure):
         ("dtype", C.c_int32),
         ("sm_scale", C.c_float),
         ("flags", C.c_int32),
-        ("reserved", C.c_int32),
+        ("pad", C.c_int32),
         ("score", ScoreSpecC),
         ("mask", MaskSpecC),
         ("map", BlockMapC),
@@ -144,6 +144,7 @@ EXPORTS = (
     "flexattn_last_error_string",
     "flexattn_tile_shape",
     "flexattn_build_block_mask",
+    "flexattn_build_block_mask_ragged",
     "flexattn_build_ds_index",
     "flexattn_fwd",
     "flexattn_fwd_noalloc",
@@ -167,6 +168,7 @@ def _bind(lib: C.CDLL) -> C.CDLL:
     lib.flexattn_build_block_mask.argtypes = [
         C.POINTER(MaskSpecC), C.c_int32, C.c_int32, C.c_int32, C.c_int32,
         C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
+    lib.flexattn_build_block_mask_ragged.argtypes = lib.flexattn_build_block_mask.argtypes
     lib.flexattn_build_ds_index.argtypes = [C.POINTER(BlockMapC), C.c_void_p, C.c_void_p, C.c_void_p]
     lib.flexattn_fwd.argtypes = [C.POINTER(FwdParamsC), C.c_void_p]
     lib.flexattn_fwd_noalloc.argtypes = [C.POINTER(FwdParamsC), C.c_void_p]
@@ -176,8 +178,8 @@ def _bind(lib: C.CDLL) -> C.CDLL:
     lib.flexattn_bwd_ds_bytes.restype = C.c_int64
     lib.flexattn_bwd_dkv.argtypes = [C.POINTER(BwdParamsC), C.c_void_p]
     lib.flexattn_bwd.argtypes = [C.POINTER(BwdParamsC), C.POINTER(BwdParamsC), C.c_void_p]
-    for name in ("flexattn_tile_shape", "flexattn_build_block_mask", "flexattn_build_ds_index", "flexattn_fwd", "flexattn_fwd_noalloc", "flexattn_bwd_delta",
-                 "flexattn_bwd_dq", "flexattn_bwd_dkv", "flexattn_bwd"):
+    for name in ("flexattn_tile_shape", "flexattn_build_block_mask", "flexattn_build_block_mask_ragged", "flexattn_build_ds_index", "flexattn_fwd",
+                 "flexattn_fwd_noalloc", "flexattn_bwd_delta", "flexattn_bwd_dq", "flexattn_bwd_dkv", "flexattn_bwd"):
         getattr(lib, name).restype = C.c_int
     return lib
 

@@ -60,12 +60,13 @@ class BlockMap:
     """Device-resident block map at (block_q x block_k) granularity.
 
     state[qb, kb]: 0 skip, 1 partial, 2 full.  kv_idx[qb, :kv_cnt[qb]] / q_idx[kb, :q_cnt[kb]] are
-    the ascending lists of blocks to visit per q-block row / kv-block column.
+    the ascending lists of blocks to visit per q-block row / kv-block column.  The last blocks of lengths that are
+    no multiples of the blocks end at the lengths (a block cut off at Sk is at most partial).
     """
 
     def __init__(self, spec: MaskSpec, Sq: int, Sk: int, block_q: int, block_k: int, device):
         self.spec, self.Sq, self.Sk, self.block_q, self.block_k = spec, Sq, Sk, block_q, block_k
-        self.nq, self.nk = Sq // block_q, Sk // block_k
+        self.nq, self.nk = -(-Sq // block_q), -(-Sk // block_k)
         self.state = torch.empty(self.nq, self.nk, dtype=torch.uint8, device=device)
         self.kv_cnt = torch.empty(self.nq, dtype=torch.int32, device=device)
         self.kv_idx = torch.empty(self.nq, self.nk, dtype=torch.int32, device=device)
@@ -219,10 +220,11 @@ def mask_spec_c(spec: MaskSpec, Sq: int, Sk: int, device) -> _lib.MaskSpecC:
 
 
 def build_block_map(spec: MaskSpec, Sq: int, Sk: int, block_q: int, block_k: int, device,
-                    cache: bool = True, score_code=None) -> BlockMap:
+                    cache: bool = True, score_code=None, ragged: bool = False) -> BlockMap:
     """Runs the GPU block-mask builder (or returns the cached map for this specification).  A compiled
     mask closure is built by the functor library that holds it (`score_code`: the compiled score closure of
-    the same call, if any, so that one library serves both)."""
+    the same call, if any, so that one library serves both).  ``ragged``: take lengths that are no multiples of the
+    blocks."""
     device = torch.device(device)
     key = (spec, Sq, Sk, block_q, block_k, str(device))
     if cache:
@@ -230,14 +232,14 @@ def build_block_map(spec: MaskSpec, Sq: int, Sk: int, block_q: int, block_k: int
         if hit is not None:
             hit.wait_ready(device)
             return hit
-    if Sq % block_q or Sk % block_k:
+    if not ragged and (Sq % block_q or Sk % block_k):
         raise ValueError(f"Sq={Sq} / Sk={Sk} not divisible by blocks {block_q} / {block_k}")
     lib = _lib.load_for(score_code if spec.custom is not None else None, spec.custom)
     bm = BlockMap(spec, Sq, Sk, block_q, block_k, device)
     mc = mask_spec_c(spec, Sq, Sk, device)
     stream = torch.cuda.current_stream(device).cuda_stream
     with torch.cuda.device(device):
-        _lib.check(lib.flexattn_build_block_mask(
+        _lib.check(lib.flexattn_build_block_mask_ragged(
             C.byref(mc), Sq, Sk, block_q, block_k, bm.state.data_ptr(), bm.kv_cnt.data_ptr(),
             bm.kv_idx.data_ptr(), bm.q_cnt.data_ptr(), bm.q_idx.data_ptr(), stream), lib)
         bm.built_on = stream

@@ -140,9 +140,18 @@ static int check_scale_flags(float sm_scale, int flags) {
   return FLEXATTN_OK;
 }
 
+// Rows of the padded lengths beyond the tensors (FLEXATTN_PAD): less than a tile, and at least one tile is left.
+static int check_pad(int pad, int Sq, int Sk, int bq, int bk) {
+  const int pad_q = pad & 0xffff, pad_k = (pad >> 16) & 0xffff;
+  if (pad < 0 || pad_q >= bq || pad_k >= bk || Sq - pad_q < bq || Sk - pad_k < bk)
+    return set_error(FLEXATTN_EINVAL, "padding of %d q and %d kv rows: must be less than a tile (%d, %d) and leave at least one", pad_q,
+                     pad_k, bq, bk);
+  return FLEXATTN_OK;
+}
+
 // `tile_pass`: the pass whose tile granularity the map must have (the dq pass reads the dk/dv kernel's dS blocks at
 // that kernel's tiles)
-static int check_shape(int pass, int B, int Hq, int Hkv, int Sq, int Sk, int D, int dtype,
+static int check_shape(int pass, int B, int Hq, int Hkv, int Sq, int Sk, int pad, int D, int dtype,
                        const flexattn_block_map& map, int tile_pass = -1) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || Sq <= 0 || Sk <= 0 || D <= 0)
     return set_error(FLEXATTN_EINVAL, "non-positive dimension (B=%d Hq=%d Hkv=%d Sq=%d Sk=%d D=%d)", B, Hq, Hkv, Sq, Sk, D);
@@ -152,6 +161,7 @@ static int check_shape(int pass, int B, int Hq, int Hkv, int Sq, int Sk, int D, 
   if (rc != FLEXATTN_OK) return rc;
   if (Sq % bq != 0) return set_error(FLEXATTN_EINVAL, "Sq=%d is not a multiple of the q tile %d", Sq, bq);
   if (Sk % bk != 0) return set_error(FLEXATTN_EINVAL, "Sk=%d is not a multiple of the kv tile %d", Sk, bk);
+  if ((rc = check_pad(pad, Sq, Sk, bq, bk)) != FLEXATTN_OK) return rc;
   if (map.state == nullptr) return set_error(FLEXATTN_EINVAL, "block map state is NULL");
   if (map.block_q != bq || map.block_k != bk || map.nq != Sq / bq || map.nk != Sk / bk)
     return set_error(FLEXATTN_EINVAL, "block map is %dx%d blocks of %dx%d, kernel needs %dx%d blocks of %dx%d",
@@ -235,13 +245,14 @@ static int to_bwd_args(const flexattn_bwd_params* p, int pass, BwdArgs* a) {
   if (pass == FLEXATTN_PASS_DKV && (!p->dk || !p->dv)) return set_error(FLEXATTN_EINVAL, "dk or dv is NULL");
   int rc = check_ds(p);
   if (rc != FLEXATTN_OK) return rc;
-  rc = check_shape(pass, p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->D, p->dtype, p->map, p->ds ? FLEXATTN_PASS_DKV : -1);
+  const int Sq = p->Sq - (p->pad & 0xffff), Sk = p->Sk - (p->pad >> 16);   // the tensors' lengths
+  rc = check_shape(pass, p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->pad, p->D, p->dtype, p->map, p->ds ? FLEXATTN_PASS_DKV : -1);
   if (rc != FLEXATTN_OK) return rc;
   if ((rc = check_scale_flags(p->sm_scale, p->flags)) != FLEXATTN_OK) return rc;
   if ((rc = check_score(p->score)) != FLEXATTN_OK) return rc;
   if ((rc = check_mask(p->mask)) != FLEXATTN_OK) return rc;
   if ((rc = check_doc_batches(p->mask, p->B)) != FLEXATTN_OK) return rc;
-  if ((rc = check_bias(p->ab, p->B, p->Hq, p->Sq, p->Sk)) != FLEXATTN_OK) return rc;
+  if ((rc = check_bias(p->ab, p->B, p->Hq, Sq, Sk)) != FLEXATTN_OK) return rc;
   if (p->dab != nullptr) {
     if (pass != FLEXATTN_PASS_DQ) return set_error(FLEXATTN_EINVAL, "dab is an output of flexattn_bwd_dq");
     if (p->ds != nullptr) return set_error(FLEXATTN_EINVAL, "dab and ds exclude each other (the dq pass from dS recomputes nothing)");
@@ -256,10 +267,10 @@ static int to_bwd_args(const flexattn_bwd_params* p, int pass, BwdArgs* a) {
   a->q = p->q; a->k = p->k; a->v = p->v; a->dout = p->dout;
   a->l = p->l; a->m = p->m; a->delta = p->delta;
   a->dq = p->dq; a->dk = p->dk; a->dv = p->dv;
-  a->B = p->B; a->Hq = p->Hq; a->Hkv = p->Hkv; a->Sq = p->Sq; a->Sk = p->Sk;
+  a->B = p->B; a->Hq = p->Hq; a->Hkv = p->Hkv; a->Sq = Sq; a->Sk = Sk;
   a->sm_scale = p->sm_scale;
   a->flags = p->flags;
-  a->score = to_args(p->score, p->ab, p->Sk);
+  a->score = to_args(p->score, p->ab, Sk);
   a->mask = to_args(p->mask);
   a->map = (pass == FLEXATTN_PASS_DKV) ? col_view(p->map) : row_view(p->map);
   return FLEXATTN_OK;
@@ -281,19 +292,20 @@ static int delta_first(BwdArgs* a, int D, int dtype, hipStream_t s) {
 static int fwd_with_map(const flexattn_fwd_params* p, const flexattn_block_map& map, hipStream_t s) {
   if (!p->q || !p->k || !p->v || !p->o) return set_error(FLEXATTN_EINVAL, "q, k, v or o is NULL");
   if ((p->l == nullptr) != (p->m == nullptr)) return set_error(FLEXATTN_EINVAL, "l and m must both be given or both NULL");
-  int rc = check_shape(FLEXATTN_PASS_FWD, p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->D, p->dtype, map);
+  const int Sq = p->Sq - (p->pad & 0xffff), Sk = p->Sk - (p->pad >> 16);   // the tensors' lengths
+  int rc = check_shape(FLEXATTN_PASS_FWD, p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->pad, p->D, p->dtype, map);
   if (rc != FLEXATTN_OK) return rc;
   if ((rc = check_scale_flags(p->sm_scale, p->flags)) != FLEXATTN_OK) return rc;
   if ((rc = check_score(p->score)) != FLEXATTN_OK) return rc;
   if ((rc = check_mask(p->mask)) != FLEXATTN_OK) return rc;
   if ((rc = check_doc_batches(p->mask, p->B)) != FLEXATTN_OK) return rc;
-  if ((rc = check_bias(p->ab, p->B, p->Hq, p->Sq, p->Sk)) != FLEXATTN_OK) return rc;
+  if ((rc = check_bias(p->ab, p->B, p->Hq, Sq, Sk)) != FLEXATTN_OK) return rc;
   FwdArgs a;
   a.q = p->q; a.k = p->k; a.v = p->v; a.o = p->o; a.l = p->l; a.m = p->m;
-  a.B = p->B; a.Hq = p->Hq; a.Hkv = p->Hkv; a.Sq = p->Sq; a.Sk = p->Sk;
+  a.B = p->B; a.Hq = p->Hq; a.Hkv = p->Hkv; a.Sq = Sq; a.Sk = Sk;
   a.sm_scale = p->sm_scale;
   a.flags = p->flags;
-  a.score = to_args(p->score, p->ab, p->Sk);
+  a.score = to_args(p->score, p->ab, Sk);
   a.mask = to_args(p->mask);
   a.map = row_view(map);
   if (p->dtype == FLEXATTN_BF16) return p->D == 256 ? fwd_bf16_d256(a, s) : fwd_bf16_d128(a, s);
@@ -361,11 +373,17 @@ int flexattn_tile_shape(int32_t pass, int32_t dtype, int32_t D, int32_t* block_q
 int flexattn_build_block_mask(const flexattn_mask_spec* mask, int32_t Sq, int32_t Sk, int32_t block_q,
                               int32_t block_k, uint8_t* state, int32_t* kv_cnt, int32_t* kv_idx,
                               int32_t* q_cnt, int32_t* q_idx, void* stream) {
+  if (Sq > 0 && Sk > 0 && block_q > 0 && block_k > 0 && (Sq % block_q != 0 || Sk % block_k != 0))
+    return set_error(FLEXATTN_EINVAL, "Sq=%d / Sk=%d not divisible by blocks %d / %d", Sq, Sk, block_q, block_k);
+  return flexattn_build_block_mask_ragged(mask, Sq, Sk, block_q, block_k, state, kv_cnt, kv_idx, q_cnt, q_idx, stream);
+}
+
+int flexattn_build_block_mask_ragged(const flexattn_mask_spec* mask, int32_t Sq, int32_t Sk, int32_t block_q,
+                                     int32_t block_k, uint8_t* state, int32_t* kv_cnt, int32_t* kv_idx,
+                                     int32_t* q_cnt, int32_t* q_idx, void* stream) {
   if (mask == nullptr || state == nullptr) return set_error(FLEXATTN_EINVAL, "mask or state is NULL");
   if (Sq <= 0 || Sk <= 0 || block_q <= 0 || block_k <= 0)
     return set_error(FLEXATTN_EINVAL, "non-positive size (Sq=%d Sk=%d block_q=%d block_k=%d)", Sq, Sk, block_q, block_k);
-  if (Sq % block_q != 0 || Sk % block_k != 0)
-    return set_error(FLEXATTN_EINVAL, "Sq=%d / Sk=%d not divisible by blocks %d / %d", Sq, Sk, block_q, block_k);
   if ((kv_cnt == nullptr) != (kv_idx == nullptr) || (q_cnt == nullptr) != (q_idx == nullptr))
     return set_error(FLEXATTN_EINVAL, "count and index arrays must be given in pairs");
   int rc = check_mask(*mask);
@@ -419,7 +437,8 @@ int flexattn_fwd_noalloc(const flexattn_fwd_params* p, void* stream) {
   // every state, every count and every list entry below its count is rewritten by the builder: nothing of
   // an earlier call is read, nothing needs clearing
   if ((rc = check_doc_batches(p->mask, p->B)) != FLEXATTN_OK) return rc;
-  rc = build_block_mask(to_args(p->mask), p->mask.doc_batches, p->Sq, p->Sk, bq, bk, base + kScratchStateOff,
+  if ((rc = check_pad(p->pad, p->Sq, p->Sk, bq, bk)) != FLEXATTN_OK) return rc;
+  rc = build_block_mask(to_args(p->mask), p->mask.doc_batches, p->Sq - (p->pad & 0xffff), p->Sk - (p->pad >> 16), bq, bk, base + kScratchStateOff,
                         reinterpret_cast<int*>(base + kScratchCntOff), reinterpret_cast<int*>(base + kScratchIdxOff),
                         nullptr, nullptr, s);
   if (rc != FLEXATTN_OK) return rc;
@@ -454,7 +473,8 @@ int flexattn_bwd(const flexattn_bwd_params* pq, const flexattn_bwd_params* pkv, 
   if ((rc = to_bwd_args(pkv, FLEXATTN_PASS_DKV, &akv)) != FLEXATTN_OK) return rc;
   if (pq->ds != nullptr || pkv->ds != nullptr)
     return set_error(FLEXATTN_EINVAL, "flexattn_bwd runs the two passes side by side: no dS hand-over (call flexattn_bwd_dkv, then flexattn_bwd_dq)");
-  if (pq->B != pkv->B || pq->Hq != pkv->Hq || pq->Hkv != pkv->Hkv || pq->Sq != pkv->Sq || pq->Sk != pkv->Sk || pq->D != pkv->D ||
+  if (pq->B != pkv->B || pq->Hq != pkv->Hq || pq->Hkv != pkv->Hkv || pq->Sq - (pq->pad & 0xffff) != pkv->Sq - (pkv->pad & 0xffff) ||
+      pq->Sk - (pq->pad >> 16) != pkv->Sk - (pkv->pad >> 16) || pq->D != pkv->D ||
       pq->dtype != pkv->dtype || pq->q != pkv->q || pq->k != pkv->k || pq->v != pkv->v || pq->dout != pkv->dout)
     return set_error(FLEXATTN_EINVAL, "flexattn_bwd: the two parameter blocks describe different problems");
   hipStream_t s = static_cast<hipStream_t>(stream);

@@ -87,13 +87,13 @@ __global__ __launch_bounds__(256) void fwd_f32_kernel(FwdArgs a) {
   float* sK = reinterpret_cast<float*>(smem_raw);
   float* sV = sK + BK * D;
 
-  const int nQ = a.Sq / BQ, nK = a.map.nk;
+  const int nQ = a.map.nq, nK = a.map.nk;
   const int wg = blockIdx.x;
   const int bh = wg / nQ, qb = nQ - 1 - (wg % nQ);
   const int b = bh / a.Hq, h = bh % a.Hq, hk = h / (a.Hq / a.Hkv);
   const MaskArgs mk = mask_of_batch(a.mask, b, a.Sq, a.Sk);
   const int tid = threadIdx.x, sub = tid & 3, r = tid >> 2;
-  const int q_idx = qb * BQ + r;
+  const int q_idx = tile_base(qb, BQ, a.Sq) + r;   // (rows before qb BQ belong to the q tile before)
 
   const float* Qg = static_cast<const float*>(a.q) + ((size_t)bh * a.Sq + q_idx) * D;
   const float* Kg = static_cast<const float*>(a.k) + (size_t)(b * a.Hkv + hk) * a.Sk * D;
@@ -117,20 +117,21 @@ __global__ __launch_bounds__(256) void fwd_f32_kernel(FwdArgs a) {
     const int kb = tile_idx[t];
     const bool partial = tile_state[kb] == 1;
     __syncthreads();
-    copy_tile<D>(sK, Kg + (size_t)kb * BK * D, BK, tid);
-    copy_tile<D>(sV, Vg + (size_t)kb * BK * D, BK, tid);
+    const int k0 = tile_base(kb, BK, a.Sk);   // (keys before kb BK belong to the kv tile before)
+    copy_tile<D>(sK, Kg + (size_t)k0 * D, BK, tid);
+    copy_tile<D>(sV, Vg + (size_t)k0 * D, BK, tid);
     __syncthreads();
     for (int j0 = 0; j0 < BK; j0 += CH) {
       float tv[CH];
       float m_new = m_run;
 #pragma unroll
       for (int jj = 0; jj < CH; ++jj) {
-        const int j = kb * BK + j0 + jj;
+        const int j = k0 + j0 + jj;
         float s = quad_sum(dot_slice<NV>(qv, sK + (j0 + jj) * D, sub));
         float x = sm.to_log2(s, q_idx, j) + sm.bias2(q_idx, j);
         if (partial) {
           const int doc_j = (mk.flags & FLEXATTN_MASK_DOC) ? mk.doc_k[j] : 0;
-          if (!keep_elem(mk, q_idx, j, doc_i, doc_j)) x = kNegInf;
+          if (!keep_elem(mk, q_idx, j, doc_i, doc_j) || j < kb * BK) x = kNegInf;
         }
         tv[jj] = x;
         m_new = fmaxf(m_new, x);
@@ -153,6 +154,7 @@ __global__ __launch_bounds__(256) void fwd_f32_kernel(FwdArgs a) {
   }
 
   const float inv = (l_run > 0.f) ? 1.0f / l_run : 0.f;
+  if (q_idx < qb * BQ) return;
   float* Og = static_cast<float*>(a.o) + ((size_t)bh * a.Sq + q_idx) * D;
   store_slice<NV>(Og, acc, sub, inv);
   if (a.l != nullptr && sub == 0) {
@@ -172,13 +174,13 @@ __global__ __launch_bounds__(256) void bwd_dq_f32_kernel(BwdArgs a) {
   float* sK = reinterpret_cast<float*>(smem_raw);
   float* sV = sK + BK * D;
 
-  const int nQ = a.Sq / BQ, nK = a.map.nk;
+  const int nQ = a.map.nq, nK = a.map.nk;
   const int wg = blockIdx.x;
   const int bh = wg / nQ, qb = nQ - 1 - (wg % nQ);
   const int b = bh / a.Hq, h = bh % a.Hq, hk = h / (a.Hq / a.Hkv);
   const MaskArgs mk = mask_of_batch(a.mask, b, a.Sq, a.Sk);
   const int tid = threadIdx.x, sub = tid & 3, r = tid >> 2;
-  const int q_idx = qb * BQ + r;
+  const int q_idx = tile_base(qb, BQ, a.Sq) + r;   // (rows before qb BQ belong to the q tile before)
   const size_t row = (size_t)bh * a.Sq + q_idx;
 
   const float* Kg = static_cast<const float*>(a.k) + (size_t)(b * a.Hkv + hk) * a.Sk * D;
@@ -204,26 +206,28 @@ __global__ __launch_bounds__(256) void bwd_dq_f32_kernel(BwdArgs a) {
     const int kb = tile_idx[t];
     const bool partial = tile_state[kb] == 1;
     __syncthreads();
-    copy_tile<D>(sK, Kg + (size_t)kb * BK * D, BK, tid);
-    copy_tile<D>(sV, Vg + (size_t)kb * BK * D, BK, tid);
+    const int k0 = tile_base(kb, BK, a.Sk);   // (keys before kb BK belong to the kv tile before)
+    copy_tile<D>(sK, Kg + (size_t)k0 * D, BK, tid);
+    copy_tile<D>(sV, Vg + (size_t)k0 * D, BK, tid);
     __syncthreads();
     for (int jj = 0; jj < BK; ++jj) {
-      const int j = kb * BK + jj;
+      const int j = k0 + jj;
       const float s = quad_sum(dot_slice<NV>(qv, sK + jj * D, sub));
       const float dp = quad_sum(dot_slice<NV>(dov, sV + jj * D, sub));
       const float tv = sm.to_log2(s, q_idx, j);  // (the score function's value: what its derivative is taken from)
       float x = tv + sm.bias2(q_idx, j);
       if (partial) {
         const int doc_j = (mk.flags & FLEXATTN_MASK_DOC) ? mk.doc_k[j] : 0;
-        if (!keep_elem(mk, q_idx, j, doc_i, doc_j)) x = kNegInf;
+        if (!keep_elem(mk, q_idx, j, doc_i, doc_j) || j < kb * BK) x = kNegInf;
       }
       const float p = exp2f(x - lse2);
       const float gl = (x == kNegInf) ? 0.f : p * (dp - dl);   // gradient with respect to the logit (the bias's share)
-      if (a.dab != nullptr && sub == 0) a.dab[row * (size_t)a.Sk + j] = gl;
+      if (a.dab != nullptr && sub == 0 && j >= kb * BK && q_idx >= qb * BQ) a.dab[row * (size_t)a.Sk + j] = gl;
       const float ds = (x == kNegInf) ? 0.f : gl * sm.dfactor(tv, s, q_idx, j);
       axpy_slice<NV>(acc, ds, sK + jj * D, sub);
     }
   }
+  if (q_idx < qb * BQ) return;
   store_slice<NV>(static_cast<float*>(a.dq) + row * D, acc, sub, 1.0f);
 }
 
@@ -240,14 +244,14 @@ __global__ __launch_bounds__(256) void bwd_dkv_f32_kernel(BwdArgs a) {
   float* sLse = sDO + BQ * D;
   float* sDl = sLse + BQ;
 
-  const int nKb = a.Sk / BK, nQ = a.map.nq;
+  const int nKb = a.map.nk, nQ = a.map.nq;
   const int wg = blockIdx.x;
   const int bhk = wg / nKb, kb = wg % nKb;
   const int b = bhk / a.Hkv, hk = bhk % a.Hkv;
   const MaskArgs mk = mask_of_batch(a.mask, b, a.Sq, a.Sk);
   const int group = a.Hq / a.Hkv;
   const int tid = threadIdx.x, sub = tid & 3, r = tid >> 2;
-  const int k_idx = kb * BK + r;
+  const int k_idx = tile_base(kb, BK, a.Sk) + r;   // (rows before kb BK belong to the kv tile before)
   const size_t krow = (size_t)bhk * a.Sk + k_idx;
 
   f32x4 kv[NV], vv[NV], dk_acc[NV], dv_acc[NV];
@@ -270,12 +274,13 @@ __global__ __launch_bounds__(256) void bwd_dkv_f32_kernel(BwdArgs a) {
     sm.init(a.score, a.sm_scale, h, b);
     for (int t = 0; t < n_tiles; ++t) {
       const int qb = tile_idx[t];
-      const bool partial = a.map.state[(size_t)qb * a.map.nk + kb] == 1;
+      const int q0 = tile_base(qb, BQ, a.Sq);   // (rows before qb BQ belong to the q tile before)
+      const bool partial = a.map.state[(size_t)qb * a.map.nk + kb] == 1 || q0 != qb * BQ;
       __syncthreads();
-      copy_tile<D>(sQ, static_cast<const float*>(a.q) + (qbase + (size_t)qb * BQ) * D, BQ, tid);
-      copy_tile<D>(sDO, static_cast<const float*>(a.dout) + (qbase + (size_t)qb * BQ) * D, BQ, tid);
+      copy_tile<D>(sQ, static_cast<const float*>(a.q) + (qbase + (size_t)q0) * D, BQ, tid);
+      copy_tile<D>(sDO, static_cast<const float*>(a.dout) + (qbase + (size_t)q0) * D, BQ, tid);
       if (tid < BQ) {
-        const size_t rr = qbase + (size_t)qb * BQ + tid;
+        const size_t rr = qbase + (size_t)q0 + tid;
         sLse[tid] = lse2_of(a.l[rr], a.m[rr]);
         sDl[tid] = a.delta[rr];
       }
@@ -290,14 +295,14 @@ __global__ __launch_bounds__(256) void bwd_dkv_f32_kernel(BwdArgs a) {
         dv_t[c] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
       for (int ii = 0; ii < BQ; ++ii) {
-        const int i = qb * BQ + ii;
+        const int i = q0 + ii;
         const float s = quad_sum(dot_slice<NV>(kv, sQ + ii * D, sub));
         const float dp = quad_sum(dot_slice<NV>(vv, sDO + ii * D, sub));
         const float tv = sm.to_log2(s, i, k_idx);
         float x = tv + sm.bias2(i, k_idx);
         if (partial) {
           const int doc_i = (mk.flags & FLEXATTN_MASK_DOC) ? mk.doc_q[i] : 0;
-          if (!keep_elem(mk, i, k_idx, doc_i, doc_j)) x = kNegInf;
+          if (!keep_elem(mk, i, k_idx, doc_i, doc_j) || i < qb * BQ) x = kNegInf;
         }
         const float p = exp2f(x - sLse[ii]);
         const float ds = (x == kNegInf) ? 0.f : p * (dp - sDl[ii]) * sm.dfactor(tv, s, i, k_idx);
@@ -311,6 +316,7 @@ __global__ __launch_bounds__(256) void bwd_dkv_f32_kernel(BwdArgs a) {
       }
     }
   }
+  if (k_idx < kb * BK) return;
   store_slice<NV>(static_cast<float*>(a.dk) + krow * D, dk_acc, sub, 1.0f);
   store_slice<NV>(static_cast<float*>(a.dv) + krow * D, dv_acc, sub, 1.0f);
 }
@@ -344,19 +350,19 @@ static int launch_with_lds(Kern kern, int grid, int lds, const Args& a, hipStrea
 
 template <int DD>
 static int fwd_f32_d(const FwdArgs& a, hipStream_t stream) {
-  const int grid = a.B * a.Hq * (a.Sq / f32_cfg::BQ);
+  const int grid = a.B * a.Hq * a.map.nq;
   const int lds = 2 * f32_cfg::BK * DD * 4;
   FA_F32_DISPATCH(fwd_f32_kernel, grid, lds, a, "flexattn_fwd f32")
 }
 template <int DD>
 static int bwd_dq_f32_d(const BwdArgs& a, hipStream_t stream) {
-  const int grid = a.B * a.Hq * (a.Sq / f32_cfg::BQ);
+  const int grid = a.B * a.Hq * a.map.nq;
   const int lds = 2 * f32_cfg::BK * DD * 4;
   FA_F32_DISPATCH(bwd_dq_f32_kernel, grid, lds, a, "flexattn_bwd_dq f32")
 }
 template <int DD>
 static int bwd_dkv_f32_d(const BwdArgs& a, hipStream_t stream) {
-  const int grid = a.B * a.Hkv * (a.Sk / f32_cfg::BK);
+  const int grid = a.B * a.Hkv * a.map.nk;
   const int lds = 2 * f32_cfg::BQ * DD * 4 + 2 * f32_cfg::BQ * 4;
   FA_F32_DISPATCH(bwd_dkv_f32_kernel, grid, lds, a, "flexattn_bwd_dkv f32")
 }

@@ -74,14 +74,15 @@ __global__ __launch_bounds__(64 * NW) void fwd_f32_mfma_kernel(FwdArgs a) {
   float (*sM)[BO] = reinterpret_cast<float (*)[BO]>(smem_raw + sizeof(float) * NW * BO * (D + 1));
   float (*sL)[BO] = sM + NW;
 
-  const int nO = a.Sq / BO, nK = a.map.nk;
+  const int nO = tiles_of(a.Sq, BO), nK = a.map.nk;
   const int wg = blockIdx.x;
   const int bh = wg / nO, ob = nO - 1 - (wg % nO);
   const int qb = ob / (BT / BO);
   const int b = bh / a.Hq, h = bh % a.Hq, hk = h / (a.Hq / a.Hkv);
   const MaskArgs mk = mask_of_batch(a.mask, b, a.Sq, a.Sk);
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
-  const int q_idx = ob * BO + l32;
+  const int o0 = tile_base(ob, BO, a.Sq);   // (first owner row; rows before ob BO belong to the owner before)
+  const int q_idx = o0 + l32;
 
   const float* Qg = static_cast<const float*>(a.q) + ((size_t)bh * a.Sq + q_idx) * D;
   const float* Kg = static_cast<const float*>(a.k) + (size_t)(b * a.Hkv + hk) * a.Sk * D;
@@ -109,8 +110,9 @@ __global__ __launch_bounds__(64 * NW) void fwd_f32_mfma_kernel(FwdArgs a) {
   for (int u = w; u < 2 * n_tiles; u += NW) {
     const int kb = tile_idx[u >> 1];
     const bool partial = tile_state[kb] == 1;
-    {
-      const int j0 = kb * BT + 32 * (u & 1);
+    const int j_first = kb * BT + 32 * (u & 1);   // (keys before it belong to the unit before)
+    if (j_first < a.Sk) {
+      const int j0 = min(j_first, a.Sk - 32);
       const f32x16 s = dot_block<D>(Kg + (size_t)(j0 + l32) * D, qf, half);
       float x[16];
       float m_blk = kNegInf;
@@ -120,7 +122,7 @@ __global__ __launch_bounds__(64 * NW) void fwd_f32_mfma_kernel(FwdArgs a) {
         float v = sm.to_log2(s[i], q_idx, j) + sm.bias2(q_idx, j);
         if (partial) {
           const int doc_j = has_doc ? mk.doc_k[j] : 0;
-          if (!keep_elem(mk, q_idx, j, doc_i, doc_j)) v = kNegInf;
+          if (!keep_elem(mk, q_idx, j, doc_i, doc_j) || j < j_first) v = kNegInf;
         }
         x[i] = v;
         m_blk = fmaxf(m_blk, v);
@@ -169,7 +171,8 @@ __global__ __launch_bounds__(64 * NW) void fwd_f32_mfma_kernel(FwdArgs a) {
     l_all += sL[ww][r] * f[ww];
   }
   const float inv = (l_all > 0.f) ? 1.0f / l_all : 0.f;
-  float* Og = static_cast<float*>(a.o) + ((size_t)bh * a.Sq + ob * BO + r) * D + c0;
+  if (o0 + r < ob * BO) return;
+  float* Og = static_cast<float*>(a.o) + ((size_t)bh * a.Sq + o0 + r) * D + c0;
 #pragma unroll
   for (int c = 0; c < CPT; ++c) {
     float o = 0.f;
@@ -178,16 +181,16 @@ __global__ __launch_bounds__(64 * NW) void fwd_f32_mfma_kernel(FwdArgs a) {
     Og[c] = o * inv;
   }
   if (a.l != nullptr && (tid % TPR) == 0) {
-    a.l[(size_t)bh * a.Sq + ob * BO + r] = l_all;
-    a.m[(size_t)bh * a.Sq + ob * BO + r] = m_all * kLn2;
+    a.l[(size_t)bh * a.Sq + o0 + r] = l_all;
+    a.m[(size_t)bh * a.Sq + o0 + r] = m_all * kLn2;
   }
 }
 
 // Sum of the waves' accumulators (each [ND][16] in MFMA layout: column = the lane's owner row) through
-// LDS, written out as rows of D floats: 2 NW threads per row, D / (2 NW) consecutive columns each.
+// LDS, written out as rows of D floats from row r_first on: 2 NW threads per row, D / (2 NW) consecutive columns each.
 template <int D, int NW>
 __device__ __forceinline__ void merge_and_store(const f32x16 (&acc)[D / 32], float (*stage)[f32m::BO][D + 1], float* out_rows,
-                                                float mul, int tid) {
+                                                int r_first, float mul, int tid) {
   const int w = tid >> 6, l32 = tid & 31, half = (tid >> 5) & 1;
 #pragma unroll
   for (int db = 0; db < D / 32; ++db)
@@ -196,6 +199,7 @@ __device__ __forceinline__ void merge_and_store(const f32x16 (&acc)[D / 32], flo
   __syncthreads();
   constexpr int TPR = 2 * NW, CPT = D / TPR;
   const int r = tid / TPR, c0 = (tid % TPR) * CPT;
+  if (r < r_first) return;
 #pragma unroll
   for (int c = 0; c < CPT; ++c) {
     float x = 0.f;
@@ -219,14 +223,15 @@ __global__ __launch_bounds__(64 * NW) void bwd_dq_f32_mfma_kernel(BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   float (*sA)[BO][D + 1] = reinterpret_cast<float (*)[BO][D + 1]>(smem_raw);
 
-  const int nO = a.Sq / BO, nK = a.map.nk;
+  const int nO = tiles_of(a.Sq, BO), nK = a.map.nk;
   const int wg = blockIdx.x;
   const int bh = wg / nO, ob = nO - 1 - (wg % nO);
   const int qb = ob / (BT / BO);
   const int b = bh / a.Hq, h = bh % a.Hq, hk = h / (a.Hq / a.Hkv);
   const MaskArgs mk = mask_of_batch(a.mask, b, a.Sq, a.Sk);
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
-  const int q_idx = ob * BO + l32;
+  const int o0 = tile_base(ob, BO, a.Sq);   // (first owner row; rows before ob BO belong to the owner before)
+  const int q_idx = o0 + l32;
   const size_t row = (size_t)bh * a.Sq + q_idx;
 
   const float* Kg = static_cast<const float*>(a.k) + (size_t)(b * a.Hkv + hk) * a.Sk * D;
@@ -254,8 +259,9 @@ __global__ __launch_bounds__(64 * NW) void bwd_dq_f32_mfma_kernel(BwdArgs a) {
   for (int u = w; u < 2 * n_tiles; u += NW) {
     const int kb = tile_idx[u >> 1];
     const bool partial = tile_state[kb] == 1;
-    {
-      const int j0 = kb * BT + 32 * (u & 1);
+    const int j_first = kb * BT + 32 * (u & 1);   // (keys before it belong to the unit before)
+    if (j_first < a.Sk) {
+      const int j0 = min(j_first, a.Sk - 32);
       const f32x16 s = dot_block<D>(Kg + (size_t)(j0 + l32) * D, qf, half);
       const f32x16 dp = dot_block<D>(Vg + (size_t)(j0 + l32) * D, dof, half);
       float ds[16];
@@ -266,17 +272,17 @@ __global__ __launch_bounds__(64 * NW) void bwd_dq_f32_mfma_kernel(BwdArgs a) {
         float x = tv + sm.bias2(q_idx, j);
         if (partial) {
           const int doc_j = has_doc ? mk.doc_k[j] : 0;
-          if (!keep_elem(mk, q_idx, j, doc_i, doc_j)) x = kNegInf;
+          if (!keep_elem(mk, q_idx, j, doc_i, doc_j) || j < j_first) x = kNegInf;
         }
         const float pe = exp2f(x - lse2);
         const float gl = (x == kNegInf) ? 0.f : pe * (dp[i] - dl);   // gradient with respect to the logit (the bias's share)
-        if (a.dab != nullptr) a.dab[row * (size_t)a.Sk + j] = gl;
+        if (a.dab != nullptr && j >= j_first && q_idx >= ob * BO) a.dab[row * (size_t)a.Sk + j] = gl;
         ds[i] = (x == kNegInf) ? 0.f : gl * sm.dfactor(tv, s[i], q_idx, j);
       }
       accumulate_rows<D>(acc, Kg + (size_t)j0 * D, ds, l32, half);
     }
   }
-  merge_and_store<D, NW>(acc, sA, static_cast<float*>(a.dq) + ((size_t)bh * a.Sq + ob * BO) * D, 1.0f, tid);
+  merge_and_store<D, NW>(acc, sA, static_cast<float*>(a.dq) + ((size_t)bh * a.Sq + o0) * D, ob * BO - o0, 1.0f, tid);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -290,14 +296,15 @@ __global__ __launch_bounds__(64 * NW) void bwd_dkv_f32_mfma_kernel(BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   float (*sA)[BO][D + 1] = reinterpret_cast<float (*)[BO][D + 1]>(smem_raw);   // (dk, then dv)
 
-  const int nO = a.Sk / BO, nQ = a.map.nq;
+  const int nO = tiles_of(a.Sk, BO), nQ = a.map.nq;
   const int wg = blockIdx.x;
   const int bhk = wg / nO, ob = wg % nO;
   const int kb = ob / (BT / BO);
   const int b = bhk / a.Hkv, hk = bhk % a.Hkv, group = a.Hq / a.Hkv;
   const MaskArgs mk = mask_of_batch(a.mask, b, a.Sq, a.Sk);
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
-  const int k_idx = ob * BO + l32;
+  const int o0 = tile_base(ob, BO, a.Sk);   // (first owner row; rows before ob BO belong to the owner before)
+  const int k_idx = o0 + l32;
   const size_t krow = (size_t)bhk * a.Sk + k_idx;
 
   const bool has_doc = (mk.flags & FLEXATTN_MASK_DOC) != 0;
@@ -323,9 +330,10 @@ __global__ __launch_bounds__(64 * NW) void bwd_dkv_f32_mfma_kernel(BwdArgs a) {
     const float* dOg = static_cast<const float*>(a.dout) + head_row * D;
     ScoreMod<SCORE> sm;
     sm.init(a.score, a.sm_scale, h, b);
-    const bool partial = state[(size_t)qb * a.map.nk + kb] == 1;
-    {
-      const int i0 = qb * BT + 32 * (u & 1);
+    const int i_first = qb * BT + 32 * (u & 1);   // (rows before it belong to the unit before)
+    const bool partial = state[(size_t)qb * a.map.nk + kb] == 1 || i_first + 32 > a.Sq;
+    if (i_first < a.Sq) {
+      const int i0 = min(i_first, a.Sq - 32);
       const f32x16 s = dot_block<D>(Qg + (size_t)(i0 + l32) * D, kf, half);
       const f32x16 dp = dot_block<D>(dOg + (size_t)(i0 + l32) * D, vf, half);
       float pv[16], ds[16];
@@ -336,7 +344,7 @@ __global__ __launch_bounds__(64 * NW) void bwd_dkv_f32_mfma_kernel(BwdArgs a) {
         float x = tv + sm.bias2(i, k_idx);
         if (partial) {
           const int doc_i = has_doc ? mk.doc_q[i] : 0;
-          if (!keep_elem(mk, i, k_idx, doc_i, doc_j)) x = kNegInf;
+          if (!keep_elem(mk, i, k_idx, doc_i, doc_j) || i < i_first) x = kNegInf;
         }
         const float pe = exp2f(x - lse2_from(a.l[head_row + i], a.m[head_row + i]));
         pv[e] = pe;
@@ -346,9 +354,9 @@ __global__ __launch_bounds__(64 * NW) void bwd_dkv_f32_mfma_kernel(BwdArgs a) {
       accumulate_rows<D>(dk_acc, Qg + (size_t)i0 * D, ds, l32, half);
     }
   }
-  merge_and_store<D, NW>(dk_acc, sA, static_cast<float*>(a.dk) + ((size_t)bhk * a.Sk + ob * BO) * D, 1.0f, tid);
+  merge_and_store<D, NW>(dk_acc, sA, static_cast<float*>(a.dk) + ((size_t)bhk * a.Sk + o0) * D, ob * BO - o0, 1.0f, tid);
   __syncthreads();  // (the stage is read by other threads than wrote it: all of dk is out before dv goes in)
-  merge_and_store<D, NW>(dv_acc, sA, static_cast<float*>(a.dv) + ((size_t)bhk * a.Sk + ob * BO) * D, 1.0f, tid);
+  merge_and_store<D, NW>(dv_acc, sA, static_cast<float*>(a.dv) + ((size_t)bhk * a.Sk + o0) * D, ob * BO - o0, 1.0f, tid);
 }
 
 template <typename Kern, typename Args>
@@ -375,33 +383,33 @@ static bool wide_groups(int D, int grid) { return D == 64 && grid <= 512; }
 
 template <int DD, int NWW>
 static int fwd_f32_mfma_d(const FwdArgs& a, hipStream_t stream) {
-  const int grid = a.B * a.Hq * (a.Sq / f32m::BO);
+  const int grid = a.B * a.Hq * tiles_of(a.Sq, f32m::BO);
   const int lds = 4 * (NWW * f32m::BO * (DD + 1) + 2 * NWW * f32m::BO);
   FA_F32M_DISPATCH(fwd_f32_mfma_kernel, grid, lds, a, "flexattn_fwd f32")
 }
 
 template <int DD, int NWW>
 static int bwd_dq_f32_mfma_d(const BwdArgs& a, hipStream_t stream) {
-  const int grid = a.B * a.Hq * (a.Sq / f32m::BO);
+  const int grid = a.B * a.Hq * tiles_of(a.Sq, f32m::BO);
   const int lds = 4 * NWW * f32m::BO * (DD + 1);
   FA_F32M_DISPATCH(bwd_dq_f32_mfma_kernel, grid, lds, a, "flexattn_bwd_dq f32")
 }
 template <int DD, int NWW>
 static int bwd_dkv_f32_mfma_d(const BwdArgs& a, hipStream_t stream) {
-  const int grid = a.B * a.Hkv * (a.Sk / f32m::BO);
+  const int grid = a.B * a.Hkv * tiles_of(a.Sk, f32m::BO);
   const int lds = 4 * NWW * f32m::BO * (DD + 1);
   FA_F32M_DISPATCH(bwd_dkv_f32_mfma_kernel, grid, lds, a, "flexattn_bwd_dkv f32")
 }
 
 int bwd_dq_f32_mfma(const BwdArgs& a, int D, hipStream_t stream) {
   if (D == 64)
-    return wide_groups(D, a.B * a.Hq * (a.Sq / f32m::BO)) ? bwd_dq_f32_mfma_d<64, 8>(a, stream) : bwd_dq_f32_mfma_d<64, 4>(a, stream);
+    return wide_groups(D, a.B * a.Hq * tiles_of(a.Sq, f32m::BO)) ? bwd_dq_f32_mfma_d<64, 8>(a, stream) : bwd_dq_f32_mfma_d<64, 4>(a, stream);
   if (D == 128) return bwd_dq_f32_mfma_d<128, 4>(a, stream);
   return set_error(FLEXATTN_ENOTSUP, "fp32 dq: head dim %d not in {64, 128}", D);
 }
 int bwd_dkv_f32_mfma(const BwdArgs& a, int D, hipStream_t stream) {
   if (D == 64)
-    return wide_groups(D, a.B * a.Hkv * (a.Sk / f32m::BO)) ? bwd_dkv_f32_mfma_d<64, 8>(a, stream)
+    return wide_groups(D, a.B * a.Hkv * tiles_of(a.Sk, f32m::BO)) ? bwd_dkv_f32_mfma_d<64, 8>(a, stream)
                                                           : bwd_dkv_f32_mfma_d<64, 4>(a, stream);
   if (D == 128) return bwd_dkv_f32_mfma_d<128, 4>(a, stream);
   return set_error(FLEXATTN_ENOTSUP, "fp32 dk/dv: head dim %d not in {64, 128}", D);
@@ -409,7 +417,7 @@ int bwd_dkv_f32_mfma(const BwdArgs& a, int D, hipStream_t stream) {
 
 int fwd_f32_mfma(const FwdArgs& a, int D, hipStream_t stream) {
   if (D == 64)
-    return wide_groups(D, a.B * a.Hq * (a.Sq / f32m::BO)) ? fwd_f32_mfma_d<64, 8>(a, stream) : fwd_f32_mfma_d<64, 4>(a, stream);
+    return wide_groups(D, a.B * a.Hq * tiles_of(a.Sq, f32m::BO)) ? fwd_f32_mfma_d<64, 8>(a, stream) : fwd_f32_mfma_d<64, 4>(a, stream);
   if (D == 128) return fwd_f32_mfma_d<128, 4>(a, stream);
   return set_error(FLEXATTN_ENOTSUP, "fp32 forward: head dim %d not in {64, 128}", D);
 }

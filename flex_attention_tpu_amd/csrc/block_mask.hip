@@ -11,9 +11,12 @@ namespace fa {
 // With a compiled mask predicate (FLEXATTN_MASK_CUSTOM) there is no closed form: the element predicate is
 // evaluated on every element of the tile, run = any kept, full = all kept, which is what the Python block
 // closure of a compiled mask returns (any(mask_fn over the tile)).
-__device__ __forceinline__ int tile_state(const MaskArgs& mk, int qb, int kb, int bq, int bk, bool sorted_ids) {
-  const int q_start = qb * bq, q_end = q_start + bq - 1;
-  const int k_start = kb * bk, k_end = k_start + bk - 1;
+// Sq, Sk: the sequence lengths; a last tile that runs past one of them ends there, and is at most partial when it
+// runs past Sk (the kernels start it early, tile_base, and mask the keys it then shares with the tile before).
+__device__ __forceinline__ int tile_state(const MaskArgs& mk, int qb, int kb, int bq, int bk, int Sq, int Sk, bool sorted_ids) {
+  const int q_start = qb * bq, q_end = min(q_start + bq, Sq) - 1;
+  const int k_start = kb * bk, k_end = min(k_start + bk, Sk) - 1;
+  const bool whole = k_end == k_start + bk - 1;
 #if FLEXATTN_CUSTOM_HAS_MASK
   if (mk.flags & FLEXATTN_MASK_CUSTOM) {
     const bool has_doc = (mk.flags & FLEXATTN_MASK_DOC) != 0;
@@ -26,7 +29,7 @@ __device__ __forceinline__ int tile_state(const MaskArgs& mk, int qb, int kb, in
         all = all & keep;
       }
     }
-    return any ? (all ? 2 : 1) : 0;
+    return any ? (all && whole ? 2 : 1) : 0;
   }
 #endif
   bool run = true, full = true;
@@ -65,7 +68,7 @@ __device__ __forceinline__ int tile_state(const MaskArgs& mk, int qb, int kb, in
     run = run && (lo <= hi);
     full = full && (qmin == qmax) && (kmin == kmax) && (qmin == kmin);
   }
-  return run ? (full ? 2 : 1) : 0;
+  return run ? (full && whole ? 2 : 1) : 0;
 }
 
 // Work-groups [0, nq) own one q-block row each: write its states and its ascending kv list.
@@ -73,7 +76,7 @@ __device__ __forceinline__ int tile_state(const MaskArgs& mk, int qb, int kb, in
 // `batches`: number of batch entries the document arrays hold a row for (1: one row for all).  The map is then the
 // union over the entries: a tile runs if it runs for any entry and is full only if it is full for every entry (an
 // entry that keeps nothing of a tile it visits masks every element of it).
-__global__ __launch_bounds__(64) void block_mask_kernel(MaskArgs mk, int batches, int nq, int nk, int bq, int bk,
+__global__ __launch_bounds__(64) void block_mask_kernel(MaskArgs mk, int batches, int Sq, int Sk, int nq, int nk, int bq, int bk,
                                                         uint8_t* state, int* kv_cnt, int* kv_idx,
                                                         int* q_cnt, int* q_idx) {
   const int lane = threadIdx.x;
@@ -83,16 +86,16 @@ __global__ __launch_bounds__(64) void block_mask_kernel(MaskArgs mk, int batches
   if (mk.flags & FLEXATTN_MASK_DOC) {
     bool ok = true;
     for (int e = 0; e < batches; ++e) {
-      const MaskArgs me = mask_of_batch(mk, e, nq * bq, nk * bk);
-      for (int i = lane + 1; i < nq * bq; i += 64) ok = ok && (me.doc_q[i - 1] <= me.doc_q[i]);
-      for (int j = lane + 1; j < nk * bk; j += 64) ok = ok && (me.doc_k[j - 1] <= me.doc_k[j]);
+      const MaskArgs me = mask_of_batch(mk, e, Sq, Sk);
+      for (int i = lane + 1; i < Sq; i += 64) ok = ok && (me.doc_q[i - 1] <= me.doc_q[i]);
+      for (int j = lane + 1; j < Sk; j += 64) ok = ok && (me.doc_k[j - 1] <= me.doc_k[j]);
     }
     sorted_ids = __ballot(!ok) == 0ull;
   }
   auto tile_state_all = [&](int qb, int kb) {
-    int st = tile_state(mk, qb, kb, bq, bk, sorted_ids);
+    int st = tile_state(mk, qb, kb, bq, bk, Sq, Sk, sorted_ids);
     for (int e = 1; e < batches; ++e) {
-      const int se = tile_state(mask_of_batch(mk, e, nq * bq, nk * bk), qb, kb, bq, bk, sorted_ids);
+      const int se = tile_state(mask_of_batch(mk, e, Sq, Sk), qb, kb, bq, bk, Sq, Sk, sorted_ids);
       st = (st == 0 && se == 0) ? 0 : ((st == 2 && se == 2) ? 2 : 1);
     }
     return st;
@@ -154,10 +157,10 @@ int build_ds_index(const uint8_t* state, const int* q_cnt, const int* q_idx, int
 
 int build_block_mask(const MaskArgs& mask, int doc_batches, int Sq, int Sk, int block_q, int block_k, uint8_t* state,
                      int* kv_cnt, int* kv_idx, int* q_cnt, int* q_idx, hipStream_t stream) {
-  const int nq = Sq / block_q, nk = Sk / block_k;
+  const int nq = tiles_of(Sq, block_q), nk = tiles_of(Sk, block_k);
   const bool want_cols = q_cnt != nullptr;
   const int grid = nq + (want_cols ? nk : 0);
-  hipLaunchKernelGGL(block_mask_kernel, dim3(grid), dim3(64), 0, stream, mask, doc_batches > 1 ? doc_batches : 1, nq, nk, block_q, block_k,
+  hipLaunchKernelGGL(block_mask_kernel, dim3(grid), dim3(64), 0, stream, mask, doc_batches > 1 ? doc_batches : 1, Sq, Sk, nq, nk, block_q, block_k,
                      state, kv_cnt, kv_idx, q_cnt, q_idx);
   return check_launch("flexattn_build_block_mask");
 }

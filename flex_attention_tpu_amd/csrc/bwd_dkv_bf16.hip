@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
   float* sLse = reinterpret_cast<float*>(sDO + 4 * kTileElems);
   float* sDl = sLse + 2 * BQ;
 
-  const int nKb = a.Sk / BNK;
+  const int nKb = a.map.nk;
   const int nQ = a.map.nq;
   const int n_wg = a.B * a.Hkv * nKb;
   const int wg = xcd_remap(blockIdx.x, n_wg);
@@ -102,8 +102,10 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
   const int hh = lane >> 5;
 
   const int kv_local = w * 32 + l32;
-  const int k_idx = kb * BNK + kv_local;
-  const size_t kv_off = ((size_t)bhk * a.Sk + (size_t)kb * BNK) * D;
+  const int k0 = tile_base(kb, BNK, a.Sk);
+  const int k_idx = k0 + kv_local;
+  const bool own_col = k_idx >= kb * BNK;   // (else a row of the kv tile before)
+  const size_t kv_off = ((size_t)bhk * a.Sk + (size_t)k0) * D;
   const bf16_t* Kg = static_cast<const bf16_t*>(a.k) + kv_off;
   const bf16_t* Vg = static_cast<const bf16_t*>(a.v) + kv_off;
   const bf16_t* Qall = static_cast<const bf16_t*>(a.q);
@@ -129,6 +131,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
 
   const int n_tiles = a.map.cnt[kb];
   const int* tile_idx = a.map.idx + (size_t)kb * nQ;
+  const bool ragged_q = nQ * BQ != a.Sq;   // (the last q tile then shares rows with the one before)
   const int n_iter = n_tiles * group;
 
   // Iteration `it` covers q tile tile_idx[it % n_tiles] of query head hk*group + it / n_tiles.
@@ -144,7 +147,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
   float lse_st = 0.f, dl_st = 0.f;
   auto issue_tile = [&](int it, int qb, int buf) {
     const int g = it / n_tiles;
-    const size_t rbase = ((size_t)(b * a.Hq + hk * group + g) * a.Sq + (size_t)qb * BQ);
+    const size_t rbase = ((size_t)(b * a.Hq + hk * group + g) * a.Sq + (size_t)tile_base(qb, BQ, a.Sq));
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       loader.load(Qall + (rbase + half * kTileRows) * D, sQ + (2 * buf + half) * kTileElems);
@@ -187,7 +190,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
   for (int it = 0; it < n_iter; ++it) {
     const int buf = it & 1;
     const int qb = __builtin_amdgcn_readfirstlane(qb_cur);
-    const bool partial = __builtin_amdgcn_readfirstlane(st_cur) == 1;
+    const bool partial = __builtin_amdgcn_readfirstlane(st_cur) == 1 || (qb == nQ - 1 && ragged_q);
     sm.init(a.score, a.sm_scale, hk * group + it / n_tiles, b);
     const int qb_n2 = (it + 2 < n_iter) ? q_block_of(it + 2) : 0;
     int st_nxt = 0;
@@ -196,7 +199,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
       st_nxt = a.map.state[(size_t)qbn * a.map.nk + kb];
       issue_tile(it + 1, qbn, buf ^ 1);
     }
-    const int q0 = qb * BQ;
+    const int q0 = tile_base(qb, BQ, a.Sq);
+    const int q_first = qb * BQ;   // (rows before it belong to the q tile before)
 #pragma unroll
     for (int cc = 0; cc < 4; ++cc) {
       const int c = cc & 1;  // 32-row block inside the 64-row LDS tile cc >> 1
@@ -246,7 +250,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
           const f32x4 dl4 = *reinterpret_cast<const f32x4*>(sDl + buf * BQ + r0);
           int di[4] = {0, 0, 0, 0};
           if (MASKED && has_doc) {
-            const auto d4 = *reinterpret_cast<const int __attribute__((ext_vector_type(4)))*>(mk.doc_q + q0 + r0);
+            const auto d4 = *reinterpret_cast<const i32x4_a4*>(mk.doc_q + q0 + r0);
             di[0] = d4[0]; di[1] = d4[1]; di[2] = d4[2]; di[3] = d4[3];
           }
           float pv[4], dsv[4];
@@ -258,7 +262,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
             float pe = fast_exp2(tv + sm.bias2(i, k_idx) - lse4[u]);
             float gd = pe * (dp_acc[e] - dl4[u]) * sm.dfactor(tv, s_acc[e], i, k_idx);
             if (MASKED) {
-              const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j);
+              const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j) & (i >= q_first) & own_col;
               pe = keep ? pe : 0.f;
               gd = keep ? gd : 0.f;
             }
@@ -304,6 +308,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
     __syncthreads();
   }
 
+  if (!own_col) return;
   bf16_t* dKg = static_cast<bf16_t*>(a.dk) + kv_off;
   bf16_t* dVg = static_cast<bf16_t*>(a.dv) + kv_off;
 #pragma unroll
@@ -338,7 +343,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
   float* sLse = reinterpret_cast<float*>(sDO + 2 * NP * kTileElems);
   float* sDl = sLse + 2 * HQ;
 
-  const int nKb = a.Sk / BNK;
+  const int nKb = a.map.nk;
   const int nQ = a.map.nq;
   const int n_wg = a.B * a.Hkv * nKb;
   const int wg = xcd_remap(blockIdx.x, n_wg);
@@ -356,8 +361,10 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
   const int hh = lane >> 5;
 
   const int kv_local = w * 32 + l32;
-  const int k_idx = kb * BNK + kv_local;
-  const size_t kv_off = ((size_t)bhk * a.Sk + (size_t)kb * BNK) * D;
+  const int k0 = tile_base(kb, BNK, a.Sk);
+  const int k_idx = k0 + kv_local;
+  const bool own_col = k_idx >= kb * BNK;   // (else a row of the kv tile before)
+  const size_t kv_off = ((size_t)bhk * a.Sk + (size_t)k0) * D;
   const bf16_t* Kg = static_cast<const bf16_t*>(a.k) + kv_off;
   const bf16_t* Vg = static_cast<const bf16_t*>(a.v) + kv_off;
   const bf16_t* Qall = static_cast<const bf16_t*>(a.q);
@@ -383,6 +390,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
 
   const int n_tiles = a.map.cnt[kb];
   const int* tile_idx = a.map.idx + (size_t)kb * nQ;
+  const bool ragged_q = nQ * BQ != a.Sq;   // (the last q tile then shares rows with the one before)
   const int n_iter = 2 * n_tiles * group;
 
   // Iteration `it` covers rows 64 (it & 1) .. of q tile tile_idx[(it / 2) % n_tiles] of query head
@@ -398,7 +406,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
   float lse_st = 0.f, dl_st = 0.f;
   auto issue_tile = [&](int it, int qb, int buf) {
     const int g = (it >> 1) / n_tiles;
-    const size_t rbase = ((size_t)(b * a.Hq + hk * group + g) * a.Sq + (size_t)qb * BQ + (size_t)(it & 1) * HQ);
+    const size_t rbase = ((size_t)(b * a.Hq + hk * group + g) * a.Sq + (size_t)tile_base(qb, BQ, a.Sq) + (size_t)(it & 1) * HQ);
 #pragma unroll
     for (int pn = 0; pn < NP; ++pn) {
       loader.load(Qall + rbase * D + 128 * pn, sQ + (buf * NP + pn) * kTileElems);
@@ -441,7 +449,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
   for (int it = 0; it < n_iter; ++it) {
     const int buf = it & 1;
     const int qb = __builtin_amdgcn_readfirstlane(qb_cur);
-    const bool partial = __builtin_amdgcn_readfirstlane(st_cur) == 1;
+    const bool partial = __builtin_amdgcn_readfirstlane(st_cur) == 1 || (qb == nQ - 1 && ragged_q);
     sm.init(a.score, a.sm_scale, hk * group + (it >> 1) / n_tiles, b);
     const int qb_n2 = (it + 2 < n_iter) ? q_block_of(it + 2) : 0;
     int st_nxt = 0;
@@ -450,7 +458,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
       st_nxt = a.map.state[(size_t)qbn * a.map.nk + kb];
       issue_tile(it + 1, qbn, buf ^ 1);
     }
-    const int q0 = qb * BQ + (it & 1) * HQ;
+    const int q0 = tile_base(qb, BQ, a.Sq) + (it & 1) * HQ;
+    const int q_first = qb * BQ;   // (rows before it belong to the q tile before)
     const char* qt = reinterpret_cast<const char*>(sQ + buf * NP * kTileElems);
     const char* dot = reinterpret_cast<const char*>(sDO + buf * NP * kTileElems);
 #pragma unroll 1   // (rolled: unrolled, the second block's operand loads are hoisted over the first block's and 72 registers spill; 2.72 -> 2.01 ms on B=4, H=16, S=4096)
@@ -489,7 +498,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
           const f32x4 dl4 = *reinterpret_cast<const f32x4*>(sDl + buf * HQ + r0);
           int di[4] = {0, 0, 0, 0};
           if (MASKED && has_doc) {
-            const auto d4 = *reinterpret_cast<const int __attribute__((ext_vector_type(4)))*>(mk.doc_q + q0 + r0);
+            const auto d4 = *reinterpret_cast<const i32x4_a4*>(mk.doc_q + q0 + r0);
             di[0] = d4[0]; di[1] = d4[1]; di[2] = d4[2]; di[3] = d4[3];
           }
           float pv[4], dsv[4];
@@ -501,7 +510,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
             float pe = fast_exp2(tv + sm.bias2(i, k_idx) - lse4[u]);
             float gd = pe * (dp_acc[e] - dl4[u]) * sm.dfactor(tv, s_acc[e], i, k_idx);
             if (MASKED) {
-              const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j);
+              const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j) & (i >= q_first) & own_col;
               pe = keep ? pe : 0.f;
               gd = keep ? gd : 0.f;
             }
@@ -552,6 +561,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
     __syncthreads();
   }
 
+  if (!own_col) return;
   bf16_t* dKg = static_cast<bf16_t*>(a.dk) + kv_off;
   bf16_t* dVg = static_cast<bf16_t*>(a.dv) + kv_off;
 #pragma unroll
@@ -578,7 +588,7 @@ static int launch_dkv_wide(const BwdArgs& a, hipStream_t stream) {
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dkv): %s", hipGetErrorString(attr));
-  const int n_wg = a.B * a.Hkv * (a.Sk / BNK);
+  const int n_wg = a.B * a.Hkv * a.map.nk;
   hipLaunchKernelGGL(kern, dim3(n_wg), dim3(256), kLds, stream, a);
   return check_launch("flexattn_bwd_dkv bf16");
 }
@@ -617,7 +627,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
   float* sLse = reinterpret_cast<float*>(sT + 8 * kTileElems);
   float* sDl = sLse + 2 * BQ;
 
-  const int nKb = a.Sk / BNK;
+  const int nKb = a.map.nk;
   const int nQ = a.map.nq;
   const int n_wg = a.B * a.Hkv * nKb;
   const int group = a.Hq / a.Hkv;
@@ -665,7 +675,9 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
     g.kb = __builtin_amdgcn_readfirstlane(g.kb);
     return g;
   };
-  auto kv_offset = [&](const Geometry& g) { return ((size_t)g.bhk * a.Sk + (size_t)g.kb * BNK) * D; };
+  auto kv_base = [&](const Geometry& g) { return tile_base(g.kb, BNK, a.Sk); };
+  auto kv_offset = [&](const Geometry& g) { return ((size_t)g.bhk * a.Sk + (size_t)kv_base(g)) * D; };
+  const bool ragged_q = nQ * BQ != a.Sq;   // (the last q tile then shares rows with the one before: always masked)
   // (DOCS) document arrays given per batch entry: the rows of the entry of a (batch, kv head) pair
   auto doc_rows = [&](int bhk, int S) { return (DOCS && a.mask.doc_batched) ? (size_t)(bhk / a.Hkv) * (size_t)S : (size_t)0; };
   // (EXPORT) dS block of the item's kv tile against the first q tile of its list, for the group's first query
@@ -703,11 +715,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
     rows_load(r.k, Kg + (size_t)(tid_here >> 6) * 32 * D, tid_here & 63);
     rows_load(r.v, Vg + (size_t)(tid_here >> 6) * 32 * D, tid_here & 63);
     const size_t dk_rows = doc_rows(g.bhk, a.Sk);
-    r.doc = (a.mask.flags & FLEXATTN_MASK_DOC) ? a.mask.doc_k[dk_rows + g.kb * BNK + kv_local] : 0;
+    r.doc = (a.mask.flags & FLEXATTN_MASK_DOC) ? a.mask.doc_k[dk_rows + kv_base(g) + kv_local] : 0;
     if constexpr (DOCS) {
       const bool have = a.mask.doc_k_range != nullptr;
-      r.qlo = have ? a.mask.doc_k_range[2 * (dk_rows + g.kb * BNK + kv_local)] : 0;
-      r.qhi = have ? a.mask.doc_k_range[2 * (dk_rows + g.kb * BNK + kv_local) + 1] : 0;
+      r.qlo = have ? a.mask.doc_k_range[2 * (dk_rows + kv_base(g) + kv_local)] : 0;
+      r.qhi = have ? a.mask.doc_k_range[2 * (dk_rows + kv_base(g) + kv_local) + 1] : 0;
     }
     const int* tile_idx = a.map.idx + (size_t)g.kb * nQ;
     r.n_tiles = a.map.cnt[g.kb];
@@ -786,7 +798,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
 
   for (int item = 0; item < n_items; ++item) {
   const int kb = geo.kb;
-  const int k_idx = kb * BNK + kv_local;
+  const int k0 = kv_base(geo);
+  const int k_idx = k0 + kv_local;
   const size_t kv_off = kv_offset(geo);
   const size_t rows0 = first_row(geo);
   const bf16_t* Qg = static_cast<const bf16_t*>(a.q) + rows0 * D;
@@ -801,7 +814,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
   const int n_tiles = cur.n_tiles;
   const int n_iter = n_tiles * group;
   const float na2 = cur.na2;
-  const int kc = kb * BNK + BNK / 2;  // j0
+  const int kc = k0 + BNK / 2;  // j0
   if (item > 0) __syncthreads();  // the previous item's list and row values are dead from here
 
   asm volatile(FA_DKV_ZERO_ACC
@@ -816,7 +829,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
     const int t = tid_p + 256 * j;
     if (t < nQ) {
       sIdx[t] = cur.idx[j];
-      sPart[t] = cur.part[j] == 1 ? 1 : 0;
+      sPart[t] = (cur.part[j] == 1 || (ragged_q && t == nQ - 1)) ? 1 : 0;
     }
   }
   if (nQ > PREFETCH_LIST) {
@@ -824,12 +837,12 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
     // (an item is then thousands of steps long: the wait does not show)
     for (int t = PREFETCH_LIST + tid_p; t < nQ; t += 256) {
       sIdx[t] = tile_idx[t];
-      sPart[t] = a.map.state[(size_t)t * a.map.nk + kb] == 1 ? 1 : 0;
+      sPart[t] = (a.map.state[(size_t)t * a.map.nk + kb] == 1 || (ragged_q && t == nQ - 1)) ? 1 : 0;
     }
   }
   if (n_iter > 0 && !resident) {
     // first step into the current buffer: tiles (LDS-direct) and the lane's row value
-    const size_t r0 = (size_t)cur.qb0 * BQ;
+    const size_t r0 = (size_t)tile_base(cur.qb0, BQ, a.Sq);
     bf16_t* dst = sT + (size_t)buf * 4 * kTileElems;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
@@ -911,7 +924,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
     unsigned km[2] = {0u, 0u};
     if (partial) {
       // the lane's keep bits: element e of q block c sits at bit 16 (c & 1) + e of km[c >> 1]
-      const int q0 = qb * BQ;
+      const int q0 = tile_base(qb, BQ, a.Sq);
       if constexpr (DOCS) {
         int* sDoc = reinterpret_cast<int*>(sPart + MAX_LIST) + w * 128;  // the wave's stage for document ids
         if (ranged) {
@@ -929,6 +942,10 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
         for (int half = 0; half < 2; ++half)
           km[half] = keep_bits32<false>(a.mask, k_idx, q0 + 64 * half + 4 * hh, doc_j, a.mask.doc_q);
       }
+      // (rows and columns that the last tiles of ragged lengths share with the tiles before them: those own them)
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+        km[half] = k_idx < kb * BNK ? 0u : km[half] & keep_bits_from(qb * BQ - q0 - 64 * half - 4 * hh);
     } else {
       // the run of full tiles ends before the next partial one: lanes look 64 steps ahead at a time
       bool found = false;
@@ -975,7 +992,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
           tbl[24] = (unsigned)qb0_n;
           if (ALIBI) {
             tbl[26] = __builtin_bit_cast(unsigned, pre.na2);
-            tbl[27] = (unsigned)(geo_n.kb * BNK + BNK / 2);
+            tbl[27] = (unsigned)(kv_base(geo_n) + BNK / 2);
           }
           if (EXPORT) {
             const size_t ds_n = ds_item_n;
@@ -1071,9 +1088,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
     bf16_t* dKg = static_cast<bf16_t*>(a.dk) + kv_off + (size_t)(w * 32) * D;
     bf16_t* dVg = static_cast<bf16_t*>(a.dv) + kv_off + (size_t)(w * 32) * D;
     const int chunk = lane_here & 15;
+    const int r_first = kb * BNK - k0 - w * 32;   // (rows before it belong to the kv tile before)
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int r = 4 * i + (lane_here >> 4);
+      if (r < r_first) continue;
       const unsigned rd = (unsigned)r * 256u + (unsigned)((chunk ^ (r & 15)) << 4);
       const u32x4 kx = *reinterpret_cast<const u32x4*>(stage + rd);
       const u32x4 vx = *reinterpret_cast<const u32x4*>(stage + 8192 + rd);
@@ -1094,7 +1113,7 @@ static int launch_dkv_on(const BwdArgs& a, hipStream_t stream) {
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dkv): %s", hipGetErrorString(attr));
-  const int n_wg = a.B * a.Hkv * (a.Sk / BNK);
+  const int n_wg = a.B * a.Hkv * a.map.nk;
   hipLaunchKernelGGL(kern, dim3(n_wg), dim3(256), LDS_BYTES, stream, a);
   return check_launch("flexattn_bwd_dkv bf16");
 }
@@ -1111,10 +1130,10 @@ static int launch_dkv_plain_on(const BwdArgs& a, hipStream_t stream) {
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dkv): %s", hipGetErrorString(attr));
-  const int n_wg = a.B * a.Hkv * (a.Sk / BNK);
+  const int n_wg = a.B * a.Hkv * a.map.nk;
   // (persistent_ok's schedule balances masks whose work per tile is linear in the tile index; document
   // masks take the longest-first schedule of sorted_items; what fits neither runs one item per work-group)
-  const bool persistent = DOCS ? sorted_schedule_ok(n_wg, a.Sk / BNK) : persistent_ok(n_wg, a.Sk / BNK);
+  const bool persistent = DOCS ? sorted_schedule_ok(n_wg, a.map.nk) : persistent_ok(n_wg, a.map.nk);
   const int grid = (persistent && n_wg > 256) ? 256 : n_wg;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(256), LDS_BYTES, stream, a);
   return check_launch("flexattn_bwd_dkv bf16");

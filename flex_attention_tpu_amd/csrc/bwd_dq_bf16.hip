@@ -27,7 +27,7 @@
   "a158", "a159", "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", \
   "a171", "a172", "a173", "a174", "a175", "a176", "a177", "a178", "a179", "a180", "a181", "a182", "a183", \
   "a184", "a185", "a186", "a187", "a188", "a189", "a190", "a191"
-#define FA_DQ_RUN_SGPRS "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", \
+#define FA_DQ_RUN_SGPRS "s59", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", \
   "s72", "s73", "s74", "s75", "s76", "s77", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", \
   "s87", "s88", "s89", "s90", "s91", "s92", "s93", "s94", "s95", "s96", "s97", "s98", "s99", "s100"
 
@@ -42,8 +42,9 @@ constexpr int D = 128;
 constexpr int LDS_BYTES = 4 * kTileElems * 2;  // K x2, V x2, per 128 columns of the head dimension
 // plain-score kernel: steps of two kv tiles, (K, K, V, V) x 2 buffers, per-wave tables, cached kv list + states
 constexpr int MAX_LIST = 4096;       // kv tiles of a row whose list and states the kernel caches in LDS (262144 tokens)
+constexpr int TBL = 20;              // dwords of a wave's table of run-loop constants
 constexpr int PREFETCH_LIST = 2048;  // of which an item's prefetch carries this many in registers; the rest is read when the item starts
-constexpr int PLAIN_LDS_BYTES = 8 * kTileElems * 2 + 4 * 16 * 4 + MAX_LIST * 5 + kDocStageBytes + kMaxSortedItems * 4;
+constexpr int PLAIN_LDS_BYTES = 8 * kTileElems * 2 + 4 * TBL * 4 + MAX_LIST * 5 + kDocStageBytes + kMaxSortedItems * 4;
 }  // namespace dq_cfg
 
 
@@ -72,7 +73,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
   bf16_t* sK = reinterpret_cast<bf16_t*>(smem_raw);
   bf16_t* sV = sK + 2 * NP * kTileElems;
 
-  const int nQ = a.Sq / BM;
+  const int nQ = a.map.nq;
   const int nK = a.map.nk;
   const int n_wg = a.B * a.Hq * nQ;
   const int wg = xcd_remap(blockIdx.x, n_wg);
@@ -89,7 +90,8 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
   const int l32 = lane & 31;
   const int hh = lane >> 5;
 
-  const size_t q_off = ((size_t)bh * a.Sq + (size_t)qb * BM) * D;
+  const int q0 = tile_base(qb, BM, a.Sq);
+  const size_t q_off = ((size_t)bh * a.Sq + (size_t)q0) * D;
   const bf16_t* Qg = static_cast<const bf16_t*>(a.q) + q_off;
   const bf16_t* dOg = static_cast<const bf16_t*>(a.dout) + q_off;
   bf16_t* dQg = static_cast<bf16_t*>(a.dq) + q_off;
@@ -97,8 +99,9 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
   const bf16_t* Vg = static_cast<const bf16_t*>(a.v) + ((size_t)(b * a.Hkv + hk) * a.Sk) * D;
 
   const int q_local = w * 32 + l32;
-  const int q_idx = qb * BM + q_local;
+  const int q_idx = q0 + q_local;
   const size_t row = (size_t)bh * a.Sq + q_idx;
+  const bool own_row = q_idx >= qb * BM;   // (else a row of the q tile before)
 
   ScoreMod<SCORE> sm;
   sm.init(a.score, a.sm_scale, h, b);
@@ -118,7 +121,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
   const uint8_t* tile_state = a.map.state + (size_t)qb * nK;
   int doc_i = 0;
   if (mk.flags & FLEXATTN_MASK_DOC) doc_i = mk.doc_q[q_idx];
-  float* dab_row = a.dab != nullptr ? a.dab + row * (size_t)a.Sk : nullptr;  // this lane's row of the bias gradient
+  float* dab_row = a.dab != nullptr && own_row ? a.dab + row * (size_t)a.Sk : nullptr;  // this lane's row of the bias gradient
 
   f32x16 dq_acc[4 * NP];
 #pragma unroll
@@ -140,8 +143,8 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
     const int kb0 = __builtin_amdgcn_readfirstlane(kb_cur);
 #pragma unroll
     for (int pn = 0; pn < NP; ++pn) {
-      loader.load(Kg + (size_t)kb0 * BN * D + 128 * pn, sK + pn * kTileElems);
-      loader.load(Vg + (size_t)kb0 * BN * D + 128 * pn, sV + pn * kTileElems);
+      loader.load(Kg + (size_t)tile_base(kb0, BN, a.Sk) * D + 128 * pn, sK + pn * kTileElems);
+      loader.load(Vg + (size_t)tile_base(kb0, BN, a.Sk) * D + 128 * pn, sV + pn * kTileElems);
     }
   }
   wait_vmem_all();
@@ -171,11 +174,12 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
       const int kbn = __builtin_amdgcn_readfirstlane(kb_nxt);
 #pragma unroll
       for (int pn = 0; pn < NP; ++pn) {
-        loader.load(Kg + (size_t)kbn * BN * D + 128 * pn, sK + ((buf ^ 1) * NP + pn) * kTileElems);
-        loader.load(Vg + (size_t)kbn * BN * D + 128 * pn, sV + ((buf ^ 1) * NP + pn) * kTileElems);
+        loader.load(Kg + (size_t)tile_base(kbn, BN, a.Sk) * D + 128 * pn, sK + ((buf ^ 1) * NP + pn) * kTileElems);
+        loader.load(Vg + (size_t)tile_base(kbn, BN, a.Sk) * D + 128 * pn, sV + ((buf ^ 1) * NP + pn) * kTileElems);
       }
     }
-    const int kv0 = kb * BN;
+    const int kv0 = tile_base(kb, BN, a.Sk);
+    const int kv_first = kb * BN;   // (keys before it belong to the tile before)
     const char* kt = reinterpret_cast<const char*>(sK + buf * NP * kTileElems);
     const char* vt = reinterpret_cast<const char*>(sV + buf * NP * kTileElems);
 
@@ -225,7 +229,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
           const int j0 = kv0 + 32 * c + 8 * g + 4 * hh;
           int dj[4] = {0, 0, 0, 0};
           if (MASKED && has_doc) {
-            const auto d4 = *reinterpret_cast<const int __attribute__((ext_vector_type(4)))*>(mk.doc_k + j0);
+            const auto d4 = *reinterpret_cast<const i32x4_a4*>(mk.doc_k + j0);
             dj[0] = d4[0]; dj[1] = d4[1]; dj[2] = d4[2]; dj[3] = d4[3];
           }
           float dsv[4];
@@ -238,14 +242,22 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
             float gl = pe * (dp_acc[e] - delta);
             float gd = gl * sm.dfactor(tv, s_acc[e], q_idx, j0 + u);
             if (MASKED) {   // (selected, not multiplied: a score function may return anything at a dropped element)
-              const bool keep = keep_elem(mk, q_idx, j0 + u, doc_i, dj[u]);
+              const bool keep = keep_elem(mk, q_idx, j0 + u, doc_i, dj[u]) & (j0 + u >= kv_first);
               gl = keep ? gl : 0.f;
               gd = keep ? gd : 0.f;
             }
             gb[u] = gl;
             dsv[u] = gd;
           }
-          if (dab_row != nullptr) *reinterpret_cast<f32x4*>(dab_row + j0) = gb;
+          if (dab_row != nullptr) {
+            if (!MASKED || j0 >= kv_first) {
+              *reinterpret_cast<f32x4_a4*>(dab_row + j0) = gb;
+            } else {
+#pragma unroll
+              for (int u = 0; u < 4; ++u)
+                if (j0 + u >= kv_first) dab_row[j0 + u] = gb[u];
+            }
+          }
           const bf16x2 d01 = pack_bf16(dsv[0], dsv[1]), d23 = pack_bf16(dsv[2], dsv[3]);
           const int o = 4 * (g & 1);
           ds[g >> 1][o] = d01[0]; ds[g >> 1][o + 1] = d01[1]; ds[g >> 1][o + 2] = d23[0]; ds[g >> 1][o + 3] = d23[1];
@@ -272,6 +284,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
     __syncthreads();
   }
 
+  if (!own_row) return;
 #pragma unroll
   for (int db = 0; db < 4 * NP; ++db) {
 #pragma unroll
@@ -291,7 +304,7 @@ static int launch_dq(const BwdArgs& a, hipStream_t stream) {
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, NP * LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dq): %s", hipGetErrorString(attr));
-  const int n_wg = a.B * a.Hq * (a.Sq / BM);
+  const int n_wg = a.B * a.Hq * a.map.nq;
   hipLaunchKernelGGL(kern, dim3(n_wg), dim3(256), NP * LDS_BYTES, stream, a);
   return check_launch("flexattn_bwd_dq bf16");
 }
@@ -324,10 +337,10 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
   bf16_t* sT = reinterpret_cast<bf16_t*>(smem_raw);  // buffer b: K tile 0, K tile 1, V tile 0, V tile 1
   unsigned* sTbl = reinterpret_cast<unsigned*>(sT + 8 * kTileElems);
-  int* sIdx = reinterpret_cast<int*>(sTbl + 4 * 16);
+  int* sIdx = reinterpret_cast<int*>(sTbl + 4 * TBL);
   unsigned char* sSt = reinterpret_cast<unsigned char*>(sIdx + MAX_LIST);
 
-  const int nQ = a.Sq / BM;
+  const int nQ = a.map.nq;
   const int nK = a.map.nk;
   const int n_wg = a.B * a.Hq * nQ;
   const int tid = threadIdx.x;
@@ -384,19 +397,20 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
   auto fetch = [&](int item, ItemRegs& r) {
     int bh, qb;
     geometry(item, bh, qb);
-    const size_t q_off = ((size_t)bh * a.Sq + (size_t)qb * BM + w * 32) * D;
+    const int q0 = tile_base(qb, BM, a.Sq);
+    const size_t q_off = ((size_t)bh * a.Sq + (size_t)q0 + w * 32) * D;
     rows_load(r.q, static_cast<const bf16_t*>(a.q) + q_off, lane);
     rows_load(r.d, static_cast<const bf16_t*>(a.dout) + q_off, lane);
-    const size_t row = (size_t)bh * a.Sq + qb * BM + q_local;
+    const size_t row = (size_t)bh * a.Sq + q0 + q_local;
     r.l = a.l[row];
     r.m = a.m[row];
     r.delta = a.delta[row];
     const size_t dq_rows = doc_rows(bh, a.Sq);
-    r.doc = (a.mask.flags & FLEXATTN_MASK_DOC) ? a.mask.doc_q[dq_rows + qb * BM + q_local] : 0;
+    r.doc = (a.mask.flags & FLEXATTN_MASK_DOC) ? a.mask.doc_q[dq_rows + q0 + q_local] : 0;
     if constexpr (DOCS) {
       const bool have = a.mask.doc_q_range != nullptr;
-      r.klo = have ? a.mask.doc_q_range[2 * (dq_rows + qb * BM + q_local)] : 0;
-      r.khi = have ? a.mask.doc_q_range[2 * (dq_rows + qb * BM + q_local) + 1] : 0;
+      r.klo = have ? a.mask.doc_q_range[2 * (dq_rows + q0 + q_local)] : 0;
+      r.khi = have ? a.mask.doc_q_range[2 * (dq_rows + q0 + q_local) + 1] : 0;
     }
     r.n_tiles = a.map.cnt[qb];
     const int* tile_idx = a.map.idx + (size_t)qb * nK;
@@ -481,10 +495,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
     geometry(item, bh, qb);
     if (item > 0) __syncthreads();  // the previous item's LDS contents are dead from here
 
-    bf16_t* dQg = static_cast<bf16_t*>(a.dq) + ((size_t)bh * a.Sq + (size_t)qb * BM) * D;
+    const int q0 = tile_base(qb, BM, a.Sq);
+    bf16_t* dQg = static_cast<bf16_t*>(a.dq) + ((size_t)bh * a.Sq + (size_t)q0) * D;
     const bf16_t* Kg = static_cast<const bf16_t*>(a.k) + ((size_t)kv_pair(bh) * a.Sk) * D;
     const bf16_t* Vg = static_cast<const bf16_t*>(a.v) + ((size_t)kv_pair(bh) * a.Sk) * D;
-    const int q_idx = qb * BM + q_local;
+    const int q_idx = q0 + q_local;
     const int* tile_idx = a.map.idx + (size_t)qb * nK;
 
     // the q tile's kv list and its state row into LDS
@@ -527,13 +542,14 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
     if (n_tiles > 0 && !resident) {
       // first step into the current buffer (a missing second entry repeats the first: finite data, masked out)
       bf16_t* dst = sT + (size_t)buf * 4 * kTileElems;
-      loader.load(Kg + (size_t)kb_first * BN * D, dst);
-      loader.load(Kg + (size_t)kb_second * BN * D, dst + kTileElems);
-      loader.load(Vg + (size_t)kb_first * BN * D, dst + 2 * kTileElems);
-      loader.load(Vg + (size_t)kb_second * BN * D, dst + 3 * kTileElems);
+      const size_t ra_ = (size_t)tile_base(kb_first, BN, a.Sk) * D, rb_ = (size_t)tile_base(kb_second, BN, a.Sk) * D;
+      loader.load(Kg + ra_, dst);
+      loader.load(Kg + rb_, dst + kTileElems);
+      loader.load(Vg + ra_, dst + 2 * kTileElems);
+      loader.load(Vg + rb_, dst + 3 * kTileElems);
       wait_vmem_all();
     }
-    unsigned* tbl = sTbl + w * 16;
+    unsigned* tbl = sTbl + w * TBL;
     const unsigned tbl_addr = (unsigned)(size_t)tbl;
     __syncthreads();
     // The next item's data lands while this item runs.  (The last item fetches itself again: every
@@ -589,8 +605,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
         int* sDoc = reinterpret_cast<int*>(sSt + MAX_LIST) + w * 128;  // the wave's stage for document ids
         if ((a.mask.flags & FLEXATTN_MASK_DOC) && !ranged) {
           const int e1 = 2 * it_part + 1 < n_tiles ? 2 * it_part + 1 : 2 * it_part;
-          stage_doc_ids(a.mask.doc_k + doc_rows(bh, a.Sk), __builtin_amdgcn_readfirstlane(sIdx[2 * it_part]) * BN,
-                        __builtin_amdgcn_readfirstlane(sIdx[e1]) * BN, lane, sDoc);
+          stage_doc_ids(a.mask.doc_k + doc_rows(bh, a.Sk), tile_base(__builtin_amdgcn_readfirstlane(sIdx[2 * it_part]), BN, a.Sk),
+                        tile_base(__builtin_amdgcn_readfirstlane(sIdx[e1]), BN, a.Sk), lane, sDoc);
         }
 #pragma unroll
         for (int hx = 0; hx < 2; ++hx) {
@@ -598,15 +614,17 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
           if (e >= n_tiles) continue;  // missing half: all dropped
           const int kt = __builtin_amdgcn_readfirstlane(sIdx[e]);
           const int state = __builtin_amdgcn_readfirstlane((int)sSt[kt]);
+          const int k0 = tile_base(kt, BN, a.Sk);
           if (state == 2) {
             km[hx] = 0xffffffffu;
           } else if (DOCS && ranged) {
-            km[hx] = keep_bits32_range<true>(a.mask, q_idx, kt * BN + 4 * hh, cur.klo, cur.khi);
+            km[hx] = keep_bits32_range<true>(a.mask, q_idx, k0 + 4 * hh, cur.klo, cur.khi);
           } else if (a.mask.flags & FLEXATTN_MASK_DOC) {
-            km[hx] = keep_bits32_staged<true>(a.mask, q_idx, kt * BN + 4 * hh, doc_i, sDoc + 64 * hx + 4 * hh);
+            km[hx] = keep_bits32_staged<true>(a.mask, q_idx, k0 + 4 * hh, doc_i, sDoc + 64 * hx + 4 * hh);
           } else {
-            km[hx] = keep_bits32<true>(a.mask, q_idx, kt * BN + 4 * hh, doc_i, nullptr);
+            km[hx] = keep_bits32<true>(a.mask, q_idx, k0 + 4 * hh, doc_i, nullptr);
           }
+          km[hx] &= keep_bits_from(kt * BN - k0 - 4 * hh);
         }
       } else {
         it_part = -1;
@@ -639,6 +657,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
           tbl[13] = (unsigned)((size_t)Kg_n >> 32);
           tbl[14] = (unsigned)(size_t)Vg_n;
           tbl[15] = (unsigned)((size_t)Vg_n >> 32);
+          tbl[16] = (unsigned)(a.Sk - BN);  // the last kv tile starts here at the latest
         }
       }
       // no scalar operands (see gen_dq_tile.py): the loop state travels in VGPRs
@@ -711,9 +730,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
       __builtin_amdgcn_wave_barrier();
       bf16_t* out_rows = dQg + (size_t)(w * 32) * D;
       const int chunk = lane_here & 15;
+      const int r_first = qb * BM - q0 - w * 32;   // (rows before it belong to the q tile before)
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int r = 4 * i + (lane_here >> 4);
+        if (r < r_first) continue;
         const u32x4 x = *reinterpret_cast<const u32x4*>(stage + (unsigned)r * 256u + (unsigned)((chunk ^ (r & 15)) << 4));
         *reinterpret_cast<u32x4*>(out_rows + (size_t)r * D + chunk * 8) = x;
       }
@@ -728,8 +749,8 @@ static int launch_dq_plain_on(const BwdArgs& a, hipStream_t stream) {
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, PLAIN_LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dq): %s", hipGetErrorString(attr));
-  const int n_wg = a.B * a.Hq * (a.Sq / BM);
-  const bool persistent = DOCS ? sorted_schedule_ok(n_wg, a.Sq / BM) : persistent_ok(n_wg, a.Sq / BM);
+  const int n_wg = a.B * a.Hq * a.map.nq;
+  const bool persistent = DOCS ? sorted_schedule_ok(n_wg, a.map.nq) : persistent_ok(n_wg, a.map.nq);
   const int grid = (persistent && n_wg > 256) ? 256 : n_wg;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(256), PLAIN_LDS_BYTES, stream, a);
   return check_launch("flexattn_bwd_dq bf16");

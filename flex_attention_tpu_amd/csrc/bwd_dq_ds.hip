@@ -132,7 +132,7 @@ __global__ __launch_bounds__(dqds_cfg::THREADS, dqds_cfg::OCC) void bwd_dq_from_
       src = ds_row + (size_t)block_of(s) * kDsBlockBytes + (size_t)(s % PARTS) * DS_STAGE_BYTES;
       dst = lds0 + (unsigned)(s % NDS) * DS_STAGE_BYTES + (unsigned)w * 4096u;
     } else {
-      src = reinterpret_cast<const char*>(Kg + ((size_t)tile_of(s) * BNK + (size_t)(s % PARTS) * STAGE_KV) * D);
+      src = reinterpret_cast<const char*>(Kg + ((size_t)tile_base(tile_of(s), BNK, a.Sk) + (size_t)(s % PARTS) * STAGE_KV) * D);
       dst = lds0 + K_RING + (unsigned)(s % NK) * K_STAGE_BYTES + (unsigned)(w - 2) * 4096u;
     }
 #pragma unroll
@@ -252,11 +252,14 @@ __global__ __launch_bounds__(dqds_cfg::THREADS, dqds_cfg::OCC) void bwd_dq_from_
   __syncthreads();
   if (!computes) return;
   const char* stage = smem_raw + w * 8192;  // wave w stores q block w
-  bf16_t* dQg = static_cast<bf16_t*>(a.dq) + ((size_t)bh * a.Sq + (size_t)qb * BQ + (size_t)w * 32) * D;
+  const int q0 = tile_base(qb, BQ, a.Sq);
+  bf16_t* dQg = static_cast<bf16_t*>(a.dq) + ((size_t)bh * a.Sq + (size_t)q0 + (size_t)w * 32) * D;
+  const int r_first = qb * BQ - q0 - w * 32;   // (rows before it belong to the q tile before)
   const int chunk = lane & 15;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int r = 4 * i + (lane >> 4);
+    if (r < r_first) continue;
     const unsigned rd = (unsigned)r * 256u + (unsigned)((chunk ^ (r & 15)) << 4);
     *reinterpret_cast<u32x4*>(dQg + (size_t)r * D + chunk * 8) = *reinterpret_cast<const u32x4*>(stage + rd);
   }
@@ -272,7 +275,7 @@ int bwd_dq_from_ds(const BwdArgs& a, float out_scale, hipStream_t stream) {
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dq from dS): %s", hipGetErrorString(attr));
-  const int n_wg = a.B * a.Hq * (a.Sq / BQ);
+  const int n_wg = a.B * a.Hq * a.map.nq;
   hipLaunchKernelGGL(kern, dim3(n_wg), dim3(THREADS), LDS_BYTES, stream, a, out_scale);
   return check_launch("flexattn_bwd_dq (from dS) bf16");
 }

@@ -32,6 +32,10 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+// (16 bytes of a row whose start is aligned to 4 bytes only)
+typedef unsigned int u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef int i32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
@@ -101,6 +105,18 @@ struct MapArgs {
   const int* idx;
   int nq, nk;
 };
+
+// Ragged lengths.  Sq and Sk below are the tensors' own lengths; the block map has ceil(S / tile) tiles a side.  A last
+// tile that would run past the end starts at S - tile instead (tile_base), so that every copy, load and row value
+// stays inside its head's rows whatever the length (at least one tile); the rows it shares with the tile before are
+// dropped: masked where they would enter a sum, not stored where they are results.  Against zero-padded copies of the
+// operands this costs no pass over memory (B=1, Hq=32, Hkv=8, S=2777, D=128 forward: the copies, their clearing and the
+// cutting back took 52 of 147 us).
+__host__ __device__ __forceinline__ int tile_base(int t, int tile, int len) {
+  const int at = t * tile;
+  return at + tile <= len ? at : len - tile;
+}
+__host__ __device__ __forceinline__ int tiles_of(int len, int tile) { return (len + tile - 1) / tile; }
 
 struct FwdArgs {
   const void* q; const void* k; const void* v;
@@ -260,7 +276,7 @@ __host__ __device__ __forceinline__ unsigned compress_even_nibbles(unsigned long
   m = (m | (m >> 16)) & 0x00000000FFFFFFFFull;
   return (unsigned)m;
 }
-// Document ids of two 64-index strips, from `first_a` and `first_b` on (multiples of 4), into a
+// Document ids of two 64-index strips, from `first_a` and `first_b` on, into a
 // wave-private LDS stage of 128 ints: lanes 0-31 load and store 16 bytes each.  keep_bits32 then reads
 // a strip's ids from LDS (pass `stage [+ 64] - first` as its doc_var) instead of one dependent global
 // load per group of four elements.
@@ -268,16 +284,21 @@ constexpr int kDocStageBytes = 4 * 128 * 4;  // four waves
 __device__ __forceinline__ void stage_doc_ids(const int* doc, int first_a, int first_b, int lane, int* stage) {
   if (lane < 32) {
     const int first = lane < 16 ? first_a : first_b;
-    const u32x4 v = *reinterpret_cast<const u32x4*>(doc + first + 4 * (lane & 15));
+    const u32x4 v = *reinterpret_cast<const u32x4_a4*>(doc + first + 4 * (lane & 15));
     *reinterpret_cast<u32x4*>(stage + 4 * lane) = v;
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
+// The keep bits of the offsets from `first` on (the rows a shifted last tile does not share with the one before).
+__host__ __device__ __forceinline__ unsigned keep_bits_from(int first) {
+  if (first <= 0) return ~0u;
+  return first > 63 ? 0u : compress_even_nibbles(~0ull << first);
+}
 template <bool KEYS>
 __host__ __device__ __forceinline__ unsigned keep_bits32(const MaskArgs& mk, int fixed, int base, int doc_fixed,
                                                 const int* doc_var) {
-  if (mk.flags != 0 && (mk.flags & ~(FLEXATTN_MASK_CAUSAL | FLEXATTN_MASK_WINDOW)) == 0) {
+  if ((mk.flags & ~(FLEXATTN_MASK_CAUSAL | FLEXATTN_MASK_WINDOW)) == 0) {
     // kept offsets form one interval [lo, hi]: with d = fixed - base, keys keep d - window < off <= d,
     // queries keep d <= off < d + window (the causal bound resp. the window bound, where present)
     const int d = fixed - base;

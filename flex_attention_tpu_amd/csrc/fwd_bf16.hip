@@ -12,7 +12,7 @@
 #include "launch.hpp"
 #include "tile_io.hpp"
 
-// registers of the generated run loop (gen_fwd_tile.py): v[66:199], a[192:255], s[60:100]
+// registers of the generated run loop (gen_fwd_tile.py): v[66:199], a[192:255], s[59:100]
 #define FA_FWD_RUN_VGPRS "v66", "v67", "v68", "v69", "v70", "v71", "v72", "v73", "v74", "v75", "v76", "v77", "v78", "v79", "v80", \
   "v81", "v82", "v83", "v84", "v85", "v86", "v87", "v88", "v89", "v90", "v91", "v92", "v93", "v94", "v95", \
   "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103", "v104", "v105", "v106", "v107", "v108", "v109", \
@@ -28,7 +28,7 @@
   "a219", "a220", "a221", "a222", "a223", "a224", "a225", "a226", "a227", "a228", "a229", "a230", "a231", \
   "a232", "a233", "a234", "a235", "a236", "a237", "a238", "a239", "a240", "a241", "a242", "a243", "a244", \
   "a245", "a246", "a247", "a248", "a249", "a250", "a251", "a252", "a253", "a254", "a255"
-#define FA_FWD_RUN_SGPRS "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", \
+#define FA_FWD_RUN_SGPRS "s59", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", \
   "s72", "s73", "s74", "s75", "s76", "s77", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", \
   "s87", "s88", "s89", "s90", "s91", "s92", "s93", "s94", "s95", "s96", "s97", "s98", "s99", "s100"
 
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
   bf16_t* sK = reinterpret_cast<bf16_t*>(smem_raw);
   bf16_t* sV = sK + 2 * NP * kTileElems;
 
-  const int nQ = a.Sq / BM;
+  const int nQ = a.map.nq;
   const int nK = a.map.nk;
   const int n_wg = a.B * a.Hq * nQ;
   const int wg = xcd_remap(blockIdx.x, n_wg);
@@ -90,13 +90,14 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
   const int l32 = lane & 31;
   const int hh = lane >> 5;
 
-  const bf16_t* Qg = static_cast<const bf16_t*>(a.q) + ((size_t)bh * a.Sq + (size_t)qb * BM) * D;
+  const int q0 = tile_base(qb, BM, a.Sq);
+  const bf16_t* Qg = static_cast<const bf16_t*>(a.q) + ((size_t)bh * a.Sq + (size_t)q0) * D;
   const bf16_t* Kg = static_cast<const bf16_t*>(a.k) + ((size_t)(b * a.Hkv + hk) * a.Sk) * D;
   const bf16_t* Vg = static_cast<const bf16_t*>(a.v) + ((size_t)(b * a.Hkv + hk) * a.Sk) * D;
-  bf16_t* Og = static_cast<bf16_t*>(a.o) + ((size_t)bh * a.Sq + (size_t)qb * BM) * D;
+  bf16_t* Og = static_cast<bf16_t*>(a.o) + ((size_t)bh * a.Sq + (size_t)q0) * D;
 
   const int q_local = w * 32 + l32;
-  const int q_idx = qb * BM + q_local;
+  const int q_idx = q0 + q_local;
 
   ScoreMod<SCORE> sm;
   sm.init(a.score, a.sm_scale, h, b);
@@ -136,8 +137,8 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
     const int kb0 = __builtin_amdgcn_readfirstlane(kb_cur);
 #pragma unroll
     for (int pn = 0; pn < NP; ++pn) {
-      loader.load(Kg + (size_t)kb0 * BN * D + 128 * pn, sK + pn * kTileElems);
-      loader.load(Vg + (size_t)kb0 * BN * D + 128 * pn, sV + pn * kTileElems);
+      loader.load(Kg + (size_t)tile_base(kb0, BN, a.Sk) * D + 128 * pn, sK + pn * kTileElems);
+      loader.load(Vg + (size_t)tile_base(kb0, BN, a.Sk) * D + 128 * pn, sV + pn * kTileElems);
     }
   }
   wait_vmem_all();
@@ -173,8 +174,8 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
     // The next tile's LDS-direct loads are issued two at a time between the MFMA stages below.
     const bool prefetch = t + 1 < n_tiles;
     const int kbn = __builtin_amdgcn_readfirstlane(kb_nxt);
-    const bf16_t* k_next = Kg + (size_t)kbn * BN * D;
-    const bf16_t* v_next = Vg + (size_t)kbn * BN * D;
+    const bf16_t* k_next = Kg + (size_t)tile_base(kbn, BN, a.Sk) * D;
+    const bf16_t* v_next = Vg + (size_t)tile_base(kbn, BN, a.Sk) * D;
 
     // ---- S^T = K Q^T : two 32(kv) x 32(q) accumulator tiles ----
     // LDS operand reads run one stage (4 MFMAs) ahead of the MFMAs that consume them, so the LDS
@@ -235,7 +236,8 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
     // ---- score mod, mask, online softmax ----
     // For the plain score the running maximum is kept on the raw dot products and the scale is
     // folded into the exponent (one FMA per element); score mods go through the log2-domain logit.
-    const int kv0 = kb * BN;
+    const int kv0 = tile_base(kb, BN, a.Sk);
+    const int kv_first = kb * BN;   // (keys before it belong to the tile before)
     constexpr bool kPlain = (SCORE == FLEXATTN_SCORE_NONE);
     float m_tile = kNegInf;
     if (!partial) {
@@ -260,14 +262,14 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
           const int j0 = kv0 + 32 * c + 8 * g + 4 * hh;
           int dj[4] = {0, 0, 0, 0};
           if (has_doc) {
-            const auto d4 = *reinterpret_cast<const int __attribute__((ext_vector_type(4)))*>(mk.doc_k + j0);
+            const auto d4 = *reinterpret_cast<const i32x4_a4*>(mk.doc_k + j0);
             dj[0] = d4[0]; dj[1] = d4[1]; dj[2] = d4[2]; dj[3] = d4[3];
           }
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const int e = 4 * g + u;
             float tv = kPlain ? s_acc[c][e] : sm.to_log2(s_acc[c][e], q_idx, j0 + u) + sm.bias2(q_idx, j0 + u);
-            tv = keep_elem(mk, q_idx, j0 + u, doc_i, dj[u]) ? tv : kNegInf;
+            tv = (keep_elem(mk, q_idx, j0 + u, doc_i, dj[u]) & (j0 + u >= kv_first)) ? tv : kNegInf;
             s_acc[c][e] = tv;
             m_tile = fmaxf(m_tile, tv);
           }
@@ -335,6 +337,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
   // ---- epilogue ----
   const float l_tot = half_sum(l_run);
   const float inv = (l_tot > 0.f) ? 1.0f / l_tot : 0.f;
+  if (q_idx < qb * BM) return;   // (a row of the q tile before)
 #pragma unroll
   for (int db = 0; db < 4 * NP; ++db) {
 #pragma unroll
@@ -359,7 +362,7 @@ static int launch_fwd(const FwdArgs& a, hipStream_t stream) {
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, NP * LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(fwd): %s", hipGetErrorString(attr));
-  const int n_wg = a.B * a.Hq * (a.Sq / BM);
+  const int n_wg = a.B * a.Hq * a.map.nq;
   hipLaunchKernelGGL(kern, dim3(n_wg), dim3(256), NP * LDS_BYTES, stream, a);
   return check_launch("flexattn_fwd bf16");
 }
@@ -398,7 +401,7 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
   unsigned char* sStA = reinterpret_cast<unsigned char*>(sList + MAX_LIST);
   unsigned char* sStB = sStA + MAX_LIST;
 
-  const int nQ = a.Sq / BM;
+  const int nQ = a.map.nq;
   const int nQ2 = (nQ + 1) >> 1;
   const int nK = a.map.nk;
   const int n_wg = a.B * a.Hq * nQ2;
@@ -481,12 +484,13 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
       const int qb = min(2 * qb2 + x, nQ - 1);  // (a missing second tile repeats the first; nothing of it is stored)
-      rows_load(r.q[x], static_cast<const bf16_t*>(a.q) + ((size_t)bh * a.Sq + (size_t)qb * BM + w_here * 32) * D, lane_here);
-      r.doc[x] = (a.mask.flags & FLEXATTN_MASK_DOC) ? a.mask.doc_q[dq_rows + qb * BM + row_here] : 0;
+      const int q0 = tile_base(qb, BM, a.Sq);
+      rows_load(r.q[x], static_cast<const bf16_t*>(a.q) + ((size_t)bh * a.Sq + (size_t)q0 + w_here * 32) * D, lane_here);
+      r.doc[x] = (a.mask.flags & FLEXATTN_MASK_DOC) ? a.mask.doc_q[dq_rows + q0 + row_here] : 0;
       if constexpr (DOCS) {
         const bool ranged = a.mask.doc_q_range != nullptr;
-        r.klo[x] = ranged ? a.mask.doc_q_range[2 * (dq_rows + qb * BM + row_here)] : 0;
-        r.khi[x] = ranged ? a.mask.doc_q_range[2 * (dq_rows + qb * BM + row_here) + 1] : 0;
+        r.klo[x] = ranged ? a.mask.doc_q_range[2 * (dq_rows + q0 + row_here)] : 0;
+        r.khi[x] = ranged ? a.mask.doc_q_range[2 * (dq_rows + q0 + row_here) + 1] : 0;
       }
       const uint8_t* row = a.map.state + (size_t)qb * nK;
       const bool valid = 2 * qb2 + x < nQ;
@@ -614,7 +618,9 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
     // (DOCS) with sorted kv ids the keys of a row's document are one interval: the keep bits of a partial tile
     // then have a closed form (keep_bits32_range) and no ids are read
     const bool ranged = DOCS && a.mask.doc_q_range != nullptr && keep_bits_have_range(a.mask);
-    const int q_idx[2] = {(2 * qb2) * BM + q_local, (2 * qb2 + 1) * BM + q_local};
+    // (first row of each q tile; the last tile of a ragged length starts early, see tile_base)
+    const int q_at[2] = {tile_base(2 * qb2, BM, a.Sq), 2 * qb2 + 1 < nQ ? tile_base(2 * qb2 + 1, BM, a.Sq) : (2 * qb2 + 1) * BM};
+    const int q_idx[2] = {q_at[0] + q_local, q_at[1] + q_local};
     // softmax state of the lane's two q rows (log2 domain): reference maximum M, running maximum
     // relative to it, sum of 2^(score - M)
     // (softcap: the reference is the constant cap and the streams leave M and Mt alone)
@@ -624,7 +630,8 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
     const float a2 = ALIBI ? a.score.slopes[bh % a.Hq] * kLog2e : 0.f;
     const float aone = hh ? (float)l32 : 1.f;
     const float mulv = hh ? 0.f : a2;
-    float addv[2] = {hh ? a2 : 0.f, hh ? a2 : 0.f};
+    // (the streams place q block 1 128 rows behind q block 0: a second tile that starts early gets the difference here)
+    float addv[2] = {hh ? a2 : 0.f, hh ? a2 : a2 * (float)(q_at[0] + BM - q_at[1])};
 
     // entry e of the list in the order the steps take it: ascending kv tiles; descending under a position
     // bias, which (slopes are positive) is largest at the last key, so that the running maximum settles early
@@ -635,10 +642,11 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
       const int ka = __builtin_amdgcn_readfirstlane(entry(0));
       const int kbb = __builtin_amdgcn_readfirstlane(entry(1));
       bf16_t* dst = sT + (size_t)buf * 4 * kTileElems;
-      loader.load(Kg + (size_t)ka * BN * D, dst);
-      loader.load(Kg + (size_t)kbb * BN * D, dst + kTileElems);
-      loader.load(Vg + (size_t)ka * BN * D, dst + 2 * kTileElems);
-      loader.load(Vg + (size_t)kbb * BN * D, dst + 3 * kTileElems);
+      const size_t ra_ = (size_t)tile_base(ka, BN, a.Sk) * D, rb_ = (size_t)tile_base(kbb, BN, a.Sk) * D;
+      loader.load(Kg + ra_, dst);
+      loader.load(Kg + rb_, dst + kTileElems);
+      loader.load(Vg + ra_, dst + 2 * kTileElems);
+      loader.load(Vg + rb_, dst + 3 * kTileElems);
       wait_vmem_all();
     }
     resident = false;
@@ -675,7 +683,7 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
       tbl[11] = (unsigned)((size_t)Kg >> 32);
       tbl[12] = (unsigned)(size_t)Vg;
       tbl[13] = (unsigned)((size_t)Vg >> 32);
-      tbl[14] = 0u;
+      tbl[14] = (unsigned)(a.Sk - BN);  // the last kv tile starts here at the latest
       tbl[15] = 0u;
     }
     // a step is full when both of its entries exist and are full for both q tiles
@@ -693,14 +701,16 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
         int* sDoc = reinterpret_cast<int*>(sStB + MAX_LIST) + w * 128;  // the wave's stage for document ids
         if constexpr (DOCS) {
           if (!ranged)
-            stage_doc_ids(a.mask.doc_k + doc_rows(bh, a.Sk), __builtin_amdgcn_readfirstlane(entry(2 * it)) * BN,
-                          __builtin_amdgcn_readfirstlane(entry(2 * it + 1)) * BN, lane, sDoc);
+            stage_doc_ids(a.mask.doc_k + doc_rows(bh, a.Sk), tile_base(__builtin_amdgcn_readfirstlane(entry(2 * it)), BN, a.Sk),
+                          tile_base(__builtin_amdgcn_readfirstlane(entry(2 * it + 1)), BN, a.Sk), lane, sDoc);
         }
 #pragma unroll
         for (int hx = 0; hx < 2; ++hx) {
           const int e = 2 * it + hx;
           if (e >= n_list) continue;  // missing half: all dropped
           const int k = __builtin_amdgcn_readfirstlane(list_at(e));
+          const int k0 = tile_base(k, BN, a.Sk);
+          const unsigned own = keep_bits_from(k * BN - k0 - 4 * hh);
 #pragma unroll
           for (int x = 0; x < 2; ++x) {
             const int state = __builtin_amdgcn_readfirstlane((int)(x == 0 ? sStA[k] : sStB[k]));
@@ -708,10 +718,11 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
               km[2 * x + hx] = 0xffffffffu;
             } else if (state == 1) {
               if constexpr (DOCS)
-                km[2 * x + hx] = ranged ? keep_bits32_range<true>(a.mask, q_idx[x], k * BN + 4 * hh, cur.klo[x], cur.khi[x])
-                                        : keep_bits32_staged<true>(a.mask, q_idx[x], k * BN + 4 * hh, doc_i[x], sDoc + 64 * hx + 4 * hh);
+                km[2 * x + hx] = ranged ? keep_bits32_range<true>(a.mask, q_idx[x], k0 + 4 * hh, cur.klo[x], cur.khi[x])
+                                        : keep_bits32_staged<true>(a.mask, q_idx[x], k0 + 4 * hh, doc_i[x], sDoc + 64 * hx + 4 * hh);
               else
-                km[2 * x + hx] = keep_bits32<true>(a.mask, q_idx[x], k * BN + 4 * hh, doc_i[x], a.mask.doc_k);
+                km[2 * x + hx] = keep_bits32<true>(a.mask, q_idx[x], k0 + 4 * hh, doc_i[x], a.mask.doc_k);
+              km[2 * x + hx] &= own;
             }
           }
         }
@@ -840,7 +851,7 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
         const float l_tot = half_sum(L[x]);
         const float mt_row = half_max(Mt[x]);  // (the streams keep the running maximum per lane)
         inv[x] = (l_tot > 0.f) ? 1.0f / l_tot : 0.f;
-        if (2 * qb2 + x < nQ && a.l != nullptr && lane_here < 32) {
+        if (2 * qb2 + x < nQ && a.l != nullptr && lane_here < 32 && q_idx[x] >= (2 * qb2 + x) * BM) {
           const size_t r = (size_t)bh * a.Sq + q_idx[x];
           // sums were taken against the reference maximum M: move them to the true maximum M + Mt
           a.l[r] = (l_tot > 0.f) ? l_tot * fast_exp2(-mt_row) : 0.f;
@@ -874,10 +885,12 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
         if (2 * qb2 + x < nQ) {
-          bf16_t* Og = static_cast<bf16_t*>(a.o) + ((size_t)bh * a.Sq + (size_t)(2 * qb2 + x) * BM + w * 32) * D;
+          bf16_t* Og = static_cast<bf16_t*>(a.o) + ((size_t)bh * a.Sq + (size_t)q_at[x] + w * 32) * D;
+          const int r_first = (2 * qb2 + x) * BM - q_at[x] - w * 32;   // (rows before it belong to the q tile before)
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
             const int r = 4 * i + (lane_here >> 4);
+            if (r < r_first) continue;
             const u32x4 v = *reinterpret_cast<const u32x4*>(stage + x * 8192 + (unsigned)r * 256u +
                                                             (unsigned)((chunk ^ (r & 15)) << 4));
             *reinterpret_cast<u32x4*>(Og + (size_t)r * D + chunk * 8) = v;
@@ -895,7 +908,7 @@ static int launch_fwd_plain_on(const FwdArgs& a, hipStream_t stream) {
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, PLAIN_LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(fwd): %s", hipGetErrorString(attr));
-  const int nQ2 = (a.Sq / BM + 1) / 2;
+  const int nQ2 = (a.map.nq + 1) / 2;
   const int n_wg = a.B * a.Hq * nQ2;
   // (document masks take the longest-first schedule of sorted_items)
   const bool persistent = DOCS ? sorted_schedule_ok(n_wg, nQ2) : persistent_ok(n_wg, nQ2);

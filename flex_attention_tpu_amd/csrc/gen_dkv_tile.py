@@ -362,6 +362,8 @@ def build(masked, alibi=False, softcap=False, export=False):
             # middle j0 of the kv tile (s64 holds -slope log2 e): the key's share 2^(slope log2(e) (j - j0))
             # is a factor of whole dk / dv rows, which the epilogue applies
             e.raw(f"s_lshl_b32 {S_T[0]}, s80, 7")
+            e.raw(f"s_sub_u32 {S_T[1]}, s62, 128")
+            e.raw(f"s_min_u32 {S_T[0]}, {S_T[0]}, {S_T[1]}")   # (a ragged length's last q tile starts early)
             e.raw(f"s_sub_i32 {S_T[0]}, {S_T[0]}, {S_KC}")
             e.valu(f"v_lshrrev_b32_e32 {vr(inf_)}, 2, %[tid4]", vset(inf_), set())
             e.valu(f"v_add_u32_e32 {vr(inf_)}, {S_T[0]}, {vr(inf_)}", vset(inf_), vset(inf_))
@@ -436,10 +438,13 @@ def run_loop(full, masked, alibi=False, softcap=False, export=False):
         "s_mov_b32 s78, 0",
         ".Lfa_dkv_same_%=:",
     ] + ds_next + [
-        # row of the next step relative to the first head of the group: min(g1, gmax) Sq + 128 qb1
+        # row of the next step relative to the first head of the group: min(g1, gmax) Sq + min(128 qb1, Sq - 128) (the
+        # last q tile of a ragged length starts early)
         f"s_min_u32 {t0}, s78, s61",
         f"s_mul_i32 {t0}, {t0}, s62",
         f"s_lshl_b32 {t1}, s80, 7",
+        f"s_sub_u32 {t2}, s62, 128",
+        f"s_min_u32 {t1}, {t1}, {t2}",
         f"s_add_u32 {t0}, {t0}, {t1}",
         f"s_lshl_b32 {t2}, {t0}, 8",
         f"s_lshr_b32 {t3}, {t0}, 24",

@@ -60,10 +60,10 @@ TILE = 16384
 # (the compiler may print a VGPR for an "s" operand once many uniform values are live).
 TABLE = ["n_tiles", "w4k", "c2", "n_steps",  # (c2: softcap and exact-scale variants; its register holds a tile index in the position-bias variant)
          "idx_lo", "idx_hi", "kg_lo", "kg_hi", "vg_lo", "vg_hi", "kban", "kbbn",
-         "kgn_lo", "kgn_hi", "vgn_lo", "vgn_hi"]
+         "kgn_lo", "kgn_hi", "vgn_lo", "vgn_hi", "klim"]   # (klim: first row of the last kv tile at the latest)
 SREG = {"n_tiles": "s60", "w4k": "s61", "c2": "s62", "n_steps": "s63", "idx_lo": "s64", "idx_hi": "s65",
         "kg_lo": "s66", "kg_hi": "s67", "vg_lo": "s68", "vg_hi": "s69", "kban": "s70", "kbbn": "s71",
-        "kgn_lo": "s78", "kgn_hi": "s79", "vgn_lo": "s80", "vgn_hi": "s81",
+        "kgn_lo": "s78", "kgn_hi": "s79", "vgn_lo": "s80", "vgn_hi": "s81", "klim": "s59",
         "it": "s72", "kba1": "s73", "kbb1": "s74", "buf": "s75", "it_end": "s76", "partial": "s77",
         "idx": "s[64:65]"}
 S_SEL = ["s82", "s83", "s96", "s97", "s98", "s99"]  # this pass's tile indices and K / V bases (next step or next item)
@@ -74,7 +74,7 @@ S_GK0, S_GK1, S_GV0, S_GV1 = "s[88:89]", "s[90:91]", "s[92:93]", "s[94:95]"
 S_LDSN = "s100"
 V_KB2 = 66       # kv tile indices of the step after the next one (2 registers), across the stream
 V_TMP = 68       # 4 temporaries of the masked variant
-V_TBL = 72       # 12 scratch VGPRs the table is read into at entry
+V_TBL = 72       # 20 scratch VGPRs the table is read into at entry
 V_S = [72, 104]
 V_DP = [88, 120]
 V_DS = 136       # dS^T as MFMA B operands: [c & 1][u] x 4 registers
@@ -101,6 +101,7 @@ def bias_ops(e, block, tile, odd):
     t0 = S_T[0]
     b = V_B[block & 1]
     e.raw(f"s_lshl_b32 {t0}, {tile}, 6")
+    e.raw(f"s_min_u32 {t0}, {t0}, {SREG['klim']}")
     if odd:
         e.raw(f"s_add_u32 {t0}, {t0}, 32")
     e.valu(f"v_sub_u32_e32 {vr(V_T)}, {t0}, %[iq]", vset(V_T), set())
@@ -295,7 +296,7 @@ def run_loop(full, masked, alibi=False, softcap=False, exact=False):
     t0, t1, t2, t3 = S_T
     S = SREG
     n_tbl = len(TABLE)
-    entry = [f"ds_read_b128 {vr(V_TBL + 4 * i, 4)}, %[tbl] offset:{16 * i}" for i in range(n_tbl // 4)]
+    entry = [f"ds_read_b128 {vr(V_TBL + 4 * i, 4)}, %[tbl] offset:{16 * i}" for i in range((n_tbl + 3) // 4)]
     entry += ["s_waitcnt lgkmcnt(0)"]  # (the streams count LDS operations from zero)
     entry += [f"v_readfirstlane_b32 {S[n]}, {vr(V_TBL + i)}" for i, n in enumerate(TABLE)]
     entry += [f"v_readfirstlane_b32 {S[n]}, %[{n}]" for n in STATE_IO + STATE_IN]
@@ -316,11 +317,13 @@ def run_loop(full, masked, alibi=False, softcap=False, exact=False):
             f"s_cselect_b32 {ka}, {S['kban']}, {S['kba1']}", f"s_cselect_b32 {kb_}, {S['kbbn']}, {S['kbb1']}",
             f"s_cselect_b32 {kglo}, {S['kgn_lo']}, {S['kg_lo']}", f"s_cselect_b32 {kghi}, {S['kgn_hi']}, {S['kg_hi']}",
             f"s_cselect_b32 {vglo}, {S['vgn_lo']}, {S['vg_lo']}", f"s_cselect_b32 {vghi}, {S['vgn_hi']}, {S['vg_hi']}"]
-    for pair, (blo, bhi), kb in ((S_GK0, (kglo, kghi), ka), (S_GK1, (kglo, kghi), kb_), (S_GV0, (vglo, vghi), ka),
-                                 (S_GV1, (vglo, vghi), kb_)):
-        n = int(pair[2:].split(":")[0])
-        top += [f"s_lshl_b32 {t2}, {kb}, 14", f"s_lshr_b32 {t3}, {kb}, 18",  # 64 rows x 256 bytes per kv tile
-                f"s_add_u32 s{n}, {blo}, {t2}", f"s_addc_u32 s{n + 1}, {bhi}, {t3}"]
+    for kb, bases in ((ka, (S_GK0, S_GV0)), (kb_, (S_GK1, S_GV1))):
+        # first row of the kv tile (64 kb; a ragged length's last tile starts early), 256 bytes a row
+        top += [f"s_lshl_b32 {t2}, {kb}, 6", f"s_min_u32 {t3}, {t2}, {S['klim']}",
+                f"s_lshl_b32 {t2}, {t3}, 8", f"s_lshr_b32 {t3}, {t3}, 24"]
+        for pair, (blo, bhi) in zip(bases, ((kglo, kghi), (vglo, vghi))):
+            n = int(pair[2:].split(":")[0])
+            top += [f"s_add_u32 s{n}, {blo}, {t2}", f"s_addc_u32 s{n + 1}, {bhi}, {t3}"]
     top += [
         f"s_xor_b32 {t1}, {S['buf']}, 1",
         f"s_lshl_b32 {t1}, {t1}, 16",

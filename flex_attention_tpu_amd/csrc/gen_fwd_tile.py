@@ -34,7 +34,7 @@ physical-register constraints):
     a[0:63], a[64:127]     O^T accumulators of q block 0, 1 (4 x 16 each)
     a[128:159], a[160:191] Q^T fragments of q block 0, 1 (8 x 4 each), pre-scaled
     a[192:255]             staging slots of the LDS fragments (clobbered)
-    v[66:199], s[60:100], vcc, m0   scratch of the run loop (clobbered)
+    v[66:199], s[59:100], vcc, m0   scratch of the run loop (clobbered)
     %[r0..r7]  byte address of the lane's row fragment ks in K half-tile 0 of the current buffer
     %[t0..t7]  byte address of the lane's transposed fragment (2 db + hi) in K half-tile 0 (the V
                tiles lie 32 KiB behind the K tiles)
@@ -73,10 +73,10 @@ SEQUENTIAL = True  # (plain scores) the S chains of the two q blocks one after t
 TILE = 16384
 # No scalar operands: constants come from a per-wave table in LDS, loop state from VGPR operands.
 TABLE = ["n_list", "w4k", "c2", "n_steps", "kg_lo", "kg_hi", "vg_lo", "vg_hi", "kban", "kbbn", "kgn_lo", "kgn_hi",
-         "vgn_lo", "vgn_hi", "pad0", "pad1"]
+         "vgn_lo", "vgn_hi", "klim", "pad1"]   # (klim: first row of the last kv tile at the latest)
 SREG = {"n_list": "s60", "w4k": "s61", "c2": "s62", "n_steps": "s63", "kg_lo": "s64", "kg_hi": "s65", "vg_lo": "s66",
         "vg_hi": "s67", "kban": "s68", "kbbn": "s69", "kgn_lo": "s70", "kgn_hi": "s71", "vgn_lo": "s78", "vgn_hi": "s79",
-        "pad0": "s80", "pad1": "s81",
+        "klim": "s59", "pad1": "s81",
         "it": "s72", "kba1": "s73", "kbb1": "s74", "buf": "s75", "it_end": "s76", "partial": "s77"}
 STATE_IO = ["it", "kba1", "kbb1", "buf"]
 STATE_IN = ["it_end", "partial"]
@@ -120,6 +120,7 @@ def bias_ops(e, c, q, tile):
     b = V_B[q]
     off = 32 * (c & 1) - 128 * q
     e.raw(f"s_lshl_b32 {t0}, {tile}, 6")
+    e.raw(f"s_min_u32 {t0}, {t0}, {SREG['klim']}")
     if off > 0:
         e.raw(f"s_add_u32 {t0}, {t0}, {off}")
     elif off < 0:
@@ -592,11 +593,13 @@ def run_loop(full, masked, alibi=False, softcap=False):
             f"s_cselect_b32 {ka}, {S['kban']}, {S['kba1']}", f"s_cselect_b32 {kb_}, {S['kbbn']}, {S['kbb1']}",
             f"s_cselect_b32 {kglo}, {S['kgn_lo']}, {S['kg_lo']}", f"s_cselect_b32 {kghi}, {S['kgn_hi']}, {S['kg_hi']}",
             f"s_cselect_b32 {vglo}, {S['vgn_lo']}, {S['vg_lo']}", f"s_cselect_b32 {vghi}, {S['vgn_hi']}, {S['vg_hi']}"]
-    for pair, (blo, bhi), kb in ((S_GK0, (kglo, kghi), ka), (S_GK1, (kglo, kghi), kb_), (S_GV0, (vglo, vghi), ka),
-                                 (S_GV1, (vglo, vghi), kb_)):
-        n = int(pair[2:].split(":")[0])
-        top += [f"s_lshl_b32 {t2}, {kb}, 14", f"s_lshr_b32 {t3}, {kb}, 18",  # 64 rows x 256 bytes per kv tile
-                f"s_add_u32 s{n}, {blo}, {t2}", f"s_addc_u32 s{n + 1}, {bhi}, {t3}"]
+    for kb, bases in ((ka, (S_GK0, S_GV0)), (kb_, (S_GK1, S_GV1))):
+        # first row of the kv tile (64 kb; a ragged length's last tile starts early), 256 bytes a row
+        top += [f"s_lshl_b32 {t2}, {kb}, 6", f"s_min_u32 {t3}, {t2}, {S['klim']}",
+                f"s_lshl_b32 {t2}, {t3}, 8", f"s_lshr_b32 {t3}, {t3}, 24"]
+        for pair, (blo, bhi) in zip(bases, ((kglo, kghi), (vglo, vghi))):
+            n = int(pair[2:].split(":")[0])
+            top += [f"s_add_u32 s{n}, {blo}, {t2}", f"s_addc_u32 s{n + 1}, {bhi}, {t3}"]
     top += [f"s_xor_b32 {t1}, {S['buf']}, 1", f"s_lshl_b32 {t1}, {t1}, 16", f"s_add_u32 {S_LDSN}, {t1}, {S['w4k']}",
             f"s_mov_b32 m0, {S_LDSN}",   # LDS destination of the step's first copy (the streams write the others)
             f"s_cmp_eq_u32 {S['partial']}, 0", "s_cbranch_scc1 .Lfa_fwd_full_%="]

@@ -30,7 +30,7 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
         check_rows(name, t, B, Hq, Sq, q.device)
     check_blocks(Sq, Sk, block_q=block_q, block_k_major=block_k_major, block_k=block_k,
                  block_q_major=block_q_major)
-    # ragged lengths: zero-padded to the kernels' tiles (padded rows carry l = 0 and dO = 0: they add nothing)
+    # (lengths below one tile: zero-padded to it; padded rows carry l = 0 and dO = 0, they add nothing)
     Sq_p, Sk_p = padded_len(Sq), padded_len(Sk)
     spec = resolve_mask(mask_fn, block_mask_fn, causal, segment_ids, Sq, Sk, Sq_p, Sk_p)
     check_doc_batches(spec, B)   # (ids of shape [B, S]: the kernels mask every batch entry by its own row)
@@ -46,7 +46,7 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
                    compiled_loop=compiled_loop, ab_c=ab_c)
     ds = None
     lib = library_for(score_fn, spec)
-    if _defer:   # (flex_attention_bwd launches this pass together with the dq pass: whole tiles only, no hand-over)
+    if _defer:   # (flex_attention_bwd launches this pass together with the dq pass: unpadded tensors only, no hand-over)
         if Sk_p != Sk or Sq_p != Sq or D != D_user or return_ds:
             return None
         return {"params": p, "lib": lib, "finish": lambda: (dk, dv), "keep": (q, k, v, do, l, m, di, ab_keep, bm)}

@@ -8,7 +8,7 @@ import torch
 
 from . import _lib
 from ._common import (on_device, bias_c, check_blocks, check_doc_batches, check_qkv, check_rows, dtype_code, kernel_block_map, kernel_head_dim, library_for,
-                      pad_seq, padded_len, mostly_partial_custom_mask, resolve_mask, score_spec_c, stream_of, tagged_closures)
+                      pad_seq, padded_len, mostly_partial_custom_mask, resolve_mask, score_spec_c, stream_of, tagged_closures, tile_lengths)
 from .block_mask import mask_spec_c
 
 
@@ -94,11 +94,12 @@ def bwd_params(q, k, v, l, m, do, d, sm_scale, score_fn, spec, bm, mod_q, mod_k,
                compiled_loop=False, ab_c=None):
     B, Hq, Sq, D = q.shape
     _, Hkv, Sk, _ = k.shape
+    Sq_c, Sk_c, pad = tile_lengths(bm)
     return _lib.BwdParamsC(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(), l.data_ptr(), m.data_ptr(), d.data_ptr(),
         dq.data_ptr() if dq is not None else None,
         dk.data_ptr() if dk is not None else None, dv.data_ptr() if dv is not None else None,
-        B, Hq, Hkv, Sq, Sk, D, dtype_code(q), float(sm_scale), _lib.FLAG_COMPILED_LOOP if compiled_loop else 0, 0,
+        B, Hq, Hkv, Sq_c, Sk_c, D, dtype_code(q), float(sm_scale), _lib.FLAG_COMPILED_LOOP if compiled_loop else 0, pad,
         score_spec_c(score_fn, Hq, q.device, mod_q, mod_k, sm_scale), mask_spec_c(spec, Sq, Sk, q.device), bm.as_c(),
         ab_c if ab_c is not None else _lib.BiasC())
 
@@ -132,7 +133,7 @@ def flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, d, *, block_b, 
     for name, t in (("l", l), ("m", m), ("d", d)):
         check_rows(name, t, B, Hq, Sq, q.device)
     check_blocks(Sq, Sk, block_q=block_q, block_k_major=block_k_major, block_k=block_k)
-    # ragged lengths: zero-padded to the kernels' tiles (padded rows carry l = 0: their probabilities vanish)
+    # (lengths below one tile: zero-padded to it; padded rows carry l = 0, their probabilities vanish)
     Sq_p, Sk_p = padded_len(Sq), padded_len(Sk)
     spec = resolve_mask(mask_fn, block_mask_fn, causal, segment_ids, Sq, Sk, Sq_p, Sk_p)
     check_doc_batches(spec, B)   # (ids of shape [B, S]: the kernels mask every batch entry by its own row)

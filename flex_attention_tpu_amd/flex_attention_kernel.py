@@ -13,7 +13,7 @@ import torch
 
 from . import _lib
 from ._common import (on_device, bias_c, check_blocks, check_doc_batches, check_qkv, dtype_code, kernel_block_map, kernel_head_dim, library_for, pad_seq,
-                      padded_len, mostly_partial_custom_mask, resolve_mask, score_spec_c, stream_of, tagged_closures)
+                      padded_len, mostly_partial_custom_mask, resolve_mask, score_spec_c, stream_of, tagged_closures, tile_lengths)
 from .block_mask import mask_spec_c
 
 
@@ -31,8 +31,8 @@ def _flex_attention_impl(q, k, v, ab, segment_ids, save_residuals, causal, sm_sc
     B, Hq, Hkv, Sq, Sk, D = check_qkv(q, k, v)
     check_blocks(Sq, Sk, block_q=block_q, block_k_major=block_k_major, block_k=block_k)
     score_fn, mask_fn, block_mask_fn = tagged_closures(score_fn, mask_fn, block_mask_fn, block_q, block_k_major)
-    # ragged lengths: the tensors are zero-padded to the kernels' tiles, a key bound drops the padded keys
-    # and the padded query rows are cut off again
+    # (lengths below one tile: the tensors are zero-padded to it, a document id of their own drops the padded keys
+    # and the padded query rows are cut off again)
     Sq_p, Sk_p = padded_len(Sq), padded_len(Sk)
     spec = resolve_mask(mask_fn, block_mask_fn, causal, segment_ids, Sq, Sk, Sq_p, Sk_p)
     check_doc_batches(spec, B)   # (ids of shape [B, S]: the kernels mask every batch entry by its own row)
@@ -47,10 +47,11 @@ def _flex_attention_impl(q, k, v, ab, segment_ids, save_residuals, causal, sm_sc
     if save_residuals:
         l = torch.empty(B, Hq, Sq_p, dtype=torch.float32, device=q.device)
         m = torch.empty(B, Hq, Sq_p, dtype=torch.float32, device=q.device)
+    Sq_c, Sk_c, pad = tile_lengths(bm)
     p = _lib.FwdParamsC(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
         l.data_ptr() if l is not None else None, m.data_ptr() if m is not None else None,
-        B, Hq, Hkv, Sq_p, Sk_p, D, dtype_code(q), float(sm_scale), _lib.FLAG_COMPILED_LOOP if compiled_loop else 0, 0,
+        B, Hq, Hkv, Sq_c, Sk_c, D, dtype_code(q), float(sm_scale), _lib.FLAG_COMPILED_LOOP if compiled_loop else 0, pad,
         score_spec_c(score_fn, Hq, q.device, block_q or 1, block_k or 1, sm_scale),
         mask_spec_c(spec, Sq_p, Sk_p, q.device), bm.as_c(), ab_c)
     with on_device(q.device):

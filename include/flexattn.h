@@ -120,6 +120,12 @@ typedef struct flexattn_bias {
  * for a call, for comparisons and tests. */
 #define FLEXATTN_FLAG_COMPILED_LOOP 1
 
+/* Ragged sequence lengths.  Sq and Sk of a call are multiples of the pass's tiles (flexattn_tile_shape); tensors whose
+ * lengths are not name the next multiples and the rows by which these exceed them: the tensors, the row vectors, the
+ * bias and the document arrays have Sq - pad_q resp. Sk - pad_k rows (at least one tile each, pads below a tile), and
+ * nothing beyond them is read or written.  The block map of such a call is flexattn_build_block_mask_ragged's. */
+#define FLEXATTN_PAD(pad_q, pad_k) ((pad_q) | ((pad_k) << 16))
+
 typedef struct flexattn_fwd_params {
   const void* q; const void* k; const void* v; /* in  */
   void* o;                                      /* out [B,Hq,Sq,D], dtype of q */
@@ -128,7 +134,7 @@ typedef struct flexattn_fwd_params {
   int32_t dtype;
   float sm_scale; /* > 0 */
   int32_t flags;  /* FLEXATTN_FLAG_* */
-  int32_t reserved;
+  int32_t pad;    /* FLEXATTN_PAD(...), 0 for lengths that are multiples of the tiles */
   flexattn_score_spec score;
   flexattn_mask_spec mask;
   flexattn_block_map map; /* granularity must equal flexattn_tile_shape(FLEXATTN_PASS_FWD, ...) */
@@ -155,7 +161,7 @@ typedef struct flexattn_bwd_params {
   int32_t dtype;
   float sm_scale; /* > 0 */
   int32_t flags;  /* FLEXATTN_FLAG_* */
-  int32_t reserved;
+  int32_t pad;    /* FLEXATTN_PAD(...), 0 for lengths that are multiples of the tiles */
   flexattn_score_spec score;
   flexattn_mask_spec mask;
   flexattn_block_map map; /* granularity of the pass being launched */
@@ -210,6 +216,13 @@ int flexattn_build_block_mask(const flexattn_mask_spec* mask, int32_t Sq, int32_
                               int32_t block_q, int32_t block_k, uint8_t* state,
                               int32_t* kv_cnt, int32_t* kv_idx, int32_t* q_cnt, int32_t* q_idx,
                               void* stream);
+
+/* The same for sequence lengths that are no multiples of the blocks: ceil(Sq / block_q) x ceil(Sk / block_k) tiles, the
+ * last ones cut off at the lengths; a tile cut off at Sk is at most partial. */
+int flexattn_build_block_mask_ragged(const flexattn_mask_spec* mask, int32_t Sq, int32_t Sk,
+                                     int32_t block_q, int32_t block_k, uint8_t* state,
+                                     int32_t* kv_cnt, int32_t* kv_idx, int32_t* q_cnt, int32_t* q_idx,
+                                     void* stream);
 
 /* Forward.  Replaces the pallas_call in _flex_attention_impl (flex_attention_kernel.py:173-187). */
 int flexattn_fwd(const flexattn_fwd_params* p, void* stream);
