@@ -200,7 +200,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
       issue_tile(it + 1, qbn, buf ^ 1);
     }
     const int q0 = tile_base(qb, BQ, a.Sq);
-    const int q_first = qb * BQ;   // (rows before it belong to the q tile before)
+    // (elements before this offset belong to the q tile before; a column of the kv tile before owns none)
+    const int own = own_col ? qb * BQ - q0 - 4 * hh : 1 << 20;
 #pragma unroll
     for (int cc = 0; cc < 4; ++cc) {
       const int c = cc & 1;  // 32-row block inside the 64-row LDS tile cc >> 1
@@ -262,7 +263,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
             float pe = fast_exp2(tv + sm.bias2(i, k_idx) - lse4[u]);
             float gd = pe * (dp_acc[e] - dl4[u]) * sm.dfactor(tv, s_acc[e], i, k_idx);
             if (MASKED) {
-              const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j) & (i >= q_first) & own_col;
+              const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j) & (32 * cc + 8 * g4 + u >= own);
               pe = keep ? pe : 0.f;
               gd = keep ? gd : 0.f;
             }
@@ -459,7 +460,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
       issue_tile(it + 1, qbn, buf ^ 1);
     }
     const int q0 = tile_base(qb, BQ, a.Sq) + (it & 1) * HQ;
-    const int q_first = qb * BQ;   // (rows before it belong to the q tile before)
+    // (elements before this offset belong to the q tile before; a column of the kv tile before owns none)
+    const int own = own_col ? qb * BQ - q0 - 4 * hh : 1 << 20;
     const char* qt = reinterpret_cast<const char*>(sQ + buf * NP * kTileElems);
     const char* dot = reinterpret_cast<const char*>(sDO + buf * NP * kTileElems);
 #pragma unroll 1   // (rolled: unrolled, the second block's operand loads are hoisted over the first block's and 72 registers spill; 2.72 -> 2.01 ms on B=4, H=16, S=4096)
@@ -510,7 +512,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
             float pe = fast_exp2(tv + sm.bias2(i, k_idx) - lse4[u]);
             float gd = pe * (dp_acc[e] - dl4[u]) * sm.dfactor(tv, s_acc[e], i, k_idx);
             if (MASKED) {
-              const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j) & (i >= q_first) & own_col;
+              const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j) & (8 * g4 + u >= own - 32 * c);
               pe = keep ? pe : 0.f;
               gd = keep ? gd : 0.f;
             }

@@ -179,7 +179,6 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
       }
     }
     const int kv0 = tile_base(kb, BN, a.Sk);
-    const int kv_first = kb * BN;   // (keys before it belong to the tile before)
     const char* kt = reinterpret_cast<const char*>(sK + buf * NP * kTileElems);
     const char* vt = reinterpret_cast<const char*>(sV + buf * NP * kTileElems);
 
@@ -224,6 +223,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
       auto elementwise = [&](auto masked) {
         constexpr bool MASKED = decltype(masked)::value;
         const bool has_doc = MASKED && (mk.flags & FLEXATTN_MASK_DOC) != 0;
+        const int own = kb * BN - kv0 - 32 * c - 4 * hh;   // (elements before this offset belong to the tile before)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const int j0 = kv0 + 32 * c + 8 * g + 4 * hh;
@@ -232,32 +232,26 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
             const auto d4 = *reinterpret_cast<const i32x4_a4*>(mk.doc_k + j0);
             dj[0] = d4[0]; dj[1] = d4[1]; dj[2] = d4[2]; dj[3] = d4[3];
           }
+          const f32x4 bias = sm.bias2x4(q_idx, j0);
           float dsv[4];
           f32x4 gb;   // the gradient with respect to the logits themselves: what an additive bias receives
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const int e = 4 * g + u;
             const float tv = sm.to_log2(s_acc[e], q_idx, j0 + u);
-            const float pe = fast_exp2(tv + sm.bias2(q_idx, j0 + u) - lse2);
+            const float pe = fast_exp2(tv + bias[u] - lse2);
             float gl = pe * (dp_acc[e] - delta);
             float gd = gl * sm.dfactor(tv, s_acc[e], q_idx, j0 + u);
             if (MASKED) {   // (selected, not multiplied: a score function may return anything at a dropped element)
-              const bool keep = keep_elem(mk, q_idx, j0 + u, doc_i, dj[u]) & (j0 + u >= kv_first);
+              const bool keep = keep_elem(mk, q_idx, j0 + u, doc_i, dj[u]);
               gl = keep ? gl : 0.f;
-              gd = keep ? gd : 0.f;
+              gd = keep & (8 * g + u >= own) ? gd : 0.f;
             }
             gb[u] = gl;
             dsv[u] = gd;
           }
-          if (dab_row != nullptr) {
-            if (!MASKED || j0 >= kv_first) {
-              *reinterpret_cast<f32x4_a4*>(dab_row + j0) = gb;
-            } else {
-#pragma unroll
-              for (int u = 0; u < 4; ++u)
-                if (j0 + u >= kv_first) dab_row[j0 + u] = gb[u];
-            }
-          }
+          // (elements of the tile before get the value that tile stores, too: the same products in the same order)
+          if (dab_row != nullptr) *reinterpret_cast<f32x4_a4*>(dab_row + j0) = gb;
           const bf16x2 d01 = pack_bf16(dsv[0], dsv[1]), d23 = pack_bf16(dsv[2], dsv[3]);
           const int o = 4 * (g & 1);
           ds[g >> 1][o] = d01[0]; ds[g >> 1][o + 1] = d01[1]; ds[g >> 1][o + 2] = d23[0]; ds[g >> 1][o + 3] = d23[1];

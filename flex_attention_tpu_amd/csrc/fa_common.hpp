@@ -35,6 +35,7 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 // (16 bytes of a row whose start is aligned to 4 bytes only)
 typedef unsigned int u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef int i32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned short u16x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr float kLog2e = 1.4426950408889634f;
@@ -460,6 +461,25 @@ struct ScoreMod {
     const float v = ab_f32 ? reinterpret_cast<const float*>(ab_base)[at]
                            : __builtin_bit_cast(float, (unsigned)reinterpret_cast<const unsigned short*>(ab_base)[at] << 16);
     return v * kLog2e;
+  }
+
+  // The same of the elements (i, j0 .. j0 + 3): one 16-byte (bf16: 8-byte) load, of any alignment.  (Four loads at
+  // j0 + u, u = 0..3, each take an address of their own in registers, because j0 + u is a 32-bit sum: 32 of them per
+  // tile made the kernels spill.)
+  __device__ __forceinline__ f32x4 bias2x4(int i, int j0) const {
+    f32x4 r = {0.f, 0.f, 0.f, 0.f};
+    if (ab_base == nullptr) return r;
+    const unsigned long long at = (unsigned long long)(unsigned)(ab_row0 + i) * (unsigned)ab_ld + (unsigned)j0;
+    if (ab_f32) {
+      r = *reinterpret_cast<const f32x4_a4*>(reinterpret_cast<const float*>(ab_base) + at);
+    } else {
+      const u16x4_a2 v = *reinterpret_cast<const u16x4_a2*>(reinterpret_cast<const unsigned short*>(ab_base) + at);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) r[u] = __builtin_bit_cast(float, (unsigned)v[u] << 16);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) r[u] *= kLog2e;
+    return r;
   }
 
   // d(s')/d(raw) in natural units, from the log2-domain modified logit t.

@@ -237,43 +237,61 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
     // For the plain score the running maximum is kept on the raw dot products and the scale is
     // folded into the exponent (one FMA per element); score mods go through the log2-domain logit.
     const int kv0 = tile_base(kb, BN, a.Sk);
-    const int kv_first = kb * BN;   // (keys before it belong to the tile before)
     constexpr bool kPlain = (SCORE == FLEXATTN_SCORE_NONE);
     float m_tile = kNegInf;
     if (!partial) {
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          if (!kPlain) {
-            const int j = kv0 + 32 * c + acc_row(e, hh);
-            s_acc[c][e] = sm.to_log2(s_acc[c][e], q_idx, j) + sm.bias2(q_idx, j);
+        for (int g = 0; g < 4; ++g) {
+          const int j0 = kv0 + 32 * c + 8 * g + 4 * hh;
+          f32x4 bias;
+          if (!kPlain) bias = sm.bias2x4(q_idx, j0);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int e = 4 * g + u;
+            if (!kPlain) s_acc[c][e] = sm.to_log2(s_acc[c][e], q_idx, j0 + u) + bias[u];
+            m_tile = fmaxf(m_tile, s_acc[c][e]);
           }
-          m_tile = fmaxf(m_tile, s_acc[c][e]);
         }
       }
     } else {
       // the lane's kv indices come in runs of 4: kv0 + 32c + 8g + 4hh + {0..3}
+      int kv0_here = kv0;   // (a copy: shared with the other branch, what depends on a key index alone is kept in 32 registers)
+      asm volatile("" : "+s"(kv0_here));
       const bool has_doc = (mk.flags & FLEXATTN_MASK_DOC) != 0;
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          const int j0 = kv0 + 32 * c + 8 * g + 4 * hh;
+          const int j0 = kv0_here + 32 * c + 8 * g + 4 * hh;
           int dj[4] = {0, 0, 0, 0};
           if (has_doc) {
             const auto d4 = *reinterpret_cast<const i32x4_a4*>(mk.doc_k + j0);
             dj[0] = d4[0]; dj[1] = d4[1]; dj[2] = d4[2]; dj[3] = d4[3];
           }
+          f32x4 bias;
+          if (!kPlain) bias = sm.bias2x4(q_idx, j0);
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const int e = 4 * g + u;
-            float tv = kPlain ? s_acc[c][e] : sm.to_log2(s_acc[c][e], q_idx, j0 + u) + sm.bias2(q_idx, j0 + u);
-            tv = (keep_elem(mk, q_idx, j0 + u, doc_i, dj[u]) & (j0 + u >= kv_first)) ? tv : kNegInf;
+            float tv = kPlain ? s_acc[c][e] : sm.to_log2(s_acc[c][e], q_idx, j0 + u) + bias[u];
+            tv = keep_elem(mk, q_idx, j0 + u, doc_i, dj[u]) ? tv : kNegInf;
             s_acc[c][e] = tv;
             m_tile = fmaxf(m_tile, tv);
           }
         }
+      }
+      if (kv0 != kb * BN) {   // (a last tile that starts early: its first elements belong to the tile before)
+        const int own = kb * BN - kv0 - 4 * hh;
+        m_tile = kNegInf;
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            s_acc[c][e] = 32 * c + 8 * (e >> 2) + (e & 3) >= own ? s_acc[c][e] : kNegInf;
+            m_tile = fmaxf(m_tile, s_acc[c][e]);
+          }
       }
     }
     m_tile = half_max(m_tile);
