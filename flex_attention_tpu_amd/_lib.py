@@ -148,6 +148,8 @@ EXPORTS = (
     "flexattn_build_ds_index",
     "flexattn_fwd",
     "flexattn_fwd_noalloc",
+    "flexattn_fwd_decode_bytes",
+    "flexattn_fwd_decode",
     "flexattn_bwd_delta",
     "flexattn_bwd_ds_bytes",
     "flexattn_bwd_dq",
@@ -172,6 +174,9 @@ def _bind(lib: C.CDLL) -> C.CDLL:
     lib.flexattn_build_ds_index.argtypes = [C.POINTER(BlockMapC), C.c_void_p, C.c_void_p, C.c_void_p]
     lib.flexattn_fwd.argtypes = [C.POINTER(FwdParamsC), C.c_void_p]
     lib.flexattn_fwd_noalloc.argtypes = [C.POINTER(FwdParamsC), C.c_void_p]
+    lib.flexattn_fwd_decode_bytes.argtypes = [C.POINTER(FwdParamsC)]
+    lib.flexattn_fwd_decode_bytes.restype = C.c_int64
+    lib.flexattn_fwd_decode.argtypes = [C.POINTER(FwdParamsC), C.c_void_p, C.c_int64, C.c_void_p]
     lib.flexattn_bwd_delta.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int32, C.c_int32, C.c_void_p]
     lib.flexattn_bwd_dq.argtypes = [C.POINTER(BwdParamsC), C.c_void_p]
     lib.flexattn_bwd_ds_bytes.argtypes = [C.POINTER(BwdParamsC)]
@@ -179,7 +184,7 @@ def _bind(lib: C.CDLL) -> C.CDLL:
     lib.flexattn_bwd_dkv.argtypes = [C.POINTER(BwdParamsC), C.c_void_p]
     lib.flexattn_bwd.argtypes = [C.POINTER(BwdParamsC), C.POINTER(BwdParamsC), C.c_void_p]
     for name in ("flexattn_tile_shape", "flexattn_build_block_mask", "flexattn_build_block_mask_ragged", "flexattn_build_ds_index", "flexattn_fwd",
-                 "flexattn_fwd_noalloc", "flexattn_bwd_delta", "flexattn_bwd_dq", "flexattn_bwd_dkv", "flexattn_bwd"):
+                 "flexattn_fwd_noalloc", "flexattn_fwd_decode", "flexattn_bwd_delta", "flexattn_bwd_dq", "flexattn_bwd_dkv", "flexattn_bwd"):
         getattr(lib, name).restype = C.c_int
     return lib
 

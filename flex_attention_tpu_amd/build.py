@@ -19,6 +19,7 @@ SOURCES = [
     "attn_f32.hip",
     "attn_f32_mfma.hip",
     "fwd_bf16.hip",
+    "fwd_decode.hip",
     "bwd_dq_bf16.hip",
     "bwd_dkv_bf16.hip",
     "bwd_dq_ds.hip",

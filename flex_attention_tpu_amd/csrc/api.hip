@@ -445,6 +445,32 @@ int flexattn_fwd_noalloc(const flexattn_fwd_params* p, void* stream) {
   return fwd_with_map(p, map, s);
 }
 
+static bool decode_ok(const flexattn_fwd_params* p) {
+  return p != nullptr && p->score.kind == FLEXATTN_SCORE_NONE && p->mask.flags == 0 && p->ab.ptr == nullptr && p->pad == 0 &&
+         p->flags == 0 && fwd_decode_ok(p->dtype, p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->D);
+}
+
+int64_t flexattn_fwd_decode_bytes(const flexattn_fwd_params* p) {
+  return decode_ok(p) ? fwd_decode_bytes(p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->D) : -1;
+}
+
+int flexattn_fwd_decode(const flexattn_fwd_params* p, void* work, int64_t work_bytes, void* stream) {
+  if (p == nullptr) return set_error(FLEXATTN_EINVAL, "params is NULL");
+  if (!p->q || !p->k || !p->v || !p->o) return set_error(FLEXATTN_EINVAL, "q, k, v or o is NULL");
+  if ((p->l == nullptr) != (p->m == nullptr)) return set_error(FLEXATTN_EINVAL, "l and m must both be given or both NULL");
+  if (!decode_ok(p)) return set_error(FLEXATTN_ENOTSUP, "not a request of flexattn_fwd_decode (flexattn_fwd_decode_bytes is -1)");
+  const int rc = check_scale_flags(p->sm_scale, p->flags);
+  if (rc != FLEXATTN_OK) return rc;
+  const int64_t need = fwd_decode_bytes(p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->D);
+  if (need > 0 && (work == nullptr || work_bytes < need))
+    return set_error(FLEXATTN_EINVAL, "work holds %lld bytes, the request needs %lld", (long long)(work ? work_bytes : 0), (long long)need);
+  FwdArgs a{};
+  a.q = p->q; a.k = p->k; a.v = p->v; a.o = p->o; a.l = p->l; a.m = p->m;
+  a.B = p->B; a.Hq = p->Hq; a.Hkv = p->Hkv; a.Sq = p->Sq; a.Sk = p->Sk;
+  a.sm_scale = p->sm_scale;
+  return fwd_decode(a, p->D, work, static_cast<hipStream_t>(stream));
+}
+
 int flexattn_bwd_delta(const void* o, const void* dout, float* delta, int64_t rows, int32_t D, int32_t dtype,
                        void* stream) {
   if (!o || !dout || !delta) return set_error(FLEXATTN_EINVAL, "o, dout or delta is NULL");

@@ -16,6 +16,10 @@ int check_launch(const char* what);
 int fwd_bf16_d128(const FwdArgs& a, hipStream_t stream);
 int fwd_bf16_d256(const FwdArgs& a, hipStream_t stream);   // (same tiles as head dim 128)
 void fwd_bf16_d128_tile(int* bq, int* bk);
+// few query rows against long keys, plain scores, no mask (head dim 64 or 128)
+bool fwd_decode_ok(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D);
+int64_t fwd_decode_bytes(int B, int Hq, int Hkv, int Sq, int Sk, int D);
+int fwd_decode(const FwdArgs& a, int D, void* work, hipStream_t stream);
 int bwd_dq_bf16_d128(const BwdArgs& a, hipStream_t stream);
 int bwd_dq_bf16_d256(const BwdArgs& a, hipStream_t stream);
 void bwd_dq_bf16_d128_tile(int* bq, int* bk);

@@ -14,7 +14,38 @@ import torch
 from . import _lib
 from ._common import (on_device, bias_c, check_blocks, check_doc_batches, check_qkv, dtype_code, kernel_block_map, kernel_head_dim, library_for, pad_seq,
                       padded_len, mostly_partial_custom_mask, resolve_mask, score_spec_c, stream_of, tagged_closures, tile_lengths)
-from .block_mask import mask_spec_c
+from .block_mask import mask_spec_c, spec_of
+
+
+def _decode(q, k, v, mask_fn, block_mask_fn, save_residuals, sm_scale):
+    """The forward of a few query rows against long keys without mask, bias or score function, or None where the
+    kernel for it does not take the call.  Nothing is padded to the 128 rows of the other kernels' tiles, and the query
+    heads of a kv head share its keys (fwd_decode.hip; B=8, Hq=32, Hkv=8, one query, 6001 keys, D=128: 198 -> 41 us).  The
+    line at 128 query rows per kv head: 1935 -> 310 us there (B=32, Hq=64, Hkv=8, 16 queries, 8192 keys); beyond it the
+    other kernels' tiles fill."""
+    B, Hq, Sq, D = q.shape
+    _, Hkv, Sk, _ = k.shape
+    if q.dtype != torch.bfloat16 or D > 128 or Hq // Hkv * Sq > 128 or spec_of(mask_fn, block_mask_fn).flags:
+        return None
+    D_user, D = D, 64 if D <= 64 else 128
+    q, k, v = pad_seq(q, D, 3), pad_seq(k, D, 3), pad_seq(v, D, 3)
+    o = torch.empty_like(q)
+    l = m = None
+    if save_residuals:
+        l = torch.empty(B, Hq, Sq, dtype=torch.float32, device=q.device)
+        m = torch.empty_like(l)
+    p = _lib.FwdParamsC(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), l.data_ptr() if l is not None else None,
+                        m.data_ptr() if m is not None else None, B, Hq, Hkv, Sq, Sk, D, _lib.BF16, float(sm_scale))
+    lib = _lib.load()
+    with on_device(q.device):
+        need = lib.flexattn_fwd_decode_bytes(C.byref(p))
+        if need < 0:
+            return None
+        work = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
+        _lib.check(lib.flexattn_fwd_decode(C.byref(p), work.data_ptr() if need else None, need, stream_of(q)), lib)
+    if D != D_user:
+        o = o[..., :D_user].contiguous()
+    return (o, l, m) if save_residuals else o
 
 
 def _flex_attention_impl(q, k, v, ab, segment_ids, save_residuals, causal, sm_scale, block_b, block_q,
@@ -31,6 +62,12 @@ def _flex_attention_impl(q, k, v, ab, segment_ids, save_residuals, causal, sm_sc
     B, Hq, Hkv, Sq, Sk, D = check_qkv(q, k, v)
     check_blocks(Sq, Sk, block_q=block_q, block_k_major=block_k_major, block_k=block_k)
     score_fn, mask_fn, block_mask_fn = tagged_closures(score_fn, mask_fn, block_mask_fn, block_q, block_k_major)
+    if score_fn is None and ab is None and segment_ids is None and not causal and not compiled_loop and Sq < 128 <= Sk:
+        out = _decode(q, k, v, mask_fn, block_mask_fn, save_residuals, sm_scale)
+        if out is not None:
+            if debug:
+                print(f"[flexattn_fwd_decode] B={B} Hq={Hq} Hkv={Hkv} Sq={Sq} Sk={Sk} D={D} dtype={q.dtype}")
+            return out
     # (lengths below one tile: the tensors are zero-padded to it, a document id of their own drops the padded keys
     # and the padded query rows are cut off again)
     Sq_p, Sk_p = padded_len(Sq), padded_len(Sk)

@@ -240,6 +240,15 @@ int flexattn_fwd(const flexattn_fwd_params* p, void* stream);
  * serialised by the caller. */
 int flexattn_fwd_noalloc(const flexattn_fwd_params* p, void* stream);
 
+/* Forward for few query rows against long keys (token generation; the reference has no kernel of its own for it): the
+ * query heads of a kv head share one pass over its keys, which is split over work-groups.  Takes bf16 at head dimension
+ * 64 or 128, plain scores, no mask, no bias, flags and pad 0, at most 128 query rows per kv head (Sq Hq / Hkv), any Sk
+ * of at least 32 (head dimension 64: 64) keys; p->map is not read.  flexattn_fwd_decode_bytes returns the bytes of
+ * device memory (float32 sums of the splits, 16-byte aligned) that the request needs as `work`, which may be 0, or -1
+ * for a request that the call does not take; it looks at shapes, dtype, score, mask flags, bias, flags and pad only. */
+int64_t flexattn_fwd_decode_bytes(const flexattn_fwd_params* p);
+int flexattn_fwd_decode(const flexattn_fwd_params* p, void* work, int64_t work_bytes, void* stream);
+
 /* delta_i = sum_c o_ic * do_ic in float32.  Replaces the caller-side reduction at
  * flex_attention_dq_bwd.py:932 and flash_attention_dkv_bwd.py:925.  rows = B*Hq*Sq. */
 int flexattn_bwd_delta(const void* o, const void* dout, float* delta, int64_t rows, int32_t D,
