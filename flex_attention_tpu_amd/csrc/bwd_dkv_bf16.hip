@@ -617,9 +617,12 @@ static int launch_dkv_wide(const BwdArgs& a, hipStream_t stream) {
 // kv tile's list) 32 KB (the index of flexattn_build_ds_index: skipped pairs take no room); inside a block wave w
 // (kv columns 32 w + L % 32) writes 1 KB per (32-row q block c, 16-row half u) at 8192 w + 1024 (2 c + u), lane L
 // its 8 values (rows 8 (e / 4) + 4 (L / 32) + e % 4 of the half) at 16 (2 (L % 32) + L / 32).  bwd_dq_ds.hip reads it.
-template <int SCORE, bool DOCS, bool EXPORT = false>
+// HD: head dimension 128, or 64 (plain scores without export; see the forward).
+template <int SCORE, bool DOCS, bool EXPORT = false, int HD = 128>
 __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs a) {
   using namespace dkv_cfg;
+  constexpr int D = HD;
+  static_assert(HD == 128 || (SCORE == FLEXATTN_SCORE_NONE && !EXPORT), "streams of head dimension 64: plain scores");
   static_assert(!(EXPORT && SCORE == FLEXATTN_SCORE_ALIBI), "the position-bias streams keep the key's share out of dS");
   constexpr bool ALIBI = SCORE == FLEXATTN_SCORE_ALIBI;
   constexpr bool SOFTCAP = SCORE == FLEXATTN_SCORE_SOFTCAP;
@@ -649,7 +652,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
   const bool lse_wave = w < 2;
   int* sIdx = reinterpret_cast<int*>(sDl + 2 * BQ) + 4 * 32;
   unsigned char* sPart = reinterpret_cast<unsigned char*>(sIdx + MAX_LIST);  // by q tile: 1 = partial with this kv tile
-  TileLoader<4> loader;
+  TileLoader<4, HD> loader;
   loader.init(w, lane);
 
   // An item is kv tile kb of (batch, kv head) pair bhk.  Its addresses are cheap to derive from the
@@ -714,8 +717,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
     const int tid_here = opaque(tid);
     const bf16_t* Kg = static_cast<const bf16_t*>(a.k) + kv_offset(g);
     const bf16_t* Vg = static_cast<const bf16_t*>(a.v) + kv_offset(g);
-    rows_load(r.k, Kg + (size_t)(tid_here >> 6) * 32 * D, tid_here & 63);
-    rows_load(r.v, Vg + (size_t)(tid_here >> 6) * 32 * D, tid_here & 63);
+    rows_load<HD>(r.k, Kg + (size_t)(tid_here >> 6) * 32 * D, tid_here & 63);
+    rows_load<HD>(r.v, Vg + (size_t)(tid_here >> 6) * 32 * D, tid_here & 63);
     const size_t dk_rows = doc_rows(g.bhk, a.Sk);
     r.doc = (a.mask.flags & FLEXATTN_MASK_DOC) ? a.mask.doc_k[dk_rows + kv_base(g) + kv_local] : 0;
     if constexpr (DOCS) {
@@ -750,8 +753,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
   auto consume = [&](const ItemRegs& r, ItemHead& c, char* stage) {
     u32x4 kw[8], vw[8];
     const int lane_here = opaque(lane);
-    rows_to_fragments(r.k, stage, lane_here, kw);
-    rows_to_fragments(r.v, stage + 8192, lane_here, vw);
+    rows_to_fragments<HD>(r.k, stage, lane_here, kw);
+    rows_to_fragments<HD>(r.v, stage + 8192, lane_here, vw);
 #define FA_PUT(KS, KR, VR)                                                                                    \
   asm volatile(FA_DKV_PUT_KV_##KS                                                                             \
                : "={" KR "}"(st.k[KS]), "={" VR "}"(st.v[KS])                                                 \
@@ -1018,6 +1021,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
                  [m1] "v"(km[1]), [tid4] "v"(tid4), [c2v] "v"(c2), ##__VA_ARGS__                                                \
                : "memory", "scc", "vcc", "m0", FA_DKV_RUN_SGPRS, "v67", FA_DKV_TILE_CLOBBERS CLOB_MORE)
 #define FA_DKV_ALIBI_CLOBBERS , "s101"
+#define FA_DKV_D64_CLOBBERS , "v200", "v201", "v202", "v203"
 #define FA_DKV_DS_CLOBBERS , "s52", "s53", "s54", "s55", "s56", "s57", "s58", "s59"
     if constexpr (EXPORT) {
       // dS block of step `it` (head it / n_tiles of the group, place p0 in the q list) and the lane's place in
@@ -1038,11 +1042,12 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
       const float k2 = -2.f * cap2;
       FA_DKV_CALL(FA_DKV_RUN_SOFTCAP, FA_DKV_ALIBI_CLOBBERS, [k2] "v"(k2));
     } else {
-      FA_DKV_CALL(FA_DKV_RUN, );
+      if constexpr (HD == 64) { FA_DKV_CALL(FA_DKV_RUN_D64, FA_DKV_D64_CLOBBERS); } else { FA_DKV_CALL(FA_DKV_RUN, ); }
     }
 #undef FA_DKV_CALL
 #undef FA_DKV_DS_CLOBBERS
 #undef FA_DKV_ALIBI_CLOBBERS
+#undef FA_DKV_D64_CLOBBERS
     it = __builtin_amdgcn_readfirstlane(it);
     p1 = __builtin_amdgcn_readfirstlane(p1);
     buf = __builtin_amdgcn_readfirstlane(buf);
@@ -1062,7 +1067,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
     const int row_here = lane_here & 31;
     const unsigned wr = (unsigned)row_here * 256u + 8u * (unsigned)(lane_here >> 5);
 #define FA_GET(T, SRC, REG, MAT, DB, SCALE)                                                                        \
-  {                                                                                                                \
+  if constexpr (32 * DB < HD) {                                                                                                                \
     float x[16];                                                                                                   \
     asm volatile(FA_DKV_GET_ACC_##T                                                                                \
                  : "=v"(x[0]), "=v"(x[1]), "=v"(x[2]), "=v"(x[3]), "=v"(x[4]), "=v"(x[5]), "=v"(x[6]), "=v"(x[7]), \
@@ -1089,18 +1094,9 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
     __builtin_amdgcn_wave_barrier();
     bf16_t* dKg = static_cast<bf16_t*>(a.dk) + kv_off + (size_t)(w * 32) * D;
     bf16_t* dVg = static_cast<bf16_t*>(a.dv) + kv_off + (size_t)(w * 32) * D;
-    const int chunk = lane_here & 15;
     const int r_first = kb * BNK - k0 - w * 32;   // (rows before it belong to the kv tile before)
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int r = 4 * i + (lane_here >> 4);
-      if (r < r_first) continue;
-      const unsigned rd = (unsigned)r * 256u + (unsigned)((chunk ^ (r & 15)) << 4);
-      const u32x4 kx = *reinterpret_cast<const u32x4*>(stage + rd);
-      const u32x4 vx = *reinterpret_cast<const u32x4*>(stage + 8192 + rd);
-      *reinterpret_cast<u32x4*>(dKg + (size_t)r * D + chunk * 8) = kx;
-      *reinterpret_cast<u32x4*>(dVg + (size_t)r * D + chunk * 8) = vx;
-    }
+    rows_store<HD>(stage, dKg, lane_here, r_first);
+    rows_store<HD>(stage + 8192, dVg, lane_here, r_first);
   }
   geo = geo_n;
   }  // work items
@@ -1125,10 +1121,10 @@ static int launch_dkv(const BwdArgs& a, hipStream_t stream) {
 }
 
 #ifndef FLEXATTN_CUSTOM_ONLY
-template <int SCORE, bool DOCS, bool EXPORT>
+template <int SCORE, bool DOCS, bool EXPORT, int HD = 128>
 static int launch_dkv_plain_on(const BwdArgs& a, hipStream_t stream) {
   using namespace dkv_cfg;
-  auto kern = bwd_dkv_bf16_d128_plain_kernel<SCORE, DOCS, EXPORT>;
+  auto kern = bwd_dkv_bf16_d128_plain_kernel<SCORE, DOCS, EXPORT, HD>;
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dkv): %s", hipGetErrorString(attr));
@@ -1192,6 +1188,17 @@ int bwd_dkv_bf16_d128(const BwdArgs& a, hipStream_t stream) {
   }
   return set_error(FLEXATTN_EINVAL, "unknown score kind %d", a.score.kind);
 #endif
+}
+
+// Head dim 64: the generated stream for plain scores (the rest: see fwd_bf16_d64).
+int bwd_dkv_bf16_d64(const BwdArgs& a, hipStream_t stream) {
+#ifndef FLEXATTN_CUSTOM_ONLY
+  if (a.score.kind == FLEXATTN_SCORE_NONE && a.ds == nullptr &&
+      bwd_dkv_bf16_d128_on_stream(a.score.kind, a.flags, a.map.nq, a.score.ab != nullptr, a.Hq, a.Hkv))
+    return (a.mask.flags & FLEXATTN_MASK_DOC) ? launch_dkv_plain_on<FLEXATTN_SCORE_NONE, true, false, 64>(a, stream)
+                                              : launch_dkv_plain_on<FLEXATTN_SCORE_NONE, false, false, 64>(a, stream);
+#endif
+  return set_error(FLEXATTN_ENOTSUP, "bf16 head dim 64: only plain scores without a bias (pad the operands to 128 columns)");
 }
 
 // Head dim 256: the kernel with a compiled main loop (two 128-column panels per row), every score kind.

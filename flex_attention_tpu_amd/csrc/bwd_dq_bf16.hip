@@ -322,9 +322,12 @@ static int launch_dq(const BwdArgs& a, hipStream_t stream) {
 // EXACT: plain scores with Q unscaled in its registers; the stream turns the raw product into the exponent with one
 // fma per element (c2 <q, k> - lse).  For scales too large to fold into bf16 Q (folded_scale_ok).
 // KIND: 0 plain, 1 ALIBI, 2 SOFTCAP, 3 EXACT.
-template <int KIND, bool DOCS>
+// HD: head dimension 128, or 64 (plain scores; see the forward).
+template <int KIND, bool DOCS, int HD = 128>
 __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs a) {
   using namespace dq_cfg;
+  constexpr int D = HD;
+  static_assert(HD == 128 || KIND == 0 || KIND == 3, "streams of head dimension 64: plain scores");
   constexpr bool ALIBI = KIND == 1;
   constexpr bool SOFTCAP = KIND == 2;
   constexpr bool EXACT = KIND == 3;
@@ -344,7 +347,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
   const int hh = lane >> 5;
   const int q_local = w * 32 + l32;
 
-  TileLoader<4> loader;
+  TileLoader<4, HD> loader;
   loader.init(w, lane);
   const int r_sw = swz(l32);
   const int t_row = 4 * hh + ((lane & 15) >> 2);
@@ -393,8 +396,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
     geometry(item, bh, qb);
     const int q0 = tile_base(qb, BM, a.Sq);
     const size_t q_off = ((size_t)bh * a.Sq + (size_t)q0 + w * 32) * D;
-    rows_load(r.q, static_cast<const bf16_t*>(a.q) + q_off, lane);
-    rows_load(r.d, static_cast<const bf16_t*>(a.dout) + q_off, lane);
+    rows_load<HD>(r.q, static_cast<const bf16_t*>(a.q) + q_off, lane);
+    rows_load<HD>(r.d, static_cast<const bf16_t*>(a.dout) + q_off, lane);
     const size_t row = (size_t)bh * a.Sq + q0 + q_local;
     r.l = a.l[row];
     r.m = a.m[row];
@@ -451,8 +454,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
   // (`stage`: the wave's 16 KB of a free LDS step buffer)
   auto consume = [&](const ItemRegs& r, ItemHead& c, char* stage) {
     u32x4 qw[8], dw[8];
-    rows_to_fragments(r.q, stage, lane, qw);
-    rows_to_fragments(r.d, stage + 8192, lane, dw);
+    rows_to_fragments<HD>(r.q, stage, lane, qw);
+    rows_to_fragments<HD>(r.d, stage + 8192, lane, dw);
 #define FA_PUT(KS, QR, DR)                                                                                    \
   asm volatile(FA_DQ_PUT_##KS                                                                                 \
                : "={" QR "}"(st.q[KS]), "={" DR "}"(st.d[KS])                                                 \
@@ -676,9 +679,9 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
         const float caplse = cap2 - lse2;
         FA_DQ_CALL(FA_DQ_RUN_SOFTCAP, , [lse] "v"(caplse));
       } else if constexpr (EXACT) {
-        FA_DQ_CALL(FA_DQ_RUN_EXACT, , [lse] "v"(lse2));
+        if constexpr (HD == 64) { FA_DQ_CALL(FA_DQ_RUN_EXACT_D64, , [lse] "v"(lse2)); } else { FA_DQ_CALL(FA_DQ_RUN_EXACT, , [lse] "v"(lse2)); }
       } else {
-        FA_DQ_CALL(FA_DQ_RUN, , [lse] "v"(lse2));
+        if constexpr (HD == 64) { FA_DQ_CALL(FA_DQ_RUN_D64, , [lse] "v"(lse2)); } else { FA_DQ_CALL(FA_DQ_RUN, , [lse] "v"(lse2)); }
       }
 #undef FA_DQ_CALL
 #undef FA_DQ_ALIBI_CLOBBERS
@@ -702,7 +705,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
       const int row_here = lane_here & 31;
       const unsigned wr = (unsigned)row_here * 256u + 8u * (unsigned)(lane_here >> 5);
 #define FA_GET(T, SRC, REG)                                                                                        \
-  {                                                                                                                \
+  if constexpr (32 * T < HD) {                                                                                                                \
     float x[16];                                                                                                   \
     asm volatile(FA_DQ_GET_ACC_##T                                                                                 \
                  : "=v"(x[0]), "=v"(x[1]), "=v"(x[2]), "=v"(x[3]), "=v"(x[4]), "=v"(x[5]), "=v"(x[6]), "=v"(x[7]), \
@@ -723,23 +726,15 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
       bf16_t* out_rows = dQg + (size_t)(w * 32) * D;
-      const int chunk = lane_here & 15;
-      const int r_first = qb * BM - q0 - w * 32;   // (rows before it belong to the q tile before)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int r = 4 * i + (lane_here >> 4);
-        if (r < r_first) continue;
-        const u32x4 x = *reinterpret_cast<const u32x4*>(stage + (unsigned)r * 256u + (unsigned)((chunk ^ (r & 15)) << 4));
-        *reinterpret_cast<u32x4*>(out_rows + (size_t)r * D + chunk * 8) = x;
-      }
+      rows_store<HD>(stage, out_rows, lane_here, qb * BM - q0 - w * 32);   // (rows before that belong to the q tile before)
     }
   }  // work items
 }
 
-template <int KIND, bool DOCS>
+template <int KIND, bool DOCS, int HD>
 static int launch_dq_plain_on(const BwdArgs& a, hipStream_t stream) {
   using namespace dq_cfg;
-  auto kern = bwd_dq_bf16_d128_plain_kernel<KIND, DOCS>;
+  auto kern = bwd_dq_bf16_d128_plain_kernel<KIND, DOCS, HD>;
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, PLAIN_LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dq): %s", hipGetErrorString(attr));
@@ -750,10 +745,10 @@ static int launch_dq_plain_on(const BwdArgs& a, hipStream_t stream) {
   return check_launch("flexattn_bwd_dq bf16");
 }
 
-template <int KIND>
+template <int KIND, int HD = 128>
 static int launch_dq_plain(const BwdArgs& a, hipStream_t stream) {
-  return (a.mask.flags & FLEXATTN_MASK_DOC) ? launch_dq_plain_on<KIND, true>(a, stream)
-                                            : launch_dq_plain_on<KIND, false>(a, stream);
+  return (a.mask.flags & FLEXATTN_MASK_DOC) ? launch_dq_plain_on<KIND, true, HD>(a, stream)
+                                            : launch_dq_plain_on<KIND, false, HD>(a, stream);
 }
 
 #endif  // FLEXATTN_CUSTOM_ONLY
@@ -785,6 +780,16 @@ int bwd_dq_bf16_d128(const BwdArgs& a, hipStream_t stream) {
   }
   return set_error(FLEXATTN_EINVAL, "unknown score kind %d", a.score.kind);
 #endif
+}
+
+// Head dim 64: the generated streams for plain scores (the rest: see fwd_bf16_d64).
+int bwd_dq_bf16_d64(const BwdArgs& a, hipStream_t stream) {
+#ifndef FLEXATTN_CUSTOM_ONLY
+  if (a.score.kind == FLEXATTN_SCORE_NONE && a.score.ab == nullptr && a.dab == nullptr && !(a.flags & FLEXATTN_FLAG_COMPILED_LOOP) &&
+      a.map.nk <= dq_cfg::MAX_LIST)
+    return folded_scale_ok(a.sm_scale * kLog2e, a.sm_scale, 64) ? launch_dq_plain<0, 64>(a, stream) : launch_dq_plain<3, 64>(a, stream);
+#endif
+  return set_error(FLEXATTN_ENOTSUP, "bf16 head dim 64: only plain scores without a bias (pad the operands to 128 columns)");
 }
 
 // Head dim 256: the kernels with a compiled main loop (two 128-column panels per row), every score kind.

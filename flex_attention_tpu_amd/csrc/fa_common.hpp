@@ -220,28 +220,51 @@ __device__ __forceinline__ bf16x2 pack_bf16(float a, float b) {
 // through 8 KB of wave-private LDS when it is needed (rows_to_fragments; 16-byte chunks
 // XOR-swizzled by row: conflict-free both ways).
 // ------------------------------------------------------------------------------------------
+// (HD = 64: a row is 8 chunks, eight rows per instruction; the fragments 4..7 are zero.)
 struct RowBlock {
   u32x4 v[8];
 };
+template <int HD = 128>
 __device__ __forceinline__ void rows_load(RowBlock& r, const bf16_t* block, int lane) {
+  constexpr int CH = HD / 8, RPI = 64 / CH;   // chunks per row, rows per instruction
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
-    r.v[i] = *reinterpret_cast<const u32x4*>(block + (size_t)(4 * i + (lane >> 4)) * 128 + (lane & 15) * 8);
+  for (int i = 0; i < 32 / RPI; ++i)
+    r.v[i] = *reinterpret_cast<const u32x4*>(block + (size_t)(RPI * i + lane / CH) * HD + (lane % CH) * 8);
 }
+template <int HD = 128>
 __device__ __forceinline__ void rows_to_fragments(const RowBlock& r, char* stage, int lane, u32x4 (&frag)[8]) {
+  constexpr int CH = HD / 8, RPI = 64 / CH;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int row = 4 * i + (lane >> 4);
-    *reinterpret_cast<u32x4*>(stage + row * 256 + (((lane & 15) ^ (row & 15)) << 4)) = r.v[i];
+  for (int i = 0; i < 32 / RPI; ++i) {
+    const int row = RPI * i + lane / CH;
+    *reinterpret_cast<u32x4*>(stage + row * 256 + (((lane % CH) ^ (row & 15)) << 4)) = r.v[i];
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
   const int l32 = lane & 31, hh = lane >> 5;
 #pragma unroll
-  for (int ks = 0; ks < 8; ++ks)
-    frag[ks] = *reinterpret_cast<const u32x4*>(stage + l32 * 256 + (((2 * ks + hh) ^ (l32 & 15)) << 4));
+  for (int ks = 0; ks < 8; ++ks) {
+    if (16 * ks < HD)
+      frag[ks] = *reinterpret_cast<const u32x4*>(stage + l32 * 256 + (((2 * ks + hh) ^ (l32 & 15)) << 4));
+    else
+      frag[ks] = u32x4{0u, 0u, 0u, 0u};
+  }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
+}
+// A wave's 32 x HD results, staged as rows of 256 bytes with their 16-byte chunks XOR-swizzled by row, to memory with
+// full-row stores; rows before r_first are left alone.
+template <int HD>
+__device__ __forceinline__ void rows_store(const char* stage, bf16_t* block, int lane, int r_first) {
+  constexpr int CH = HD / 8, RPI = 64 / CH;
+  const int chunk = lane % CH;
+#pragma unroll
+  for (int i = 0; i < 32 / RPI; ++i) {
+    const int r = RPI * i + lane / CH;
+    if (r < r_first) continue;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(stage + (unsigned)r * 256u + (unsigned)((chunk ^ (r & 15)) << 4));
+    *reinterpret_cast<u32x4*>(block + (size_t)r * HD + chunk * 8) = v;
+  }
 }
 
 // ------------------------------------------------------------------------------------------

@@ -406,9 +406,16 @@ static int launch_fwd(const FwdArgs& a, hipStream_t stream) {
 // is all the backward kernels take from them.  (Caps up to 50 / log2(e): beyond, p could leave the range of the
 // accumulation; the compiled kernel takes those.)
 // KIND: 0 plain, 1 ALIBI, 2 SOFTCAP.
-template <int KIND, bool DOCS>
+// HD: head dimension 128, or 64 (plain scores): the streams then leave out the k-steps and column blocks that are not
+// there, on LDS tiles of the same layout whose rows are half used.  (Zero-padded copies of the operands and the cutting
+// back of the results took 590 of 1210 us of a training step on B=8, H=16, S=2048, D=64; kernels padded -> here:
+// forward 157 -> 131 us, dq 195 -> 149, dk/dv 244 -> 199: bound by the element-wise work, which the head dimension does
+// not shrink; the step 1206 -> 441 us.)
+template <int KIND, bool DOCS, int HD = 128>
 __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) {
   using namespace fwd_cfg;
+  constexpr int D = HD;
+  static_assert(HD == 128 || KIND == 0, "streams of head dimension 64: plain scores");
   constexpr bool ALIBI = KIND == 1;
   constexpr bool SOFTCAP = KIND == 2;
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
@@ -430,7 +437,7 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
   const int hh = lane >> 5;
   const int q_local = w * 32 + l32;
 
-  TileLoader<4> loader;
+  TileLoader<4, HD> loader;
   loader.init(w, lane);
   const int r_sw = swz(l32);
   const int t_row = 4 * hh + ((lane & 15) >> 2);
@@ -503,7 +510,7 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
     for (int x = 0; x < 2; ++x) {
       const int qb = min(2 * qb2 + x, nQ - 1);  // (a missing second tile repeats the first; nothing of it is stored)
       const int q0 = tile_base(qb, BM, a.Sq);
-      rows_load(r.q[x], static_cast<const bf16_t*>(a.q) + ((size_t)bh * a.Sq + (size_t)q0 + w_here * 32) * D, lane_here);
+      rows_load<HD>(r.q[x], static_cast<const bf16_t*>(a.q) + ((size_t)bh * a.Sq + (size_t)q0 + w_here * 32) * D, lane_here);
       r.doc[x] = (a.mask.flags & FLEXATTN_MASK_DOC) ? a.mask.doc_q[dq_rows + q0 + row_here] : 0;
       if constexpr (DOCS) {
         const bool ranged = a.mask.doc_q_range != nullptr;
@@ -543,8 +550,8 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
   auto consume = [&](const ItemRegs& r, ItemHead& c, char* stage) {
     u32x4 q0[8], q1[8];
     const int lane_here = opaque(lane);
-    rows_to_fragments(r.q[0], stage, lane_here, q0);
-    rows_to_fragments(r.q[1], stage + 8192, lane_here, q1);
+    rows_to_fragments<HD>(r.q[0], stage, lane_here, q0);
+    rows_to_fragments<HD>(r.q[1], stage + 8192, lane_here, q1);
 #define FA_PUT(KS, Q0, Q1)                                                                                        \
   asm volatile(FA_FWD_PUT_##KS                                                                                    \
                : "={" Q0 "}"(st.q[KS]), "={" Q1 "}"(st.q[8 + KS])                                                 \
@@ -840,7 +847,7 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
       } else if constexpr (SOFTCAP) {
         FA_FWD_CALL(FA_FWD_RUN_SOFTCAP, , );
       } else {
-        FA_FWD_CALL(FA_FWD_RUN, , );
+        if constexpr (HD == 64) { FA_FWD_CALL(FA_FWD_RUN_D64, , ); } else { FA_FWD_CALL(FA_FWD_RUN, , ); }
       }
 #undef FA_FWD_ADDV
 #undef FA_FWD_ALIBI_CLOBBERS
@@ -877,7 +884,7 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
         }
       }
 #define FA_GET(T, SRC, REG)                                                                                        \
-  {                                                                                                                \
+  if constexpr (32 * (T % 4) < HD) {                                                                                                                \
     float xv[16];                                                                                                  \
     asm volatile(FA_FWD_GET_ACC_##T                                                                                \
                  : "=v"(xv[0]), "=v"(xv[1]), "=v"(xv[2]), "=v"(xv[3]), "=v"(xv[4]), "=v"(xv[5]), "=v"(xv[6]),      \
@@ -899,30 +906,22 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
 #undef FA_GET
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
-      const int chunk = lane_here & 15;
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
         if (2 * qb2 + x < nQ) {
           bf16_t* Og = static_cast<bf16_t*>(a.o) + ((size_t)bh * a.Sq + (size_t)q_at[x] + w * 32) * D;
-          const int r_first = (2 * qb2 + x) * BM - q_at[x] - w * 32;   // (rows before it belong to the q tile before)
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const int r = 4 * i + (lane_here >> 4);
-            if (r < r_first) continue;
-            const u32x4 v = *reinterpret_cast<const u32x4*>(stage + x * 8192 + (unsigned)r * 256u +
-                                                            (unsigned)((chunk ^ (r & 15)) << 4));
-            *reinterpret_cast<u32x4*>(Og + (size_t)r * D + chunk * 8) = v;
-          }
+          // (rows before r_first belong to the q tile before)
+          rows_store<HD>(stage + x * 8192, Og, lane_here, (2 * qb2 + x) * BM - q_at[x] - w * 32);
         }
       }
     }
   }  // work items
 }
 
-template <int KIND, bool DOCS>
+template <int KIND, bool DOCS, int HD>
 static int launch_fwd_plain_on(const FwdArgs& a, hipStream_t stream) {
   using namespace fwd_cfg;
-  auto kern = fwd_bf16_d128_plain_kernel<KIND, DOCS>;
+  auto kern = fwd_bf16_d128_plain_kernel<KIND, DOCS, HD>;
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, PLAIN_LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(fwd): %s", hipGetErrorString(attr));
@@ -935,10 +934,10 @@ static int launch_fwd_plain_on(const FwdArgs& a, hipStream_t stream) {
   return check_launch("flexattn_fwd bf16");
 }
 
-template <int KIND>
+template <int KIND, int HD = 128>
 static int launch_fwd_plain(const FwdArgs& a, hipStream_t stream) {
-  return (a.mask.flags & FLEXATTN_MASK_DOC) ? launch_fwd_plain_on<KIND, true>(a, stream)
-                                            : launch_fwd_plain_on<KIND, false>(a, stream);
+  return (a.mask.flags & FLEXATTN_MASK_DOC) ? launch_fwd_plain_on<KIND, true, HD>(a, stream)
+                                            : launch_fwd_plain_on<KIND, false, HD>(a, stream);
 }
 
 #endif  // FLEXATTN_CUSTOM_ONLY
@@ -976,6 +975,17 @@ int fwd_bf16_d128(const FwdArgs& a, hipStream_t stream) {
   }
   return set_error(FLEXATTN_EINVAL, "unknown score kind %d", a.score.kind);
 #endif
+}
+
+// Head dim 64: the generated stream for plain scores (with a scale that folds into bf16 Q); everything else runs
+// zero-padded to 128 columns, which the caller sees to.
+int fwd_bf16_d64(const FwdArgs& a, hipStream_t stream) {
+#ifndef FLEXATTN_CUSTOM_ONLY
+  if (a.score.kind == FLEXATTN_SCORE_NONE && a.score.ab == nullptr && !(a.flags & FLEXATTN_FLAG_COMPILED_LOOP) &&
+      a.map.nk <= fwd_cfg::MAX_LIST && folded_scale_ok(a.sm_scale * kLog2e, a.sm_scale, 64))
+    return launch_fwd_plain<0, 64>(a, stream);
+#endif
+  return set_error(FLEXATTN_ENOTSUP, "bf16 head dim 64: only plain scores without a bias (pad the operands to 128 columns)");
 }
 
 // Head dim 256: the kernels with a compiled main loop (two 128-column panels per row), every score kind.

@@ -43,6 +43,9 @@ physical-register constraints; prologue / epilogue macros are generated here too
     %[ldsn]    LDS byte address of the wave's first block in the next step's buffer
     %[m0], %[m1]  (masked stream only) the lane's keep bits: bit 16 (c & 1) + e of m[c >> 1] is
                element e of the S accumulator of q block c; dropped elements get P = 0
+    (head dimension 64, `d64`: rows of 128 bytes in memory; an LDS row keeps its 256 bytes, of which the second half is
+    neither filled for use nor read: k-steps 4-7 and column blocks 2, 3 with their registers drop out of the streams;
+    v[200:203] are clobbered too)
 LDS layout of one step buffer (bytes): Q half 0, Q half 1, dO half 0, dO half 1 (16 KiB each);
 -lse [128] floats, -delta 1 KiB after it.
 """
@@ -89,6 +92,7 @@ S_KC = "s101"     # (position-bias variant) 128 kb + 64: the middle of the item'
 # cap' - lse - 2 cap' r with cap' = cap log2(e) (LDS holds cap' - lse; s64 = cap', s101 = -2 cap'), and
 # ds'/ds = 1 - tanh^2 = 4 r (1 - r), whose factor 4 the epilogue applies to dk.
 S_CAP, S_K2 = "s64", "s101"
+CAP_D64 = 12      # ... at head dimension 64 (64 MFMAs a step for the same element-wise work instead of 128)
 CAP_SOFTCAP = 8   # instructions per MFMA gap in the softcap variant (8 VALU ops per element instead of 2)
 # dS export variant: the step's bf16 dS (the B operand registers of the dk product) also goes to a buffer in
 # global memory, one 32 KB block per (query head, kept tile pair), from which the dq pass takes it.  The blocks of
@@ -99,6 +103,7 @@ S_DSB, S_PAIRS, S_DS, S_DSN = "s[52:53]", "s54", "s[56:57]", "s[58:59]"
 V_QB2 = 67      # q block index of the step after the next one, across the stream
 ROW_SLOT = 28   # MFMA slot at which the next step's lse / delta values are turned around
 V_ROW = 144     # 4 temporaries for that, inside pb[1] (first written by E(1), after ROW_SLOT)
+V_ROW_D64 = 200 # (head dimension 64: above the other scratch)
 V_S = [72, 104]
 V_DP = [88, 120]
 V_PB = 136
@@ -110,18 +115,22 @@ V_TMP = 68    # 4 temporaries of the masked variant
 DL_OFFSET = 1024
 
 
-def build(masked, alibi=False, softcap=False, export=False):
+def build(masked, alibi=False, softcap=False, export=False, d64=False):
+    assert not (d64 and (alibi or softcap or export))
+    KS, ND = (4, 2) if d64 else (8, 4)   # k-steps of a score, column blocks of dk and dv
+    near = 3 if d64 else 6               # MFMAs between a row value's read and the chains before and behind it
+    row_slot, v_row = (40, V_ROW_D64) if d64 else (ROW_SLOT, V_ROW)
     em = Emitter()
     em.wait_old = WAIT_OLD
 
     # ---- MFMA pairs in issue order -------------------------------------------------------
     pairs = []
     def add_A(c):
-        for ks in range(8):
+        for ks in range(KS):
             pairs.append(("A", c, ks))
     def add_B(c):
         for u in range(2):
-            for db in range(4):
+            for db in range(ND):
                 pairs.append(("B", c, (u, db)))
     add_A(0); add_A(1); add_A(2); add_B(0); add_A(3); add_B(1); add_B(2); add_B(3)
     n_mfma = 2 * len(pairs)
@@ -129,9 +138,9 @@ def build(masked, alibi=False, softcap=False, export=False):
     for k, key in enumerate(pairs):
         idx[key] = 2 * k
     first_A = {c: idx[("A", c, 0)] for c in range(4)}
-    last_A = {c: idx[("A", c, 7)] + 1 for c in range(4)}
+    last_A = {c: idx[("A", c, KS - 1)] + 1 for c in range(4)}
     first_B = {(c, u): idx[("B", c, (u, 0))] for c in range(4) for u in range(2)}
-    last_B = {(c, u): idx[("B", c, (u, 3))] + 1 for c in range(4) for u in range(2)}
+    last_B = {(c, u): idx[("B", c, (u, ND - 1))] + 1 for c in range(4) for u in range(2)}
 
     def half_off(c):
         return (c >> 1) * TILE + (c & 1) * (TILE // 2)
@@ -306,7 +315,7 @@ def build(masked, alibi=False, softcap=False, export=False):
                 if reg == V_LSE:
                     continue   # (used by E(c), not by the chain: read there, block 0 below)
                 rows.append(lds(f"ds_read_b128 {vr(reg + 4 * g, 4)}, %[la] offset:{(32 * c + 8 * g) * 4 + off}", vset(reg + 4 * g, 4),
-                                earliest=first_A[c - 1] + 6 if c else 0, deadline=max(0, first_A[c] - 6)))
+                                earliest=first_A[c - 1] + near if c else 0, deadline=max(0, first_A[c] - near)))
     chains.append(rows)
     first_rows = [lse_read(0, g) for g in range(4)]
     first_rows[-1].deadline = last_A[0]
@@ -345,7 +354,7 @@ def build(masked, alibi=False, softcap=False, export=False):
         # LDS-direct load) have arrived once at most as many vector-memory operations are open as
         # LDS-direct loads were issued.  Waves 0, 1: (l, m) -> -lse = -m log2(e) - log2(l), -inf where
         # l = 0; waves 2, 3: -delta (%[lsew] is non-zero resp. zero).  One LDS store into the next buffer.
-        ra_, rb_, rt_, inf_ = V_ROW, V_ROW + 1, V_ROW + 2, V_ROW + 3
+        ra_, rb_, rt_, inf_ = v_row, v_row + 1, v_row + 2, v_row + 3
         e.raw(f"s_waitcnt vmcnt({state['direct']})")
         # (-lse by one fused multiply-add, m (-log2 e) - log2 l: the same rounding as the kernel's own set-up of an
         # item's first step, so that a step's row values do not depend on who prepared them)
@@ -377,9 +386,10 @@ def build(masked, alibi=False, softcap=False, export=False):
         e.lds_write(f"ds_write_b32 %[lw], {vr(rt_)}", vset(rt_))
 
     # V_ROW lies inside pb[1] (first written by E(1)): the turn-around runs before E(1) may start
-    chains.append([Op(row_turnaround, cost=8, earliest=ROW_SLOT, deadline=last_A[1] + 3)])
+    # (d64: registers of its own, later in the step: the values have as long to arrive)
+    chains.append([Op(row_turnaround, cost=8, earliest=row_slot, deadline=row_slot + 8 if d64 else last_A[1] + 3)])
 
-    schedule(em, mfmas, chains, CAP_SOFTCAP if softcap else CAP)
+    schedule(em, mfmas, chains, CAP_D64 if d64 else CAP_SOFTCAP if softcap else CAP)
     em.drain()
     if export:
         # the step's copies have landed once only the stores issued behind the last of them are open
@@ -387,12 +397,13 @@ def build(masked, alibi=False, softcap=False, export=False):
     return em
 
 
-def run_loop(full, masked, alibi=False, softcap=False, export=False):
+def run_loop(full, masked, alibi=False, softcap=False, export=False, d64=False):
     """One asm statement: a run of consecutive steps [it, it_end) of one work-group, all full or a
     single partial one.  At entry the step's Q / dO tiles and row values are resident in LDS buffer
     s81; each pass computes the next step's addresses, streams the tile (which copies the next
     step's data into the other buffer), synchronises the work-group and advances."""
     t0, t1, t2, t3 = S_T
+    v_row = V_ROW_D64 if d64 else V_ROW
     lo = lambda pair: pair[2:].split(":")[0]  # "s[88:89]" -> "88"
     entry = [f"ds_read_b128 {vr(V_TBL + 4 * i, 4)}, %[tbl] offset:{16 * i}" for i in range(4)]
     entry += ["s_waitcnt lgkmcnt(0)"]  # (the streams count LDS operations from zero)
@@ -446,13 +457,13 @@ def run_loop(full, masked, alibi=False, softcap=False, export=False):
         f"s_sub_u32 {t2}, s62, 128",
         f"s_min_u32 {t1}, {t1}, {t2}",
         f"s_add_u32 {t0}, {t0}, {t1}",
-        f"s_lshl_b32 {t2}, {t0}, 8",
-        f"s_lshr_b32 {t3}, {t0}, 24",
+        f"s_lshl_b32 {t2}, {t0}, {7 if d64 else 8}",
+        f"s_lshr_b32 {t3}, {t0}, {25 if d64 else 24}",
     ]
     for pair, base in ((S_GQ0, "qg"), (S_GD0, "dog")):
         n = int(lo(pair))
         top += [f"s_add_u32 s{n}, {SREG[base + '_lo']}, {t2}", f"s_addc_u32 s{n + 1}, {SREG[base + '_hi']}, {t3}",
-                f"s_add_u32 s{n + 2}, s{n}, 0x4000", f"s_addc_u32 s{n + 3}, s{n + 1}, 0"]
+                f"s_add_u32 s{n + 2}, s{n}, {'0x2000' if d64 else '0x4000'}", f"s_addc_u32 s{n + 3}, s{n + 1}, 0"]
     top += [f"s_lshl_b32 {t2}, {t0}, 2", f"s_lshr_b32 {t3}, {t0}, 30"]
     for pair, base in ((S_RA, "rowa"), (S_RB, "rowb")):
         n = int(lo(pair))
@@ -467,8 +478,8 @@ def run_loop(full, masked, alibi=False, softcap=False, export=False):
         f"s_lshl_b32 {t1}, s79, 2",
         f"v_mov_b32_e32 {vr(V_QB2)}, {t1}",
         f"global_load_dword {vr(V_QB2)}, {vr(V_QB2)}, s[66:67]",
-        f"global_load_dword {vr(V_ROW)}, %[tid4], {S_RA}",
-        f"global_load_dword {vr(V_ROW + 1)}, %[tid4], {S_RB}",
+        f"global_load_dword {vr(v_row)}, %[tid4], {S_RA}",
+        f"global_load_dword {vr(v_row + 1)}, %[tid4], {S_RB}",
         "s_bitcmp0_b32 s83, 0",
         "s_cbranch_scc1 .Lfa_dkv_full_%=",
     ]
@@ -519,6 +530,10 @@ def main():
             f.write(f"#define {name} \\\n")
             f.write(" \\\n".join(f'  "{line}\\n"' for line in lines))
             f.write("\n\n")
+        lines = run_loop(build(False, d64=True), build(True, d64=True), d64=True)
+        f.write("#define FA_DKV_RUN_D64 \\\n")
+        f.write(" \\\n".join(f'  "{line}\\n"' for line in lines))
+        f.write("\n\n")
         for name, em in (("full", full), ("masked", masked)):
             print(f"{path}: {name}: {len(em.out)} instructions, {em.stats}", file=sys.stderr)
 

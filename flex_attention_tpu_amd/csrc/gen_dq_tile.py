@@ -31,6 +31,8 @@ physical-register constraints):
     %[m0], %[m1]  (partial steps) the lane's keep bits: bit 16 (c & 1) + e of m[c >> 1] is element e
                of the S^T accumulator of kv block c; dropped elements get dS = 0
     %[tbl]     LDS byte address of the wave's table of work-group constants (TABLE below)
+    (head dimension 64, `d64`: rows of 128 bytes in memory; an LDS row keeps its 256 bytes, of which the second half is
+    neither filled for use nor read: k-steps 4-7 and column blocks 2, 3 with their registers drop out of the streams)
     %[it], %[kba1], %[kbb1], %[buf]  loop state (in/out); %[it_end] (in); %[partial] (in): the step of the
                run that is partial and takes the masked stream with the keep bits (-1: none)
 LDS layout of one step buffer (bytes): K tile 0, K tile 1, V tile 0, V tile 1 (16 KiB each); the two
@@ -52,6 +54,7 @@ LOAD_EVERY = 3   # gaps between two of them
 LOAD_COST = 3    # share of an MFMA gap one of them takes
 TRANS_COST = 2   # share of an MFMA gap a transcendental takes (it holds the wave's issue for two slots)
 CAP_SOFTCAP = 8  # instructions per MFMA gap in the softcap variant (8 VALU ops per element instead of 2)
+CAP_D64 = 10     # ... at head dimension 64 (48 MFMAs a step for the same element-wise work instead of 96)
 S_K2 = "s62"     # (softcap variant) -2 cap log2(e): the table's c2 entry
 DROP = ()        # instruction classes left out (--drop, timing studies only)
 
@@ -110,26 +113,27 @@ def bias_ops(e, block, tile, odd):
     e.mfma_f32x2(vr(V_NL, 16), "%[aone]", vr(b), vset(V_NL, 16), set(), vset(b))
 
 
-def build(masked, alibi=False, softcap=False, exact=False):
+def build(masked, alibi=False, softcap=False, exact=False, d64=False):
     em = Emitter()
     em.wait_old = WAIT_OLD
     pairs = []
+    KS, NJ = (4, 1) if d64 else (8, 2)   # k-steps of a score, pairs of column blocks of dq
 
     def add_A(c):
-        for ks in range(8):
+        for ks in range(KS):
             pairs.append(("A", c, ks))
 
     def add_B(c):
         for u in range(2):
-            for j in range(2):
+            for j in range(NJ):
                 pairs.append(("B", c, (u, j)))
 
     add_A(0); add_A(1); add_A(2); add_B(0); add_A(3); add_B(1); add_B(2); add_B(3)
     idx = {key: 2 * k for k, key in enumerate(pairs)}  # number of the pair's first MFMA
     first_A = {c: idx[("A", c, 0)] for c in range(4)}
-    last_A = {c: idx[("A", c, 7)] + 1 for c in range(4)}
+    last_A = {c: idx[("A", c, KS - 1)] + 1 for c in range(4)}
     first_B = {(c, u): idx[("B", c, (u, 0))] for c in range(4) for u in range(2)}
-    last_B = {(c, u): idx[("B", c, (u, 1))] + 1 for c in range(4) for u in range(2)}
+    last_B = {(c, u): idx[("B", c, (u, NJ - 1))] + 1 for c in range(4) for u in range(2)}
 
     def half_off(c):
         return (c >> 1) * TILE + (c & 1) * (TILE // 2)
@@ -261,7 +265,7 @@ def build(masked, alibi=False, softcap=False, exact=False):
     k = 0
     for t, gbase in enumerate((S_GK0, S_GK1, S_GV0, S_GV1)):  # half tiles in LDS order
         for i in range(4):
-            at = LOAD_FIRST + LOAD_EVERY * k
+            at = LOAD_FIRST + (2 if d64 else LOAD_EVERY) * k
 
             # (M0 of load k + 1 is written behind load k; the loop top writes the first one's)
             nxt = None if k == 15 else ((k + 1) // 4) * TILE + ((k + 1) % 4) * 1024
@@ -283,12 +287,12 @@ def build(masked, alibi=False, softcap=False, exact=False):
                            deadline=first_A[c] - 6 if c < 4 else None))
         chains.append(bias)
 
-    schedule(em, mfmas, chains, CAP_SOFTCAP if softcap else CAP)
+    schedule(em, mfmas, chains, CAP_D64 if d64 else CAP_SOFTCAP if softcap else CAP)
     em.drain()
     return em
 
 
-def run_loop(full, masked, alibi=False, softcap=False, exact=False):
+def run_loop(full, masked, alibi=False, softcap=False, exact=False, d64=False):
     """One asm statement: a run of consecutive steps [it, it_end) of one work item, at most one of
     them partial.  At entry the step's K / V tiles are resident in LDS buffer %[buf]; each pass
     computes the next step's addresses, streams the step (which copies the next step's tiles into the
@@ -318,9 +322,9 @@ def run_loop(full, masked, alibi=False, softcap=False, exact=False):
             f"s_cselect_b32 {kglo}, {S['kgn_lo']}, {S['kg_lo']}", f"s_cselect_b32 {kghi}, {S['kgn_hi']}, {S['kg_hi']}",
             f"s_cselect_b32 {vglo}, {S['vgn_lo']}, {S['vg_lo']}", f"s_cselect_b32 {vghi}, {S['vgn_hi']}, {S['vg_hi']}"]
     for kb, bases in ((ka, (S_GK0, S_GV0)), (kb_, (S_GK1, S_GV1))):
-        # first row of the kv tile (64 kb; a ragged length's last tile starts early), 256 bytes a row
+        # first row of the kv tile (64 kb; a ragged length's last tile starts early), 256 bytes a row (head dimension 64: 128)
         top += [f"s_lshl_b32 {t2}, {kb}, 6", f"s_min_u32 {t3}, {t2}, {S['klim']}",
-                f"s_lshl_b32 {t2}, {t3}, 8", f"s_lshr_b32 {t3}, {t3}, 24"]
+                f"s_lshl_b32 {t2}, {t3}, {7 if d64 else 8}", f"s_lshr_b32 {t3}, {t3}, {25 if d64 else 24}"]
         for pair, (blo, bhi) in zip(bases, ((kglo, kghi), (vglo, vghi))):
             n = int(pair[2:].split(":")[0])
             top += [f"s_add_u32 s{n}, {blo}, {t2}", f"s_addc_u32 s{n + 1}, {bhi}, {t3}"]
@@ -385,6 +389,8 @@ def main():
         macro("FA_DQ_RUN_ALIBI", run_loop(build(False, True), build(True, True), True))
         macro("FA_DQ_RUN_SOFTCAP", run_loop(build(False, softcap=True), build(True, softcap=True), softcap=True))
         macro("FA_DQ_RUN_EXACT", run_loop(build(False, exact=True), build(True, exact=True), exact=True))
+        macro("FA_DQ_RUN_D64", run_loop(build(False, d64=True), build(True, d64=True), d64=True))
+        macro("FA_DQ_RUN_EXACT_D64", run_loop(build(False, exact=True, d64=True), build(True, exact=True, d64=True), exact=True, d64=True))
         for name, em in (("full", full), ("masked", masked)):
             print(f"{args.out}: {name}: {len(em.out)} instructions, {em.stats}", file=sys.stderr)
         macro("FA_DQ_ZERO_ACC", [f"v_accvgpr_write_b32 a{A_DQ + i}, 0" for i in range(64)])

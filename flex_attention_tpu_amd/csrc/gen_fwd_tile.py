@@ -46,6 +46,8 @@ physical-register constraints):
     %[tbl]     LDS byte address of the wave's table of work-group constants (TABLE below)
     %[lst]     LDS byte address of the item's merged kv tile list (int32 entries)
     %[it], %[kba1], %[kbb1], %[buf]  loop state (in/out); %[it_end], %[partial]  (in)
+    (head dimension 64, `d64`: rows of 128 bytes in memory; an LDS row keeps its 256 bytes, of which the second half is
+    neither filled for use nor read: k-steps 4-7 and column blocks 2, 3 with their registers drop out of the streams)
 LDS layout of one step buffer (bytes): K tile 0, K tile 1, V tile 0, V tile 1 (16 KiB each); the two
 buffers are 64 KiB apart and the first starts at LDS address 0.
 """
@@ -66,6 +68,7 @@ TAU = "0x40c00000"  # 6.0: M moves when the running maximum relative to it leave
 TRANS_COST = 2   # share of an MFMA gap a transcendental takes (it holds the wave's issue for two slots)
 ROUNDED_SUM = False  # row sums add the bf16-rounded probabilities (v_dot2c on the packed pairs) instead of the fp32 ones
 DROP = ()        # instruction classes left out (--drop, timing studies only)
+CAP_D64 = 10     # ... at head dimension 64 (64 MFMAs a step for the same softmax work instead of 128)
 CAP_SOFTCAP = 8  # instructions per MFMA gap in the softcap variant (6.5 VALU ops per score instead of 2.5)
 S_K2 = "s62"     # (softcap variant) -2 cap log2(e): the table's c2 entry
 SEQUENTIAL = True  # (plain scores) the S chains of the two q blocks one after the other instead of alternating
@@ -139,7 +142,9 @@ def v_p(c, x, u):
     return V_P0 + 8 * x + 4 * u
 
 
-def build(masked, alibi=False, softcap=False):
+def build(masked, alibi=False, softcap=False, d64=False):
+    assert not (d64 and alibi)
+    KS, NJ = (4, 1) if d64 else (8, 2)   # k-steps of a score, pairs of column blocks of O
     em = Emitter()
     em.wait_old = WAIT_OLD
     # MFMA pairs (2 MFMAs each), in issue order.  The two q blocks of a kv block are processed half a
@@ -153,7 +158,7 @@ def build(masked, alibi=False, softcap=False):
 
     def add_B(c, q):
         for u in range(2):
-            for j in range(2):
+            for j in range(NJ):
                 pairs.append(("B", c, (q, u, j)))
 
     # Without a position bias the S chains of the two q blocks run one after the other (a chain's eight
@@ -163,7 +168,7 @@ def build(masked, alibi=False, softcap=False):
     sequential = SEQUENTIAL and not alibi
 
     def add_S(c, q):
-        for j in range(4):
+        for j in range(KS // 2):
             pairs.append(("A", c, (q, j)))
 
     if sequential:
@@ -193,7 +198,7 @@ def build(masked, alibi=False, softcap=False):
         return idx[("B", c, (q, u, 0))]
 
     def b_last(c, q, u):
-        return idx[("B", c, (q, u, 1))] + 1
+        return idx[("B", c, (q, u, NJ - 1))] + 1
 
     def half_off(c):
         return (c >> 1) * TILE + (c & 1) * (TILE // 2)
@@ -211,11 +216,17 @@ def build(masked, alibi=False, softcap=False):
     def k_slot(k):
         return A_STG + 32 + 4 * (a_index[k] % 8)
 
-    def ks_slot(ks):          # (sequential chains: the fragment of k-step ks has its own slot, read once for both chains)
-        return A_STG + 32 + 4 * ks
+    # (d64: half the fragments; two kv blocks' worth then fit and take the places in turn)
+    behind = 2 if d64 else 1   # a place's last user belongs to the block `behind` before
 
-    def v_place(u, db):
-        return A_STG + 4 * (4 * u + db)
+    def ks_slot(c, ks):       # (sequential chains: the fragment of k-step ks has its own slot, read once for both chains)
+        return A_STG + 32 + 4 * (ks + (4 * (c & 1) if d64 else 0))
+
+    def v_slot(c, db):
+        return db + (2 * (c & 1) if d64 else 0)
+
+    def v_place(c, u, db):
+        return A_STG + 4 * (4 * u + v_slot(c, db))
 
     holds = {}  # V^T place -> kv block whose fragment was last read into it
 
@@ -229,8 +240,8 @@ def build(masked, alibi=False, softcap=False):
         if kind == "A" and sequential:
             q, j = x
             for ks in (2 * j, 2 * j + 1) if q == 0 else ():
-                text, dst = f"ds_read_b128 {ar(ks_slot(ks), 4)}, %[r{ks}] offset:{half_off(c)}", aset(ks_slot(ks), 4)
-                earliest = a_mfma(c - 1, ks, 1) + 1 if c > 0 else 0   # (the slot's last user: the second chain of block c - 1)
+                text, dst = f"ds_read_b128 {ar(ks_slot(c, ks), 4)}, %[r{ks}] offset:{half_off(c)}", aset(ks_slot(c, ks), 4)
+                earliest = a_mfma(c - behind, ks, 1) + 1 if c >= behind else 0   # (the slot's last user: the second chain of block c - 1)
                 reads.append((2 * k, Op((lambda e, t=text, d=dst: e.lds_read(t, d)) if "lds" not in DROP else (lambda e: None),
                                         earliest=earliest, deadline=max(0, 2 * (k - MIN_AHEAD)))))
                 read_texts.append((text, max(0, 2 * (k - MIN_AHEAD))))
@@ -246,14 +257,14 @@ def build(masked, alibi=False, softcap=False):
             off = 2 * TILE + half_off(c) + u * 4096
             for db in (2 * j, 2 * j + 1):
                 for hi in range(2):
-                    reg = v_place(u, db) + 2 * hi
+                    reg = v_place(c, u, db) + 2 * hi
                     text, dst = f"ds_read_b64_tr_b16 {ar(reg, 2)}, %[t{2 * db + hi}] offset:{off}", aset(reg, 2)
 
-                    def emit(e, t=text, d=dst, key=(u, db), blk=c):
+                    def emit(e, t=text, d=dst, key=(u, v_slot(c, db)), blk=c):
                         holds[key] = blk
                         if "lds" not in DROP:
                             e.lds_read(t, d)
-                    earliest = b_last(c - 1, 1, u) + 1 if c > 0 else 0
+                    earliest = b_last(c - behind, 1, u) + 1 if c >= behind else 0
                     reads.append((2 * k, Op(emit, earliest=earliest, deadline=2 * (k - MIN_AHEAD))))
                     read_texts.append((text, 2 * (k - MIN_AHEAD)))
     reads.sort(key=lambda r: r[0])  # (stable: in the order of their use)
@@ -263,7 +274,7 @@ def build(masked, alibi=False, softcap=False):
         if kind == "A":
             if sequential:
                 q, ks = x[0], 2 * x[1] + j
-                slot = ks_slot(ks)
+                slot = ks_slot(c, ks)
             else:
                 ks, q = x, j
                 slot = k_slot(k)
@@ -279,11 +290,11 @@ def build(masked, alibi=False, softcap=False):
         db = 2 * jj + j
         p = v_p(c, q, u)
         acc = A_O + 64 * q + 16 * db
-        vt = v_place(u, db)
+        vt = v_place(c, u, db)
         args = (ar(acc, 16), ar(vt, 4), vr(p, 4), ar(acc, 16), aset(acc, 16), aset(vt, 4), vset(p, 4), aset(acc, 16))
 
         def emit(e):
-            assert holds.get((u, db)) == c, f"B({c}, {q}) would multiply with the V^T fragment of block {holds.get((u, db))}"
+            assert holds.get((u, v_slot(c, db))) == c, f"B({c}, {q}) would multiply with the V^T fragment of block {holds.get((u, v_slot(c, db)))}"
             e.mfma(*args)
         return emit
 
@@ -351,7 +362,7 @@ def build(masked, alibi=False, softcap=False):
                 for u in range(4):
                     e = 4 * g + u
                     ops.append(valu(f"v_add_f32_e32 {L}, {L}, {vr(s + e)}", kL, kL | vset(s + e)))
-            ops[0].earliest = max(ops[0].earliest, a_mfma(c, 7, q) + 4)   # the chain's last result needs 12 wait states
+            ops[0].earliest = max(ops[0].earliest, a_mfma(c, KS - 1, q) + 4)   # the chain's last result needs 12 wait states
             if c + 2 < 4:
                 ops[-1].deadline = min(ops[-1].deadline or (1 << 30), a_mfma(c + 2, 0, q))  # A(c + 2) writes the same S registers
             return ops
@@ -410,7 +421,7 @@ def build(masked, alibi=False, softcap=False):
                  ("valu", f"v_sub_f32_e32 {Mt}, {Mt}, {vr(D)}", kMt, kMt | vset(D), False),
                  ("valu", f"v_add_f32_e32 {M}, {M}, {vr(D)}", kM, kM | vset(D), False),
                  ("valu", f"v_mul_f32_e32 {L}, {L}, {vr(AL)}", kL, kL | vset(AL), False)]
-        for i in range(64):
+        for i in range(32 * NJ):
             t = T[5 + (i % 4)]
             acc = A_O + 64 * q + i
             rare.append(("valu", f"v_accvgpr_read_b32 {vr(t)}, {ar(acc)}", vset(t), aset(acc), False))
@@ -497,7 +508,7 @@ def build(masked, alibi=False, softcap=False):
             if g < 3:
                 exps(g + 1)
             dots(g)
-        ops[0].earliest = max(ops[0].earliest, a_mfma(c, 7, q) + 4)   # the chain's last result needs 12 wait states
+        ops[0].earliest = max(ops[0].earliest, a_mfma(c, KS - 1, q) + 4)   # the chain's last result needs 12 wait states
         if c + 2 < 4:
             ops[-1].deadline = min(ops[-1].deadline or (1 << 30), a_mfma(c + 2, 0, q))  # A(c + 2) writes the same S registers
         return ops
@@ -537,7 +548,7 @@ def build(masked, alibi=False, softcap=False):
 
     if masked:
         em.valu(f"v_mov_b32_e32 {vr(V_NEGINF)}, 0xff800000", vset(V_NEGINF), set())
-    schedule(em, mfmas, chains, CAP_SOFTCAP if softcap else CAP)
+    schedule(em, mfmas, chains, CAP_D64 if d64 else CAP_SOFTCAP if softcap else CAP)
     em.drain()
     return em
 
@@ -567,7 +578,7 @@ def out_of_line(lines):
     return hot, cold
 
 
-def run_loop(full, masked, alibi=False, softcap=False):
+def run_loop(full, masked, alibi=False, softcap=False, d64=False):
     """One asm statement: a run of consecutive steps [it, it_end) of one work item, all full or a
     single partial one.  At entry the step's K / V tiles are resident in LDS buffer %[buf]."""
     t0, t1, t2, t3 = S_T
@@ -594,9 +605,9 @@ def run_loop(full, masked, alibi=False, softcap=False):
             f"s_cselect_b32 {kglo}, {S['kgn_lo']}, {S['kg_lo']}", f"s_cselect_b32 {kghi}, {S['kgn_hi']}, {S['kg_hi']}",
             f"s_cselect_b32 {vglo}, {S['vgn_lo']}, {S['vg_lo']}", f"s_cselect_b32 {vghi}, {S['vgn_hi']}, {S['vg_hi']}"]
     for kb, bases in ((ka, (S_GK0, S_GV0)), (kb_, (S_GK1, S_GV1))):
-        # first row of the kv tile (64 kb; a ragged length's last tile starts early), 256 bytes a row
+        # first row of the kv tile (64 kb; a ragged length's last tile starts early), 256 bytes a row (head dimension 64: 128)
         top += [f"s_lshl_b32 {t2}, {kb}, 6", f"s_min_u32 {t3}, {t2}, {S['klim']}",
-                f"s_lshl_b32 {t2}, {t3}, 8", f"s_lshr_b32 {t3}, {t3}, 24"]
+                f"s_lshl_b32 {t2}, {t3}, {7 if d64 else 8}", f"s_lshr_b32 {t3}, {t3}, {25 if d64 else 24}"]
         for pair, (blo, bhi) in zip(bases, ((kglo, kghi), (vglo, vghi))):
             n = int(pair[2:].split(":")[0])
             top += [f"s_add_u32 s{n}, {blo}, {t2}", f"s_addc_u32 s{n + 1}, {bhi}, {t3}"]
@@ -661,6 +672,7 @@ def main():
         macro("FA_FWD_RUN", run_loop(full, masked))
         macro("FA_FWD_RUN_ALIBI", run_loop(build(False, True), build(True, True), True))
         macro("FA_FWD_RUN_SOFTCAP", run_loop(build(False, softcap=True), build(True, softcap=True), softcap=True))
+        macro("FA_FWD_RUN_D64", run_loop(build(False, d64=True), build(True, d64=True), d64=True))
         for name, em in (("full", full), ("masked", masked)):
             print(f"{args.out}: {name}: {len(em.out)} instructions, {em.stats}", file=sys.stderr)
         macro("FA_FWD_ZERO_ACC", [f"v_accvgpr_write_b32 a{A_O + i}, 0" for i in range(128)])

@@ -14,6 +14,7 @@ int check_launch(const char* what);
 
 // bf16, head dim 128 (MFMA kernels)
 int fwd_bf16_d128(const FwdArgs& a, hipStream_t stream);
+int fwd_bf16_d64(const FwdArgs& a, hipStream_t stream);    // (same tiles as head dim 128; plain scores)
 int fwd_bf16_d256(const FwdArgs& a, hipStream_t stream);   // (same tiles as head dim 128)
 void fwd_bf16_d128_tile(int* bq, int* bk);
 // few query rows against long keys, plain scores, no mask (head dim 64 or 128)
@@ -21,9 +22,11 @@ bool fwd_decode_ok(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D);
 int64_t fwd_decode_bytes(int B, int Hq, int Hkv, int Sq, int Sk, int D);
 int fwd_decode(const FwdArgs& a, int D, void* work, hipStream_t stream);
 int bwd_dq_bf16_d128(const BwdArgs& a, hipStream_t stream);
+int bwd_dq_bf16_d64(const BwdArgs& a, hipStream_t stream);
 int bwd_dq_bf16_d256(const BwdArgs& a, hipStream_t stream);
 void bwd_dq_bf16_d128_tile(int* bq, int* bk);
 int bwd_dkv_bf16_d128(const BwdArgs& a, hipStream_t stream);
+int bwd_dkv_bf16_d64(const BwdArgs& a, hipStream_t stream);
 int bwd_dkv_bf16_d256(const BwdArgs& a, hipStream_t stream);
 // (the dk/dv pass of such a request runs the generated stream: its exported dS then lacks sm_scale and the soft-cap's
 // factor 4; the kernel with a compiled main loop exports dS complete)

@@ -28,7 +28,8 @@ __host__ __device__ __forceinline__ constexpr int tile_off(int row, int chunk) {
 }
 
 // Asynchronous copy of a 64 x 128 bf16 tile (global row stride ROW elements: 128, or the head dimension where a
-// tile is one 128-column panel of wider rows) into LDS with
+// tile is one 128-column panel of wider rows; 64: an LDS row's second half gets a copy of its first, from the same cache
+// lines, and is not used) into LDS with
 // global_load_lds_dwordx4: the data never passes through registers.  Each instruction fills one
 // contiguous 1 KB block (4 tile rows); lane L's 16 bytes land at block + 16*L, so the swizzle is
 // applied on the global side.  The NWAVES waves of a work-group each copy 16/NWAVES blocks.  The
@@ -45,7 +46,7 @@ struct TileLoader {
 #pragma unroll
     for (int i = 0; i < kBlocks; ++i) {
       const int row = (wave * kBlocks + i) * 4 + (lane >> 4);
-      const int chunk = (lane & 15) ^ swz(row);
+      const int chunk = ((lane & 15) ^ swz(row)) & (ROW / 8 - 1);
       goff[i] = (unsigned)(row * ROW + chunk * 8) * 2u;
     }
   }

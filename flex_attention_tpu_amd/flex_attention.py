@@ -15,6 +15,8 @@ from typing import Callable, Optional, Tuple
 
 import torch
 
+from ._common import call_head_dim
+from .block_mask import spec_of
 from .flex_attention_dkv_kernel import flash_attention_bwd_dkv
 from .flex_attention_dq_bwd import compute_delta, ds_exchange_pays, flex_attention_bwd_dq
 from .flex_attention_kernel import _flex_attention_impl
@@ -81,7 +83,9 @@ class _FlexAttention(torch.autograd.Function):
         dq = dk = dv = ds = dab = None
         want_dkv = ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
         want_dq = ctx.needs_input_grad[0] or want_dab
+        # (not at the head dimension 64 kernels, which hand nothing over: recomputing there beats 128 padded columns)
         exchange = (want_dkv and ctx.needs_input_grad[0] and ab is None and q.dtype == torch.bfloat16 and
+                    call_head_dim(q.shape[-1], q.dtype, sm_scale, score_fn, ab, spec_of(mask_fn, block_mask_fn), q.shape[2], k.shape[2]) != 64 and
                     ds_exchange_pays(score_fn, mask_fn, segment_ids))
         # di = sum(o * do), float32 [B, H, Sq] (jax_exp.py:276-278): taken by the dq pass itself where that pass runs
         # first (no dS hand-over), else by its own launch

@@ -8,7 +8,7 @@ import ctypes as C
 import torch
 
 from . import _lib
-from ._common import (on_device, bias_c, check_blocks, check_doc_batches, check_qkv, check_rows, kernel_block_map, kernel_head_dim, library_for, pad_seq,
+from ._common import (on_device, bias_c, check_blocks, check_doc_batches, check_qkv, check_rows, kernel_block_map, call_head_dim, kernel_head_dim, library_for, pad_seq,
                       padded_len, resolve_mask, stream_of, tagged_closures)
 from .flex_attention_dq_bwd import DsBlocks, alloc_ds, bwd_params
 
@@ -36,7 +36,9 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
     check_doc_batches(spec, B)   # (ids of shape [B, S]: the kernels mask every batch entry by its own row)
     q, do, k, v = pad_seq(q, Sq_p), pad_seq(do, Sq_p), pad_seq(k, Sk_p), pad_seq(v, Sk_p)
     l, m, di = pad_seq(l, Sq_p), pad_seq(m, Sq_p), pad_seq(di, Sq_p)
-    D_user, D = D, kernel_head_dim(D, q.dtype)   # smaller head dimensions: zero-padded columns
+    # (a dS hand-over is at 128 columns)
+    D_user, D = D, (call_head_dim(D, q.dtype, sm_scale, score_fn, ab, spec, Sq, Sk, compiled_loop) if not return_ds
+                    else kernel_head_dim(D, q.dtype))   # smaller head dimensions: zero-padded columns
     q, do, k, v = pad_seq(q, D, 3), pad_seq(do, D, 3), pad_seq(k, D, 3), pad_seq(v, D, 3)
     bm = kernel_block_map(_lib.PASS_DKV, spec, q, Sq_p, Sk_p, D, score_fn)
     dk = torch.empty_like(k)

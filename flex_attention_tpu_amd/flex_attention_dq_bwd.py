@@ -7,7 +7,7 @@ import ctypes as C
 import torch
 
 from . import _lib
-from ._common import (on_device, bias_c, check_blocks, check_doc_batches, check_qkv, check_rows, dtype_code, kernel_block_map, kernel_head_dim, library_for,
+from ._common import (on_device, bias_c, check_blocks, check_doc_batches, check_qkv, check_rows, dtype_code, kernel_block_map, call_head_dim, kernel_head_dim, library_for,
                       pad_seq, padded_len, mostly_partial_custom_mask, resolve_mask, score_spec_c, stream_of, tagged_closures, tile_lengths)
 from .block_mask import mask_spec_c
 
@@ -139,7 +139,9 @@ def flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, d, *, block_b, 
     check_doc_batches(spec, B)   # (ids of shape [B, S]: the kernels mask every batch entry by its own row)
     q, do, k, v = pad_seq(q, Sq_p), pad_seq(do, Sq_p), pad_seq(k, Sk_p), pad_seq(v, Sk_p)
     l, m, d_p = pad_seq(l, Sq_p), pad_seq(m, Sq_p), pad_seq(d, Sq_p)
-    D_user, D = D, kernel_head_dim(D, q.dtype)   # smaller head dimensions: zero-padded columns
+    # (a dS hand-over is at 128 columns)
+    D_user, D = D, (call_head_dim(D, q.dtype, sm_scale, score_fn, ab, spec, Sq, Sk, compiled_loop) if ds is None
+                    else kernel_head_dim(D, q.dtype))   # smaller head dimensions: zero-padded columns
     q, do, k, v = pad_seq(q, D, 3), pad_seq(do, D, 3), pad_seq(k, D, 3), pad_seq(v, D, 3)
     o_p = pad_seq(pad_seq(o, Sq_p), D, 3) if fuse_delta else None
     if ds is not None and (ds.buf is None or ds.index is None or ds.shape != (B, Hq, Sq_p, Sk_p) or ds.buf.device != q.device

@@ -8,7 +8,8 @@
  *
  * Conventions
  *  - All tensors are contiguous row-major [B, H, S, D] device memory owned by the caller.
- *    Head dimension D: 128 or 256 for bf16, 64 or 128 for float32 (anything else: FLEXATTN_ENOTSUP).
+ *    Head dimension D: 128 or 256 for bf16, 64 or 128 for float32 (anything else: FLEXATTN_ENOTSUP); bf16 also 64 for
+ *    plain scores without a bias, without dS hand-over and with flags 0 (pad the operands of others to 128 columns).
  *    q/o/do/dq have Hq heads, k/v/dk/dv have Hkv heads, Hq % Hkv == 0 (kv head = h / (Hq/Hkv)).
  *  - l, m, delta are float32 [B, Hq, Sq].
  *  - Every function returns FLEXATTN_OK or a negative error code, never throws or aborts, and
@@ -203,7 +204,7 @@ const char* flexattn_last_error_string(void);
 const char* flexattn_custom_tag(void);
 
 /* Tile granularity (block_q, block_k) the kernels of `pass` expect of the block map for this
- * dtype and head dimension (bf16 head dimension 256 runs on the tiles of 128). */
+ * dtype and head dimension (bf16 head dimensions 64 and 256 run on the tiles of 128). */
 int flexattn_tile_shape(int32_t pass, int32_t dtype, int32_t D, int32_t* block_q, int32_t* block_k);
 
 /* Block-mask builder.  Replaces the per-grid-step evaluation of the `block_mask_fn` closures

@@ -368,15 +368,15 @@ def test_fwd_tile_streams_respect_hazards():
         assert pending is None
 
 
-def check_dataflow(lines, reads_per_fragment, reads_per_packed):
+def check_dataflow(lines, reads_per_fragment, reads_per_packed, chain_len=8):
     """What the hazard rules cannot see: that the scheduler kept every value alive until its users
     were issued.  Re-derived from the text alone:
       * a staging register filled by an LDS read is read by exactly `reads_per_fragment` MFMAs (as A
         operand) before the next LDS read overwrites it;
       * a register written by v_cvt_pk_bf16_f32 (P, dS) is read by exactly `reads_per_packed` MFMAs
         (as B operand) before it is packed again;
-      * an accumulation chain (first MFMA: C input is not its destination) consists of 8 MFMAs, and
-        no other instruction touches its destination before the eighth has been issued."""
+      * an accumulation chain (first MFMA: C input is not its destination) consists of `chain_len` MFMAs, and
+        no other instruction touches its destination before the last of them has been issued."""
     frag_reads, packed_reads, chain = {}, {}, {}
     skip = None
     for line in lines:
@@ -399,11 +399,11 @@ def check_dataflow(lines, reads_per_fragment, reads_per_packed):
             if dst and next(iter(dst))[0] == "v":  # S / dP chains live in VGPRs
                 key = min(dst)
                 if c != dst:
-                    assert chain.get(key, 8) == 8, f"a chain restarts after {chain[key]} MFMAs: {line}"
+                    assert chain.get(key, chain_len) == chain_len, f"a chain restarts after {chain[key]} MFMAs: {line}"
                     chain[key] = 1
                 else:
                     chain[key] += 1
-                    assert chain[key] <= 8, f"more than 8 MFMAs in a chain: {line}"
+                    assert chain[key] <= chain_len, f"more than {chain_len} MFMAs in a chain: {line}"
         elif op.startswith("ds_read"):
             for r in regs_of(ops[0]):
                 if r[0] == "a":
@@ -414,7 +414,7 @@ def check_dataflow(lines, reads_per_fragment, reads_per_packed):
             touched = set().union(*[regs_of(x) for x in ops]) if ops else set()
             for key, n in chain.items():
                 tup = {(key[0], key[1] + i) for i in range(16)}
-                assert not (touched & tup) or n == 8, f"chain at {key} used after {n} of 8 MFMAs: {line}"
+                assert not (touched & tup) or n == chain_len, f"chain at {key} used after {n} of {chain_len} MFMAs: {line}"
             if op.startswith("v_cvt_pk_bf16"):
                 for r in regs_of(ops[0]):
                     assert packed_reads.get(r, reads_per_packed) == reads_per_packed, \
@@ -425,7 +425,7 @@ def check_dataflow(lines, reads_per_fragment, reads_per_packed):
         assert n == reads_per_fragment, f"fragment in {r} used {n} times at the end of the stream"
     for r, n in packed_reads.items():
         assert n == reads_per_packed, f"packed operand {r} used {n} times at the end of the stream"
-    assert all(n == 8 for n in chain.values())
+    assert all(n == chain_len for n in chain.values())
 
 
 def test_streams_keep_values_alive_for_their_users():
@@ -611,3 +611,25 @@ def test_vmem_queue_checker_catches_open_loads():
     bad = [".Ltop:", "s_barrier", "global_load_lds_dwordx4 v70, s[20:21]", "s_cbranch_scc1 .Ltop", "s_waitcnt vmcnt(0)"]
     with pytest.raises(AssertionError, match="s_barrier with loads in flight"):
         check_vmem_queue(bad)
+
+
+def test_head_dim_64_streams():
+    """The streams of head dimension 64: half the MFMAs of a step (four k-steps, half the column blocks), the same
+    element-wise work; hazards, data flow (chains of four, two column blocks per packed operand) and open loads as above."""
+    import gen_dkv_tile, gen_dq_tile, gen_fwd_tile
+
+    for masked in (False, True):
+        for g, n_mfma, scratch, reads, kw in ((gen_dkv_tile, 64, (68, 203, 255), 1, {}), (gen_dq_tile, 48, (66, 183, 191), 1, {}),
+                                              (gen_dq_tile, 48, (66, 183, 191), 1, {"exact": True}),
+                                              (gen_fwd_tile, 64, (66, 199, 255), 2, {})):
+            em = g.build(masked, d64=True, **kw)
+            n = check_stream(em.out)
+            assert em.stats["mfma"] == n_mfma
+            assert n == em.stats["mfma"] + em.stats["valu"] + em.stats["lds"] + em.stats["vmem"]
+            scratch_ok(em.out, *scratch)
+            check_dataflow(em.out, reads, 2, chain_len=4)
+            # nothing beyond the 64 columns: fragments ks < 4, transposed fragments of the column blocks 0 and 1
+            assert not any(f"%[{x}{i}]" in line for line in em.out for x in "rt" for i in range(4, 8))
+    for g, kw in ((gen_dkv_tile, {}), (gen_dq_tile, {}), (gen_dq_tile, {"exact": True}), (gen_fwd_tile, {})):
+        lines = g.run_loop(g.build(False, d64=True, **kw), g.build(True, d64=True, **kw), d64=True, **kw)
+        assert check_vmem_queue(lines) > len(lines)
