@@ -67,6 +67,8 @@ struct DqPinned {
 template <int SCORE, int NP>
 __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdArgs a) {
   using namespace dq_cfg;
+  constexpr bool kBias = NP == 1 && SCORE == kScoreBiasOnly;   // a bias and no score function: launched as a kind of its own
+  constexpr bool kNoBias = NP == 1 && SCORE == FLEXATTN_SCORE_NONE;
   constexpr int D = 128 * NP;
   constexpr int kPanel = kTileElems * 2;   // bytes
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
@@ -182,8 +184,14 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
     const char* kt = reinterpret_cast<const char*>(sK + buf * NP * kTileElems);
     const char* vt = reinterpret_cast<const char*>(sV + buf * NP * kTileElems);
 
-#pragma clang loop unroll_count(NP == 1 ? 2 : 1)   // (wider rows: rolled, which keeps the second block's operand loads out of the first block's registers: 1.37 -> 1.25 ms on B=4, H=16, S=4096, D=256)
+#pragma clang loop unroll_count(NP == 1 && !kBias ? 2 : 1)   // (wider rows: rolled, which keeps the second block's operand loads out of the first block's registers: 1.37 -> 1.25 ms on B=4, H=16, S=4096, D=256)
     for (int c = 0; c < 2; ++c) {
+      // (an additive bias: loaded in front of the products, which hide the latency)
+      f32x4 bias_pre[4];
+      if (kBias) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) bias_pre[g] = sm.bias2x4(q_idx, kv0 + 32 * c + 8 * g + 4 * hh);
+      }
       // ---- S^T and dP^T for kv rows [32c, 32c+32) ----
       f32x16 s_acc, dp_acc;
 #pragma unroll
@@ -232,7 +240,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
             const auto d4 = *reinterpret_cast<const i32x4_a4*>(mk.doc_k + j0);
             dj[0] = d4[0]; dj[1] = d4[1]; dj[2] = d4[2]; dj[3] = d4[3];
           }
-          const f32x4 bias = sm.bias2x4(q_idx, j0);
+          const f32x4 bias = kBias ? bias_pre[g] : kNoBias ? f32x4{0.f, 0.f, 0.f, 0.f} : sm.bias2x4(q_idx, j0);
           float dsv[4];
           f32x4 gb;   // the gradient with respect to the logits themselves: what an additive bias receives
 #pragma unroll
@@ -293,6 +301,8 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
 
 template <int SCORE, int NP = 1>
 static int launch_dq(const BwdArgs& a, hipStream_t stream) {
+  if constexpr (SCORE == FLEXATTN_SCORE_NONE && NP == 1)
+    if (a.score.ab != nullptr) return launch_dq<kScoreBiasOnly, 1>(a, stream);
   using namespace dq_cfg;
   auto kern = bwd_dq_bf16_kernel<SCORE, NP>;
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),

@@ -479,7 +479,7 @@ struct ScoreMod {
   // depend on the dot product (mha_reference.py:50-51 adds it behind the score function).
   __device__ __forceinline__ bool has_bias() const { return ab_base != nullptr; }
   __device__ __forceinline__ float bias2(int i, int j) const {
-    if (ab_base == nullptr) return 0.f;
+    if (KIND != kScoreBiasOnly && ab_base == nullptr) return 0.f;
     const unsigned long long at = (unsigned long long)(unsigned)(ab_row0 + i) * (unsigned)ab_ld + (unsigned)j;
     const float v = ab_f32 ? reinterpret_cast<const float*>(ab_base)[at]
                            : __builtin_bit_cast(float, (unsigned)reinterpret_cast<const unsigned short*>(ab_base)[at] << 16);
@@ -491,7 +491,7 @@ struct ScoreMod {
   // tile made the kernels spill.)
   __device__ __forceinline__ f32x4 bias2x4(int i, int j0) const {
     f32x4 r = {0.f, 0.f, 0.f, 0.f};
-    if (ab_base == nullptr) return r;
+    if (KIND != kScoreBiasOnly && ab_base == nullptr) return r;   // (that kind is launched with a bias only)
     const unsigned long long at = (unsigned long long)(unsigned)(ab_row0 + i) * (unsigned)ab_ld + (unsigned)j0;
     if (ab_f32) {
       r = *reinterpret_cast<const f32x4_a4*>(reinterpret_cast<const float*>(ab_base) + at);

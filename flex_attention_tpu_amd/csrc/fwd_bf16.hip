@@ -190,7 +190,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
     s16x4 vlo[4][4 * NP], vhi[4][4 * NP];  // [tt][db]
     // Plain scores fetch the first half of V^T ahead of the softmax, which hides the latency; a score function's
     // own arithmetic, or the wider rows, need those registers in the softmax (the compiler spilled otherwise)
-    constexpr bool kEarlyV = NP == 1 && (SCORE == FLEXATTN_SCORE_NONE || SCORE == kScoreBiasOnly);
+    constexpr bool kEarlyV = NP == 1 && SCORE == FLEXATTN_SCORE_NONE;
     auto read_k = [&](int g) {
       const int c = g / (2 * NP), pn = (g % (2 * NP)) >> 1;
 #pragma unroll
@@ -208,6 +208,14 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int e = 0; e < 16; ++e) s_acc[c][e] = 0.f;
+    // (an additive bias: the tile's 32 values per lane are loaded in front of the products, which hide the latency)
+    constexpr bool kBias = NP == 1 && SCORE == kScoreBiasOnly;
+    f32x4 bias_pre[8];
+    if (kBias) {
+      const int kv0_b = tile_base(kb, BN, a.Sk);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) bias_pre[i] = sm.bias2x4(q_idx, kv0_b + 32 * (i >> 2) + 8 * (i & 3) + 4 * hh);
+    }
     read_k(0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -246,7 +254,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
         for (int g = 0; g < 4; ++g) {
           const int j0 = kv0 + 32 * c + 8 * g + 4 * hh;
           f32x4 bias;
-          if (!kPlain) bias = sm.bias2x4(q_idx, j0);
+          if (!kPlain) bias = kBias ? bias_pre[4 * c + g] : sm.bias2x4(q_idx, j0);
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const int e = 4 * g + u;
@@ -271,7 +279,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
             dj[0] = d4[0]; dj[1] = d4[1]; dj[2] = d4[2]; dj[3] = d4[3];
           }
           f32x4 bias;
-          if (!kPlain) bias = sm.bias2x4(q_idx, j0);
+          if (!kPlain) bias = kBias ? bias_pre[4 * c + g] : sm.bias2x4(q_idx, j0);
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const int e = 4 * g + u;
@@ -408,9 +416,7 @@ static int launch_fwd(const FwdArgs& a, hipStream_t stream) {
 // KIND: 0 plain, 1 ALIBI, 2 SOFTCAP.
 // HD: head dimension 128, or 64 (plain scores): the streams then leave out the k-steps and column blocks that are not
 // there, on LDS tiles of the same layout whose rows are half used.  (Zero-padded copies of the operands and the cutting
-// back of the results took 590 of 1210 us of a training step on B=8, H=16, S=2048, D=64; kernels padded -> here:
-// forward 157 -> 131 us, dq 195 -> 149, dk/dv 244 -> 199: bound by the element-wise work, which the head dimension does
-// not shrink; the step 1206 -> 441 us.)
+// back of the results took 590 of 1210 us of a training step on B=8, H=16, S=2048, D=64.)
 template <int KIND, bool DOCS, int HD = 128>
 __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) {
   using namespace fwd_cfg;

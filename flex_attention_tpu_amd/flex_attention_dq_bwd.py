@@ -161,8 +161,10 @@ def flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, d, *, block_b, 
     if return_dab:
         if ab is None or ds is not None:
             raise ValueError("return_dab needs the additive bias `ab` and excludes `ds`")
-        # (only the tiles the block map visits are written: masked-out pairs have no gradient)
-        dab_full = torch.zeros(B, Hq, Sq_p, Sk_p, dtype=torch.float32, device=q.device)
+        # (only the tiles the block map visits are written: masked-out pairs have no gradient; without a mask that is
+        # every element, and the clearing, 70 us for B=4, H=16, S=1500, is left out)
+        new = torch.empty if spec.flags == 0 else torch.zeros
+        dab_full = new(B, Hq, Sq_p, Sk_p, dtype=torch.float32, device=q.device)
         p.dab = dab_full.data_ptr()
     if ds is not None:
         p.ds, p.ds_bytes = ds.buf.data_ptr(), ds.buf.numel()
