@@ -75,11 +75,12 @@ struct PinnedState {
 // EXPORT: the kernel also writes the tile's bf16 dS (the B operands of the dk product: here with the score function's
 // derivative and sm_scale in them) to a.ds, in the block layout of the generated streams' export (see there), for
 // the dq pass from dS: a score function is then evaluated in one backward pass instead of two.
-template <int SCORE, bool EXPORT = false>
+// AB: the call may have an additive bias (false: splits_bias() kinds without one).
+template <int SCORE, bool EXPORT, bool AB>
 __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
   using namespace dkv_cfg;
   constexpr bool kBias = SCORE == kScoreBiasOnly;             // a bias and no score function: launched as a kind of its own
-  constexpr bool kNoBias = SCORE == FLEXATTN_SCORE_NONE;
+  constexpr bool kNoBias = SCORE == FLEXATTN_SCORE_NONE || !AB;
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
   bf16_t* sQ = reinterpret_cast<bf16_t*>(smem_raw);
   bf16_t* sDO = sQ + 4 * kTileElems;
@@ -349,9 +350,10 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
 // 64-row tile one LDS tile (tile_io.hpp) at [buffer][panel]; a loop iteration covers 64 q rows (half an entry of the
 // kv tile's list: the two buffers of Q and dO panels then take the LDS the 128-row steps take at head dim 128), the
 // contractions of S and dP run over the panels, dk^T and dv^T have four accumulators per panel.
-template <int SCORE, int NP>
+template <int SCORE, int NP, bool AB>
 __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
   using namespace dkv_cfg;
+  constexpr bool kNoBias = SCORE == FLEXATTN_SCORE_NONE || !AB;   // (a bias without a score function: kScoreBiasOnly)
   constexpr int D = 128 * NP;
   constexpr int HQ = 64;                  // q rows per iteration
   constexpr int kPanel = kTileElems * 2;  // bytes
@@ -526,7 +528,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
             const int e = 4 * g4 + u;
             const int i = q0 + r0 + u;
             const float tv = sm.to_log2(s_acc[e], i, k_idx);
-            float pe = fast_exp2(tv + sm.bias2(i, k_idx) - lse4[u]);
+            float pe = fast_exp2(tv + (kNoBias ? 0.f : sm.bias2(i, k_idx)) - lse4[u]);
             float gd = pe * (dp_acc[e] - dl4[u]) * sm.dfactor(tv, s_acc[e], i, k_idx);
             if (MASKED) {
               const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j) & (8 * g4 + u >= own - 32 * c);
@@ -599,11 +601,15 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
   }
 }
 
-template <int SCORE, int NP>
+template <int SCORE, int NP, bool AB = true>
 static int launch_dkv_wide(const BwdArgs& a, hipStream_t stream) {
+  if constexpr (AB && splits_bias(SCORE))
+    if (a.score.ab == nullptr) return launch_dkv_wide<SCORE, NP, false>(a, stream);
+  if constexpr (SCORE == FLEXATTN_SCORE_NONE)
+    if (a.score.ab != nullptr) return launch_dkv_wide<kScoreBiasOnly, NP>(a, stream);
   using namespace dkv_cfg;
   constexpr int kLds = 4 * NP * kTileElems * 2 + 4 * 64 * 4;   // (Q, dO) x 2 buffers x NP panels; lse, delta x 2 buffers
-  auto kern = bwd_dkv_bf16_wide_kernel<SCORE, NP>;
+  auto kern = bwd_dkv_bf16_wide_kernel<SCORE, NP, AB>;
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dkv): %s", hipGetErrorString(attr));
@@ -1121,10 +1127,12 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
 
 #endif  // FLEXATTN_CUSTOM_ONLY
 
-template <int SCORE, bool EXPORT>
+template <int SCORE, bool EXPORT, bool AB = true>
 static int launch_dkv_on(const BwdArgs& a, hipStream_t stream) {
+  if constexpr (AB && splits_bias(SCORE))
+    if (a.score.ab == nullptr) return launch_dkv_on<SCORE, EXPORT, false>(a, stream);
   using namespace dkv_cfg;
-  auto kern = bwd_dkv_bf16_d128_kernel<SCORE, EXPORT>;
+  auto kern = bwd_dkv_bf16_d128_kernel<SCORE, EXPORT, AB>;
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dkv): %s", hipGetErrorString(attr));

@@ -64,11 +64,12 @@ struct DqPinned {
 // Head dimension 128 NP: a row of K or V is NP panels of 128 columns, each panel of a 64-row tile one LDS tile
 // (tile_io.hpp) at [buffer][panel]; the contractions of S and dP run over the panels, dq^T has four accumulators
 // per panel.
-template <int SCORE, int NP>
+// AB: the call may have an additive bias (false: splits_bias() kinds without one).
+template <int SCORE, int NP, bool AB>
 __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdArgs a) {
   using namespace dq_cfg;
   constexpr bool kBias = NP == 1 && SCORE == kScoreBiasOnly;   // a bias and no score function: launched as a kind of its own
-  constexpr bool kNoBias = NP == 1 && SCORE == FLEXATTN_SCORE_NONE;
+  constexpr bool kNoBias = SCORE == FLEXATTN_SCORE_NONE || !AB;
   constexpr int D = 128 * NP;
   constexpr int kPanel = kTileElems * 2;   // bytes
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
@@ -253,7 +254,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
             if (MASKED) {   // (selected, not multiplied: a score function may return anything at a dropped element)
               const bool keep = keep_elem(mk, q_idx, j0 + u, doc_i, dj[u]);
               gl = keep ? gl : 0.f;
-              gd = keep & (8 * g + u >= own) ? gd : 0.f;
+              gd = (keep & (8 * g + u >= own)) ? gd : 0.f;
             }
             gb[u] = gl;
             dsv[u] = gd;
@@ -299,12 +300,14 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
   }
 }
 
-template <int SCORE, int NP = 1>
+template <int SCORE, int NP = 1, bool AB = true>
 static int launch_dq(const BwdArgs& a, hipStream_t stream) {
-  if constexpr (SCORE == FLEXATTN_SCORE_NONE && NP == 1)
-    if (a.score.ab != nullptr) return launch_dq<kScoreBiasOnly, 1>(a, stream);
+  if constexpr (AB && splits_bias(SCORE))
+    if (a.score.ab == nullptr) return launch_dq<SCORE, NP, false>(a, stream);
+  if constexpr (SCORE == FLEXATTN_SCORE_NONE)
+    if (a.score.ab != nullptr) return launch_dq<kScoreBiasOnly, NP>(a, stream);
   using namespace dq_cfg;
-  auto kern = bwd_dq_bf16_kernel<SCORE, NP>;
+  auto kern = bwd_dq_bf16_kernel<SCORE, NP, AB>;
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, NP * LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dq): %s", hipGetErrorString(attr));

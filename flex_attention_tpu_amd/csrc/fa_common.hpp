@@ -422,6 +422,12 @@ __device__ __forceinline__ unsigned keep_bits32_staged(const MaskArgs& mk, int f
 // running maximum on the raw dot products when there is no score function at all; with a bias it must
 // take the log2-domain route of the score functions.)
 constexpr int kScoreBiasOnly = 100;
+// Whether the kernels with a compiled main loop have a variant of this kind without the code of an additive bias (its
+// pointers and strides take registers through the loop, and kernels at the limit spill: symmetric ALiBi closure, B=8, H=4,
+// S=2048, 399 -> 375 us; tile-local ALiBi forward 28 spilled registers -> none).  Plain scores have no such
+// code at all, see kScoreBiasOnly; the global position bias and the soft-cap take the generated streams where there is no
+// bias, and keep one variant.
+constexpr bool splits_bias(int kind) { return kind == FLEXATTN_SCORE_CUSTOM || kind == FLEXATTN_SCORE_ALIBI_TILE; }
 
 template <int KIND>
 struct ScoreMod {

@@ -65,7 +65,8 @@ struct FwdPinned {
 
 // Head dimension 128 NP: a row of K or V is NP panels of 128 columns, each panel of a 64-row tile one LDS tile
 // (tile_io.hpp) at [buffer][panel]; the contraction of S runs over the panels, O^T has four accumulators per panel.
-template <int SCORE, int NP>
+// AB: the call may have an additive bias (false: splits_bias() kinds without one).
+template <int SCORE, int NP, bool AB>
 __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs a) {
   using namespace fwd_cfg;
   constexpr int D = 128 * NP;
@@ -254,7 +255,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
         for (int g = 0; g < 4; ++g) {
           const int j0 = kv0 + 32 * c + 8 * g + 4 * hh;
           f32x4 bias;
-          if (!kPlain) bias = kBias ? bias_pre[4 * c + g] : sm.bias2x4(q_idx, j0);
+          if (!kPlain) bias = kBias ? bias_pre[4 * c + g] : AB ? sm.bias2x4(q_idx, j0) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const int e = 4 * g + u;
@@ -279,7 +280,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
             dj[0] = d4[0]; dj[1] = d4[1]; dj[2] = d4[2]; dj[3] = d4[3];
           }
           f32x4 bias;
-          if (!kPlain) bias = kBias ? bias_pre[4 * c + g] : sm.bias2x4(q_idx, j0);
+          if (!kPlain) bias = kBias ? bias_pre[4 * c + g] : AB ? sm.bias2x4(q_idx, j0) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const int e = 4 * g + u;
@@ -381,10 +382,12 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
   }
 }
 
-template <int SCORE, int NP = 1>
+template <int SCORE, int NP = 1, bool AB = true>
 static int launch_fwd(const FwdArgs& a, hipStream_t stream) {
   using namespace fwd_cfg;
-  auto kern = fwd_bf16_kernel<SCORE, NP>;
+  if constexpr (AB && splits_bias(SCORE))
+    if (a.score.ab == nullptr) return launch_fwd<SCORE, NP, false>(a, stream);
+  auto kern = fwd_bf16_kernel<SCORE, NP, AB>;
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, NP * LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(fwd): %s", hipGetErrorString(attr));
