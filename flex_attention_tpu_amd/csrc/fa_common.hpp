@@ -583,13 +583,32 @@ __device__ __forceinline__ PersistentPlan persistent_plan(int j, int n_wg, int n
   }
   return p;
 }
+// One item per work-group, started in the order of the ids: (batch, head) pair and rank of work-group j, ranks ascending
+// in work under causal masks from the caller's end.  An XCD (ids j % 8) takes a contiguous share of the heads and starts
+// the blocks of equal rank of several heads together, longest first: with the blocks of one head behind each other the
+// longest of the share's last head start when the chip is already running dry (B=1, Hq=32, S=2777 forward, 352 items of
+// 2 to 22 steps on 256 CUs: 94.6 us against 77.2 us).  The heads taken together are those that kSetItems items make, so that
+// the K / V of few heads are in use at a time.
+constexpr int kSetItems = 64;
+__host__ __device__ inline void single_item(int j, int n_wg, int nKb, int& head, int& kb) {
+  const int heads = n_wg / nKb;
+  if (heads % 8 != 0) {
+    const int wg = (n_wg % 8 != 0) ? j : (j % 8) * (n_wg / 8) + j / 8;
+    head = wg / nKb;
+    kb = wg % nKb;
+    return;
+  }
+  const int share = heads / 8, set = nKb >= kSetItems ? 1 : kSetItems / nKb;   // heads of an XCD, heads taken together
+  const int t = j >> 3, first = t / (set * nKb) * set;                         // first head of the item's set
+  const int in = t - first * nKb, n = share - first < set ? share - first : set;
+  head = (j & 7) * share + first + in % n;
+  kb = in / n;
+}
 // (batch, head) pair and block of item number `item` of work-group j
 __device__ __forceinline__ void persistent_item(const PersistentPlan& p, int j, int item, int grid, int n_wg, int nKb,
                                                 int& head, int& kb) {
   if (grid == n_wg) {  // one item per work-group, no static schedule
-    const int wg = xcd_remap(j, n_wg);
-    head = wg / nKb;
-    kb = wg % nKb;
+    single_item(j, n_wg, nKb, head, kb);
     return;
   }
   int hd;
