@@ -141,6 +141,9 @@ def tagged_closures(score_fn, mask_fn, block_mask_fn, block_q, block_k):
     sizes, which also derives the block closure (a block closure without a mask function cannot be compiled: it
     says which tiles run, not which elements).  Closures that carry a ``.spec`` pass through; the compiled form of
     a function object is kept while the function lives."""
+    if (score_fn is None or isinstance(getattr(score_fn, "spec", None), ScoreSpec)) and \
+            (mask_fn is None or getattr(mask_fn, "spec", None) is not None):
+        return score_fn, mask_fn, block_mask_fn   # (the usual case)
     import inspect
 
     def arity(fn):

@@ -10,16 +10,18 @@ flex_attention_kernel.py:66-83 carried through.
 """
 from __future__ import annotations
 
+import ctypes as C
 import math
 from typing import Callable, Optional, Tuple
 
 import torch
 
-from ._common import call_head_dim
+from . import _lib, _plans
+from ._common import call_head_dim, check_blocks, check_qkv, check_rows, on_device, stream_of, tagged_closures
 from .block_mask import spec_of
 from .flex_attention_dkv_kernel import flash_attention_bwd_dkv
 from .flex_attention_dq_bwd import compute_delta, ds_exchange_pays, flex_attention_bwd_dq
-from .flex_attention_kernel import _flex_attention_impl
+from .flex_attention_kernel import _CAUSAL, _flex_attention_impl
 
 
 # The backward hands dS from the dk/dv pass to the dq pass (DsBlocks in flex_attention_dq_bwd.py) when both
@@ -34,9 +36,17 @@ def flex_attention_bwd(q, k, v, ab, segment_ids, l, m, o, do, *, block_q, block_
     reference's custom_vjp wiring, jax_exp.py:276-321) from one call through the C ABI (flexattn_bwd): small
     problems are bound by the host's path to a launch.  No dS hand-over (see flash_attention_bwd_dkv(return_ds=True) for that) and no bias
     gradient (flex_attention_bwd_dq(return_dab=True))."""
-    import ctypes as C
-    from . import _lib
-    from ._common import on_device, stream_of
+    if score_fn is None and ab is None and segment_ids is None and not compiled_loop:
+        B, Hq, _, Sq, Sk, _ = check_qkv(q, k, v, do, o)
+        check_blocks(Sq, Sk, block_q=block_q, block_k_major=block_k, block_k=block_k)
+        check_rows("l", l, B, Hq, Sq, q.device)
+        check_rows("m", m, B, Hq, Sq, q.device)
+        _, mask_fn, block_mask_fn = tagged_closures(None, mask_fn, block_mask_fn, block_q, block_k)
+        spec = spec_of(mask_fn, block_mask_fn)
+        if causal:
+            spec = spec.combine(_CAUSAL)
+        if _plans.takes(q, k, spec, sm_scale):
+            return _plans.backward(q, k, v, l, m, o, do, spec, float(sm_scale))
     kw = dict(sm_scale=sm_scale, debug=False, score_fn=score_fn, mask_fn=mask_fn, block_mask_fn=block_mask_fn,
               compiled_loop=compiled_loop)
     dq_call = flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, None, block_b=1, block_q=block_q,
@@ -85,8 +95,8 @@ class _FlexAttention(torch.autograd.Function):
         want_dq = ctx.needs_input_grad[0] or want_dab
         # (not at the head dimension 64 kernels, which hand nothing over: recomputing there beats 128 padded columns)
         exchange = (want_dkv and ctx.needs_input_grad[0] and ab is None and q.dtype == torch.bfloat16 and
-                    call_head_dim(q.shape[-1], q.dtype, sm_scale, score_fn, ab, spec_of(mask_fn, block_mask_fn), q.shape[2], k.shape[2]) != 64 and
-                    ds_exchange_pays(score_fn, mask_fn, segment_ids))
+                    ds_exchange_pays(score_fn, mask_fn, segment_ids) and
+                    call_head_dim(q.shape[-1], q.dtype, sm_scale, score_fn, ab, spec_of(mask_fn, block_mask_fn), q.shape[2], k.shape[2]) != 64)
         # di = sum(o * do), float32 [B, H, Sq] (jax_exp.py:276-278): taken by the dq pass itself where that pass runs
         # first (no dS hand-over), else by its own launch
         di = None
@@ -148,7 +158,6 @@ def flex_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, score_fn: 
         mask_fn, block_mask_fn = mask_fns, None
     else:
         mask_fn, block_mask_fn = mask_fns if mask_fns is not None else (None, None)
-    from ._common import tagged_closures
     score_fn, mask_fn, block_mask_fn = tagged_closures(score_fn, mask_fn, block_mask_fn, block_q, block_k)
     opts = (score_fn, mask_fn, block_mask_fn, segment_ids, bool(causal), float(sm_scale), int(block_q), int(block_k))
     return _FlexAttention.apply(q, k, v, ab, opts)

@@ -14,7 +14,11 @@ import torch
 from . import _lib
 from ._common import (on_device, bias_c, check_blocks, check_doc_batches, check_qkv, dtype_code, kernel_block_map, call_head_dim, library_for, pad_seq,
                       padded_len, mostly_partial_custom_mask, resolve_mask, score_spec_c, stream_of, tagged_closures, tile_lengths)
+from . import _plans
 from .block_mask import mask_spec_c, spec_of
+from .masks import MaskSpec
+
+_CAUSAL = MaskSpec(flags=_lib.MASK_CAUSAL)
 
 
 def _decode(q, k, v, mask_fn, block_mask_fn, save_residuals, sm_scale):
@@ -68,6 +72,12 @@ def _flex_attention_impl(q, k, v, ab, segment_ids, save_residuals, causal, sm_sc
             if debug:
                 print(f"[flexattn_fwd_decode] B={B} Hq={Hq} Hkv={Hkv} Sq={Sq} Sk={Sk} D={D} dtype={q.dtype}")
             return out
+    if score_fn is None and ab is None and segment_ids is None and not compiled_loop and not debug:
+        spec = spec_of(mask_fn, block_mask_fn)
+        if causal:
+            spec = spec.combine(_CAUSAL)
+        if _plans.takes(q, k, spec, sm_scale):
+            return _plans.forward(q, k, v, spec, float(sm_scale), save_residuals)
     # (lengths below one tile: the tensors are zero-padded to it, a document id of their own drops the padded keys
     # and the padded query rows are cut off again)
     Sq_p, Sk_p = padded_len(Sq), padded_len(Sk)
