@@ -33,6 +33,7 @@ MASK_S2 = 8
 MASK_CUSTOM = 16
 
 FLAG_COMPILED_LOOP = 1
+FLAG_WIDE_DS = 16
 
 PASS_FWD = 0
 PASS_DQ = 1

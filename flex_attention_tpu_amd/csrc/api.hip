@@ -136,7 +136,7 @@ static int tile_shape(int pass, int dtype, int D, int* bq, int* bk) {
 static int check_scale_flags(float sm_scale, int flags) {
   if (!(sm_scale > 0.f) || !(sm_scale < __builtin_huge_valf()))
     return set_error(FLEXATTN_EINVAL, "sm_scale must be positive and finite (got %g)", (double)sm_scale);
-  if (flags & ~FLEXATTN_FLAG_COMPILED_LOOP) return set_error(FLEXATTN_EINVAL, "unknown flags 0x%x", flags);
+  if (flags & ~(FLEXATTN_FLAG_COMPILED_LOOP | FLEXATTN_FLAG_WIDE_DS)) return set_error(FLEXATTN_EINVAL, "unknown flags 0x%x", flags);
   return FLEXATTN_OK;
 }
 
@@ -195,9 +195,10 @@ static bool dkv_on_stream(const flexattn_bwd_params* p) {
 // bias out of their dS), and so does the dk/dv kernel with a compiled main loop, for every score (compiled score
 // functions among them: the dq pass from dS then evaluates none).  Looks at shapes, score, flags and the map's size.
 static bool ds_exchange_ok(const flexattn_bwd_params* p) {
-  if (p == nullptr || p->dtype != FLEXATTN_BF16 || p->D != 128) return false;
+  if (p == nullptr || p->dtype != FLEXATTN_BF16) return false;
+  if (p->D != 128 && !(p->D == 256 && (p->flags & FLEXATTN_FLAG_WIDE_DS))) return false;
   if (p->B <= 0 || p->Hq <= 0 || p->Hkv <= 0 || p->Sq <= 0 || p->Sk <= 0) return false;
-  if (dkv_on_stream(p) && p->score.kind != FLEXATTN_SCORE_NONE && p->score.kind != FLEXATTN_SCORE_SOFTCAP) return false;
+  if (p->D == 128 && dkv_on_stream(p) && p->score.kind != FLEXATTN_SCORE_NONE && p->score.kind != FLEXATTN_SCORE_SOFTCAP) return false;
   int bq = 0, bk = 0;
   bwd_dkv_bf16_d128_tile(&bq, &bk);
   if (p->Sq % bq != 0 || p->Sk % bk != 0) return false;
@@ -208,7 +209,7 @@ static bool ds_exchange_ok(const flexattn_bwd_params* p) {
 // What the dq pass multiplies K by: the streams export dS without sm_scale (softcap: without its factor 4 either),
 // the kernel with a compiled main loop exports it complete.
 static float ds_out_scale(const flexattn_bwd_params* p) {
-  if (!dkv_on_stream(p)) return 1.0f;
+  if (p->D != 128 || !dkv_on_stream(p)) return 1.0f;
   return (p->score.kind == FLEXATTN_SCORE_SOFTCAP ? 4.f : 1.f) * p->sm_scale;
 }
 
@@ -479,7 +480,7 @@ int flexattn_bwd_delta(const void* o, const void* dout, float* delta, int64_t ro
 }
 
 static int launch_dq(const flexattn_bwd_params* p, BwdArgs a, hipStream_t s) {
-  if (p->ds != nullptr) return bwd_dq_from_ds(a, ds_out_scale(p), s);
+  if (p->ds != nullptr) return bwd_dq_from_ds(a, p->D, ds_out_scale(p), s);
   if (p->dtype == FLEXATTN_BF16) {
     if (a.dab != nullptr) a.flags |= FLEXATTN_FLAG_COMPILED_LOOP;  // (the generated streams store no bias gradient)
     return p->D == 256 ? bwd_dq_bf16_d256(a, s) : p->D == 64 ? bwd_dq_bf16_d64(a, s) : bwd_dq_bf16_d128(a, s);

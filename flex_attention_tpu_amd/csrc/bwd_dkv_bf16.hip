@@ -350,7 +350,10 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
 // 64-row tile one LDS tile (tile_io.hpp) at [buffer][panel]; a loop iteration covers 64 q rows (half an entry of the
 // kv tile's list: the two buffers of Q and dO panels then take the LDS the 128-row steps take at head dim 128), the
 // contractions of S and dP run over the panels, dk^T and dv^T have four accumulators per panel.
-template <int SCORE, int NP, bool AB>
+// EXPORT: the pass also writes its bf16 dS, as bwd_dkv_bf16_d128_kernel does: at two panels the dq pass that recomputes S
+// and dP costs three products of a 256-deep contraction, from dS one (B=4, H=16, S=4096, causal, forward and backward: 3.61
+// -> 3.08 ms).
+template <int SCORE, int NP, bool EXPORT, bool AB>
 __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
   using namespace dkv_cfg;
   constexpr bool kNoBias = SCORE == FLEXATTN_SCORE_NONE || !AB;   // (a bias without a score function: kScoreBiasOnly)
@@ -550,6 +553,14 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
       } else {
         elementwise(std::false_type{});
       }
+      if constexpr (EXPORT) {
+        // (the block layout of bwd_dkv_bf16_d128_kernel's export; 32-row block 2 (it & 1) + c of the q tile)
+        char* blk = static_cast<char*>(a.ds) +
+                    ((size_t)(b * a.Hq + hk * group + (it >> 1) / n_tiles) * (size_t)a.ds_pairs + (size_t)a.ds_col[kb] +
+                     (size_t)((it >> 1) % n_tiles)) * kDsBlockBytes + 8192 * w + 16 * (2 * l32 + hh);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) *reinterpret_cast<bf16x8*>(blk + 1024 * (4 * (it & 1) + 2 * c + u)) = dsb[u];
+      }
 
       // dv^T += dO^T P, dk^T += Q^T dS, a panel at a time (the transposed fragments of one panel are live at once)
 #pragma unroll
@@ -601,21 +612,25 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
   }
 }
 
-template <int SCORE, int NP, bool AB = true>
-static int launch_dkv_wide(const BwdArgs& a, hipStream_t stream) {
+template <int SCORE, int NP, bool EXPORT, bool AB = true>
+static int launch_dkv_wide_on(const BwdArgs& a, hipStream_t stream) {
   if constexpr (AB && splits_bias(SCORE))
-    if (a.score.ab == nullptr) return launch_dkv_wide<SCORE, NP, false>(a, stream);
+    if (a.score.ab == nullptr) return launch_dkv_wide_on<SCORE, NP, EXPORT, false>(a, stream);
   if constexpr (SCORE == FLEXATTN_SCORE_NONE)
-    if (a.score.ab != nullptr) return launch_dkv_wide<kScoreBiasOnly, NP>(a, stream);
+    if (a.score.ab != nullptr) return launch_dkv_wide_on<kScoreBiasOnly, NP, EXPORT>(a, stream);
   using namespace dkv_cfg;
   constexpr int kLds = 4 * NP * kTileElems * 2 + 4 * 64 * 4;   // (Q, dO) x 2 buffers x NP panels; lse, delta x 2 buffers
-  auto kern = bwd_dkv_bf16_wide_kernel<SCORE, NP, AB>;
+  auto kern = bwd_dkv_bf16_wide_kernel<SCORE, NP, EXPORT, AB>;
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dkv): %s", hipGetErrorString(attr));
   const int n_wg = a.B * a.Hkv * a.map.nk;
   hipLaunchKernelGGL(kern, dim3(n_wg), dim3(256), kLds, stream, a);
   return check_launch("flexattn_bwd_dkv bf16");
+}
+template <int SCORE, int NP>
+static int launch_dkv_wide(const BwdArgs& a, hipStream_t stream) {
+  return a.ds != nullptr ? launch_dkv_wide_on<SCORE, NP, true>(a, stream) : launch_dkv_wide_on<SCORE, NP, false>(a, stream);
 }
 
 #ifndef FLEXATTN_CUSTOM_ONLY

@@ -1,4 +1,4 @@
-// dq from exported dS (bf16, head dim 128): dq = out_scale * dS K, one contraction per (q tile, kv tile) pair
+// dq from exported dS (bf16, head dim 128, or 256 as two panels of 128 columns): dq = out_scale * dS K, one contraction per (q tile, kv tile) pair
 // instead of the three of the recomputing dq kernel (S = Q K^T, dP = dO V^T, dq += dS K).
 //
 // The dk/dv stream kernel (bwd_dkv_bf16.hip, EXPORT) leaves every step's bf16 dS in a buffer of 32 KB blocks, one
@@ -26,11 +26,10 @@ namespace fa {
 namespace dqds_cfg {
 constexpr int BQ = 128;
 constexpr int BNK = 128;
-constexpr int D = 128;
 constexpr int STAGE_KV = 32;                       // kv columns per pipeline stage: one wave's share of a dS block
 constexpr int PARTS = BNK / STAGE_KV;              // stages per kv tile
 constexpr int DS_STAGE_BYTES = BQ * STAGE_KV * 2;  // 8 KB
-constexpr int K_STAGE_BYTES = STAGE_KV * D * 2;    // 8 KB: 32 rows of a K tile in the layout of tile_io.hpp
+constexpr int K_PANEL_BYTES = STAGE_KV * 128 * 2;  // 8 KB: 32 rows of a panel of K in the layout of tile_io.hpp
 #ifndef DQDS_NDS
 #define DQDS_NDS 6
 #define DQDS_NK 3
@@ -51,12 +50,19 @@ constexpr int OCC = DQDS_OCC;                      // work-groups per CU
 constexpr bool PRODUCERS = DQDS_PRODUCERS != 0;
 constexpr int THREADS = PRODUCERS ? 512 : 256;
 constexpr int MAX_LIST = 1024;
-constexpr int K_RING = NDS * DS_STAGE_BYTES;       // LDS offset of the K ring
-constexpr int LDS_BYTES = NDS * DS_STAGE_BYTES + NK * K_STAGE_BYTES + MAX_LIST * 4;
 constexpr size_t kDsBlockBytes = (size_t)BQ * BNK * 2;
-static_assert(NK >= 2 && NDS >= 2 && NDS <= 17 && NK <= 10, "the wait counts are written for up to 15 stages behind");
-static_assert(LDS_BYTES <= 160 * 1024 / OCC, "the rings must fit the CU's LDS");
-static_assert(NDS * DS_STAGE_BYTES >= 4 * 8192, "the epilogue stages 8 KB per wave in the dS ring");
+// The rings of NP panels.  Two panels double the accumulators: one work-group per CU then, with deeper rings.
+template <int NP>
+struct Rings {
+  static constexpr int NDS = NP == 1 ? dqds_cfg::NDS : 10;
+  static constexpr int NK = NP == 1 ? dqds_cfg::NK : 4;
+  static constexpr int K_STAGE_BYTES = NP * K_PANEL_BYTES;
+  static constexpr int K_RING = NDS * DS_STAGE_BYTES;       // LDS offset of the K ring
+  static constexpr int LDS_BYTES = NDS * DS_STAGE_BYTES + NK * K_STAGE_BYTES + MAX_LIST * 4;
+  static_assert(NK >= 2 && NDS >= 2 && NDS <= 17 && NP * NK <= 10, "the wait counts are written for up to 15 stages behind");
+  static_assert(LDS_BYTES <= 160 * 1024 / (NP == 1 ? OCC : 1), "the rings must fit the CU's LDS");
+  static_assert(NDS * DS_STAGE_BYTES >= 4 * 8192, "the epilogue stages 8 KB per wave in the dS ring");
+};
 static_assert(MAX_LIST == 1024, "a list entry packs the kv tile into 10 bits");
 }  // namespace dqds_cfg
 
@@ -66,10 +72,15 @@ __device__ __forceinline__ void wait_vmem_but() {
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
+// NP: panels of 128 columns of K and dq.  A work-group takes both panels of its q tile: dS, which is what the launch
+// waits for, is read once.
+template <int NP>
 __global__ __launch_bounds__(dqds_cfg::THREADS, dqds_cfg::OCC) void bwd_dq_from_ds_kernel(BwdArgs a, float out_scale) {
   using namespace dqds_cfg;
+  constexpr int D = 128 * NP;
+  constexpr int NDS = Rings<NP>::NDS, NK = Rings<NP>::NK, K_STAGE_BYTES = Rings<NP>::K_STAGE_BYTES, K_RING = Rings<NP>::K_RING;
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
-  int* sIdx = reinterpret_cast<int*>(smem_raw + NDS * DS_STAGE_BYTES + NK * K_STAGE_BYTES);
+  int* sIdx = reinterpret_cast<int*>(smem_raw + K_RING + NK * K_STAGE_BYTES);
 
   const int nQ = a.map.nq, nK = a.map.nk;
   const int n_wg = a.B * a.Hq * nQ;
@@ -115,7 +126,7 @@ __global__ __launch_bounds__(dqds_cfg::THREADS, dqds_cfg::OCC) void bwd_dq_from_
     // the two 16-lane groups of a half-wave read pieces u = 0 and u = 1 at the same offset, which would be the same
     // banks; the swap puts them on the two halves of the banks)
     goff[i] = w < 2 ? (unsigned)piece * 1024u + (lane16 ^ (128u * (unsigned)(piece & 1)))
-                    : (unsigned)(row * kTileD + (((lane & 15) ^ swz(row)) << 3)) * 2u;
+                    : (unsigned)(row * D + (((lane & 15) ^ swz(row)) << 3)) * 2u;
   }
 
   // stage s = part s % PARTS of the list's kv tile s / PARTS: that part's dS as it lies in the block and its 32 K
@@ -136,17 +147,19 @@ __global__ __launch_bounds__(dqds_cfg::THREADS, dqds_cfg::OCC) void bwd_dq_from_
       dst = lds0 + K_RING + (unsigned)(s % NK) * K_STAGE_BYTES + (unsigned)(w - 2) * 4096u;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < 4; ++i) {   // (K: a piece of every panel each)
       if (ds_wave)  // (dS is read once: nt keeps it from displacing the head's K in the L2)
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
                      :
                      : "v"(goff[i]), "s"(src), "s"(dst + 1024u * i)
                      : "memory", "m0", "vcc");
       else
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                     :
-                     : "v"(goff[i]), "s"(src), "s"(dst + 1024u * i)
-                     : "memory", "m0", "vcc");
+#pragma unroll
+        for (int pn = 0; pn < NP; ++pn)
+          asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                       :
+                       : "v"(goff[i]), "s"(src + 256 * pn), "s"(dst + 1024u * i + (unsigned)(K_PANEL_BYTES * pn))
+                       : "memory", "m0", "vcc");
     }
   };
   const int ring = ds_wave ? NDS : NK;  // the wave's kind of stage is copied ring - 1 stages ahead
@@ -168,11 +181,11 @@ __global__ __launch_bounds__(dqds_cfg::THREADS, dqds_cfg::OCC) void bwd_dq_from_
   const int k_chunk = 2 * ((lane & 31) >> 4) + ((l16 & 3) >> 1);
   const int k_half = 4 * (l16 & 1);
 
-  f32x16 acc[2][2];  // [qi][di]
+  f32x16 acc[2][2 * NP];  // [qi][2 panel + di]
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < 4 * NP; ++t)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[t >> 1][t & 1][i] = 0.f;
+    for (int i = 0; i < 16; ++i) acc[t & 1][t >> 1][i] = 0.f;
 
   const int n_stages = PARTS * n_list;
   if (copies)
@@ -181,7 +194,7 @@ __global__ __launch_bounds__(dqds_cfg::THREADS, dqds_cfg::OCC) void bwd_dq_from_
     // the wave's copy of stage s has landed once only its copies of the stages behind it are open
     int behind = n_stages - 1 - s;
     if (behind > ring - 2) behind = ring - 2;
-    if (copies) switch (behind) {
+    if (copies) switch (ds_wave ? behind : NP * behind) {   // (four copies a piece of each panel)
       case 0: wait_vmem_but<0>(); break;
       case 1: wait_vmem_but<4>(); break;
       case 2: wait_vmem_but<8>(); break;
@@ -206,7 +219,7 @@ __global__ __launch_bounds__(dqds_cfg::THREADS, dqds_cfg::OCC) void bwd_dq_from_
     const bf16_t* sK = reinterpret_cast<const bf16_t*>(smem_raw + K_RING + (s % NK) * K_STAGE_BYTES);
 #pragma unroll
     for (int ks = 0; ks < STAGE_KV / 16; ++ks) {
-      bf16x8 bfrag[2], afrag[2];
+      bf16x8 bfrag[2], afrag[2 * NP];
 #pragma unroll
       for (int qi = 0; qi < 2; ++qi) {
         const char* dsp = st + 8192 * (ks >> 1) + 512 * (ks & 1) + 2048 * qi + ds_off;
@@ -215,17 +228,18 @@ __global__ __launch_bounds__(dqds_cfg::THREADS, dqds_cfg::OCC) void bwd_dq_from_
         bfrag[qi] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7));
       }
 #pragma unroll
-      for (int di = 0; di < 2; ++di) {
+      for (int di = 0; di < 2 * NP; ++di) {
         const int r = 16 * ks + k_row;
-        const int db = 2 * wd + di;
-        const s16x4 a0 = lds_read_tr16(sK + tile_off(r, 4 * db + k_chunk) + k_half);
-        const s16x4 a1 = lds_read_tr16(sK + tile_off(r + 4, 4 * db + k_chunk) + k_half);
+        const int db = 2 * wd + (di & 1);
+        const bf16_t* panel = sK + (di >> 1) * (K_PANEL_BYTES / 2);
+        const s16x4 a0 = lds_read_tr16(panel + tile_off(r, 4 * db + k_chunk) + k_half);
+        const s16x4 a1 = lds_read_tr16(panel + tile_off(r + 4, 4 * db + k_chunk) + k_half);
         afrag[di] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
       }
 #pragma unroll
       for (int qi = 0; qi < 2; ++qi)
 #pragma unroll
-        for (int di = 0; di < 2; ++di) acc[qi][di] = mfma32(afrag[di], bfrag[qi], acc[qi][di]);
+        for (int di = 0; di < 2 * NP; ++di) acc[qi][di] = mfma32(afrag[di], bfrag[qi], acc[qi][di]);
     }
   }
   __syncthreads();  // the rings are free: the start of LDS stages the tile's 128 dq rows, 8 KB per 32-row q block
@@ -234,50 +248,60 @@ __global__ __launch_bounds__(dqds_cfg::THREADS, dqds_cfg::OCC) void bwd_dq_from_
   // four complete 256-byte rows; lane: q row lane & 31 of block 2 wq + qi, head columns 32 (2 wd + di) + 8 g + 4 hh + 0..3
   const int row_here = lane & 31;
   const unsigned wr = (unsigned)row_here * 256u + 8u * (unsigned)hh;
-  if (computes) {
-#pragma unroll
-    for (int qi = 0; qi < 2; ++qi)
-#pragma unroll
-      for (int di = 0; di < 2; ++di)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x16& x = acc[qi][di];
-          const bf16x2 lo = pack_bf16(x[4 * g] * out_scale, x[4 * g + 1] * out_scale);
-          const bf16x2 hi = pack_bf16(x[4 * g + 2] * out_scale, x[4 * g + 3] * out_scale);
-          const bf16x4 out = {lo[0], lo[1], hi[0], hi[1]};
-          *reinterpret_cast<bf16x4*>(smem_raw + (2 * wq + qi) * 8192 + wr
-                                     + (unsigned)(((4 * (2 * wd + di) + g) ^ (row_here & 15)) << 4)) = out;
-        }
-  }
-  __syncthreads();
-  if (!computes) return;
-  const char* stage = smem_raw + w * 8192;  // wave w stores q block w
   const int q0 = tile_base(qb, BQ, a.Sq);
-  bf16_t* dQg = static_cast<bf16_t*>(a.dq) + ((size_t)bh * a.Sq + (size_t)q0 + (size_t)w * 32) * D;
   const int r_first = qb * BQ - q0 - w * 32;   // (rows before it belong to the q tile before)
-  const int chunk = lane & 15;
+  bf16_t* dQg = static_cast<bf16_t*>(a.dq) + ((size_t)bh * a.Sq + (size_t)q0 + (size_t)w * 32) * D;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = 4 * i + (lane >> 4);
-    if (r < r_first) continue;
-    const unsigned rd = (unsigned)r * 256u + (unsigned)((chunk ^ (r & 15)) << 4);
-    *reinterpret_cast<u32x4*>(dQg + (size_t)r * D + chunk * 8) = *reinterpret_cast<const u32x4*>(stage + rd);
+  for (int pn = 0; pn < NP; ++pn) {
+    if (pn > 0) __syncthreads();   // (the panel before has been read from the stage)
+    if (computes) {
+#pragma unroll
+      for (int qi = 0; qi < 2; ++qi)
+#pragma unroll
+        for (int di = 0; di < 2; ++di)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x16& x = acc[qi][2 * pn + di];
+            const bf16x2 lo = pack_bf16(x[4 * g] * out_scale, x[4 * g + 1] * out_scale);
+            const bf16x2 hi = pack_bf16(x[4 * g + 2] * out_scale, x[4 * g + 3] * out_scale);
+            const bf16x4 out = {lo[0], lo[1], hi[0], hi[1]};
+            *reinterpret_cast<bf16x4*>(smem_raw + (2 * wq + qi) * 8192 + wr
+                                       + (unsigned)(((4 * (2 * wd + di) + g) ^ (row_here & 15)) << 4)) = out;
+          }
+    }
+    __syncthreads();
+    if (computes) {
+      const char* stage = smem_raw + w * 8192;  // wave w stores q block w
+      const int chunk = lane & 15;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = 4 * i + (lane >> 4);
+        if (r < r_first) continue;
+        const unsigned rd = (unsigned)r * 256u + (unsigned)((chunk ^ (r & 15)) << 4);
+        *reinterpret_cast<u32x4*>(dQg + (size_t)r * D + 128 * pn + chunk * 8) = *reinterpret_cast<const u32x4*>(stage + rd);
+      }
+    }
   }
 }
 
+template <int NP>
+static int launch_from_ds(const BwdArgs& a, float out_scale, hipStream_t stream) {
+  using namespace dqds_cfg;
+  auto kern = bwd_dq_from_ds_kernel<NP>;
+  constexpr int kLds = Rings<NP>::LDS_BYTES;
+  static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+  if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dq from dS): %s", hipGetErrorString(attr));
+  hipLaunchKernelGGL(kern, dim3(a.B * a.Hq * a.map.nq), dim3(THREADS), kLds, stream, a, out_scale);
+  return check_launch("flexattn_bwd_dq (from dS) bf16");
+}
+
 // `a.map`: row lists of the block map at the dk/dv kernel's 128 x 128 tiles; `a.ds`: the buffer that kernel filled.
-int bwd_dq_from_ds(const BwdArgs& a, float out_scale, hipStream_t stream) {
+int bwd_dq_from_ds(const BwdArgs& a, int D, float out_scale, hipStream_t stream) {
   using namespace dqds_cfg;
   if (a.map.nk > MAX_LIST) return set_error(FLEXATTN_ENOTSUP, "dq from dS: %d kv tiles, at most %d", a.map.nk, MAX_LIST);
   if (a.ds_rank == nullptr || a.ds_pairs <= 0 || a.ds_pairs > (1ll << 20))
     return set_error(FLEXATTN_EINVAL, "dq from dS: no index of the dS blocks (or more than 2^20 kept tile pairs)");
-  auto kern = bwd_dq_from_ds_kernel;
-  static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
-  if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dq from dS): %s", hipGetErrorString(attr));
-  const int n_wg = a.B * a.Hq * a.map.nq;
-  hipLaunchKernelGGL(kern, dim3(n_wg), dim3(THREADS), LDS_BYTES, stream, a, out_scale);
-  return check_launch("flexattn_bwd_dq (from dS) bf16");
+  return D == 256 ? launch_from_ds<2>(a, out_scale, stream) : launch_from_ds<1>(a, out_scale, stream);
 }
 
 }  // namespace fa

@@ -93,9 +93,11 @@ class _FlexAttention(torch.autograd.Function):
         dq = dk = dv = ds = dab = None
         want_dkv = ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
         want_dq = ctx.needs_input_grad[0] or want_dab
+        # (at head dimension 256 always: the recomputing dq pass costs three products of twice the depth.  On B=4, H=16,
+        # S=4096, causal, forward and backward: 3.61 -> 3.08 ms.)
         # (not at the head dimension 64 kernels, which hand nothing over: recomputing there beats 128 padded columns)
         exchange = (want_dkv and ctx.needs_input_grad[0] and ab is None and q.dtype == torch.bfloat16 and
-                    ds_exchange_pays(score_fn, mask_fn, segment_ids) and
+                    (q.shape[-1] > 128 or ds_exchange_pays(score_fn, mask_fn, segment_ids)) and
                     call_head_dim(q.shape[-1], q.dtype, sm_scale, score_fn, ab, spec_of(mask_fn, block_mask_fn), q.shape[2], k.shape[2]) != 64)
         # di = sum(o * do), float32 [B, H, Sq] (jax_exp.py:276-278): taken by the dq pass itself where that pass runs
         # first (no dS hand-over), else by its own launch
@@ -120,7 +122,7 @@ class _FlexAttention(torch.autograd.Function):
             dk, dv, ds = flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, block_b=1, block_q=block_q,
                                                  block_q_major=block_q, block_k_major=block_k, block_k=block_k,
                                                  sm_scale=sm_scale, causal=causal, debug=False, score_fn=score_fn,
-                                                 mask_fn=mask_fn, block_mask_fn=block_mask_fn, return_ds=True) \
+                                                 mask_fn=mask_fn, block_mask_fn=block_mask_fn, return_ds=True, _wide_ds=True) \
                 if exchange else (*flash_attention_bwd_dkv(
                     k, v, q, ab, segment_ids, l, m, di, do, block_b=1, block_q=block_q, block_q_major=block_q,
                     block_k_major=block_k, block_k=block_k, sm_scale=sm_scale, causal=causal, debug=False,

@@ -15,7 +15,7 @@ from .flex_attention_dq_bwd import DsBlocks, alloc_ds, bwd_params
 
 def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=None, block_q, block_q_major,
                             block_k_major, block_k, sm_scale, causal, debug, score_fn=None, mask_fn=None,
-                            block_mask_fn=None, compiled_loop=False, return_ds=False, _defer=False):
+                            block_mask_fn=None, compiled_loop=False, return_ds=False, _defer=False, _wide_ds=False):
     """(dk, dv): dv = P^T do, dk = dS^T * d(score)/dk with P recomputed from (l, m) and
     dS = P (dP - di) (flex_attention_dkv_kernel.py:237-272).  With grouped KV heads the gradients
     of all query heads of a group are summed inside the kernel.  ``causal`` is honoured
@@ -54,6 +54,8 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
         return {"params": p, "lib": lib, "finish": lambda: (dk, dv), "keep": (q, k, v, do, l, m, di, ab_keep, bm)}
     with on_device(q.device):
         if return_ds:
+            if _wide_ds and D == 256:   # (flex_attention's own backward: head dimension 256 hands dS over too)
+                p.flags |= _lib.FLAG_WIDE_DS
             p.ds_index.pairs = 1   # (asks whether the kernels of the call exchange at all, before the index is built)
             if lib.flexattn_bwd_ds_bytes(C.byref(p)) > 0:
                 p.ds_index = bm.ds_index_c()

@@ -168,6 +168,8 @@ def flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, d, *, block_b, 
         p.dab = dab_full.data_ptr()
     if ds is not None:
         p.ds, p.ds_bytes = ds.buf.data_ptr(), ds.buf.numel()
+        if D == 256:
+            p.flags |= _lib.FLAG_WIDE_DS
         col, rank, pairs = ds.index   # (the index the dk/dv pass wrote the blocks by)
         p.ds_index = _lib.DsIndexC(col.data_ptr(), rank.data_ptr(), pairs)
     if return_delta and return_dab:

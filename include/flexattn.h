@@ -120,6 +120,9 @@ typedef struct flexattn_bias {
  * score kind and list length).  Both meet the stated tolerances; the flag selects the compiled one
  * for a call, for comparisons and tests. */
 #define FLEXATTN_FLAG_COMPILED_LOOP 1
+/* backward, bf16, head dimension 256: the call hands dS over too (flexattn_bwd_ds_bytes is 0 at that head dimension
+ * without the flag); the dk/dv call, the dq call and the question for the bytes must agree on it. */
+#define FLEXATTN_FLAG_WIDE_DS 16
 
 /* Ragged sequence lengths.  Sq and Sk of a call are multiples of the pass's tiles (flexattn_tile_shape); tensors whose
  * lengths are not name the next multiples and the rows by which these exceed them: the tensors, the row vectors, the
@@ -267,7 +270,7 @@ int flexattn_build_ds_index(const flexattn_block_map* map, int32_t* col, int32_t
  * instead of two).  Returns the bytes `ds` must hold for the request
  * described by p (B Hq ds_index.pairs 32 KB: one block per query head and kept tile pair; only shapes, dtype, D,
  * flags, score, ab, the map's nq and ds_index.pairs are looked at), or 0 when the kernels of the request exchange
- * nothing (fp32, head dimension 256, the global position bias with one query head per kv head, more than
+ * nothing (fp32, head dimension 64, 256 without FLEXATTN_FLAG_WIDE_DS, the global position bias with one query head per kv head, more than
  * 1024 tiles along a sequence, ds_index.pairs <= 0): then ds must stay NULL.
  * Order: flexattn_bwd_dkv with p->ds set, then flexattn_bwd_dq with the same p->ds on the same stream (or
  * ordered behind it) and the same score, ab and flags (they decide which dk/dv kernel wrote the buffer, and with
