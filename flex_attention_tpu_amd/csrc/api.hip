@@ -255,8 +255,9 @@ static int to_bwd_args(const flexattn_bwd_params* p, int pass, BwdArgs* a) {
   if ((rc = check_doc_batches(p->mask, p->B)) != FLEXATTN_OK) return rc;
   if ((rc = check_bias(p->ab, p->B, p->Hq, Sq, Sk)) != FLEXATTN_OK) return rc;
   if (p->dab != nullptr) {
-    if (pass != FLEXATTN_PASS_DQ) return set_error(FLEXATTN_EINVAL, "dab is an output of flexattn_bwd_dq");
-    if (p->ds != nullptr) return set_error(FLEXATTN_EINVAL, "dab and ds exclude each other (the dq pass from dS recomputes nothing)");
+    if (pass == FLEXATTN_PASS_DKV && (p->ds == nullptr || p->ab.ptr == nullptr || p->D != 128))
+      return set_error(FLEXATTN_EINVAL, "dab is an output of flexattn_bwd_dq, or of a flexattn_bwd_dkv call with ab and ds at head dim 128");
+    if (pass == FLEXATTN_PASS_DQ && p->ds != nullptr) return set_error(FLEXATTN_EINVAL, "dab and ds exclude each other (the dq pass from dS recomputes nothing)");
   }
   a->dab = p->dab;
   a->o = p->o;

@@ -81,6 +81,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
   using namespace dkv_cfg;
   constexpr bool kBias = SCORE == kScoreBiasOnly;             // a bias and no score function: launched as a kind of its own
   constexpr bool kNoBias = SCORE == FLEXATTN_SCORE_NONE || !AB;
+  constexpr bool kDab = EXPORT && !kNoBias;
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
   bf16_t* sQ = reinterpret_cast<bf16_t*>(smem_raw);
   bf16_t* sDO = sQ + 4 * kTileElems;
@@ -208,10 +209,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
     // An additive bias: the values of a 32-row block are loaded a block ahead of their use (the first block's in front of
     // its products).  Loaded where they are added, behind the products, the latency of every load showed: 1310 -> 456 us
     // on B=4, H=16, S=1500 (dq, the same: 841 -> 400; forward 532 -> 166).
+    const unsigned lane_off = (unsigned)(4 * hh) * (unsigned)a.Sk + (unsigned)k_idx;   // (of a bias or its gradient)
     float bias_next[16];
     auto load_bias = [&](int row0) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) bias_next[e] = sm.bias2(row0 + acc_row(e, hh), k_idx);
+      for (int e = 0; e < 16; ++e) bias_next[e] = sm.bias2_rows(row0 + acc_row(e, 0), lane_off);
     };
     if (kBias) load_bias(q0);
 #pragma unroll
@@ -259,6 +261,10 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
         }
 
       bf16x8 pb[2], dsb[2];
+      // (EXPORT with a bias: the bias gradient too, where the call asks for it: float32 [B, Hq, Sq, Sk], a row's 32 columns per store)
+      char* dab_block = nullptr;   // (the same in every lane)
+      if (kDab && a.dab != nullptr)
+        dab_block = reinterpret_cast<char*>(a.dab + ((size_t)(b * a.Hq + hk * group + it / n_tiles) * a.Sq + (size_t)(q0 + 32 * cc)) * a.Sk);
       auto elementwise = [&](auto masked) {
         constexpr bool MASKED = decltype(masked)::value;
         const bool has_doc = MASKED && (mk.flags & FLEXATTN_MASK_DOC) != 0;
@@ -279,12 +285,17 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
             const int i = q0 + r0 + u;
             const float tv = sm.to_log2(s_acc[e], i, k_idx);
             float pe = fast_exp2(tv + (kBias ? bias[e] : kNoBias ? 0.f : sm.bias2(i, k_idx)) - lse4[u]);
-            float gd = pe * (dp_acc[e] - dl4[u]) * sm.dfactor(tv, s_acc[e], i, k_idx);
+            float gl = pe * (dp_acc[e] - dl4[u]);   // the gradient of the logit itself: what an additive bias receives
+            if (!kNoBias) asm("" : "+v"(gl));   // (rounded here with and without export: dk and dv keep their bits)
+            float gd = gl * sm.dfactor(tv, s_acc[e], i, k_idx);
             if (MASKED) {
-              const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j) & (32 * cc + 8 * g4 + u >= own);
+              const bool kept = keep_elem(mk, i, k_idx, di[u], doc_j);
+              const bool keep = kept & (32 * cc + 8 * g4 + u >= own);
+              if (kDab) gl = kept ? gl : 0.f;   // (rows and columns of the tiles before get the value those store, too)
               pe = keep ? pe : 0.f;
               gd = keep ? gd : 0.f;
             }
+            if (kDab && a.dab != nullptr) *reinterpret_cast<float*>(dab_block + (size_t)(unsigned)((8 * g4 + u) * a.Sk) * 4 + 4u * lane_off) = gl;
             pv[u] = pe;
             dsv[u] = gd;
           }

@@ -492,6 +492,15 @@ struct ScoreMod {
     return v * kLog2e;
   }
 
+  // The same of element (i + 4 hh, j), i the same in every lane: a scalar address and one offset per lane, lane_off =
+  // 4 hh ab_ld + j.
+  __device__ __forceinline__ float bias2_rows(int i, unsigned lane_off) const {
+    const unsigned long long at = (unsigned long long)(unsigned)(ab_row0 + i) * (unsigned)ab_ld;
+    const float v = ab_f32 ? *reinterpret_cast<const float*>(ab_base + 4 * at + 4u * lane_off)
+                           : __builtin_bit_cast(float, (unsigned)*reinterpret_cast<const unsigned short*>(ab_base + 2 * at + 2u * lane_off) << 16);
+    return v * kLog2e;
+  }
+
   // The same of the elements (i, j0 .. j0 + 3): one 16-byte (bf16: 8-byte) load, of any alignment.  (Four loads at
   // j0 + u, u = 0..3, each take an address of their own in registers, because j0 + u is a 32-bit sum: 32 of them per
   // tile made the kernels spill.)

@@ -10,12 +10,12 @@ import torch
 from . import _lib
 from ._common import (on_device, bias_c, check_blocks, check_doc_batches, check_qkv, check_rows, kernel_block_map, call_head_dim, kernel_head_dim, library_for, pad_seq,
                       padded_len, resolve_mask, stream_of, tagged_closures)
-from .flex_attention_dq_bwd import DsBlocks, alloc_ds, bwd_params
+from .flex_attention_dq_bwd import DsBlocks, alloc_dab, alloc_ds, bwd_params, reduce_dab
 
 
 def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=None, block_q, block_q_major,
                             block_k_major, block_k, sm_scale, causal, debug, score_fn=None, mask_fn=None,
-                            block_mask_fn=None, compiled_loop=False, return_ds=False, _defer=False, _wide_ds=False):
+                            block_mask_fn=None, compiled_loop=False, return_ds=False, _defer=False, _wide_ds=False, _dab=False):
     """(dk, dv): dv = P^T do, dk = dS^T * d(score)/dk with P recomputed from (l, m) and
     dS = P (dP - di) (flex_attention_dkv_kernel.py:237-272).  With grouped KV heads the gradients
     of all query heads of a group are summed inside the kernel.  ``causal`` is honoured
@@ -52,6 +52,7 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
         if Sk_p != Sk or Sq_p != Sq or D != D_user or return_ds:
             return None
         return {"params": p, "lib": lib, "finish": lambda: (dk, dv), "keep": (q, k, v, do, l, m, di, ab_keep, bm)}
+    dab = None
     with on_device(q.device):
         if return_ds:
             if _wide_ds and D == 256:   # (flex_attention's own backward: head dimension 256 hands dS over too)
@@ -64,9 +65,14 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
                 if buf is not None:
                     ds = DsBlocks(buf, (B, Hq, Sq_p, Sk_p), index=bm.ds_index(), compiled_loop=bool(compiled_loop))
                     p.ds, p.ds_bytes = buf.data_ptr(), need
+                    if _dab and D == 128:   # (flex_attention's own backward: the bias gradient next to the dS it comes from)
+                        dab = alloc_dab(spec, B, Hq, Sq_p, Sk_p, q.device)
+                        p.dab = dab.data_ptr()
             if ds is None:
                 p.ds_index = _lib.DsIndexC()
         _lib.check(lib.flexattn_bwd_dkv(C.byref(p), stream_of(q)), lib)
     if Sk_p != Sk or D != D_user:
         dk, dv = dk[:, :, :Sk, :D_user].contiguous(), dv[:, :, :Sk, :D_user].contiguous()
+    if _dab:
+        return dk, dv, ds, reduce_dab(dab, ab, Sq, Sk) if dab is not None else None
     return (dk, dv, ds) if return_ds else (dk, dv)

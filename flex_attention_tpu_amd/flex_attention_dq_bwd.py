@@ -64,6 +64,23 @@ def alloc_ds(nbytes: int, device):
         return None
 
 
+def alloc_dab(spec, B, Hq, Sq, Sk, device):
+    """The kernels' output for the bias gradient, one value per logit.  (Only the tiles the block map visits are written:
+    masked-out pairs have no gradient; without a mask that is every element, and the clearing, 70 us for B=4, H=16,
+    S=1500, is left out.)"""
+    new = torch.empty if spec.flags == 0 else torch.zeros
+    return new(B, Hq, Sq, Sk, dtype=torch.float32, device=device)
+
+
+def reduce_dab(dab, ab, Sq, Sk):
+    """The bias gradient in ab's shape and dtype: padding cut off, summed over the dimensions ``ab`` broadcasts."""
+    dab = dab[:, :, :Sq, :Sk]
+    for dim in (0, 1):
+        if ab.shape[dim] == 1 and dab.shape[dim] > 1:
+            dab = dab.sum(dim, keepdim=True)
+    return dab.to(ab.dtype).contiguous()
+
+
 def ds_exchange_pays(score_fn, mask_fn=None, segment_ids=None) -> bool:
     """Whether handing dS from the dk/dv pass to the dq pass is expected to shorten the backward: yes with the
     softcap score (eight element-wise operations per score in the recomputing dq kernel) and with masks that
@@ -161,10 +178,7 @@ def flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, d, *, block_b, 
     if return_dab:
         if ab is None or ds is not None:
             raise ValueError("return_dab needs the additive bias `ab` and excludes `ds`")
-        # (only the tiles the block map visits are written: masked-out pairs have no gradient; without a mask that is
-        # every element, and the clearing, 70 us for B=4, H=16, S=1500, is left out)
-        new = torch.empty if spec.flags == 0 else torch.zeros
-        dab_full = new(B, Hq, Sq_p, Sk_p, dtype=torch.float32, device=q.device)
+        dab_full = alloc_dab(spec, B, Hq, Sq_p, Sk_p, q.device)
         p.dab = dab_full.data_ptr()
     if ds is not None:
         p.ds, p.ds_bytes = ds.buf.data_ptr(), ds.buf.numel()
@@ -186,12 +200,7 @@ def flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, d, *, block_b, 
             d_out = d_p[:, :, :Sq].contiguous()
         if not return_dab:
             return (out, d_out) if return_delta else out
-        dab = dab_full[:, :, :Sq, :Sk]
-        if ab.shape[0] == 1 and B > 1:
-            dab = dab.sum(0, keepdim=True)
-        if ab.shape[1] == 1 and Hq > 1:
-            dab = dab.sum(1, keepdim=True)
-        return out, dab.to(ab.dtype).contiguous()
+        return out, reduce_dab(dab_full, ab, Sq, Sk)
 
     if _defer:   # (flex_attention_bwd launches this pass together with the dk/dv pass)
         return {"params": p, "lib": lib, "finish": finish, "keep": keep, "delta": d if d_p is d else None}

@@ -174,7 +174,8 @@ typedef struct flexattn_bwd_params {
   void* ds;
   int64_t ds_bytes;
   flexattn_ds_index ds_index; /* needed with ds; for the map at the granularity of FLEXATTN_PASS_DKV */
-  /* Gradient of the additive bias, or NULL: out of flexattn_bwd_dq, float32 [B, Hq, Sq, Sk] (full shape: the caller
+  /* Gradient of the additive bias, or NULL: out of flexattn_bwd_dq, or of a flexattn_bwd_dkv call that hands dS over (ds
+   * and ab set, head dimension 128; the dq call from that dS has none), float32 [B, Hq, Sq, Sk] (full shape: the caller
    * sums over the dimensions its bias broadcasts).  dab = P (dP - delta), the gradient with respect to the logits
    * (the reference declares this output next to dk, dv, flash_attention_dkv_bwd.py:103-107,130-138, and its upstream
    * dq kernel writes it, jax_exp.py:1252-1255, there multiplied by sm_scale).  Only the tiles the block map visits

@@ -1,0 +1,49 @@
+"""flex_attention's gradients with a trained bias (the bias gradient out of the dk/dv pass, dq from its dS) at the edges of
+the tiles, for every way a bias broadcasts, masks, grouped heads, scores and bias dtypes, against the oracle on the kernels'
+own forward.  Tolerances: helpers.assert_close; the bias gradient P (dP - delta) by its values, relative where they
+exceed 1, as the dq pass's is in test_gpu_ragged."""
+import math
+
+import pytest
+import torch
+
+from helpers import assert_close, same_residual_grads
+from oracle import mha_oracle as O
+from test_gpu_ragged import surrounded
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D", [(1, 2, 2, 128, 128, 128), (2, 4, 2, 129, 257, 128), (3, 2, 1, 321, 255, 64), (2, 2, 2, 100, 300, 96)])
+@pytest.mark.parametrize("ab_shape", ["11", "1h", "b1", "bh"])
+@pytest.mark.parametrize("kind", ["plain", "causal", "softcap", "bf16 bias"])
+def test_bias_gradient(kind, ab_shape, B, Hq, Hkv, Sq, Sk, D):
+    import flex_attention_tpu_amd as F
+    from flex_attention_tpu_amd import masks, scores
+    sc, pair, sfn, okw = 1 / math.sqrt(D), None, None, {}
+    if kind == "causal":
+        pair, okw = masks.make_causal_mask_fns(128, 128), dict(causal=True)
+    elif kind == "softcap":
+        sfn, okw = scores.make_softcap_score_fn(5.0), dict(score_mod=O.score_mod_softcap(5.0))
+    ab = torch.randn(B if ab_shape[0] == "b" else 1, Hq if ab_shape[1] == "h" else 1, Sq, Sk, generator=torch.Generator().manual_seed(3))
+    if kind == "bf16 bias":
+        ab = ab.bfloat16()
+    okw["ab"] = ab.float().expand(B, Hq, Sq, Sk)
+    q, k, v, do = O.make_inputs(B, Hq, Hkv, Sq, Sk, D, dtype=torch.bfloat16, seed=Sq + D)
+    qg, kg, vg, abg = [surrounded(x).requires_grad_(True) for x in (q, k, v, ab)]
+    o = F.flex_attention(qg, kg, vg, sfn, pair, sm_scale=sc, ab=abg)
+    dq, dk, dv, dab = torch.autograd.grad(o, (qg, kg, vg, abg), surrounded(do))
+    mf = pair or (None, None)
+    with torch.no_grad():
+        o2, l, m = F._flex_attention_impl(qg, kg, vg, abg, None, True, False, sc, 1, 128, 128, 128, False, mf[1], mf[0], sfn)
+    assert torch.equal(o2, o)
+    same = same_residual_grads(q, k, v, do, o, l, m, sm_scale=sc, **okw)
+    for name, t, r in zip(("dq", "dk", "dv"), (dq, dk, dv), same):
+        assert_close(name, t, r, torch.bfloat16)
+    ref = O.mha_bwd_reference(q, k, v, o.detach().float().cpu(), do, l.cpu(), m.cpu(), sm_scale=sc, return_dab=True, **okw)[3]
+    for dim in (0, 1):
+        if ab.shape[dim] == 1:
+            ref = ref.sum(dim, keepdim=True)
+    assert dab.shape == ab.shape and dab.dtype == ab.dtype
+    err = (dab.cpu().double() - ref).abs()
+    assert O.rel_l2(dab, ref) <= 1e-2 and bool((err <= 1e-2 * ref.abs().clamp(min=1.0)).all()), float(err.max())
