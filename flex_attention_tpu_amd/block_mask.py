@@ -40,7 +40,10 @@ class LRU:
     def get(self, key):
         v = self._d.get(key)
         if v is not None:
-            self._d.move_to_end(key)
+            try:
+                self._d.move_to_end(key)
+            except KeyError:   # (dropped by another thread in between: the value in hand is as good)
+                pass
         return v
 
     def put(self, key, value):

@@ -76,12 +76,14 @@ struct PinnedState {
 // derivative and sm_scale in them) to a.ds, in the block layout of the generated streams' export (see there), for
 // the dq pass from dS: a score function is then evaluated in one backward pass instead of two.
 // AB: the call may have an additive bias (false: splits_bias() kinds without one).
-template <int SCORE, bool EXPORT, bool AB>
+// DAB (with EXPORT and a bias): the kernel stores the bias gradient as well.  (A variant of its own: with the stores behind
+// a test the compiler associates the element-wise sums differently, and dk and dv would change a bit with the export.)
+template <int SCORE, bool EXPORT, bool AB, bool DAB>
 __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
   using namespace dkv_cfg;
   constexpr bool kBias = SCORE == kScoreBiasOnly;             // a bias and no score function: launched as a kind of its own
   constexpr bool kNoBias = SCORE == FLEXATTN_SCORE_NONE || !AB;
-  constexpr bool kDab = EXPORT && !kNoBias;
+  static_assert(!DAB || (EXPORT && !kNoBias), "the bias gradient comes with the export of a call with a bias");
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
   bf16_t* sQ = reinterpret_cast<bf16_t*>(smem_raw);
   bf16_t* sDO = sQ + 4 * kTileElems;
@@ -267,9 +269,9 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
         }
 
       bf16x8 pb[2], dsb[2];
-      // (EXPORT with a bias: the bias gradient too, where the call asks for it: float32 [B, Hq, Sq, Sk], a row's 32 columns per store)
+      // (DAB: the bias gradient, float32 [B, Hq, Sq, Sk], a row's 32 columns per store)
       char* dab_block = nullptr;   // (the same in every lane)
-      if (kDab && a.dab != nullptr)
+      if (DAB)
         dab_block = reinterpret_cast<char*>(a.dab + ((size_t)(b * a.Hq + hk * group + it / n_tiles) * a.Sq + (size_t)(q0 + 32 * cc)) * a.Sk);
       auto elementwise = [&](auto masked) {
         constexpr bool MASKED = decltype(masked)::value;
@@ -293,16 +295,15 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
             const float tv = sm.to_log2(s_acc[e], i, k_idx);
             float pe = fast_exp2(tv + (kBias ? bias[e] : kNoBias ? 0.f : sm.bias2(i, k_idx)) - lse4[u]);
             float gl = pe * (dp_acc[e] - dl4[u]);   // the gradient of the logit itself: what an additive bias receives
-            if (!kNoBias) asm("" : "+v"(gl));   // (rounded here with and without export: dk and dv keep their bits)
             float gd = gl * sm.dfactor(tv, s_acc[e], i, k_idx);
             if (MASKED) {
               const bool kept = keep_elem(mk, i, k_idx, di[u], doc_j);
               const bool keep = kept & (32 * cc + 8 * g4 + u >= own);
-              if (kDab) gl = kept ? gl : 0.f;   // (rows and columns of the tiles before get the value those store, too)
+              if (DAB) gl = kept ? gl : 0.f;   // (rows and columns of the tiles before get the value those store, too)
               pe = keep ? pe : 0.f;
               gd = keep ? gd : 0.f;
             }
-            if (kDab && a.dab != nullptr) *reinterpret_cast<float*>(dab_block + (size_t)(unsigned)((8 * g4 + u) * a.Sk) * 4 + 4u * lane_off) = gl;
+            if (DAB) *reinterpret_cast<float*>(dab_block + (size_t)(unsigned)((8 * g4 + u) * a.Sk) * 4 + 4u * lane_off) = gl;
             pv[u] = pe;
             dsv[u] = gd;
           }
@@ -1171,12 +1172,14 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
 
 #endif  // FLEXATTN_CUSTOM_ONLY
 
-template <int SCORE, bool EXPORT, bool AB = true>
+template <int SCORE, bool EXPORT, bool AB = true, bool DAB = false>
 static int launch_dkv_on(const BwdArgs& a, hipStream_t stream) {
   if constexpr (AB && splits_bias(SCORE))
     if (a.score.ab == nullptr) return launch_dkv_on<SCORE, EXPORT, false>(a, stream);
+  if constexpr (EXPORT && AB && !DAB && SCORE != FLEXATTN_SCORE_NONE)
+    if (a.dab != nullptr) return launch_dkv_on<SCORE, true, true, true>(a, stream);   // (the caller has checked that there is a bias)
   using namespace dkv_cfg;
-  auto kern = bwd_dkv_bf16_d128_kernel<SCORE, EXPORT, AB>;
+  auto kern = bwd_dkv_bf16_d128_kernel<SCORE, EXPORT, AB, DAB>;
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dkv): %s", hipGetErrorString(attr));
