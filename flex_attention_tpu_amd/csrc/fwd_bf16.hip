@@ -517,7 +517,9 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
     r.sa = r.sb = r.head = 0u;
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
-      const int qb = min(2 * qb2 + x, nQ - 1);  // (a missing second tile repeats the first; nothing of it is stored)
+      // (a missing second tile repeats the first, states and all, and nothing of it is stored: with states of its own, empty
+      // ones, every step of the item, the longest under a causal mask, would be a masked one)
+      const int qb = min(2 * qb2 + x, nQ - 1);
       const int q0 = tile_base(qb, BM, a.Sq);
       rows_load<HD>(r.q[x], static_cast<const bf16_t*>(a.q) + ((size_t)bh * a.Sq + (size_t)q0 + w_here * 32) * D, lane_here);
       r.doc[x] = (a.mask.flags & FLEXATTN_MASK_DOC) ? a.mask.doc_q[dq_rows + q0 + row_here] : 0;
@@ -527,16 +529,15 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
         r.khi[x] = ranged ? a.mask.doc_q_range[2 * (dq_rows + q0 + row_here) + 1] : 0;
       }
       const uint8_t* row = a.map.state + (size_t)qb * nK;
-      const bool valid = 2 * qb2 + x < nQ;
       unsigned packed = 0u;
 #pragma unroll
       for (int j = 0; j < kListRegs; ++j) {
         const int t = tid_here + 256 * j;
-        const unsigned v = (valid && t < nK) ? row[t] : 0u;
+        const unsigned v = t < nK ? row[t] : 0u;
         packed |= v << (8 * j);
       }
       if (x == 0) r.sa = packed; else r.sb = packed;
-      const unsigned hv = (valid && lane_here < nK) ? row[lane_here] : 0u;
+      const unsigned hv = lane_here < nK ? row[lane_here] : 0u;
       r.head |= hv << (8 * x);
     }
   };
@@ -627,7 +628,6 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
       // rows longer than the prefetched part (more than 65536 tokens): the rest of the two state rows straight
       // from global memory (an item is then thousands of steps long: the wait does not show)
       const int qa = min(2 * qb2, nQ - 1), qb_ = min(2 * qb2 + 1, nQ - 1);
-      const bool valid_b = 2 * qb2 + 1 < nQ;
       const uint8_t* row_a = a.map.state + (size_t)qa * nK;
       const uint8_t* row_b = a.map.state + (size_t)qb_ * nK;
       for (int base = PREFETCH_LIST; base < nK; base += 256) {
@@ -635,7 +635,7 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
         unsigned sa = 0u, sb = 0u;
         if (t < nK) {
           sa = row_a[t];
-          sb = valid_b ? row_b[t] : 0u;
+          sb = row_b[t];
           sStA[t] = (unsigned char)sa;
           sStB[t] = (unsigned char)sb;
         }
@@ -653,7 +653,7 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
     // then have a closed form (keep_bits32_range) and no ids are read
     const bool ranged = DOCS && a.mask.doc_q_range != nullptr && keep_bits_have_range(a.mask);
     // (first row of each q tile; the last tile of a ragged length starts early, see tile_base)
-    const int q_at[2] = {tile_base(2 * qb2, BM, a.Sq), 2 * qb2 + 1 < nQ ? tile_base(2 * qb2 + 1, BM, a.Sq) : (2 * qb2 + 1) * BM};
+    const int q_at[2] = {tile_base(2 * qb2, BM, a.Sq), tile_base(min(2 * qb2 + 1, nQ - 1), BM, a.Sq)};
     const int q_idx[2] = {q_at[0] + q_local, q_at[1] + q_local};
     // softmax state of the lane's two q rows (log2 domain): reference maximum M, running maximum
     // relative to it, sum of 2^(score - M)
