@@ -117,6 +117,13 @@ __host__ __device__ __forceinline__ int tile_base(int t, int tile, int len) {
   const int at = t * tile;
   return at + tile <= len ? at : len - tile;
 }
+// The elements of tile t that are its own, counted from row `from` behind the strip's first row `row0`: those at or behind
+// the returned offset; none where the strip's column belongs to the tile before (`own_col` false).  What a work-group
+// writes to memory besides its result rows (the bias gradient) it writes for its own elements only: another
+// work-group writes the others, in no order to this one.
+__host__ __device__ __forceinline__ int first_owned(int t, int tile, int row0, int from, bool own_col) {
+  return own_col ? t * tile - row0 - from : 1 << 20;
+}
 __host__ __device__ __forceinline__ int tiles_of(int len, int tile) { return (len + tile - 1) / tile; }
 
 struct FwdArgs {

@@ -47,3 +47,26 @@ def test_bias_gradient(kind, ab_shape, B, Hq, Hkv, Sq, Sk, D):
     assert dab.shape == ab.shape and dab.dtype == ab.dtype
     err = (dab.cpu().double() - ref).abs()
     assert O.rel_l2(dab, ref) <= 1e-2 and bool((err <= 1e-2 * ref.abs().clamp(min=1.0)).all()), float(err.max())
+
+
+@pytest.mark.parametrize("kind", ["plain", "causal", "alibi"])
+def test_bias_gradient_repeats_bit_for_bit(kind):
+    """Elements that the last tile of a ragged length shares with the tile before have one writer: the same bits from
+    every run, on a grid that fills the chip (4 x 16 heads, 12 kv tiles)."""
+    import flex_attention_tpu_amd as F
+    from flex_attention_tpu_amd import masks, scores
+    B, H, S, D = 4, 16, 1500, 128
+    pair = masks.make_causal_mask_fns(128, 128) if kind == "causal" else None
+    sfn = scores.make_alibi_global_score_fn(H) if kind == "alibi" else None
+    q, k, v, do = (x.cuda() for x in O.make_inputs(B, H, H, S, S, D, dtype=torch.bfloat16, seed=9))
+    ab = torch.randn(B, H, S, S, generator=torch.Generator().manual_seed(1)).cuda()
+    for t in (q, k, v, ab):
+        t.requires_grad_(True)
+
+    def call():
+        o = F.flex_attention(q, k, v, sfn, pair, sm_scale=1.0 if sfn else 1 / math.sqrt(D), ab=ab)
+        return torch.autograd.grad(o, (q, k, v, ab), do)
+    want = call()
+    for _ in range(4):
+        for name, a, b in zip(("dq", "dk", "dv", "dab"), call(), want):
+            assert torch.equal(a, b), name
