@@ -24,10 +24,34 @@ from .flex_attention_dq_bwd import compute_delta, ds_exchange_pays, flex_attenti
 from .flex_attention_kernel import _CAUSAL, _flex_attention_impl
 
 
-# The backward hands dS from the dk/dv pass to the dq pass (DsBlocks in flex_attention_dq_bwd.py) when both
-# gradients are wanted and the hand-over is expected to pay (ds_exchange_pays).  The buffer holds one 32 KB block
-# per query head and kept pair of 128 x 128 tiles (what the mask skips takes no room); the dk/dv entry point
-# declines it, and the dq pass recomputes, when it would take more than half of the free device memory.
+def _hands_ds_over(q, k, ab, segment_ids, sm_scale, score_fn, mask_fn, block_mask_fn, want_dab) -> bool:
+    """Whether a backward that wants every gradient hands dS from the dk/dv pass to the dq pass (DsBlocks in
+    flex_attention_dq_bwd.py).  The buffer holds one 32 KB block per query head and kept pair of 128 x 128 tiles (what the
+    mask skips takes no room)."""
+    if q.dtype != torch.bfloat16:
+        return False
+    D = q.shape[-1]
+    if want_dab:   # (the bias gradient is the fp32 dS that the dk/dv pass rounds for the hand-over: one pass makes both, and the dq
+        return D <= 128   # pass is one product instead of three; B=4, H=16, S=1500, forward and backward: 1.19 -> 1.03 ms)
+    if ab is not None:
+        return False
+    # (at head dimension 256 always: the recomputing dq pass costs three products of twice the depth.  On B=4, H=16,
+    # S=4096, causal, forward and backward: 3.61 -> 3.08 ms.  Not at the head dimension 64 kernels, which hand nothing over.)
+    return ((D > 128 or ds_exchange_pays(score_fn, mask_fn, segment_ids)) and
+            call_head_dim(D, q.dtype, sm_scale, score_fn, ab, spec_of(mask_fn, block_mask_fn), q.shape[2], k.shape[2]) != 64)
+
+
+def _bwd_with_ds(q, k, v, ab, segment_ids, l, m, o, do, want_dab, *, block_q, block_k, **kw):
+    """(dq, dk, dv, dab or None) with dS handed from the dk/dv pass to the dq pass; where the dk/dv entry point declines
+    to (no room for the buffer, kernels that exchange nothing), the dq pass recomputes."""
+    kw.update(block_b=1, block_q=block_q, block_k_major=block_k, block_k=block_k, debug=False)
+    di = compute_delta(o, do)
+    dk, dv, ds, *dab = flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, block_q_major=block_q, return_ds=True,
+                                               _wide_ds=not want_dab, _dab=want_dab, **kw)
+    if ds is None and want_dab:
+        dq, dab = flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, di, return_dab=True, **kw)
+        return dq, dk, dv, dab
+    return flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, di, ds=ds, **kw), dk, dv, (dab[0] if want_dab else None)
 
 
 def flex_attention_bwd(q, k, v, ab, segment_ids, l, m, o, do, *, block_q, block_k, sm_scale, causal=False, score_fn=None,
@@ -90,60 +114,32 @@ class _FlexAttention(torch.autograd.Function):
         score_fn, mask_fn, block_mask_fn, segment_ids, causal, sm_scale, block_q, block_k = ctx.opts
         want_dab = ab is not None and ctx.needs_input_grad[3]
         do = do.contiguous()
-        dq = dk = dv = ds = dab = None
+        dq = dk = dv = dab = None
         want_dkv = ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
         want_dq = ctx.needs_input_grad[0] or want_dab
-        # (at head dimension 256 always: the recomputing dq pass costs three products of twice the depth.  On B=4, H=16,
-        # S=4096, causal, forward and backward: 3.61 -> 3.08 ms.)
-        # (not at the head dimension 64 kernels, which hand nothing over: recomputing there beats 128 padded columns)
-        exchange = (want_dkv and ctx.needs_input_grad[0] and ab is None and q.dtype == torch.bfloat16 and
-                    (q.shape[-1] > 128 or ds_exchange_pays(score_fn, mask_fn, segment_ids)) and
-                    call_head_dim(q.shape[-1], q.dtype, sm_scale, score_fn, ab, spec_of(mask_fn, block_mask_fn), q.shape[2], k.shape[2]) != 64)
+        kw = dict(block_q=block_q, block_k=block_k, sm_scale=sm_scale, causal=causal, score_fn=score_fn, mask_fn=mask_fn,
+                  block_mask_fn=block_mask_fn)
+        if want_dkv and ctx.needs_input_grad[0] and _hands_ds_over(q, k, ab, segment_ids, sm_scale, score_fn, mask_fn, block_mask_fn, want_dab):
+            try:
+                return (*_bwd_with_ds(q, k, v, ab, segment_ids, l, m, o, do, want_dab, **kw), None)
+            except torch.cuda.OutOfMemoryError:
+                pass   # (beside the dS buffer there was no room for the rest: below nothing needs one)
+        if want_dkv and ctx.needs_input_grad[0] and not want_dab:
+            return (*flex_attention_bwd(q, k, v, ab, segment_ids, l, m, o, do, **kw), None, None)
+        kw.update(block_b=1, block_k_major=block_k, debug=False)
         # di = sum(o * do), float32 [B, H, Sq] (jax_exp.py:276-278): taken by the dq pass itself where that pass runs
-        # first (no dS hand-over), else by its own launch
+        # first, else by its own launch
         di = None
-        if want_dkv and ctx.needs_input_grad[0] and not want_dab and not exchange:
-            dq, dk, dv = flex_attention_bwd(q, k, v, ab, segment_ids, l, m, o, do, block_q=block_q, block_k=block_k,
-                                            sm_scale=sm_scale, causal=causal, score_fn=score_fn, mask_fn=mask_fn,
-                                            block_mask_fn=block_mask_fn)
-            return dq, dk, dv, None, None
-        if want_dab and want_dkv and ctx.needs_input_grad[0] and q.dtype == torch.bfloat16 and q.shape[-1] <= 128:
-            # (the bias gradient is the fp32 dS that the dk/dv pass rounds for the hand-over: one pass makes both, and the dq
-            # pass is one product instead of three; B=4, H=16, S=1500, forward and backward: 1.19 -> 1.03 ms)
-            di = compute_delta(o, do)
-            kw = dict(block_b=1, block_q=block_q, block_k_major=block_k, block_k=block_k, sm_scale=sm_scale, debug=False,
-                      score_fn=score_fn, mask_fn=mask_fn, block_mask_fn=block_mask_fn, causal=causal)
-            dk, dv, ds, dab = flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, block_q_major=block_q, return_ds=True,
-                                                      _dab=True, **kw)
-            if ds is not None:
-                return flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, di, ds=ds, **kw), dk, dv, dab, None
-            dq, dab = flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, di, return_dab=True, **kw)
-            return dq, dk, dv, dab, None
-        if want_dq and not exchange:
-            dq = flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, None, block_b=1, block_q=block_q,
-                                       block_k_major=block_k, block_k=block_k, sm_scale=sm_scale, debug=False,
-                                       score_fn=score_fn, mask_fn=mask_fn, block_mask_fn=block_mask_fn, causal=causal,
-                                       return_dab=want_dab, return_delta=not want_dab)
+        if want_dq:
+            dq = flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, None, return_dab=want_dab, return_delta=not want_dab, **kw)
             if want_dab:
                 dq, dab = dq
             else:
                 dq, di = dq
-        if di is None and want_dkv:
-            di = compute_delta(o, do)
         if want_dkv:
-            dk, dv, ds = flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, block_b=1, block_q=block_q,
-                                                 block_q_major=block_q, block_k_major=block_k, block_k=block_k,
-                                                 sm_scale=sm_scale, causal=causal, debug=False, score_fn=score_fn,
-                                                 mask_fn=mask_fn, block_mask_fn=block_mask_fn, return_ds=True, _wide_ds=True) \
-                if exchange else (*flash_attention_bwd_dkv(
-                    k, v, q, ab, segment_ids, l, m, di, do, block_b=1, block_q=block_q, block_q_major=block_q,
-                    block_k_major=block_k, block_k=block_k, sm_scale=sm_scale, causal=causal, debug=False,
-                    score_fn=score_fn, mask_fn=mask_fn, block_mask_fn=block_mask_fn), None)
-        if want_dq and exchange:
-            dq = flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, di, block_b=1, block_q=block_q,
-                                       block_k_major=block_k, block_k=block_k, sm_scale=sm_scale, debug=False,
-                                       score_fn=score_fn, mask_fn=mask_fn, block_mask_fn=block_mask_fn, causal=causal,
-                                       ds=ds)
+            if di is None:
+                di = compute_delta(o, do)
+            dk, dv = flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, block_q_major=block_q, **kw)
         return dq if ctx.needs_input_grad[0] else None, dk, dv, dab, None
 
 

@@ -21,9 +21,10 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
     of all query heads of a group are summed inside the kernel.  ``causal`` is honoured
     (the reference's north-star file ignores it; its mask-aware twin gets the same effect from
     ``mask_fn``).  ``return_ds=True`` returns (dk, dv, ds): ds is the pass's dS as a DsBlocks for
-    ``flex_attention_bwd_dq(..., ds=ds)``, or None when the kernels of the call exchange nothing (fp32, head
-    dimension 256, the global position bias with one query head per kv head) or the device has too little free memory for the buffer (one 32 KB
-    block per query head and kept pair of 128 x 128 tiles): the dq pass then recomputes as usual."""
+    ``flex_attention_bwd_dq(..., ds=ds)``, or None when the kernels of the call exchange nothing (fp32, the global position
+    bias with one query head per kv head, head dimension 256 unless flex_attention's own backward asks) or the device
+    has too little free memory for the buffer (one 32 KB block per query head and kept pair of 128 x 128 tiles): the dq
+    pass then recomputes as usual."""
     B, Hq, Hkv, Sq, Sk, D = check_qkv(q, k, v, do)
     score_fn, mask_fn, block_mask_fn = tagged_closures(score_fn, mask_fn, block_mask_fn, block_q, block_k_major)
     for name, t in (("l", l), ("m", m), ("di", di)):
@@ -59,17 +60,20 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
                 p.flags |= _lib.FLAG_WIDE_DS
             p.ds_index.pairs = 1   # (asks whether the kernels of the call exchange at all, before the index is built)
             if lib.flexattn_bwd_ds_bytes(C.byref(p)) > 0:
+                if _dab and D == 128:   # (flex_attention's own backward: the bias gradient next to the dS it comes from.  It is
+                    # needed with and without the hand-over, dS only with it: dS is what gives way where both do not fit)
+                    dab = alloc_dab(spec, B, Hq, Sq_p, Sk_p, q.device)
                 p.ds_index = bm.ds_index_c()
                 need = lib.flexattn_bwd_ds_bytes(C.byref(p))
                 buf = alloc_ds(need, q.device)
                 if buf is not None:
                     ds = DsBlocks(buf, (B, Hq, Sq_p, Sk_p), index=bm.ds_index(), compiled_loop=bool(compiled_loop))
                     p.ds, p.ds_bytes = buf.data_ptr(), need
-                    if _dab and D == 128:   # (flex_attention's own backward: the bias gradient next to the dS it comes from)
-                        dab = alloc_dab(spec, B, Hq, Sq_p, Sk_p, q.device)
+                    if dab is not None:
                         p.dab = dab.data_ptr()
             if ds is None:
                 p.ds_index = _lib.DsIndexC()
+                dab = None
         _lib.check(lib.flexattn_bwd_dkv(C.byref(p), stream_of(q)), lib)
     if Sk_p != Sk or D != D_user:
         dk, dv = dk[:, :, :Sk, :D_user].contiguous(), dv[:, :, :Sk, :D_user].contiguous()
