@@ -116,6 +116,11 @@ class BlockMap:
             self._ds_index = (col, rank, pairs)
         return self._ds_index
 
+    def ds_index_at_hand(self) -> bool:
+        """Whether ds_index() can be had here: it copies the number of pairs to the host when it is first built, which a
+        stream that is being captured refuses."""
+        return self._ds_index is not None or not torch.cuda.is_current_stream_capturing()
+
     def partial_share(self) -> float:
         """Share of the tiles that run which are partly masked (read back from the device once per map)."""
         if self._partial_share is None:

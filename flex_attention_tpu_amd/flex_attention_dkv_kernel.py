@@ -22,9 +22,10 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
     (the reference's north-star file ignores it; its mask-aware twin gets the same effect from
     ``mask_fn``).  ``return_ds=True`` returns (dk, dv, ds): ds is the pass's dS as a DsBlocks for
     ``flex_attention_bwd_dq(..., ds=ds)``, or None when the kernels of the call exchange nothing (fp32, the global position
-    bias with one query head per kv head, head dimension 256 unless flex_attention's own backward asks) or the device
-    has too little free memory for the buffer (one 32 KB block per query head and kept pair of 128 x 128 tiles): the dq
-    pass then recomputes as usual."""
+    bias with one query head per kv head, head dimension 256 unless flex_attention's own backward asks), the device has
+    too little free memory for the buffer (one 32 KB block per query head and kept pair of 128 x 128 tiles), or the call
+    is being captured into a graph and the mask's tile pairs have not been counted by a call before: the dq pass then
+    recomputes as usual."""
     B, Hq, Hkv, Sq, Sk, D = check_qkv(q, k, v, do)
     score_fn, mask_fn, block_mask_fn = tagged_closures(score_fn, mask_fn, block_mask_fn, block_q, block_k_major)
     for name, t in (("l", l), ("m", m), ("di", di)):
@@ -59,7 +60,7 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
             if _wide_ds and D == 256:   # (flex_attention's own backward: head dimension 256 hands dS over too)
                 p.flags |= _lib.FLAG_WIDE_DS
             p.ds_index.pairs = 1   # (asks whether the kernels of the call exchange at all, before the index is built)
-            if lib.flexattn_bwd_ds_bytes(C.byref(p)) > 0:
+            if lib.flexattn_bwd_ds_bytes(C.byref(p)) > 0 and bm.ds_index_at_hand():
                 if _dab and D == 128:   # (flex_attention's own backward: the bias gradient next to the dS it comes from.  It is
                     # needed with and without the hand-over, dS only with it: dS is what gives way where both do not fit)
                     dab = alloc_dab(spec, B, Hq, Sq_p, Sk_p, q.device)

@@ -1,5 +1,5 @@
 """The backward that hands dS from the dk/dv to the dq pass, where there is no room for the buffer, or not beside what else
-the backward needs: it falls back to the recomputing passes and returns what those
+the backward needs, or where its index cannot be built: it falls back to the recomputing passes and returns what those
 return, bit for bit."""
 import math
 import sys
@@ -76,3 +76,25 @@ def test_the_bias_gradient_is_allocated_before_ds(monkeypatch):
     monkeypatch.setattr(dkv, "alloc_dab", lambda *a: order.append("dab") or dab(*a))
     call()
     assert order == ["dab", "ds"]
+
+
+@pytest.mark.parametrize("kind", ["d256", "bias", "softcap"])
+def test_captured_without_a_call_before(kind):
+    """A capture of a shape that no call has had (the kernels themselves loaded by another shape): the number of tile pairs
+    would have to come back to the host, so the captured backward recomputes."""
+    from flex_attention_tpu_amd import _plans, block_mask
+    step(kind)[0]()
+    step(kind)[1]()
+    call, recompute = step(kind, S=467)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        got = call()
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        block_mask._map_cache.clear()   # (the captured call's map lives in the graph)
+        _plans._plans.clear()
+        assert same(got, recompute())
