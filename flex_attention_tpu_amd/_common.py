@@ -283,6 +283,12 @@ def call_head_dim(D: int, dtype, sm_scale, score_fn, ab, spec: MaskSpec, Sq: int
     return kernel_head_dim(D, dtype)
 
 
+def aligned(t: torch.Tensor) -> torch.Tensor:
+    """`t` at an address that is a multiple of 16 bytes, as the kernels' loads and their copies into LDS take it: a copy of
+    a view that starts at another one (a contiguous slice of a flat buffer, say)."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def pad_seq(t: torch.Tensor, n: int, dim: int = 2) -> torch.Tensor:
     """`t` zero-padded to n positions along `dim` (a copy only when padding is needed)."""
     have = t.shape[dim]

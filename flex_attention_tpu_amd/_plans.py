@@ -16,7 +16,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from ._common import call_head_dim, dtype_code, on_device, stream_of, tile_lengths
+from ._common import aligned, call_head_dim, dtype_code, on_device, stream_of, tile_lengths
 from .block_mask import LRU, build_block_map, mask_spec_c
 from .masks import MaskSpec
 
@@ -67,6 +67,7 @@ def takes(q, k, spec: MaskSpec, sm_scale) -> bool:
 def forward(q, k, v, spec: MaskSpec, sm_scale, save_residuals):
     """(o, l, m), or o, of a call that `takes` accepts."""
     plan = _plan((0, q.shape, k.shape, q.dtype, q.device, spec, sm_scale), q, k, spec, sm_scale, _lib.FwdParamsC, (_lib.PASS_FWD,))
+    q, k, v = aligned(q), aligned(k), aligned(v)
     o = torch.empty_like(q)
     l = m = None
     if save_residuals:
@@ -85,6 +86,7 @@ def backward(q, k, v, l, m, o, do, spec: MaskSpec, sm_scale):
     """(dq, dk, dv) of a call that `takes` accepts: delta, the dq and the dk/dv pass (flexattn_bwd)."""
     plan = _plan((1, q.shape, k.shape, q.dtype, q.device, spec, sm_scale), q, k, spec, sm_scale, _lib.BwdParamsC,
                  (_lib.PASS_DQ, _lib.PASS_DKV))
+    q, k, v, o, do = aligned(q), aligned(k), aligned(v), aligned(o), aligned(do)
     dq, dk, dv, delta = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v), torch.empty_like(l)
     pq = _lib.BwdParamsC.from_buffer_copy(plan.templates[0])
     pkv = _lib.BwdParamsC.from_buffer_copy(plan.templates[1])

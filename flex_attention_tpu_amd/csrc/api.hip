@@ -1,6 +1,8 @@
 // C ABI of libflexattn.so: argument validation and dispatch to the gfx950 kernels.
 #include <cstdarg>
+#include <cstdint>
 #include <cstdio>
+#include <initializer_list>
 #include <mutex>
 
 #include "fa_common.hpp"
@@ -149,6 +151,15 @@ static int check_pad(int pad, int Sq, int Sk, int bq, int bk) {
   return FLEXATTN_OK;
 }
 
+// Requests of ragged lengths and of bf16 head dimension 64: their operands lie where the caller's tensors lie, and the
+// kernels' 16-byte loads and copies into LDS take them from there.
+static int check_aligned(int pad, int dtype, int D, std::initializer_list<const void*> ptrs) {
+  if (pad == 0 && !(dtype == FLEXATTN_BF16 && D == 64)) return FLEXATTN_OK;
+  for (const void* q : ptrs)
+    if (reinterpret_cast<uintptr_t>(q) & 15) return set_error(FLEXATTN_EINVAL, "a tensor's address is no multiple of 16 bytes");
+  return FLEXATTN_OK;
+}
+
 // `tile_pass`: the pass whose tile granularity the map must have (the dq pass reads the dk/dv kernel's dS blocks at
 // that kernel's tiles)
 static int check_shape(int pass, int B, int Hq, int Hkv, int Sq, int Sk, int pad, int D, int dtype,
@@ -246,6 +257,7 @@ static int to_bwd_args(const flexattn_bwd_params* p, int pass, BwdArgs* a) {
   if (pass == FLEXATTN_PASS_DKV && (!p->dk || !p->dv)) return set_error(FLEXATTN_EINVAL, "dk or dv is NULL");
   int rc = check_ds(p);
   if (rc != FLEXATTN_OK) return rc;
+  if ((rc = check_aligned(p->pad, p->dtype, p->D, {p->q, p->k, p->v, p->dout, p->o, p->dq, p->dk, p->dv})) != FLEXATTN_OK) return rc;
   const int Sq = p->Sq - (p->pad & 0xffff), Sk = p->Sk - (p->pad >> 16);   // the tensors' lengths
   rc = check_shape(pass, p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->pad, p->D, p->dtype, p->map, p->ds ? FLEXATTN_PASS_DKV : -1);
   if (rc != FLEXATTN_OK) return rc;
@@ -295,7 +307,9 @@ static int fwd_with_map(const flexattn_fwd_params* p, const flexattn_block_map& 
   if (!p->q || !p->k || !p->v || !p->o) return set_error(FLEXATTN_EINVAL, "q, k, v or o is NULL");
   if ((p->l == nullptr) != (p->m == nullptr)) return set_error(FLEXATTN_EINVAL, "l and m must both be given or both NULL");
   const int Sq = p->Sq - (p->pad & 0xffff), Sk = p->Sk - (p->pad >> 16);   // the tensors' lengths
-  int rc = check_shape(FLEXATTN_PASS_FWD, p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->pad, p->D, p->dtype, map);
+  int rc = check_aligned(p->pad, p->dtype, p->D, {p->q, p->k, p->v, p->o});
+  if (rc != FLEXATTN_OK) return rc;
+  rc = check_shape(FLEXATTN_PASS_FWD, p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->pad, p->D, p->dtype, map);
   if (rc != FLEXATTN_OK) return rc;
   if ((rc = check_scale_flags(p->sm_scale, p->flags)) != FLEXATTN_OK) return rc;
   if ((rc = check_score(p->score)) != FLEXATTN_OK) return rc;
@@ -461,8 +475,9 @@ int flexattn_fwd_decode(const flexattn_fwd_params* p, void* work, int64_t work_b
   if (!p->q || !p->k || !p->v || !p->o) return set_error(FLEXATTN_EINVAL, "q, k, v or o is NULL");
   if ((p->l == nullptr) != (p->m == nullptr)) return set_error(FLEXATTN_EINVAL, "l and m must both be given or both NULL");
   if (!decode_ok(p)) return set_error(FLEXATTN_ENOTSUP, "not a request of flexattn_fwd_decode (flexattn_fwd_decode_bytes is -1)");
-  const int rc = check_scale_flags(p->sm_scale, p->flags);
+  int rc = check_scale_flags(p->sm_scale, p->flags);
   if (rc != FLEXATTN_OK) return rc;
+  if ((rc = check_aligned(1, p->dtype, p->D, {p->q, p->k, p->v, p->o, work})) != FLEXATTN_OK) return rc;
   const int64_t need = fwd_decode_bytes(p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->D);
   if (need > 0 && (work == nullptr || work_bytes < need))
     return set_error(FLEXATTN_EINVAL, "work holds %lld bytes, the request needs %lld", (long long)(work ? work_bytes : 0), (long long)need);

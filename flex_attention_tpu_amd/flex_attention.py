@@ -17,7 +17,7 @@ from typing import Callable, Optional, Tuple
 import torch
 
 from . import _lib, _plans
-from ._common import call_head_dim, check_blocks, check_qkv, check_rows, on_device, stream_of, tagged_closures
+from ._common import aligned, call_head_dim, check_blocks, check_qkv, check_rows, on_device, stream_of, tagged_closures
 from .block_mask import spec_of
 from .flex_attention_dkv_kernel import flash_attention_bwd_dkv
 from .flex_attention_dq_bwd import compute_delta, ds_exchange_pays, flex_attention_bwd_dq
@@ -71,6 +71,7 @@ def flex_attention_bwd(q, k, v, ab, segment_ids, l, m, o, do, *, block_q, block_
             spec = spec.combine(_CAUSAL)
         if _plans.takes(q, k, spec, sm_scale):
             return _plans.backward(q, k, v, l, m, o, do, spec, float(sm_scale))
+    q, k, v, do = aligned(q), aligned(k), aligned(v), aligned(do)   # (the two passes share them)
     kw = dict(sm_scale=sm_scale, debug=False, score_fn=score_fn, mask_fn=mask_fn, block_mask_fn=block_mask_fn,
               compiled_loop=compiled_loop)
     dq_call = flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, None, block_b=1, block_q=block_q,
@@ -100,7 +101,7 @@ class _FlexAttention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, ab, opts):
         score_fn, mask_fn, block_mask_fn, segment_ids, causal, sm_scale, block_q, block_k = opts
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+        q, k, v = (aligned(t.contiguous()) for t in (q, k, v))
         o, l, m = _flex_attention_impl(q, k, v, ab, segment_ids, True, causal, sm_scale, 1, block_q, block_k, block_k,
                                        False, block_mask_fn, mask_fn, score_fn)
         ctx.save_for_backward(q, k, v, o, l, m, *([ab] if ab is not None else []))
@@ -113,7 +114,7 @@ class _FlexAttention(torch.autograd.Function):
         ab = rest[0] if rest else None
         score_fn, mask_fn, block_mask_fn, segment_ids, causal, sm_scale, block_q, block_k = ctx.opts
         want_dab = ab is not None and ctx.needs_input_grad[3]
-        do = do.contiguous()
+        do = aligned(do.contiguous())
         dq = dk = dv = dab = None
         want_dkv = ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
         want_dq = ctx.needs_input_grad[0] or want_dab

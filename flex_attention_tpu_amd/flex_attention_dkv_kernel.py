@@ -8,7 +8,7 @@ import ctypes as C
 import torch
 
 from . import _lib
-from ._common import (on_device, bias_c, check_blocks, check_doc_batches, check_qkv, check_rows, kernel_block_map, call_head_dim, kernel_head_dim, library_for, pad_seq,
+from ._common import (aligned, on_device, bias_c, check_blocks, check_doc_batches, check_qkv, check_rows, kernel_block_map, call_head_dim, kernel_head_dim, library_for, pad_seq,
                       padded_len, resolve_mask, stream_of, tagged_closures)
 from .flex_attention_dq_bwd import DsBlocks, alloc_dab, alloc_ds, bwd_params, reduce_dab
 
@@ -41,7 +41,7 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
     # (a dS hand-over is at 128 columns)
     D_user, D = D, (call_head_dim(D, q.dtype, sm_scale, score_fn, ab, spec, Sq, Sk, compiled_loop) if not return_ds
                     else kernel_head_dim(D, q.dtype))   # smaller head dimensions: zero-padded columns
-    q, do, k, v = pad_seq(q, D, 3), pad_seq(do, D, 3), pad_seq(k, D, 3), pad_seq(v, D, 3)
+    q, do, k, v = (aligned(pad_seq(t, D, 3)) for t in (q, do, k, v))
     bm = kernel_block_map(_lib.PASS_DKV, spec, q, Sq_p, Sk_p, D, score_fn)
     dk = torch.empty_like(k)
     dv = torch.empty_like(v)

@@ -7,7 +7,7 @@ import ctypes as C
 import torch
 
 from . import _lib
-from ._common import (on_device, bias_c, check_blocks, check_doc_batches, check_qkv, check_rows, dtype_code, kernel_block_map, call_head_dim, kernel_head_dim, library_for,
+from ._common import (aligned, on_device, bias_c, check_blocks, check_doc_batches, check_qkv, check_rows, dtype_code, kernel_block_map, call_head_dim, kernel_head_dim, library_for,
                       pad_seq, padded_len, mostly_partial_custom_mask, resolve_mask, score_spec_c, stream_of, tagged_closures, tile_lengths)
 from .block_mask import mask_spec_c
 
@@ -23,6 +23,7 @@ def compute_delta(o: torch.Tensor, do: torch.Tensor) -> torch.Tensor:
     if D not in (64, 128) and not (D == 256 and o.dtype == torch.bfloat16):   # (zero columns add nothing to the sum)
         D = kernel_head_dim(D, o.dtype)
         o, do = pad_seq(o, D, 3), pad_seq(do, D, 3)
+    o, do = aligned(o), aligned(do)
     d = torch.empty(B, H, S, dtype=torch.float32, device=o.device)
     with on_device(o.device):
         _lib.check(_lib.load().flexattn_bwd_delta(o.data_ptr(), do.data_ptr(), d.data_ptr(), B * H * S, D,
@@ -159,8 +160,8 @@ def flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, d, *, block_b, 
     # (a dS hand-over is at 128 columns)
     D_user, D = D, (call_head_dim(D, q.dtype, sm_scale, score_fn, ab, spec, Sq, Sk, compiled_loop) if ds is None
                     else kernel_head_dim(D, q.dtype))   # smaller head dimensions: zero-padded columns
-    q, do, k, v = pad_seq(q, D, 3), pad_seq(do, D, 3), pad_seq(k, D, 3), pad_seq(v, D, 3)
-    o_p = pad_seq(pad_seq(o, Sq_p), D, 3) if fuse_delta else None
+    q, do, k, v = (aligned(pad_seq(t, D, 3)) for t in (q, do, k, v))
+    o_p = aligned(pad_seq(pad_seq(o, Sq_p), D, 3)) if fuse_delta else None
     if ds is not None and (ds.buf is None or ds.index is None or ds.shape != (B, Hq, Sq_p, Sk_p) or ds.buf.device != q.device
                            or ds.compiled_loop != bool(compiled_loop)):
         raise ValueError("ds does not come from a dk/dv pass of these arguments")

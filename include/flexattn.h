@@ -11,6 +11,8 @@
  *    Head dimension D: 128 or 256 for bf16, 64 or 128 for float32 (anything else: FLEXATTN_ENOTSUP); bf16 also 64 for
  *    plain scores without a bias, without dS hand-over and with flags 0 (pad the operands of others to 128 columns).
  *    q/o/do/dq have Hq heads, k/v/dk/dv have Hkv heads, Hq % Hkv == 0 (kv head = h / (Hq/Hkv)).
+ *    In requests with pad != 0, of bf16 head dimension 64 and of flexattn_fwd_decode they start at multiples of 16 bytes
+ *    (else FLEXATTN_EINVAL).
  *  - l, m, delta are float32 [B, Hq, Sq].
  *  - Every function returns FLEXATTN_OK or a negative error code, never throws or aborts, and
  *    records a message readable with flexattn_last_error_string() (thread-local).
