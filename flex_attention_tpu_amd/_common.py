@@ -238,6 +238,12 @@ def resolve_mask(mask_fn, block_mask_fn, causal, segment_ids, Sq, Sk, Sq_pad=Non
         dq_p = DocIds(np.pad(ids_q, tail(ids_q, Sq_pad - Sq), mode="edge"))
         dk_p = DocIds(np.pad(ids_k, tail(ids_k, Sk_pad - Sk), constant_values=pad_id))
         spec = MaskSpec(spec.flags | _lib.MASK_DOC, spec.window, spec.stride, dq_p, spec.custom, None if dk_p == dq_p else dk_p)
+    elif spec.flags & _lib.MASK_DOC and (Sq % SEQ_ALIGN or Sk % SEQ_ALIGN):
+        # (ids may cover more positions than a call of ragged lengths has: it takes the first ones)
+        ids_q, ids_k = spec.doc_ids, spec.doc_ids_k if spec.doc_ids_k is not None else spec.doc_ids
+        if (len(ids_q) > Sq or len(ids_k) > Sk) and len(ids_q) >= Sq and len(ids_k) >= Sk:
+            dq_p, dk_p = DocIds(ids_q.array[..., :Sq]), DocIds(ids_k.array[..., :Sk])
+            spec = MaskSpec(spec.flags, spec.window, spec.stride, dq_p, spec.custom, None if dk_p == dq_p else dk_p)
     return spec
 
 
