@@ -1,6 +1,7 @@
 """Host-side helpers shared by the three entry points: argument checks and C struct assembly."""
 from __future__ import annotations
 
+import functools
 import warnings
 import weakref
 from typing import Callable, Optional
@@ -278,13 +279,18 @@ def kernel_head_dim(D: int, dtype) -> int:
     return 128 if D <= 128 else 256
 
 
-def call_head_dim(D: int, dtype, sm_scale, score_fn, ab, spec: MaskSpec, Sq: int, Sk: int, compiled_loop=False) -> int:
-    """kernel_head_dim of one call: bf16 head dimensions up to 64 run at 64 where the generated streams take the call
-    (plain scores, no bias, no compiled mask, a scale that folds into bf16 Q as folded_scale_ok in fa_common.hpp says,
-    lists that fit their LDS caches), and zero-padded to 128 on the other kernels.  A training step on B=8, H=16,
-    S=2048, D=64, causal: 1.21 ms padded, of which 0.59 ms copies, clears and cuts, against 0.44 ms."""
+@functools.lru_cache(maxsize=256)
+def _head_dim_64_ok(pass_id: int, sm_scale: float, Sq: int, Sk: int) -> bool:
+    return bool(_lib.load().flexattn_takes_head_dim_64(pass_id, sm_scale, Sq, Sk))
+
+
+def call_head_dim(pass_id: int, D: int, dtype, sm_scale, score_fn, ab, spec: MaskSpec, Sq: int, Sk: int, compiled_loop=False) -> int:
+    """kernel_head_dim of one pass of a call: bf16 head dimensions up to 64 run at 64 where the generated streams take the
+    pass (plain scores, no bias, no compiled mask, lengths and, in the forward, a scale as flexattn_takes_head_dim_64 says),
+    and zero-padded to 128 on the other kernels.  A training step on B=8, H=16, S=2048, D=64, causal: 1.21 ms padded, of
+    which 0.59 ms copies, clears and cuts, against 0.44 ms."""
     if (dtype == torch.bfloat16 and 0 < D <= 64 and score_fn is None and ab is None and spec.custom is None and not compiled_loop
-            and 0.0 < sm_scale * 1.4426950408889634 * 8.0 <= 2.9 and max(Sq, Sk) <= 262144):
+            and _head_dim_64_ok(pass_id, float(sm_scale), Sq, Sk)):
         return 64
     return kernel_head_dim(D, dtype)
 

@@ -55,26 +55,28 @@ def _plan(key, q, k, spec, sm_scale, cls, passes) -> _Plan:
     return plan
 
 
-def takes(q, k, spec: MaskSpec, sm_scale) -> bool:
-    """Whether a checked call without score function and bias is a prepared one.  (Document ids keep arrays per stream,
+def takes(q, k, spec: MaskSpec, sm_scale, *passes: int) -> bool:
+    """Whether these passes of a checked call without score function and bias are prepared ones.  (Document ids keep arrays per stream,
     compiled masks their own libraries, and padded calls copy their operands: those go the general way.)"""
     Sq, D = q.shape[2], q.shape[3]
     Sk = k.shape[2]
     return (spec.doc_ids is None and spec.custom is None and Sq >= 128 and Sk >= 128
-            and call_head_dim(D, q.dtype, sm_scale, None, None, spec, Sq, Sk) == D)
+            and (D == 128 or all([call_head_dim(p, D, q.dtype, sm_scale, None, None, spec, Sq, Sk) == D for p in passes])))
 
 
 def forward(q, k, v, spec: MaskSpec, sm_scale, save_residuals):
     """(o, l, m), or o, of a call that `takes` accepts."""
     plan = _plan((0, q.shape, k.shape, q.dtype, q.device, spec, sm_scale), q, k, spec, sm_scale, _lib.FwdParamsC, (_lib.PASS_FWD,))
-    q, k, v = aligned(q), aligned(k), aligned(v)
+    qp, kp, vp = q.data_ptr(), k.data_ptr(), v.data_ptr()
+    if (qp | kp | vp) % 16:
+        return forward(aligned(q), aligned(k), aligned(v), spec, sm_scale, save_residuals)
     o = torch.empty_like(q)
     l = m = None
     if save_residuals:
         l = torch.empty(q.shape[:3], dtype=torch.float32, device=q.device)
         m = torch.empty_like(l)
     p = _lib.FwdParamsC.from_buffer_copy(plan.templates[0])
-    _FWD_POINTERS.pack_into(p, 0, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+    _FWD_POINTERS.pack_into(p, 0, qp, kp, vp, o.data_ptr(),
                             l.data_ptr() if save_residuals else 0, m.data_ptr() if save_residuals else 0)
     lib = _lib.load()
     with on_device(q.device):
@@ -86,15 +88,17 @@ def backward(q, k, v, l, m, o, do, spec: MaskSpec, sm_scale):
     """(dq, dk, dv) of a call that `takes` accepts: delta, the dq and the dk/dv pass (flexattn_bwd)."""
     plan = _plan((1, q.shape, k.shape, q.dtype, q.device, spec, sm_scale), q, k, spec, sm_scale, _lib.BwdParamsC,
                  (_lib.PASS_DQ, _lib.PASS_DKV))
-    q, k, v, o, do = aligned(q), aligned(k), aligned(v), aligned(o), aligned(do)
+    head = (q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(), l.data_ptr(), m.data_ptr())
+    op = o.data_ptr()
+    if (head[0] | head[1] | head[2] | head[3] | op) % 16:
+        return backward(aligned(q), aligned(k), aligned(v), l, m, aligned(o), aligned(do), spec, sm_scale)
     dq, dk, dv, delta = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v), torch.empty_like(l)
     pq = _lib.BwdParamsC.from_buffer_copy(plan.templates[0])
     pkv = _lib.BwdParamsC.from_buffer_copy(plan.templates[1])
-    head = (q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(), l.data_ptr(), m.data_ptr())
     d = delta.data_ptr()
     _BWD_POINTERS.pack_into(pq, 0, *head, 0, dq.data_ptr(), 0, 0)
     _BWD_POINTERS.pack_into(pkv, 0, *head, d, 0, dk.data_ptr(), dv.data_ptr())
-    pq.o, pq.delta_out = o.data_ptr(), d
+    pq.o, pq.delta_out = op, d
     lib = _lib.load()
     with on_device(q.device):
         _lib.check(lib.flexattn_bwd(C.byref(pq), C.byref(pkv), stream_of(q)), lib)

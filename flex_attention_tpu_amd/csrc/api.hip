@@ -386,6 +386,16 @@ int flexattn_tile_shape(int32_t pass, int32_t dtype, int32_t D, int32_t* block_q
   return FLEXATTN_OK;
 }
 
+int flexattn_takes_head_dim_64(int32_t pass, float sm_scale, int32_t Sq, int32_t Sk) {
+  if (Sq <= 0 || Sk <= 0 || !(sm_scale > 0.f) || !(sm_scale < __builtin_huge_valf())) return 0;
+  int bq = 0, bk = 0;
+  if (tile_shape(pass, FLEXATTN_BF16, 64, &bq, &bk) != FLEXATTN_OK) return 0;
+  const int nq = tiles_of(Sq, bq), nk = tiles_of(Sk, bk);
+  if (pass == FLEXATTN_PASS_FWD) return fwd_bf16_d64_ok(sm_scale, nk);
+  if (pass == FLEXATTN_PASS_DQ) return bwd_dq_bf16_d64_ok(nk);
+  return bwd_dkv_bf16_d128_on_stream(FLEXATTN_SCORE_NONE, 0, nq, false, 1, 1);
+}
+
 int flexattn_build_block_mask(const flexattn_mask_spec* mask, int32_t Sq, int32_t Sk, int32_t block_q,
                               int32_t block_k, uint8_t* state, int32_t* kv_cnt, int32_t* kv_idx,
                               int32_t* q_cnt, int32_t* q_idx, void* stream) {

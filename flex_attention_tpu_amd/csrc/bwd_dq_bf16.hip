@@ -795,12 +795,20 @@ int bwd_dq_bf16_d128(const BwdArgs& a, hipStream_t stream) {
 #endif
 }
 
-// Head dim 64: the generated streams for plain scores (the rest: see fwd_bf16_d64).
+// Head dim 64: the generated streams for plain scores, of any scale (the rest: see fwd_bf16_d64).
+bool bwd_dq_bf16_d64_ok(int nk) {
+#ifdef FLEXATTN_CUSTOM_ONLY
+  (void)nk;
+  return false;
+#else
+  return nk <= dq_cfg::MAX_LIST;
+#endif
+}
 int bwd_dq_bf16_d64(const BwdArgs& a, hipStream_t stream) {
 #ifndef FLEXATTN_CUSTOM_ONLY
   if (a.score.kind == FLEXATTN_SCORE_NONE && a.score.ab == nullptr && a.dab == nullptr && !(a.flags & FLEXATTN_FLAG_COMPILED_LOOP) &&
-      a.map.nk <= dq_cfg::MAX_LIST)
-    return folded_scale_ok(a.sm_scale * kLog2e, a.sm_scale, 64) ? launch_dq_plain<0, 64>(a, stream) : launch_dq_plain<3, 64>(a, stream);
+      bwd_dq_bf16_d64_ok(a.map.nk))
+    return folded_scale_ok(a.sm_scale * kLog2e, a.sm_scale, 128) ? launch_dq_plain<0, 64>(a, stream) : launch_dq_plain<3, 64>(a, stream);
 #endif
   return set_error(FLEXATTN_ENOTSUP, "bf16 head dim 64: only plain scores without a bias (pad the operands to 128 columns)");
 }

@@ -987,14 +987,23 @@ int fwd_bf16_d128(const FwdArgs& a, hipStream_t stream) {
 }
 
 // Head dim 64: the generated stream for plain scores (with a scale that folds into bf16 Q); everything else runs
-// zero-padded to 128 columns, which the caller sees to.
+// zero-padded to 128 columns, which the caller sees to.  (The scales that fold are those of 128 columns: a call that the
+// kernels there scale in fp32 loses nothing here.)
+bool fwd_bf16_d64_ok(float sm_scale, int nk) {
+#ifdef FLEXATTN_CUSTOM_ONLY
+  (void)sm_scale; (void)nk;
+  return false;
+#else
+  return nk <= fwd_cfg::MAX_LIST && folded_scale_ok(sm_scale * kLog2e, sm_scale, 128);
+#endif
+}
 int fwd_bf16_d64(const FwdArgs& a, hipStream_t stream) {
 #ifndef FLEXATTN_CUSTOM_ONLY
   if (a.score.kind == FLEXATTN_SCORE_NONE && a.score.ab == nullptr && !(a.flags & FLEXATTN_FLAG_COMPILED_LOOP) &&
-      a.map.nk <= fwd_cfg::MAX_LIST && folded_scale_ok(a.sm_scale * kLog2e, a.sm_scale, 64))
+      fwd_bf16_d64_ok(a.sm_scale, a.map.nk))
     return launch_fwd_plain<0, 64>(a, stream);
 #endif
-  return set_error(FLEXATTN_ENOTSUP, "bf16 head dim 64: only plain scores without a bias (pad the operands to 128 columns)");
+  return set_error(FLEXATTN_ENOTSUP, "bf16 head dim 64: only plain scores without a bias and with a scale that folds (pad the operands to 128 columns)");
 }
 
 // Head dim 256: the kernels with a compiled main loop (two 128-column panels per row), every score kind.

@@ -15,6 +15,7 @@ int check_launch(const char* what);
 // bf16, head dim 128 (MFMA kernels)
 int fwd_bf16_d128(const FwdArgs& a, hipStream_t stream);
 int fwd_bf16_d64(const FwdArgs& a, hipStream_t stream);    // (same tiles as head dim 128; plain scores)
+bool fwd_bf16_d64_ok(float sm_scale, int nk);
 int fwd_bf16_d256(const FwdArgs& a, hipStream_t stream);   // (same tiles as head dim 128)
 void fwd_bf16_d128_tile(int* bq, int* bk);
 // few query rows against long keys, plain scores, no mask (head dim 64 or 128)
@@ -23,6 +24,7 @@ int64_t fwd_decode_bytes(int B, int Hq, int Hkv, int Sq, int Sk, int D);
 int fwd_decode(const FwdArgs& a, int D, void* work, hipStream_t stream);
 int bwd_dq_bf16_d128(const BwdArgs& a, hipStream_t stream);
 int bwd_dq_bf16_d64(const BwdArgs& a, hipStream_t stream);
+bool bwd_dq_bf16_d64_ok(int nk);
 int bwd_dq_bf16_d256(const BwdArgs& a, hipStream_t stream);
 void bwd_dq_bf16_d128_tile(int* bq, int* bk);
 int bwd_dkv_bf16_d128(const BwdArgs& a, hipStream_t stream);

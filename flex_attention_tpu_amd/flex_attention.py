@@ -38,7 +38,7 @@ def _hands_ds_over(q, k, ab, segment_ids, sm_scale, score_fn, mask_fn, block_mas
     # (at head dimension 256 always: the recomputing dq pass costs three products of twice the depth.  On B=4, H=16,
     # S=4096, causal, forward and backward: 3.61 -> 3.08 ms.  Not at the head dimension 64 kernels, which hand nothing over.)
     return ((D > 128 or ds_exchange_pays(score_fn, mask_fn, segment_ids)) and
-            call_head_dim(D, q.dtype, sm_scale, score_fn, ab, spec_of(mask_fn, block_mask_fn), q.shape[2], k.shape[2]) != 64)
+            call_head_dim(_lib.PASS_DKV, D, q.dtype, sm_scale, score_fn, ab, spec_of(mask_fn, block_mask_fn), q.shape[2], k.shape[2]) != 64)
 
 
 def _bwd_with_ds(q, k, v, ab, segment_ids, l, m, o, do, want_dab, *, block_q, block_k, **kw):
@@ -69,7 +69,7 @@ def flex_attention_bwd(q, k, v, ab, segment_ids, l, m, o, do, *, block_q, block_
         spec = spec_of(mask_fn, block_mask_fn)
         if causal:
             spec = spec.combine(_CAUSAL)
-        if _plans.takes(q, k, spec, sm_scale):
+        if _plans.takes(q, k, spec, sm_scale, _lib.PASS_DQ, _lib.PASS_DKV):
             return _plans.backward(q, k, v, l, m, o, do, spec, float(sm_scale))
     q, k, v, do = aligned(q), aligned(k), aligned(v), aligned(do)   # (the two passes share them)
     kw = dict(sm_scale=sm_scale, debug=False, score_fn=score_fn, mask_fn=mask_fn, block_mask_fn=block_mask_fn,
@@ -101,7 +101,7 @@ class _FlexAttention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, ab, opts):
         score_fn, mask_fn, block_mask_fn, segment_ids, causal, sm_scale, block_q, block_k = opts
-        q, k, v = (aligned(t.contiguous()) for t in (q, k, v))
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
         o, l, m = _flex_attention_impl(q, k, v, ab, segment_ids, True, causal, sm_scale, 1, block_q, block_k, block_k,
                                        False, block_mask_fn, mask_fn, score_fn)
         ctx.save_for_backward(q, k, v, o, l, m, *([ab] if ab is not None else []))
@@ -114,7 +114,7 @@ class _FlexAttention(torch.autograd.Function):
         ab = rest[0] if rest else None
         score_fn, mask_fn, block_mask_fn, segment_ids, causal, sm_scale, block_q, block_k = ctx.opts
         want_dab = ab is not None and ctx.needs_input_grad[3]
-        do = aligned(do.contiguous())
+        do = do.contiguous()
         dq = dk = dv = dab = None
         want_dkv = ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
         want_dq = ctx.needs_input_grad[0] or want_dab

@@ -39,7 +39,7 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
     q, do, k, v = pad_seq(q, Sq_p), pad_seq(do, Sq_p), pad_seq(k, Sk_p), pad_seq(v, Sk_p)
     l, m, di = pad_seq(l, Sq_p), pad_seq(m, Sq_p), pad_seq(di, Sq_p)
     # (a dS hand-over is at 128 columns)
-    D_user, D = D, (call_head_dim(D, q.dtype, sm_scale, score_fn, ab, spec, Sq, Sk, compiled_loop) if not return_ds
+    D_user, D = D, (call_head_dim(_lib.PASS_DKV, D, q.dtype, sm_scale, score_fn, ab, spec, Sq, Sk, compiled_loop) if not return_ds
                     else kernel_head_dim(D, q.dtype))   # smaller head dimensions: zero-padded columns
     q, do, k, v = (aligned(pad_seq(t, D, 3)) for t in (q, do, k, v))
     bm = kernel_block_map(_lib.PASS_DKV, spec, q, Sq_p, Sk_p, D, score_fn)

@@ -158,7 +158,7 @@ def flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, d, *, block_b, 
     q, do, k, v = pad_seq(q, Sq_p), pad_seq(do, Sq_p), pad_seq(k, Sk_p), pad_seq(v, Sk_p)
     l, m, d_p = pad_seq(l, Sq_p), pad_seq(m, Sq_p), pad_seq(d, Sq_p)
     # (a dS hand-over is at 128 columns)
-    D_user, D = D, (call_head_dim(D, q.dtype, sm_scale, score_fn, ab, spec, Sq, Sk, compiled_loop) if ds is None
+    D_user, D = D, (call_head_dim(_lib.PASS_DQ, D, q.dtype, sm_scale, score_fn, ab, spec, Sq, Sk, compiled_loop) if ds is None
                     else kernel_head_dim(D, q.dtype))   # smaller head dimensions: zero-padded columns
     q, do, k, v = (aligned(pad_seq(t, D, 3)) for t in (q, do, k, v))
     o_p = aligned(pad_seq(pad_seq(o, Sq_p), D, 3)) if fuse_delta else None

@@ -76,7 +76,7 @@ def _flex_attention_impl(q, k, v, ab, segment_ids, save_residuals, causal, sm_sc
         spec = spec_of(mask_fn, block_mask_fn)
         if causal:
             spec = spec.combine(_CAUSAL)
-        if _plans.takes(q, k, spec, sm_scale):
+        if _plans.takes(q, k, spec, sm_scale, _lib.PASS_FWD):
             return _plans.forward(q, k, v, spec, float(sm_scale), save_residuals)
     # (lengths below one tile: the tensors are zero-padded to it, a document id of their own drops the padded keys
     # and the padded query rows are cut off again)
@@ -84,7 +84,7 @@ def _flex_attention_impl(q, k, v, ab, segment_ids, save_residuals, causal, sm_sc
     spec = resolve_mask(mask_fn, block_mask_fn, causal, segment_ids, Sq, Sk, Sq_p, Sk_p)
     check_doc_batches(spec, B)   # (ids of shape [B, S]: the kernels mask every batch entry by its own row)
     q, k, v = pad_seq(q, Sq_p), pad_seq(k, Sk_p), pad_seq(v, Sk_p)
-    D_user, D = D, call_head_dim(D, q.dtype, sm_scale, score_fn, ab, spec, Sq, Sk, compiled_loop)   # smaller head dimensions: zero-padded columns
+    D_user, D = D, call_head_dim(_lib.PASS_FWD, D, q.dtype, sm_scale, score_fn, ab, spec, Sq, Sk, compiled_loop)   # smaller head dimensions: zero-padded columns
     q, k, v = (aligned(pad_seq(t, D, 3)) for t in (q, k, v))
     bm = kernel_block_map(_lib.PASS_FWD, spec, q, Sq_p, Sk_p, D, score_fn)
     compiled_loop = compiled_loop or mostly_partial_custom_mask(spec, bm)

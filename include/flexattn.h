@@ -8,8 +8,8 @@
  *
  * Conventions
  *  - All tensors are contiguous row-major [B, H, S, D] device memory owned by the caller.
- *    Head dimension D: 128 or 256 for bf16, 64 or 128 for float32 (anything else: FLEXATTN_ENOTSUP); bf16 also 64 for
- *    plain scores without a bias, without dS hand-over and with flags 0 (pad the operands of others to 128 columns).
+ *    Head dimension D: 128 or 256 for bf16, 64 or 128 for float32 (anything else: FLEXATTN_ENOTSUP); bf16 also 64 where
+ *    flexattn_takes_head_dim_64 says so, without dS hand-over (pad the operands of others to 128 columns).
  *    q/o/do/dq have Hq heads, k/v/dk/dv have Hkv heads, Hq % Hkv == 0 (kv head = h / (Hq/Hkv)).
  *    In requests with pad != 0, of bf16 head dimension 64 and of flexattn_fwd_decode they start at multiples of 16 bytes
  *    (else FLEXATTN_EINVAL).
@@ -212,6 +212,11 @@ const char* flexattn_custom_tag(void);
 /* Tile granularity (block_q, block_k) the kernels of `pass` expect of the block map for this
  * dtype and head dimension (bf16 head dimensions 64 and 256 run on the tiles of 128). */
 int flexattn_tile_shape(int32_t pass, int32_t dtype, int32_t D, int32_t* block_q, int32_t* block_k);
+
+/* Whether the kernels of bf16 head dimension 64 take a call of these lengths and scale in `pass` (plain scores without a
+ * bias, flags 0): 1 or 0.  The forward folds the scale into bf16 Q and leaves scales that would lose by it to 128
+ * columns; the backward takes every scale. */
+int flexattn_takes_head_dim_64(int32_t pass, float sm_scale, int32_t Sq, int32_t Sk);
 
 /* Block-mask builder.  Replaces the per-grid-step evaluation of the `block_mask_fn` closures
  * (masks.py:20-28, 63-81, 113-139, 161-177; consumed at flex_attention_kernel.py:97-106,231-236,

@@ -150,3 +150,24 @@ def test_ds_exchange_sizes_and_argument_checks(lib):
     assert lib.flexattn_build_ds_index(None, None, None, None) == _lib.EINVAL
     m = _lib.BlockMapC()
     assert lib.flexattn_build_ds_index(C.byref(m), C.addressof(dummy), C.addressof(dummy), None) == _lib.EINVAL
+
+
+def test_head_dim_64_requests(lib):
+    """Which passes take bf16 head dimension 64: the entry points ask the library, which decides by the rules its launchers
+    follow (scales in float32, lists that fit the LDS)."""
+    from flex_attention_tpu_amd._common import call_head_dim
+    from flex_attention_tpu_amd.masks import MaskSpec
+    takes = lib.flexattn_takes_head_dim_64
+    F, DQ, DKV = _lib.PASS_FWD, _lib.PASS_DQ, _lib.PASS_DKV
+    limit = 2.9 / (1.4426950408889634 * 128 ** 0.5)          # the bound of the 128-column kernels' fold
+    for scale, fwd in ((0.125, 1), (limit * 0.999, 1), (limit * 1.001, 0), (0.25, 0), (1.0, 0)):
+        assert takes(F, scale, 512, 512) == fwd
+        assert takes(DQ, scale, 512, 512) == 1 and takes(DKV, scale, 512, 512) == 1
+    for bad in (0.0, -1.0, float("inf"), float("nan")):
+        assert not any(takes(p, bad, 512, 512) for p in (F, DQ, DKV))
+    assert takes(F, 0.125, 1 << 20, 262144) == 1 and takes(F, 0.125, 128, 262145) == 0
+    assert takes(DQ, 0.125, 1 << 20, 262144) == 1 and takes(DQ, 0.125, 128, 262145) == 0
+    assert takes(DKV, 0.125, 262144, 1 << 20) == 1 and takes(DKV, 0.125, 262145, 128) == 0
+    for D in (16, 32, 64):
+        for p, want in ((F, 64 if D > 16 else 128), (DQ, 64), (DKV, 64)):
+            assert call_head_dim(p, D, torch.bfloat16, D ** -0.5, None, None, MaskSpec(), 512, 512) == want

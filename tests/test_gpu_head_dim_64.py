@@ -67,3 +67,29 @@ def test_exact_scale_dq_stream_is_reached():
     _lib.check(_lib.load().flexattn_bwd_dq(C.byref(p), stream_of(q)))
     same = same_residual_grads(*(x.cpu() for x in (q, k, v, do)), o, l, m, sm_scale=sc)
     assert_close("dq", dq, same[0], torch.bfloat16, tensor_scale=True)
+
+
+@pytest.mark.parametrize("D", [8, 16, 24])
+@pytest.mark.parametrize("mask", ["none", "causal"])
+def test_scales_that_do_not_fold(mask, D):
+    """1 / sqrt(D) of the smallest head dimensions is a scale that the kernels of 128 columns do not fold into bf16 Q: o, l
+    and m are theirs, and the backward (at 64 columns, dq by the stream that scales the fp32 product) gives what they
+    give on zero-padded operands."""
+    import flex_attention_tpu_amd as F
+    from flex_attention_tpu_amd import masks
+    mf = masks.make_causal_mask_fns(128, 128) if mask == "causal" else (None, None)
+    B, H, S, sc = 2, 2, 321, 1 / math.sqrt(D)
+    ts = O.make_inputs(B, H, H, S, S, D, dtype=torch.bfloat16, seed=D)
+
+    def passes(q, k, v, do):
+        o, l, m = F._flex_attention_impl(q, k, v, None, None, True, False, sc, 1, 128, 128, 128, False, mf[1], mf[0], None)
+        kw = dict(block_b=1, block_q=128, block_k_major=128, block_k=128, sm_scale=sc, debug=False, mask_fn=mf[0], block_mask_fn=mf[1])
+        dq, d = F.flex_attention_bwd_dq(q, k, v, None, None, l, m, o, do, None, return_delta=True, **kw)
+        return (o, l, m, dq, *F.flash_attention_bwd_dkv(k, v, q, None, None, l, m, d, do, block_q_major=128, causal=False, **kw))
+    got = passes(*(x.cuda() for x in ts))
+    want = passes(*(torch.nn.functional.pad(x, (0, 128 - D)).cuda() for x in ts))
+    for name, a, b in zip(("o", "l", "m", "dq", "dk", "dv"), got, want):
+        assert torch.equal(a, b[..., :D] if b.ndim == 4 else b), name
+    same = same_residual_grads(*ts, *got[:3], sm_scale=sc, **(dict(causal=True) if mask == "causal" else {}))
+    for name, t, r in zip(("dq", "dk", "dv"), got[3:], same):
+        assert_close(name, t, r, torch.bfloat16)
