@@ -107,15 +107,11 @@ __global__ __launch_bounds__(64 * NW) void fwd_f32_mfma_kernel(FwdArgs a) {
   const uint8_t* tile_state = a.map.state + (size_t)qb * nK;
 
   static_assert(BT == 64, "a list entry is two units of 32 rows");
-  // (A unit behind the end of a ragged length repeats the last 32 rows with every element dropped: a test around the unit's
-  // work instead cost the loads their lead and the backward its second wave per SIMD; B=1, H=8, S=2048, D=128, causal,
-  // forward and backward: 2175 us with it, 2093 without.  The list entry is the same in every lane of a wave; told so, the compiler
-  // keeps the unit's rows out of vector registers, and the 8-wave kernels at 128 of those.)
   for (int u = w; u < 2 * n_tiles; u += NW) {
-    const int kb = __builtin_amdgcn_readfirstlane(tile_idx[u >> 1]);
+    const int kb = tile_idx[u >> 1];
     const bool partial = tile_state[kb] == 1;
     const int j_first = kb * BT + 32 * (u & 1);   // (keys before it belong to the unit before)
-    {
+    if (j_first < a.Sk) {
       const int j0 = min(j_first, a.Sk - 32);
       const f32x16 s = dot_block<D>(Kg + (size_t)(j0 + l32) * D, qf, half);
       float x[16];
@@ -261,10 +257,10 @@ __global__ __launch_bounds__(64 * NW) void bwd_dq_f32_mfma_kernel(BwdArgs a) {
   const int* tile_idx = a.map.idx + (size_t)qb * nK;
   const uint8_t* tile_state = a.map.state + (size_t)qb * nK;
   for (int u = w; u < 2 * n_tiles; u += NW) {
-    const int kb = __builtin_amdgcn_readfirstlane(tile_idx[u >> 1]);
+    const int kb = tile_idx[u >> 1];
     const bool partial = tile_state[kb] == 1;
     const int j_first = kb * BT + 32 * (u & 1);   // (keys before it belong to the unit before)
-    {
+    if (j_first < a.Sk) {
       const int j0 = min(j_first, a.Sk - 32);
       const f32x16 s = dot_block<D>(Kg + (size_t)(j0 + l32) * D, qf, half);
       const f32x16 dp = dot_block<D>(Vg + (size_t)(j0 + l32) * D, dof, half);
@@ -327,7 +323,7 @@ __global__ __launch_bounds__(64 * NW) void bwd_dkv_f32_mfma_kernel(BwdArgs a) {
   const uint8_t* state = a.map.state;
   for (int u = w; u < 2 * group * n_tiles; u += NW) {
     const int it = u >> 1;
-    const int g = it / n_tiles, qb = __builtin_amdgcn_readfirstlane(tile_idx[it - g * n_tiles]);
+    const int g = it / n_tiles, qb = tile_idx[it - g * n_tiles];
     const int h = hk * group + g;
     const size_t head_row = (size_t)(b * a.Hq + h) * a.Sq;
     const float* Qg = static_cast<const float*>(a.q) + head_row * D;
@@ -336,7 +332,7 @@ __global__ __launch_bounds__(64 * NW) void bwd_dkv_f32_mfma_kernel(BwdArgs a) {
     sm.init(a.score, a.sm_scale, h, b);
     const int i_first = qb * BT + 32 * (u & 1);   // (rows before it belong to the unit before)
     const bool partial = state[(size_t)qb * a.map.nk + kb] == 1 || i_first + 32 > a.Sq;
-    {
+    if (i_first < a.Sq) {
       const int i0 = min(i_first, a.Sq - 32);
       const f32x16 s = dot_block<D>(Qg + (size_t)(i0 + l32) * D, kf, half);
       const f32x16 dp = dot_block<D>(dOg + (size_t)(i0 + l32) * D, vf, half);
