@@ -107,6 +107,10 @@ __global__ __launch_bounds__(64 * NW) void fwd_f32_mfma_kernel(FwdArgs a) {
   const uint8_t* tile_state = a.map.state + (size_t)qb * nK;
 
   static_assert(BT == 64, "a list entry is two units of 32 rows");
+  // (The test leaves out a unit behind the end of a ragged length.  It costs whole tiles nothing: with such a unit repeating
+  // the last rows, all dropped, instead, the compiler holds the operands of two units and the kernels of head dimension 64
+  // lose wavefronts per SIMD; B=2, H=16, S=2048, D=64, causal, forward and backward: 1930 us with the test, 2200 us
+  // without; B=1, H=8, S=2048, D=128: 2115 and 2112 us.)
   for (int u = w; u < 2 * n_tiles; u += NW) {
     const int kb = tile_idx[u >> 1];
     const bool partial = tile_state[kb] == 1;
