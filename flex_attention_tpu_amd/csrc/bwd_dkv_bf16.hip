@@ -735,7 +735,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
   struct Geometry {
     int bhk, kb;
   };
-  const PersistentPlan plan = persistent_plan((int)blockIdx.x, n_wg, nKb);
+  const PersistentPlan plan = persistent_plan((int)blockIdx.x, (int)gridDim.x, n_wg, nKb);
   // under document masks a persistent work-group takes its items from the longest-first schedule (sorted_items)
   const bool sorted = DOCS && gridDim.x != (unsigned)n_wg;
   int* sItems = reinterpret_cast<int*>(sPart + MAX_LIST) + 4 * 128;
@@ -749,7 +749,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
       g.bhk = v >> 16;
       g.kb = v & 0xffff;
     } else {
-      persistent_item(plan, (int)blockIdx.x, item, (int)gridDim.x, n_wg, nKb, g.bhk, g.kb);
+      persistent_item(plan, item, (int)gridDim.x, n_wg, nKb, g.bhk, g.kb);
     }
     g.bhk = __builtin_amdgcn_readfirstlane(g.bhk);
     g.kb = __builtin_amdgcn_readfirstlane(g.kb);
@@ -1022,10 +1022,13 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
         for (int half = 0; half < 2; ++half)
           km[half] = keep_bits32<false>(a.mask, k_idx, q0 + 64 * half + 4 * hh, doc_j, a.mask.doc_q);
       }
-      // (rows and columns that the last tiles of ragged lengths share with the tiles before them: those own them)
+      // (rows and columns that the last tiles of ragged lengths share with the tiles before them: those own them.  opaque():
+      // what only these tiles need is not kept through the runs)
+      if (q0 != qb * BQ || k0 != kb * BNK) {
 #pragma unroll
-      for (int half = 0; half < 2; ++half)
-        km[half] = k_idx < kb * BNK ? 0u : km[half] & keep_bits_from(qb * BQ - q0 - 64 * half - 4 * hh);
+        for (int half = 0; half < 2; ++half)
+          km[half] = opaque(kv_local) < kb * BNK - k0 ? 0u : km[half] & keep_bits_from(qb * BQ - q0 - 64 * half - 4 * (opaque(lane) >> 5));
+      }
     } else {
       // the run of full tiles ends before the next partial one: lanes look 64 steps ahead at a time
       bool found = false;
@@ -1170,8 +1173,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_plain_kernel(BwdArgs
     bf16_t* dKg = static_cast<bf16_t*>(a.dk) + kv_off + (size_t)(w * 32) * D;
     bf16_t* dVg = static_cast<bf16_t*>(a.dv) + kv_off + (size_t)(w * 32) * D;
     const int r_first = kb * BNK - k0 - w * 32;   // (rows before it belong to the kv tile before)
-    rows_store<HD>(stage, dKg, lane_here, r_first);
-    rows_store<HD>(stage + 8192, dVg, lane_here, r_first);
+    rows_store<HD, 2>(stage, {dKg, dVg}, lane_here, r_first);
   }
   geo = geo_n;
   }  // work items

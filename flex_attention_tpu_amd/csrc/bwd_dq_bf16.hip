@@ -382,7 +382,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
     unsigned char st[kListRegs];   // state of kv tile tid + 256 j in the q tile's state row
   };
   const int n_items = n_wg / (int)gridDim.x;
-  const PersistentPlan plan = persistent_plan((int)blockIdx.x, n_wg, nQ);
+  const PersistentPlan plan = persistent_plan((int)blockIdx.x, (int)gridDim.x, n_wg, nQ);
   const int group = a.Hq / a.Hkv;
   const float inv_group = 1.0f / (float)group;
   const bool sorted = DOCS && gridDim.x != (unsigned)n_wg;
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
       qb = v & 0xffff;
       return;
     }
-    persistent_item(plan, (int)blockIdx.x, item, (int)gridDim.x, n_wg, nQ, bh, qb);
+    persistent_item(plan, item, (int)gridDim.x, n_wg, nQ, bh, qb);
     if (gridDim.x == (unsigned)n_wg) qb = nQ - 1 - qb;  // one item each: longest first
   };
   // (batch, kv head) pair of a (batch, q head) pair: bh / group, exact for the small numbers involved
@@ -634,7 +634,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
           } else {
             km[hx] = keep_bits32<true>(a.mask, q_idx, k0 + 4 * hh, doc_i, nullptr);
           }
-          km[hx] &= keep_bits_from(kt * BN - k0 - 4 * hh);
+          if (k0 != kt * BN) km[hx] &= keep_bits_from(kt * BN - k0 - 4 * hh);
         }
       } else {
         it_part = -1;
@@ -739,7 +739,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_d128_plain_kernel(BwdArgs 
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
       bf16_t* out_rows = dQg + (size_t)(w * 32) * D;
-      rows_store<HD>(stage, out_rows, lane_here, qb * BM - q0 - w * 32);   // (rows before that belong to the q tile before)
+      rows_store<HD, 1>(stage, {out_rows}, lane_here, qb * BM - q0 - w * 32);   // (rows before that belong to the q tile before)
     }
   }  // work items
 }

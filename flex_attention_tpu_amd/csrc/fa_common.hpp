@@ -259,19 +259,28 @@ __device__ __forceinline__ void rows_to_fragments(const RowBlock& r, char* stage
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
-// A wave's 32 x HD results, staged as rows of 256 bytes with their 16-byte chunks XOR-swizzled by row, to memory with
-// full-row stores; rows before r_first are left alone.
-template <int HD>
-__device__ __forceinline__ void rows_store(const char* stage, bf16_t* block, int lane, int r_first) {
+// A wave's N blocks of 32 x HD results, staged 8 KB apart as rows of 256 bytes with their 16-byte chunks XOR-swizzled by
+// row, to memory with full-row stores; rows before r_first are left alone.
+template <int HD, int N>
+__device__ __forceinline__ void rows_store(const char* stage, bf16_t* const (&block)[N], int lane, int r_first) {
   constexpr int CH = HD / 8, RPI = 64 / CH;
   const int chunk = lane % CH;
+  auto rows = [&](int r) {
+    u32x4 v[N];
 #pragma unroll
-  for (int i = 0; i < 32 / RPI; ++i) {
-    const int r = RPI * i + lane / CH;
-    if (r < r_first) continue;
-    const u32x4 v = *reinterpret_cast<const u32x4*>(stage + (unsigned)r * 256u + (unsigned)((chunk ^ (r & 15)) << 4));
-    *reinterpret_cast<u32x4*>(block + (size_t)r * HD + chunk * 8) = v;
+    for (int n = 0; n < N; ++n)
+      v[n] = *reinterpret_cast<const u32x4*>(stage + n * 8192 + (unsigned)r * 256u + (unsigned)((chunk ^ (r & 15)) << 4));
+#pragma unroll
+    for (int n = 0; n < N; ++n) *reinterpret_cast<u32x4*>(block[n] + (size_t)r * HD + chunk * 8) = v[n];
+  };
+  if (r_first <= 0) {   // (the usual case: no test per store, which would order the reads and the stores one by one)
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; ++i) rows(RPI * i + lane / CH);
+    return;
   }
+#pragma unroll 1
+  for (int r = lane / CH; r < 32; r += RPI)
+    if (r >= r_first) rows(r);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -580,14 +589,45 @@ __host__ __device__ inline bool persistent_ok(int n_wg, int nKb) {
   if (nKb % 32 == 0) return true;
   return 32 % nKb == 0 && heads % (32 / nKb) == 0;
 }
+// One item per work-group, started in the order of the ids: (batch, head) pair and rank of work-group j, ranks ascending
+// in work under causal masks from the caller's end.  An XCD (ids j % 8) takes a contiguous share of the heads and starts
+// the blocks of equal rank of several heads together, longest first: with the blocks of one head behind each other the
+// longest of the share's last head start when the chip is already running dry (B=1, Hq=32, S=2777 forward, 352 items of
+// 2 to 22 steps on 256 CUs: 94.6 us against 77.2 us).  The heads taken together are those that kSetItems items make, so that
+// the K / V of few heads are in use at a time.
+constexpr int kSetItems = 64;
+__host__ __device__ inline void single_item(int j, int n_wg, int nKb, int& head, int& kb) {
+  const unsigned per = (unsigned)n_wg >> 3;   // items of an XCD
+  if ((n_wg & 7) != 0 || per % (unsigned)nKb != 0) {
+    const int wg = (n_wg & 7) != 0 ? j : (j & 7) * (int)per + (j >> 3);
+    head = (int)((unsigned)wg / (unsigned)nKb);
+    kb = wg - head * nKb;
+    return;
+  }
+  const int share = (int)(per / (unsigned)nKb);                                 // heads of an XCD
+  const int set = nKb >= kSetItems ? 1 : (int)((float)kSetItems / ((float)nKb - 0.001f));  // heads taken together
+  const int t = j >> 3, first = (int)((unsigned)t / (unsigned)(set * nKb)) * set;   // first head of the item's set
+  const int in = t - first * nKb, n = share - first < set ? share - first : set;
+  kb = (int)(((float)in + 0.5f) / (float)n);
+  head = (j & 7) * share + first + in - kb * n;
+}
 // The work-group's walk through its items with the divisions done once (the kernels locate an item
 // three times per item): `base` = first (batch, head) pair of the XCD's share, x, y = (c, blocks per
-// head / 32) when a head has at least 32 blocks, else (c / nKb, c % nKb), c = position in the XCD.
+// head / 32) when a head has at least 32 blocks, else (c / nKb, c % nKb), c = position in the XCD.  Without a static
+// schedule (one item per work-group) base and x are the item itself.
 struct PersistentPlan {
   int base, x, y;
 };
-__device__ __forceinline__ PersistentPlan persistent_plan(int j, int n_wg, int nKb) {
+__device__ __forceinline__ PersistentPlan persistent_plan(int j, int grid, int n_wg, int nKb) {
   PersistentPlan p;
+  if (grid == n_wg) {
+    int head, kb;
+    single_item(j, n_wg, nKb, head, kb);
+    p.base = __builtin_amdgcn_readfirstlane(head);   // (the same in every lane; the compiler loses sight of it)
+    p.x = __builtin_amdgcn_readfirstlane(kb);
+    p.y = 0;
+    return p;
+  }
   const int c = j >> 3;
   p.base = (j & 7) * (n_wg / 8 / nKb);
   if (nKb >= 32) {
@@ -599,32 +639,11 @@ __device__ __forceinline__ PersistentPlan persistent_plan(int j, int n_wg, int n
   }
   return p;
 }
-// One item per work-group, started in the order of the ids: (batch, head) pair and rank of work-group j, ranks ascending
-// in work under causal masks from the caller's end.  An XCD (ids j % 8) takes a contiguous share of the heads and starts
-// the blocks of equal rank of several heads together, longest first: with the blocks of one head behind each other the
-// longest of the share's last head start when the chip is already running dry (B=1, Hq=32, S=2777 forward, 352 items of
-// 2 to 22 steps on 256 CUs: 94.6 us against 77.2 us).  The heads taken together are those that kSetItems items make, so that
-// the K / V of few heads are in use at a time.
-constexpr int kSetItems = 64;
-__host__ __device__ inline void single_item(int j, int n_wg, int nKb, int& head, int& kb) {
-  const int heads = n_wg / nKb;
-  if (heads % 8 != 0) {
-    const int wg = (n_wg % 8 != 0) ? j : (j % 8) * (n_wg / 8) + j / 8;
-    head = wg / nKb;
-    kb = wg % nKb;
-    return;
-  }
-  const int share = heads / 8, set = nKb >= kSetItems ? 1 : kSetItems / nKb;   // heads of an XCD, heads taken together
-  const int t = j >> 3, first = t / (set * nKb) * set;                         // first head of the item's set
-  const int in = t - first * nKb, n = share - first < set ? share - first : set;
-  head = (j & 7) * share + first + in % n;
-  kb = in / n;
-}
-// (batch, head) pair and block of item number `item` of work-group j
-__device__ __forceinline__ void persistent_item(const PersistentPlan& p, int j, int item, int grid, int n_wg, int nKb,
-                                                int& head, int& kb) {
+// (batch, head) pair and block of the work-group's item number `item`
+__device__ __forceinline__ void persistent_item(const PersistentPlan& p, int item, int grid, int n_wg, int nKb, int& head, int& kb) {
   if (grid == n_wg) {  // one item per work-group, no static schedule
-    single_item(j, n_wg, nKb, head, kb);
+    head = p.base;
+    kb = p.x;
     return;
   }
   int hd;

@@ -483,7 +483,7 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
     unsigned head;      // states of kv tile `lane` in both rows: where the merged list starts
   };
   const int n_items = n_wg / (int)gridDim.x;
-  const PersistentPlan plan = persistent_plan((int)blockIdx.x, n_wg, nQ2);
+  const PersistentPlan plan = persistent_plan((int)blockIdx.x, (int)gridDim.x, n_wg, nQ2);
   const int group = a.Hq / a.Hkv;
   const float inv_group = 1.0f / (float)group;
   // under document masks a persistent work-group takes its items from the longest-first schedule (sorted_items)
@@ -499,7 +499,7 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
       qb2 = v & 0xffff;
       return;
     }
-    persistent_item(plan, (int)blockIdx.x, item, (int)gridDim.x, n_wg, nQ2, bh, qb2);
+    persistent_item(plan, item, (int)gridDim.x, n_wg, nQ2, bh, qb2);
     if (gridDim.x == (unsigned)n_wg) qb2 = nQ2 - 1 - qb2;  // one item each: longest first
   };
   // (batch, kv head) pair of a (batch, q head) pair: bh / group, exact for the small numbers involved
@@ -517,9 +517,7 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
     r.sa = r.sb = r.head = 0u;
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
-      // (a missing second tile repeats the first, states and all, and nothing of it is stored: with states of its own, empty
-      // ones, every step of the item, the longest under a causal mask, would be a masked one)
-      const int qb = min(2 * qb2 + x, nQ - 1);
+      const int qb = min(2 * qb2 + x, nQ - 1);  // (a missing second tile repeats the first; nothing of it is stored)
       const int q0 = tile_base(qb, BM, a.Sq);
       rows_load<HD>(r.q[x], static_cast<const bf16_t*>(a.q) + ((size_t)bh * a.Sq + (size_t)q0 + w_here * 32) * D, lane_here);
       r.doc[x] = (a.mask.flags & FLEXATTN_MASK_DOC) ? a.mask.doc_q[dq_rows + q0 + row_here] : 0;
@@ -529,15 +527,16 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
         r.khi[x] = ranged ? a.mask.doc_q_range[2 * (dq_rows + q0 + row_here) + 1] : 0;
       }
       const uint8_t* row = a.map.state + (size_t)qb * nK;
+      const bool valid = 2 * qb2 + x < nQ;
       unsigned packed = 0u;
 #pragma unroll
       for (int j = 0; j < kListRegs; ++j) {
         const int t = tid_here + 256 * j;
-        const unsigned v = t < nK ? row[t] : 0u;
+        const unsigned v = (valid && t < nK) ? row[t] : 0u;
         packed |= v << (8 * j);
       }
       if (x == 0) r.sa = packed; else r.sb = packed;
-      const unsigned hv = lane_here < nK ? row[lane_here] : 0u;
+      const unsigned hv = (valid && lane_here < nK) ? row[lane_here] : 0u;
       r.head |= hv << (8 * x);
     }
   };
@@ -595,12 +594,15 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
     // the two state rows into LDS, then the merged list of kv tiles that are non-empty for either
     // q tile, in ascending order (ballot compaction per wave, wave offsets through LDS)
     const int tid_p = opaque(tid);  // (fresh per item: see opaque())
+    // (a missing second tile gets the first one's states: with empty ones of its own every step of the item, the longest
+    // under a causal mask, would be a masked one)
+    const unsigned states_b = 2 * qb2 + 1 < nQ ? cur.sb : cur.sa;
 #pragma unroll
     for (int j = 0; j < kListRegs; ++j) {
       const int t = tid_p + 256 * j;
       if (t < nK) {
         sStA[t] = (unsigned char)((cur.sa >> (8 * j)) & 0xffu);
-        sStB[t] = (unsigned char)((cur.sb >> (8 * j)) & 0xffu);
+        sStB[t] = (unsigned char)((states_b >> (8 * j)) & 0xffu);
       }
     }
     int n_list = 0;
@@ -744,7 +746,6 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
           if (e >= n_list) continue;  // missing half: all dropped
           const int k = __builtin_amdgcn_readfirstlane(list_at(e));
           const int k0 = tile_base(k, BN, a.Sk);
-          const unsigned own = keep_bits_from(k * BN - k0 - 4 * hh);
 #pragma unroll
           for (int x = 0; x < 2; ++x) {
             const int state = __builtin_amdgcn_readfirstlane((int)(x == 0 ? sStA[k] : sStB[k]));
@@ -756,8 +757,9 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
                                         : keep_bits32_staged<true>(a.mask, q_idx[x], k0 + 4 * hh, doc_i[x], sDoc + 64 * hx + 4 * hh);
               else
                 km[2 * x + hx] = keep_bits32<true>(a.mask, q_idx[x], k0 + 4 * hh, doc_i[x], a.mask.doc_k);
-              km[2 * x + hx] &= own;
             }
+            // (keys that the last tile of a ragged length shares with the tile before, which owns them)
+            if (k0 != k * BN) km[2 * x + hx] &= keep_bits_from(k * BN - k0 - 4 * hh);
           }
         }
       } else {
@@ -920,7 +922,7 @@ __global__ __launch_bounds__(256, 1) void fwd_bf16_d128_plain_kernel(FwdArgs a) 
         if (2 * qb2 + x < nQ) {
           bf16_t* Og = static_cast<bf16_t*>(a.o) + ((size_t)bh * a.Sq + (size_t)q_at[x] + w * 32) * D;
           // (rows before r_first belong to the q tile before)
-          rows_store<HD>(stage + x * 8192, Og, lane_here, (2 * qb2 + x) * BM - q_at[x] - w * 32);
+          rows_store<HD, 1>(stage + x * 8192, {Og}, lane_here, (2 * qb2 + x) * BM - q_at[x] - w * 32);
         }
       }
     }
