@@ -98,13 +98,14 @@ S_CUR = ["s62", "s101"]  # kv tiles of the current step
 A_DQ, A_Q, A_DO, A_STG = 0, 64, 96, 128
 
 
-def bias_ops(e, block, tile, odd):
+def bias_ops(e, block, tile, odd, clamp=True):
     """The accumulator input of S chain `block` (its parity picks the B register) for the 32 keys from
     64 `tile` + 32 `odd` on."""
     t0 = S_T[0]
     b = V_B[block & 1]
     e.raw(f"s_lshl_b32 {t0}, {tile}, 6")
-    e.raw(f"s_min_u32 {t0}, {t0}, {SREG['klim']}")
+    if clamp:   # (see gen_fwd_tile.py)
+        e.raw(f"s_min_u32 {t0}, {t0}, {SREG['klim']}")
     if odd:
         e.raw(f"s_add_u32 {t0}, {t0}, 32")
     e.valu(f"v_sub_u32_e32 {vr(V_T)}, {t0}, %[iq]", vset(V_T), set())
@@ -283,7 +284,7 @@ def build(masked, alibi=False, softcap=False, exact=False, d64=False):
         bias = []
         for c in (1, 2, 3, 4):
             tile = S_SEL[0] if c == 4 else S_CUR[c >> 1]
-            bias.append(Op(lambda e, c=c, tile=tile: bias_ops(e, c, tile, c & 1), cost=CAP, earliest=first_A[c - 1] + 1,
+            bias.append(Op(lambda e, c=c, tile=tile: bias_ops(e, c, tile, c & 1, masked or c == 4), cost=CAP, earliest=first_A[c - 1] + 1,
                            deadline=first_A[c] - 6 if c < 4 else None))
         chains.append(bias)
 

@@ -117,13 +117,15 @@ V_END_ALIBI = 201
 S_CUR = ["s62", "s101"]  # kv tiles of the current step
 
 
-def bias_ops(e, c, q, tile):
-    """The accumulator input of the S chain (c, q): keys from 64 `tile` + 32 (c & 1) on, q rows 128 q on."""
+def bias_ops(e, c, q, tile, clamp=True):
+    """The accumulator input of the S chain (c, q): keys from 64 `tile` + 32 (c & 1) on, q rows 128 q on.  (clamp: the tile
+    may be the last one of a ragged length, which starts early; a full step's own tiles are not, that one is never full.)"""
     t0 = S_T[0]
     b = V_B[q]
     off = 32 * (c & 1) - 128 * q
     e.raw(f"s_lshl_b32 {t0}, {tile}, 6")
-    e.raw(f"s_min_u32 {t0}, {t0}, {SREG['klim']}")
+    if clamp:
+        e.raw(f"s_min_u32 {t0}, {t0}, {SREG['klim']}")
     if off > 0:
         e.raw(f"s_add_u32 {t0}, {t0}, {off}")
     elif off < 0:
@@ -458,7 +460,7 @@ def build(masked, alibi=False, softcap=False, d64=False):
             # the registers, is out by then; 20 wait states before the chain's first MFMA.
             cn = c + 2
             tile = S_CUR[1] if cn < 4 else S_SEL[0]
-            ops.append(Op(lambda e: bias_ops(e, cn & 3, q, tile), cost=CAP, earliest=rare_earliest,
+            ops.append(Op(lambda e: bias_ops(e, cn & 3, q, tile, masked or cn == 4), cost=CAP, earliest=rare_earliest,
                           deadline=a_mfma(cn, 0, q) - 6 if cn < 4 else None))
         ops.append(block(rare, earliest=rare_earliest, deadline=rare_deadline))
 
@@ -526,7 +528,7 @@ def build(masked, alibi=False, softcap=False, d64=False):
         f"v_xor_b32_e32 %[{name}], 0x10000, %[{name}]", {("op", name)}, {("op", name)}, earliest=at)))
     if alibi:
         # chain (1, q): behind the first MFMA of chain (0, q) and before this step's first softmax
-        chains.append([Op(lambda e, q=q: bias_ops(e, 1, q, S_CUR[0]), cost=CAP, earliest=2 + q, deadline=a_mfma(1, 0, q) - 6)
+        chains.append([Op(lambda e, q=q: bias_ops(e, 1, q, S_CUR[0], masked), cost=CAP, earliest=2 + q, deadline=a_mfma(1, 0, q) - 6)
                        for q in range(2)])
 
     # ---- next step's K / V tiles: 16 LDS-direct loads per wave spread over the stream ------------
