@@ -1,0 +1,50 @@
+"""Registers that the compiler spills in the kernels around the generated streams (bf16, plain scores, position bias,
+soft-cap): a wave holds its accumulators and the next item's operands through the run loop, so whatever else lives across it
+goes to scratch memory.  The bounds are what the present code reaches; a change that keeps more alive shows here without a
+GPU."""
+import concurrent.futures
+import os
+import re
+import subprocess
+
+import pytest
+
+from flex_attention_tpu_amd import build
+
+# (kernel, score, documents, export of dS, head dimension) -> most spilled VGPRs per lane.  score: 0 plain, 1 position bias,
+# 2 soft-cap, 3 (dq) plain with the scale applied in fp32
+BOUNDS = {
+    ("fwd", 0, 0, 0, 128): 0, ("fwd", 0, 1, 0, 128): 15, ("fwd", 1, 0, 0, 128): 8, ("fwd", 1, 1, 0, 128): 24,
+    ("fwd", 2, 0, 0, 128): 2, ("fwd", 2, 1, 0, 128): 17, ("fwd", 0, 0, 0, 64): 0, ("fwd", 0, 1, 0, 64): 16,
+    ("dkv", 0, 0, 0, 128): 3, ("dkv", 0, 0, 1, 128): 12, ("dkv", 0, 1, 0, 128): 60, ("dkv", 0, 1, 1, 128): 58,
+    ("dkv", 1, 0, 0, 128): 7, ("dkv", 1, 1, 0, 128): 41, ("dkv", 2, 0, 0, 128): 7, ("dkv", 2, 0, 1, 128): 16,
+    ("dkv", 2, 1, 0, 128): 60, ("dkv", 2, 1, 1, 128): 60, ("dkv", 0, 0, 0, 64): 0, ("dkv", 0, 1, 0, 64): 58,
+    **{("dq", s, d, 0, hd): 0 for s in range(4) for d in range(2) for hd in (64, 128)},
+}
+PATTERN = re.compile(r"(fwd|bwd_dq|bwd_dkv)_bf16_d128_plain_kernelILi(\d)ELb(\d)E(?:Lb(\d)E)?Li(\d+)EE")
+
+
+def spills(src, out):
+    cmd = [build.HIPCC, *build.FLAGS, "--cuda-device-only", "-Rpass-analysis=kernel-resource-usage", "-c", os.path.join(build.CSRC, src), "-o", out]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
+    got, name = {}, None
+    for line in r.stderr.splitlines():
+        if "Function Name:" in line:
+            m = PATTERN.search(line)
+            name = (m.group(1)[-3:].lstrip("_"), int(m.group(2)), int(m.group(3)), int(m.group(4) or 0), int(m.group(5))) if m else None
+        m = re.search(r"VGPRs Spill: (\d+)", line)
+        if m and name:
+            got[name] = int(m.group(1))
+    return got
+
+
+@pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="needs hipcc")
+def test_spilled_registers_of_the_stream_kernels(tmp_path):
+    build.generate_streams()
+    with concurrent.futures.ThreadPoolExecutor(3) as ex:
+        parts = list(ex.map(lambda s: spills(s, str(tmp_path / (s + ".o"))), ("fwd_bf16.hip", "bwd_dkv_bf16.hip", "bwd_dq_bf16.hip")))
+    got = {k: v for p in parts for k, v in p.items()}
+    assert set(got) >= {k for k in BOUNDS if not (k[0] == "dq" and k[4] == 64 and k[1] in (1, 2))}
+    over = {k: (v, BOUNDS.get(k)) for k, v in got.items() if v > BOUNDS.get(k, -1)}
+    assert not over, f"(spilled, bound): {over}"
