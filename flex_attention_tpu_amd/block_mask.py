@@ -234,14 +234,14 @@ def build_block_map(spec: MaskSpec, Sq: int, Sk: int, block_q: int, block_k: int
     the same call, if any, so that one library serves both).  ``ragged``: take lengths that are no multiples of the
     blocks."""
     device = torch.device(device)
+    if not ragged and (Sq % block_q or Sk % block_k):
+        raise ValueError(f"Sq={Sq} / Sk={Sk} not divisible by blocks {block_q} / {block_k}")
     key = (spec, Sq, Sk, block_q, block_k, str(device))
     if cache:
         hit = _map_cache.get(key)
         if hit is not None:
             hit.wait_ready(device)
             return hit
-    if not ragged and (Sq % block_q or Sk % block_k):
-        raise ValueError(f"Sq={Sq} / Sk={Sk} not divisible by blocks {block_q} / {block_k}")
     lib = _lib.load_for(score_code if spec.custom is not None else None, spec.custom)
     bm = BlockMap(spec, Sq, Sk, block_q, block_k, device)
     mc = mask_spec_c(spec, Sq, Sk, device)
