@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import collections
 import ctypes as C
+import threading
 from typing import Callable, Optional
 
 import torch
@@ -36,6 +37,7 @@ class LRU:
     def __init__(self, maxsize: int):
         self.maxsize = maxsize
         self._d = collections.OrderedDict()
+        self._lock = threading.Lock()   # (of what adds and drops entries; a lookup only reorders them)
 
     def get(self, key):
         v = self._d.get(key)
@@ -47,13 +49,15 @@ class LRU:
         return v
 
     def put(self, key, value):
-        self._d[key] = value
-        self._d.move_to_end(key)
-        while len(self._d) > self.maxsize:
-            self._d.popitem(last=False)
+        with self._lock:
+            self._d[key] = value
+            self._d.move_to_end(key)
+            while len(self._d) > self.maxsize:
+                self._d.popitem(last=False)
 
     def clear(self):
-        self._d.clear()
+        with self._lock:
+            self._d.clear()
 
     def __len__(self):
         return len(self._d)

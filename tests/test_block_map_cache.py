@@ -17,3 +17,31 @@ def test_ragged_lengths_are_refused_whether_cached_or_not(monkeypatch):
             cache.put((MaskSpec(), 200, 256, 128, 128, "cuda"), object())
         with pytest.raises(ValueError, match="divisible"):
             block_mask.create_block_mask(MaskSpec(), 200, 256, 128, 128)
+
+
+def test_lru_shared_by_threads():
+    """Threads that look up, add and drop entries of one small cache at once: no lookup and no addition raises, and the
+    bound holds."""
+    lru, errors, interval = block_mask.LRU(2), [], sys.getswitchinterval()
+
+    def work(seed):
+        try:
+            for i in range(20000):
+                k = (seed * 7 + i * 3) % 5
+                if lru.get(k) is None:
+                    lru.put(k, object())
+                if i % 500 == 0:
+                    lru.clear()
+        except Exception as e:   # (reported by the test's own thread)
+            errors.append(e)
+    sys.setswitchinterval(1e-6)
+    try:
+        threads = [threading.Thread(target=work, args=(s,)) for s in range(8)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        sys.setswitchinterval(interval)
+    assert not errors, errors[:3]
+    assert len(lru) <= 2
