@@ -1,4 +1,5 @@
 """The host side of the block maps' caches."""
+import collections
 import sys
 import threading
 
@@ -45,3 +46,20 @@ def test_lru_shared_by_threads():
         sys.setswitchinterval(interval)
     assert not errors, errors[:3]
     assert len(lru) <= 2
+
+
+def test_lru_entry_dropped_while_it_is_added():
+    """Another thread fills the cache right behind an addition's first step: the addition still ends without an error."""
+    lru = block_mask.LRU(1)
+
+    class Interrupted(collections.OrderedDict):
+        def __setitem__(self, key, value):
+            super().__setitem__(key, value)
+            if key == "a":
+                other.start()
+                other.join(0.3)   # (done by then, or waiting for this addition)
+    other = threading.Thread(target=lambda: (lru.put("b", 1), lru.put("c", 1)))
+    lru._d = Interrupted()
+    lru.put("a", 1)
+    other.join()
+    assert len(lru) == 1
