@@ -135,10 +135,10 @@ static int tile_shape(int pass, int dtype, int D, int* bq, int* bk) {
 
 // sm_scale must be positive (the kernels track maxima of unscaled products and fold the scale into an
 // operand); flags must be known.
-static int check_scale_flags(float sm_scale, int flags) {
+static int check_scale_flags(float sm_scale, int flags, int known) {
   if (!(sm_scale > 0.f) || !(sm_scale < __builtin_huge_valf()))
     return set_error(FLEXATTN_EINVAL, "sm_scale must be positive and finite (got %g)", (double)sm_scale);
-  if (flags & ~(FLEXATTN_FLAG_COMPILED_LOOP | FLEXATTN_FLAG_WIDE_DS)) return set_error(FLEXATTN_EINVAL, "unknown flags 0x%x", flags);
+  if (flags & ~known) return set_error(FLEXATTN_EINVAL, "unknown flags 0x%x", flags);
   return FLEXATTN_OK;
 }
 
@@ -261,7 +261,8 @@ static int to_bwd_args(const flexattn_bwd_params* p, int pass, BwdArgs* a) {
   const int Sq = p->Sq - (p->pad & 0xffff), Sk = p->Sk - (p->pad >> 16);   // the tensors' lengths
   rc = check_shape(pass, p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->pad, p->D, p->dtype, p->map, p->ds ? FLEXATTN_PASS_DKV : -1);
   if (rc != FLEXATTN_OK) return rc;
-  if ((rc = check_scale_flags(p->sm_scale, p->flags)) != FLEXATTN_OK) return rc;
+  if ((rc = check_scale_flags(p->sm_scale, p->flags, FLEXATTN_FLAG_COMPILED_LOOP |
+                                  (p->dtype == FLEXATTN_BF16 && p->D == 256 ? FLEXATTN_FLAG_WIDE_DS : 0))) != FLEXATTN_OK) return rc;
   if ((rc = check_score(p->score)) != FLEXATTN_OK) return rc;
   if ((rc = check_mask(p->mask)) != FLEXATTN_OK) return rc;
   if ((rc = check_doc_batches(p->mask, p->B)) != FLEXATTN_OK) return rc;
@@ -311,7 +312,7 @@ static int fwd_with_map(const flexattn_fwd_params* p, const flexattn_block_map& 
   if (rc != FLEXATTN_OK) return rc;
   rc = check_shape(FLEXATTN_PASS_FWD, p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->pad, p->D, p->dtype, map);
   if (rc != FLEXATTN_OK) return rc;
-  if ((rc = check_scale_flags(p->sm_scale, p->flags)) != FLEXATTN_OK) return rc;
+  if ((rc = check_scale_flags(p->sm_scale, p->flags, FLEXATTN_FLAG_COMPILED_LOOP)) != FLEXATTN_OK) return rc;
   if ((rc = check_score(p->score)) != FLEXATTN_OK) return rc;
   if ((rc = check_mask(p->mask)) != FLEXATTN_OK) return rc;
   if ((rc = check_doc_batches(p->mask, p->B)) != FLEXATTN_OK) return rc;
@@ -485,7 +486,7 @@ int flexattn_fwd_decode(const flexattn_fwd_params* p, void* work, int64_t work_b
   if (!p->q || !p->k || !p->v || !p->o) return set_error(FLEXATTN_EINVAL, "q, k, v or o is NULL");
   if ((p->l == nullptr) != (p->m == nullptr)) return set_error(FLEXATTN_EINVAL, "l and m must both be given or both NULL");
   if (!decode_ok(p)) return set_error(FLEXATTN_ENOTSUP, "not a request of flexattn_fwd_decode (flexattn_fwd_decode_bytes is -1)");
-  int rc = check_scale_flags(p->sm_scale, p->flags);
+  int rc = check_scale_flags(p->sm_scale, p->flags, 0);
   if (rc != FLEXATTN_OK) return rc;
   if ((rc = check_aligned(1, p->dtype, p->D, {p->q, p->k, p->v, p->o, work})) != FLEXATTN_OK) return rc;
   const int64_t need = fwd_decode_bytes(p->B, p->Hq, p->Hkv, p->Sq, p->Sk, p->D);

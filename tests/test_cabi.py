@@ -171,3 +171,20 @@ def test_head_dim_64_requests(lib):
     for D in (16, 32, 64):
         for p, want in ((F, 64 if D > 16 else 128), (DQ, 64), (DKV, 64)):
             assert call_head_dim(p, D, torch.bfloat16, D ** -0.5, None, None, MaskSpec(), 512, 512) == want
+
+
+def test_the_wide_ds_flag_belongs_to_one_kind_of_backward(lib):
+    """FLEXATTN_FLAG_WIDE_DS is known to bf16 backward calls of head dimension 256; everything else refuses it, as it
+    refuses any flag that it does not know."""
+    dummy = C.create_string_buffer(64)
+    base = C.addressof(dummy)
+    for D, dtype, cls, fn, which in ((128, _lib.BF16, _lib.FwdParamsC, lib.flexattn_fwd, _lib.PASS_FWD),
+                                     (256, _lib.BF16, _lib.FwdParamsC, lib.flexattn_fwd, _lib.PASS_FWD),
+                                     (128, _lib.BF16, _lib.BwdParamsC, lib.flexattn_bwd_dq, _lib.PASS_DQ),
+                                     (128, _lib.F32, _lib.BwdParamsC, lib.flexattn_bwd_dkv, _lib.PASS_DKV)):
+        p = cls(q=base, k=base, v=base, B=1, Hq=1, Hkv=1, Sq=256, Sk=256, D=D, dtype=dtype, sm_scale=1.0, flags=_lib.FLAG_WIDE_DS)
+        for name in ("o",) if cls is _lib.FwdParamsC else ("dout", "l", "m", "delta", "dq", "dk", "dv"):
+            setattr(p, name, base)
+        bq, bk = _lib.tile_shape(which, dtype, D)
+        p.map = _lib.BlockMapC(base, base, base, base, base, 256 // bq, 256 // bk, bq, bk)
+        assert fn(C.byref(p), None) == _lib.EINVAL and b"unknown flags" in lib.flexattn_last_error_string(), (D, dtype)
