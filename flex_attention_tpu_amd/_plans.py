@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes as C
 import struct
+import weakref
 from typing import Optional
 
 import torch
@@ -20,17 +21,18 @@ from ._common import aligned, call_head_dim, dtype_code, on_device, stream_of, t
 from .block_mask import LRU, build_block_map, mask_spec_c
 from .masks import MaskSpec
 
-_plans = LRU(64)   # (pass, q shape, k shape, dtype, device, mask, scale) -> _Plan; bounded, holds block maps only
+_plans = LRU(64)   # (pass, q shape, k shape, dtype, device, mask, scale) -> _Plan; bounded, holds no device memory
 _FWD_POINTERS = struct.Struct("6P")     # q, k, v, o, l, m
 _BWD_POINTERS = struct.Struct("10P")    # q, k, v, dout, l, m, delta, dq, dk, dv
 
 
 class _Plan:
-    """Parameter templates (bytes) of one combination and the block maps they point at."""
+    """Parameter templates (bytes) of one combination and weak references to the block maps they point at: the maps
+    belong to their own bounded cache, and a plan whose map has been dropped there is made again."""
     __slots__ = ("templates", "maps")
 
     def __init__(self, templates, maps):
-        self.templates, self.maps = templates, maps
+        self.templates, self.maps = templates, tuple(weakref.ref(bm) for bm in maps)
 
 
 def _template(cls, pass_id, q, k, spec, sm_scale):
@@ -45,14 +47,17 @@ def _template(cls, pass_id, q, k, spec, sm_scale):
     return bytes(p), bm
 
 
-def _plan(key, q, k, spec, sm_scale, cls, passes) -> _Plan:
+def _plan(key, q, k, spec, sm_scale, cls, passes):
+    """(templates, block maps) of a combination; the caller holds the maps until its launch is out."""
     plan = _plans.get(key)
-    if plan is None:
-        plan = _Plan(*zip(*(_template(cls, pass_id, q, k, spec, sm_scale) for pass_id in passes)))
+    maps = [ref() for ref in plan.maps] if plan is not None else [None]
+    if None in maps:
+        templates, maps = zip(*(_template(cls, pass_id, q, k, spec, sm_scale) for pass_id in passes))
+        plan = _Plan(templates, maps)
         _plans.put(key, plan)
-    for bm in plan.maps:   # (a map built on another stream: this one waits for it)
+    for bm in maps:   # (a map built on another stream: this one waits for it)
         bm.wait_ready(q.device)
-    return plan
+    return plan.templates, maps
 
 
 def takes(q, k, spec: MaskSpec, sm_scale, *passes: int) -> bool:
@@ -66,7 +71,7 @@ def takes(q, k, spec: MaskSpec, sm_scale, *passes: int) -> bool:
 
 def forward(q, k, v, spec: MaskSpec, sm_scale, save_residuals):
     """(o, l, m), or o, of a call that `takes` accepts."""
-    plan = _plan((0, q.shape, k.shape, q.dtype, q.device, spec, sm_scale), q, k, spec, sm_scale, _lib.FwdParamsC, (_lib.PASS_FWD,))
+    templates, maps = _plan((0, q.shape, k.shape, q.dtype, q.device, spec, sm_scale), q, k, spec, sm_scale, _lib.FwdParamsC, (_lib.PASS_FWD,))
     qp, kp, vp = q.data_ptr(), k.data_ptr(), v.data_ptr()
     if (qp | kp | vp) % 16:
         return forward(aligned(q), aligned(k), aligned(v), spec, sm_scale, save_residuals)
@@ -75,7 +80,7 @@ def forward(q, k, v, spec: MaskSpec, sm_scale, save_residuals):
     if save_residuals:
         l = torch.empty(q.shape[:3], dtype=torch.float32, device=q.device)
         m = torch.empty_like(l)
-    p = _lib.FwdParamsC.from_buffer_copy(plan.templates[0])
+    p = _lib.FwdParamsC.from_buffer_copy(templates[0])
     _FWD_POINTERS.pack_into(p, 0, qp, kp, vp, o.data_ptr(),
                             l.data_ptr() if save_residuals else 0, m.data_ptr() if save_residuals else 0)
     lib = _lib.load()
@@ -86,15 +91,15 @@ def forward(q, k, v, spec: MaskSpec, sm_scale, save_residuals):
 
 def backward(q, k, v, l, m, o, do, spec: MaskSpec, sm_scale):
     """(dq, dk, dv) of a call that `takes` accepts: delta, the dq and the dk/dv pass (flexattn_bwd)."""
-    plan = _plan((1, q.shape, k.shape, q.dtype, q.device, spec, sm_scale), q, k, spec, sm_scale, _lib.BwdParamsC,
-                 (_lib.PASS_DQ, _lib.PASS_DKV))
+    templates, maps = _plan((1, q.shape, k.shape, q.dtype, q.device, spec, sm_scale), q, k, spec, sm_scale, _lib.BwdParamsC,
+                            (_lib.PASS_DQ, _lib.PASS_DKV))
     head = (q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(), l.data_ptr(), m.data_ptr())
     op = o.data_ptr()
     if (head[0] | head[1] | head[2] | head[3] | op) % 16:
         return backward(aligned(q), aligned(k), aligned(v), l, m, aligned(o), aligned(do), spec, sm_scale)
     dq, dk, dv, delta = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v), torch.empty_like(l)
-    pq = _lib.BwdParamsC.from_buffer_copy(plan.templates[0])
-    pkv = _lib.BwdParamsC.from_buffer_copy(plan.templates[1])
+    pq = _lib.BwdParamsC.from_buffer_copy(templates[0])
+    pkv = _lib.BwdParamsC.from_buffer_copy(templates[1])
     d = delta.data_ptr()
     _BWD_POINTERS.pack_into(pq, 0, *head, 0, dq.data_ptr(), 0, 0)
     _BWD_POINTERS.pack_into(pkv, 0, *head, d, 0, dk.data_ptr(), dv.data_ptr())
