@@ -70,3 +70,49 @@ def test_bias_gradient_repeats_bit_for_bit(kind):
     for _ in range(4):
         for name, a, b in zip(("dq", "dk", "dv", "dab"), call(), want):
             assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D", [(2, 4, 4, 257, 128), (2, 4, 2, 300, 64)])
+@pytest.mark.parametrize("kind", ["alibi", "tile_alibi", "closure", "compiled mask", "documents", "ids per entry"])
+def test_bias_gradient_of_every_kernel(kind, B, Hq, Hkv, S, D):
+    """The kernels that store the bias gradient are variants of their own per score kind and library: position biases, a
+    compiled score function, a compiled mask, documents, segment ids with a row per batch entry."""
+    import custom_functors as cf
+    import flex_attention_tpu_amd as F
+    from flex_attention_tpu_amd import masks, scores
+    sc, pair, sfn, sid, okw = 1 / math.sqrt(D), None, None, None, {}
+    if kind == "alibi":
+        sfn, okw = scores.make_alibi_global_score_fn(Hq), dict(score_mod=O.score_mod_alibi_global(O.alibi_slopes(Hq)))
+    elif kind == "tile_alibi":
+        sfn, okw = scores.make_alibi_score_fn(0.02), dict(score_mod=O.score_mod_alibi_tile_local(0.02, 128, 128))
+    elif kind == "closure":
+        sfn, okw = cf.compiled()["mixed_mod"][0], dict(score_mod=cf.mixed_mod)
+    elif kind == "compiled mask":
+        i = torch.arange(S)
+        pair, okw = cf.compiled()["checker"][1], dict(mask=cf.checker_mask(i, i))
+    elif kind == "documents":
+        lens = [100, 29, S - 129]
+        pair = masks.make_jagged_mask_fns(128, 128, lens)
+        okw = dict(causal=True, segment_ids=O.doc_ids_from_lengths(lens))
+    else:
+        sid = torch.stack([torch.arange(S) * (3 + b) // S for b in range(B)])
+        okw = dict(segment_ids=sid)
+    ab = torch.randn(1, Hq, S, S, generator=torch.Generator().manual_seed(3))
+    okw["ab"] = ab.expand(B, Hq, S, S)
+    q, k, v, do = O.make_inputs(B, Hq, Hkv, S, S, D, dtype=torch.bfloat16, seed=S + D)
+    qg, kg, vg, abg = [surrounded(x).requires_grad_(True) for x in (q, k, v, ab)]
+    o = F.flex_attention(qg, kg, vg, sfn, pair, segment_ids=sid, sm_scale=sc, ab=abg)
+    dq, dk, dv, dab = torch.autograd.grad(o, (qg, kg, vg, abg), surrounded(do))
+    mf = pair or (None, None)
+    with torch.no_grad():
+        o2, l, m = F._flex_attention_impl(qg, kg, vg, abg, sid, True, False, sc, 1, 128, 128, 128, False, mf[1], mf[0], sfn)
+    assert torch.equal(o2, o)
+    same = same_residual_grads(q, k, v, do, o, l, m, sm_scale=sc, **okw)
+    for name, t, r in zip(("dq", "dk", "dv"), (dq, dk, dv), same):
+        # (without a causal mask the position bias leaves most of every row's weight on the last keys: their dv sums P dO over
+        # all rows, each term with the 2^-9 that P loses in bf16, so the error is of the sum of the terms' sizes, which the
+        # tensor's largest entry shows, not of the element that is left after they cancel)
+        assert_close(name, t, r, torch.bfloat16, tensor_scale=kind == "alibi")
+    ref = O.mha_bwd_reference(q, k, v, o.detach().float().cpu(), do, l.cpu(), m.cpu(), sm_scale=sc, return_dab=True, **okw)[3].sum(0, keepdim=True)
+    err = (dab.cpu().double() - ref).abs()
+    assert O.rel_l2(dab, ref) <= 1e-2 and bool((err <= 1e-2 * ref.abs().clamp(min=1.0)).all()), float(err.max())
