@@ -221,7 +221,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
     // S and dP of a 32-row block (cc: block of the 128 rows).  kAhead: a block's products are issued while the block before
     // goes through its element-wise work, which needs neither: the matrix pipe and the vector unit then work at the same
     // time (one wave per SIMD: nothing else overlaps them; symmetric ALiBi closure, B=8, H=4, S=2048, forward and backward:
-    // 375.7 -> 367.3 us).  With the code of a bias there are no registers for it.
+    // 383.5 -> 378.8 us, two builds in turn).  With the code of a bias there are no registers for it.
     constexpr bool kAhead = kNoBias;
     auto products = [&](int cc, f32x16& s, f32x16& dp) {
       const char* qt = reinterpret_cast<const char*>(sQ + (2 * buf + (cc >> 1)) * kTileElems) + (cc & 1) * 32 * kTileD * 2;

@@ -259,7 +259,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
             gb[u] = gl;
             dsv[u] = gd;
           }
-          // (elements of the tile before get the value that tile stores, too: the same products in the same order)
+          // (elements shared with the tile before: the same lane stores them for both tiles, one after the other)
           if (dab_row != nullptr) *reinterpret_cast<f32x4_a4*>(dab_row + j0) = gb;
           const bf16x2 d01 = pack_bf16(dsv[0], dsv[1]), d23 = pack_bf16(dsv[2], dsv[3]);
           const int o = 4 * (g & 1);

@@ -36,7 +36,9 @@ def _hands_ds_over(q, k, ab, segment_ids, sm_scale, score_fn, mask_fn, block_mas
     if ab is not None:
         return False
     # (at head dimension 256 always: the recomputing dq pass costs three products of twice the depth.  On B=4, H=16,
-    # S=4096, causal, forward and backward: 3.61 -> 3.08 ms.  Not at the head dimension 64 kernels, which hand nothing over.)
+    # S=4096, causal, forward and backward: 3.61 -> 3.08 ms.  Not at the head dimension 64 kernels, which hand nothing over:
+    # recomputing there beats the hand-over on 128 padded columns also where that pays at 128 columns; documents, B=4, H=16,
+    # S=4096: 1.40 -> 0.71 ms, GQA 4:1, S=16384: 1.81 -> 1.16 ms; causal window 1025, B=2, H=16, S=8192: 0.97 -> 0.46 ms.)
     return ((D > 128 or ds_exchange_pays(score_fn, mask_fn, segment_ids)) and
             call_head_dim(_lib.PASS_DKV, D, q.dtype, sm_scale, score_fn, ab, spec_of(mask_fn, block_mask_fn), q.shape[2], k.shape[2]) != 64)
 
