@@ -50,7 +50,7 @@ def _template(cls, pass_id, q, k, spec, sm_scale):
 def _plan(key, q, k, spec, sm_scale, cls, passes):
     """(templates, block maps) of a combination; the caller holds the maps until its launch is out."""
     plan = _plans.get(key)
-    maps = [ref() for ref in plan.maps] if plan is not None else [None]
+    maps = [ref() for ref in plan.maps] if plan is not None else (None,)
     if None in maps:
         templates, maps = zip(*(_template(cls, pass_id, q, k, spec, sm_scale) for pass_id in passes))
         plan = _Plan(templates, maps)
@@ -63,10 +63,13 @@ def _plan(key, q, k, spec, sm_scale, cls, passes):
 def takes(q, k, spec: MaskSpec, sm_scale, *passes: int) -> bool:
     """Whether these passes of a checked call without score function and bias are prepared ones.  (Document ids keep arrays per stream,
     compiled masks their own libraries, and padded calls copy their operands: those go the general way.)"""
-    Sq, D = q.shape[2], q.shape[3]
+    _, _, Sq, D = q.shape
     Sk = k.shape[2]
-    return (spec.doc_ids is None and spec.custom is None and Sq >= 128 and Sk >= 128
-            and (D == 128 or all([call_head_dim(p, D, q.dtype, sm_scale, None, None, spec, Sq, Sk) == D for p in passes])))
+    if spec.doc_ids is not None or spec.custom is not None or Sq < 128 or Sk < 128:
+        return False
+    if D == 128 or (D == 64 and q.dtype is torch.float32):   # (no question to the library in the usual cases)
+        return True
+    return all([call_head_dim(p, D, q.dtype, sm_scale, None, None, spec, Sq, Sk) == D for p in passes])
 
 
 def forward(q, k, v, spec: MaskSpec, sm_scale, save_residuals):

@@ -25,11 +25,9 @@ from .flex_attention_kernel import _CAUSAL, _flex_attention_impl
 
 
 def _hands_ds_over(q, k, ab, segment_ids, sm_scale, score_fn, mask_fn, block_mask_fn, want_dab) -> bool:
-    """Whether a backward that wants every gradient hands dS from the dk/dv pass to the dq pass (DsBlocks in
+    """Whether a bf16 backward that wants every gradient hands dS from the dk/dv pass to the dq pass (DsBlocks in
     flex_attention_dq_bwd.py).  The buffer holds one 32 KB block per query head and kept pair of 128 x 128 tiles (what the
     mask skips takes no room)."""
-    if q.dtype != torch.bfloat16:
-        return False
     D = q.shape[-1]
     if want_dab:   # (the bias gradient is the fp32 dS that the dk/dv pass rounds for the hand-over: one pass makes both, and the dq
         return D <= 128   # pass is one product instead of three; B=4, H=16, S=1500, forward and backward: 1.19 -> 1.03 ms)
@@ -43,17 +41,20 @@ def _hands_ds_over(q, k, ab, segment_ids, sm_scale, score_fn, mask_fn, block_mas
             call_head_dim(_lib.PASS_DKV, D, q.dtype, sm_scale, score_fn, ab, spec_of(mask_fn, block_mask_fn), q.shape[2], k.shape[2]) != 64)
 
 
-def _bwd_with_ds(q, k, v, ab, segment_ids, l, m, o, do, want_dab, *, block_q, block_k, **kw):
-    """(dq, dk, dv, dab or None) with dS handed from the dk/dv pass to the dq pass; where the dk/dv entry point declines
-    to (no room for the buffer, kernels that exchange nothing), the dq pass recomputes."""
-    kw.update(block_b=1, block_q=block_q, block_k_major=block_k, block_k=block_k, debug=False)
+def _bwd_with_ds(q, k, v, ab, segment_ids, l, m, o, do, want_dab, block_q, block_k, sm_scale, causal, score_fn, mask_fn, block_mask_fn):
+    """The gradients of q, k, v and the bias (or None) as the autograd function returns them, with dS handed from the dk/dv
+    pass to the dq pass; where the dk/dv entry point declines to (no room for the buffer, kernels that exchange nothing),
+    the dq pass recomputes."""
+    kw = dict(block_b=1, block_q=block_q, block_k_major=block_k, block_k=block_k, sm_scale=sm_scale, causal=causal, debug=False,
+              score_fn=score_fn, mask_fn=mask_fn, block_mask_fn=block_mask_fn)
     di = compute_delta(o, do)
     dk, dv, ds, *dab = flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, block_q_major=block_q, return_ds=True,
                                                _wide_ds=not want_dab, _dab=want_dab, **kw)
     if ds is None and want_dab:
         dq, dab = flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, di, return_dab=True, **kw)
-        return dq, dk, dv, dab
-    return flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, di, ds=ds, **kw), dk, dv, (dab[0] if want_dab else None)
+        return dq, dk, dv, dab, None
+    dq = flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, di, ds=ds, **kw)
+    return dq, dk, dv, (dab[0] if want_dab else None), None
 
 
 def flex_attention_bwd(q, k, v, ab, segment_ids, l, m, o, do, *, block_q, block_k, sm_scale, causal=False, score_fn=None,
@@ -73,7 +74,8 @@ def flex_attention_bwd(q, k, v, ab, segment_ids, l, m, o, do, *, block_q, block_
             spec = spec.combine(_CAUSAL)
         if _plans.takes(q, k, spec, sm_scale, _lib.PASS_DQ, _lib.PASS_DKV):
             return _plans.backward(q, k, v, l, m, o, do, spec, float(sm_scale))
-    q, k, v, do = aligned(q), aligned(k), aligned(v), aligned(do)   # (the two passes share them)
+    if (q.data_ptr() | k.data_ptr() | v.data_ptr() | do.data_ptr()) % 16:   # (the two passes share them)
+        q, k, v, do = aligned(q), aligned(k), aligned(v), aligned(do)
     kw = dict(sm_scale=sm_scale, debug=False, score_fn=score_fn, mask_fn=mask_fn, block_mask_fn=block_mask_fn,
               compiled_loop=compiled_loop)
     dq_call = flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, None, block_b=1, block_q=block_q,
@@ -120,16 +122,20 @@ class _FlexAttention(torch.autograd.Function):
         dq = dk = dv = dab = None
         want_dkv = ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
         want_dq = ctx.needs_input_grad[0] or want_dab
-        kw = dict(block_q=block_q, block_k=block_k, sm_scale=sm_scale, causal=causal, score_fn=score_fn, mask_fn=mask_fn,
-                  block_mask_fn=block_mask_fn)
-        if want_dkv and ctx.needs_input_grad[0] and _hands_ds_over(q, k, ab, segment_ids, sm_scale, score_fn, mask_fn, block_mask_fn, want_dab):
-            try:
-                return (*_bwd_with_ds(q, k, v, ab, segment_ids, l, m, o, do, want_dab, **kw), None)
-            except torch.cuda.OutOfMemoryError:
-                pass   # (beside the dS buffer there was no room for the rest: below nothing needs one)
-        if want_dkv and ctx.needs_input_grad[0] and not want_dab:
-            return (*flex_attention_bwd(q, k, v, ab, segment_ids, l, m, o, do, **kw), None, None)
-        kw.update(block_b=1, block_k_major=block_k, debug=False)
+        if want_dkv and ctx.needs_input_grad[0]:
+            if q.dtype is torch.bfloat16 and _hands_ds_over(q, k, ab, segment_ids, sm_scale, score_fn, mask_fn, block_mask_fn, want_dab):
+                try:
+                    return _bwd_with_ds(q, k, v, ab, segment_ids, l, m, o, do, want_dab, block_q, block_k, sm_scale, causal, score_fn,
+                                        mask_fn, block_mask_fn)
+                except torch.cuda.OutOfMemoryError:
+                    pass   # (beside the dS buffer there was no room for the rest: below nothing needs one)
+            if not want_dab:
+                dq, dk, dv = flex_attention_bwd(q, k, v, ab, segment_ids, l, m, o, do, block_q=block_q, block_k=block_k,
+                                                sm_scale=sm_scale, causal=causal, score_fn=score_fn, mask_fn=mask_fn,
+                                                block_mask_fn=block_mask_fn)
+                return dq, dk, dv, None, None
+        kw = dict(block_b=1, block_q=block_q, block_k=block_k, block_k_major=block_k, sm_scale=sm_scale, causal=causal, debug=False,
+                  score_fn=score_fn, mask_fn=mask_fn, block_mask_fn=block_mask_fn)
         # di = sum(o * do), float32 [B, H, Sq] (jax_exp.py:276-278): taken by the dq pass itself where that pass runs
         # first, else by its own launch
         di = None

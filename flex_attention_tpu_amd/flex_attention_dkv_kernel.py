@@ -41,7 +41,10 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
     # (a dS hand-over is at 128 columns)
     D_user, D = D, (call_head_dim(_lib.PASS_DKV, D, q.dtype, sm_scale, score_fn, ab, spec, Sq, Sk, compiled_loop) if not return_ds
                     else kernel_head_dim(D, q.dtype))   # smaller head dimensions: zero-padded columns
-    q, do, k, v = (aligned(pad_seq(t, D, 3)) for t in (q, do, k, v))
+    if D != D_user:
+        q, do, k, v = pad_seq(q, D, 3), pad_seq(do, D, 3), pad_seq(k, D, 3), pad_seq(v, D, 3)
+    if (q.data_ptr() | do.data_ptr() | k.data_ptr() | v.data_ptr()) % 16:
+        q, do, k, v = aligned(q), aligned(do), aligned(k), aligned(v)
     bm = kernel_block_map(_lib.PASS_DKV, spec, q, Sq_p, Sk_p, D, score_fn)
     dk = torch.empty_like(k)
     dv = torch.empty_like(v)

@@ -23,7 +23,8 @@ def compute_delta(o: torch.Tensor, do: torch.Tensor) -> torch.Tensor:
     if D not in (64, 128) and not (D == 256 and o.dtype == torch.bfloat16):   # (zero columns add nothing to the sum)
         D = kernel_head_dim(D, o.dtype)
         o, do = pad_seq(o, D, 3), pad_seq(do, D, 3)
-    o, do = aligned(o), aligned(do)
+    if (o.data_ptr() | do.data_ptr()) % 16:
+        o, do = aligned(o), aligned(do)
     d = torch.empty(B, H, S, dtype=torch.float32, device=o.device)
     with on_device(o.device):
         _lib.check(_lib.load().flexattn_bwd_delta(o.data_ptr(), do.data_ptr(), d.data_ptr(), B * H * S, D,
@@ -160,7 +161,10 @@ def flex_attention_bwd_dq(q, k, v, ab, segment_ids, l, m, o, do, d, *, block_b, 
     # (a dS hand-over is at 128 columns)
     D_user, D = D, (call_head_dim(_lib.PASS_DQ, D, q.dtype, sm_scale, score_fn, ab, spec, Sq, Sk, compiled_loop) if ds is None
                     else kernel_head_dim(D, q.dtype))   # smaller head dimensions: zero-padded columns
-    q, do, k, v = (aligned(pad_seq(t, D, 3)) for t in (q, do, k, v))
+    if D != D_user:
+        q, do, k, v = pad_seq(q, D, 3), pad_seq(do, D, 3), pad_seq(k, D, 3), pad_seq(v, D, 3)
+    if (q.data_ptr() | do.data_ptr() | k.data_ptr() | v.data_ptr()) % 16:
+        q, do, k, v = aligned(q), aligned(do), aligned(k), aligned(v)
     o_p = aligned(pad_seq(pad_seq(o, Sq_p), D, 3)) if fuse_delta else None
     if ds is not None and (ds.buf is None or ds.index is None or ds.shape != (B, Hq, Sq_p, Sk_p) or ds.buf.device != q.device
                            or ds.compiled_loop != bool(compiled_loop)):

@@ -32,7 +32,10 @@ def _decode(q, k, v, mask_fn, block_mask_fn, save_residuals, sm_scale):
     if q.dtype != torch.bfloat16 or D > 128 or Hq // Hkv * Sq > 128 or spec_of(mask_fn, block_mask_fn).flags:
         return None
     D_user, D = D, 64 if D <= 64 else 128
-    q, k, v = (aligned(pad_seq(t, D, 3)) for t in (q, k, v))
+    if D != D_user:
+        q, k, v = pad_seq(q, D, 3), pad_seq(k, D, 3), pad_seq(v, D, 3)
+    if (q.data_ptr() | k.data_ptr() | v.data_ptr()) % 16:
+        q, k, v = aligned(q), aligned(k), aligned(v)
     o = torch.empty_like(q)
     l = m = None
     if save_residuals:
@@ -85,7 +88,10 @@ def _flex_attention_impl(q, k, v, ab, segment_ids, save_residuals, causal, sm_sc
     check_doc_batches(spec, B)   # (ids of shape [B, S]: the kernels mask every batch entry by its own row)
     q, k, v = pad_seq(q, Sq_p), pad_seq(k, Sk_p), pad_seq(v, Sk_p)
     D_user, D = D, call_head_dim(_lib.PASS_FWD, D, q.dtype, sm_scale, score_fn, ab, spec, Sq, Sk, compiled_loop)   # smaller head dimensions: zero-padded columns
-    q, k, v = (aligned(pad_seq(t, D, 3)) for t in (q, k, v))
+    if D != D_user:
+        q, k, v = pad_seq(q, D, 3), pad_seq(k, D, 3), pad_seq(v, D, 3)
+    if (q.data_ptr() | k.data_ptr() | v.data_ptr()) % 16:
+        q, k, v = aligned(q), aligned(k), aligned(v)
     bm = kernel_block_map(_lib.PASS_FWD, spec, q, Sq_p, Sk_p, D, score_fn)
     compiled_loop = compiled_loop or mostly_partial_custom_mask(spec, bm)
     ab_c, ab_keep = bias_c(ab, B, Hq, Sq, Sk, Sq_p, Sk_p, q.device)
