@@ -53,6 +53,8 @@ constexpr int MAX_LIST = 2048;       // longest q tile list the plain-score kern
 constexpr int PREFETCH_LIST = 1024;  // of which an item's prefetch carries this many in registers; the rest is read when the item starts
 // (Q, dO) x 2 buffers x 2 tiles, lse x2, delta x2, run-loop tables, cached q tile list and its partial flags
 constexpr int LDS_BYTES = 8 * kTileElems * 2 + 4 * BQ * 4 + 4 * 32 * 4 + MAX_LIST * 5 + kDocStageBytes + kMaxSortedItems * 4;
+// compiled loop: K, V and (Q, dO) x 2 buffers of 64 rows, lse x2, delta x2 of 64 rows
+constexpr int LOOP_LDS_BYTES = 8 * kTileElems * 2 + 4 * 64 * 4;
 }  // namespace dkv_cfg
 
 
@@ -71,7 +73,14 @@ struct PinnedState {
       "+{a[160:163]}"(st.v[0]), "+{a[164:167]}"(st.v[1]), "+{a[168:171]}"(st.v[2]), "+{a[172:175]}"(st.v[3]), \
       "+{a[176:179]}"(st.v[4]), "+{a[180:183]}"(st.v[5]), "+{a[184:187]}"(st.v[6]), "+{a[188:191]}"(st.v[7])
 
-// Score modifications: compiled C++ path, one 128 x 128 tile per loop iteration.
+// Score modifications: compiled C++ path.  One work-group = 8 waves = one 128-row kv tile; a loop iteration covers 64 q rows,
+// half an entry of the kv tile's list.  Wave w takes kv rows 32 (w & 3) and q rows 32 (w >> 2) of the iteration: one 32 x 32
+// block of S and dP, its element-wise work, and its share of dk and dv, which the two waves of a kv block add up through LDS
+// at the end.  K and V lie in LDS (64 KB) beside the double-buffered Q and dO (64 KB).
+// BOUND: the element-wise work (about 270 vector instructions per block, against 32 MFMAs of 32 cycles) and what of it the other
+// wave's products do not cover.  Two waves a SIMD, of at most 256 registers each; four waves with K and V in registers and
+// 128-row iterations had one wave a SIMD: symmetric ALiBi closure, B=8, H=4, S=2048, dk/dv with export 240 -> 180-198 us; bias,
+// B=4, H=16, S=1500, 478 -> 350-378 us.  A higher priority for one of a SIMD's waves, or around the products, changed nothing.
 // EXPORT: the kernel also writes the tile's bf16 dS (the B operands of the dk product: here with the score function's
 // derivative and sm_scale in them) to a.ds, in the block layout of the generated streams' export (see there), for
 // the dq pass from dS: a score function is then evaluated in one backward pass instead of two.
@@ -79,16 +88,17 @@ struct PinnedState {
 // DAB (with EXPORT and a bias): the kernel stores the bias gradient as well.  (A variant of its own: with the stores behind
 // a test the compiler associates the element-wise sums differently, and dk and dv would change a bit with the export.)
 template <int SCORE, bool EXPORT, bool AB, bool DAB>
-__global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
+__global__ __launch_bounds__(512, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
   using namespace dkv_cfg;
   constexpr bool kBias = SCORE == kScoreBiasOnly;             // a bias and no score function: launched as a kind of its own
   constexpr bool kNoBias = SCORE == FLEXATTN_SCORE_NONE || !AB;
   static_assert(!DAB || (EXPORT && !kNoBias), "the bias gradient comes with the export of a call with a bias");
+  constexpr int HQ = 64;   // q rows per iteration
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
-  bf16_t* sQ = reinterpret_cast<bf16_t*>(smem_raw);
-  bf16_t* sDO = sQ + 4 * kTileElems;
-  float* sLse = reinterpret_cast<float*>(sDO + 4 * kTileElems);
-  float* sDl = sLse + 2 * BQ;
+  bf16_t* sK = reinterpret_cast<bf16_t*>(smem_raw);   // K rows 0-63, 64-127, V the same
+  bf16_t* sQ = sK + 4 * kTileElems;                   // buffer b: Q at tile 2 b, dO at 2 b + 1
+  float* sLse = reinterpret_cast<float*>(sQ + 4 * kTileElems);
+  float* sDl = sLse + 2 * HQ;
 
   const int nKb = a.map.nk;
   const int nQ = a.map.nq;
@@ -103,26 +113,16 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
 
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wk = w & 3, wq = w >> 2;   // the wave's kv block and its q block of an iteration
   const int lane = tid & 63;
   const int l32 = lane & 31;
   const int hh = lane >> 5;
 
-  const int kv_local = w * 32 + l32;
+  const int kv_local = wk * 32 + l32;
   const int k0 = tile_base(kb, BNK, a.Sk);
   const int k_idx = k0 + kv_local;
   const bool own_col = k_idx >= kb * BNK;   // (else a row of the kv tile before)
   const size_t kv_off = ((size_t)bhk * a.Sk + (size_t)k0) * D;
-  const bf16_t* Kg = static_cast<const bf16_t*>(a.k) + kv_off;
-  const bf16_t* Vg = static_cast<const bf16_t*>(a.v) + kv_off;
-  const bf16_t* Qall = static_cast<const bf16_t*>(a.q);
-  const bf16_t* dOall = static_cast<const bf16_t*>(a.dout);
-
-  bf16x8 kreg[8], vreg[8];
-#pragma unroll
-  for (int ks = 0; ks < 8; ++ks) {
-    kreg[ks] = *reinterpret_cast<const bf16x8*>(Kg + (size_t)kv_local * D + ks * 16 + hh * 8);
-    vreg[ks] = *reinterpret_cast<const bf16x8*>(Vg + (size_t)kv_local * D + ks * 16 + hh * 8);
-  }
   int doc_j = 0;
   if (mk.flags & FLEXATTN_MASK_DOC) doc_j = mk.doc_k[k_idx];
 
@@ -138,41 +138,52 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
   const int n_tiles = a.map.cnt[kb];
   const int* tile_idx = a.map.idx + (size_t)kb * nQ;
   const bool ragged_q = nQ * BQ != a.Sq;   // (the last q tile then shares rows with the one before)
-  const int n_iter = n_tiles * group;
+  const int n_iter = 2 * n_tiles * group;
 
-  // Iteration `it` covers q tile tile_idx[it % n_tiles] of query head hk*group + it / n_tiles.
-  // Its q block index is fetched two iterations ahead, its state one iteration ahead.
-  auto q_block_of = [&](int it) { return tile_idx[it % n_tiles]; };
-  int qb_cur = 0, qb_nxt = 0, st_cur = 0;
-  if (n_iter > 0) qb_cur = q_block_of(0);
-  if (n_iter > 1) qb_nxt = q_block_of(1);
-  if (n_iter > 0) st_cur = a.map.state[(size_t)qb_cur * a.map.nk + kb];
-
-  TileLoader<4> loader;
+  TileLoader<8> loader;
   loader.init(w, lane);
-  float lse_st = 0.f, dl_st = 0.f;
-  auto issue_tile = [&](int it, int qb, int buf) {
-    const int g = it / n_tiles;
-    const size_t rbase = ((size_t)(b * a.Hq + hk * group + g) * a.Sq + (size_t)tile_base(qb, BQ, a.Sq));
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      loader.load(Qall + (rbase + half * kTileRows) * D, sQ + (2 * buf + half) * kTileElems);
-      loader.load(dOall + (rbase + half * kTileRows) * D, sDO + (2 * buf + half) * kTileElems);
-    }
-    if (tid < BQ) {
-      const float l_i = a.l[rbase + tid], m_i = a.m[rbase + tid];
-      lse_st = (l_i > 0.f) ? __builtin_fmaf(m_i, kLog2e, log2f(l_i)) : __builtin_huge_valf();
+  // Iteration `it` covers rows 64 (it & 1) .. of list entry t of query head hk group + g, it = 2 (g n_tiles + t) + (it & 1).
+  // `at` walks the entries one ahead of the iteration that computes; its q block index and state are fetched an entry ahead.
+  int g_at = 0, t_at = 0;   // entry that is copied next
+  int qb_at = 0, st_at = 0, qb_next = 0;
+  if (n_iter > 0) {
+    qb_at = __builtin_amdgcn_readfirstlane(tile_idx[0]);
+    st_at = a.map.state[(size_t)qb_at * nKb + kb];
+    qb_next = n_tiles > 1 ? tile_idx[1] : qb_at;
+  }
+  float l_st = 0.f, m_st = 0.f, dl_st = 0.f;
+  auto issue_rows = [&](int half, int buf) {
+    const size_t rbase = ((size_t)(b * a.Hq + hk * group + g_at) * a.Sq + (size_t)(tile_base(qb_at, BQ, a.Sq) + half * HQ));
+    loader.load(static_cast<const bf16_t*>(a.q) + rbase * D, sQ + 2 * buf * kTileElems);
+    loader.load(static_cast<const bf16_t*>(a.dout) + rbase * D, sQ + (2 * buf + 1) * kTileElems);
+    if (tid < HQ) {
+      l_st = a.l[rbase + tid];
+      m_st = a.m[rbase + tid];
       dl_st = a.delta[rbase + tid];
     }
   };
   auto store_rows = [&](int buf) {
-    if (tid < BQ) {
-      sLse[buf * BQ + tid] = lse_st;
-      sDl[buf * BQ + tid] = dl_st;
+    if (tid < HQ) {   // (the loads' values are first touched here: touched where they are issued, every iteration waits for its copies there)
+      sLse[buf * HQ + tid] = (l_st > 0.f) ? __builtin_fmaf(m_st, kLog2e, log2f(l_st)) : __builtin_huge_valf();
+      sDl[buf * HQ + tid] = dl_st;
     }
   };
+  auto advance = [&]() {   // `at` to the next entry
+    if (++t_at == n_tiles) {
+      t_at = 0;
+      ++g_at;
+    }
+    qb_at = __builtin_amdgcn_readfirstlane(qb_next);
+    st_at = a.map.state[(size_t)qb_at * nKb + kb];
+    qb_next = tile_idx[t_at + 1 < n_tiles ? t_at + 1 : 0];
+  };
   if (n_iter > 0) {
-    issue_tile(0, __builtin_amdgcn_readfirstlane(qb_cur), 0);
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      loader.load(static_cast<const bf16_t*>(a.k) + kv_off + half * kTileElems, sK + half * kTileElems);
+      loader.load(static_cast<const bf16_t*>(a.v) + kv_off + half * kTileElems, sK + (2 + half) * kTileElems);
+    }
+    issue_rows(0, 0);
     store_rows(0);
   }
   wait_vmem_all();
@@ -191,195 +202,219 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
     t_off[db][0] = (unsigned)(tile_off(t_row, 4 * db + t_chunk) + t_half) * 2u;
     t_off[db][1] = (unsigned)(tile_off(t_row + 8, 4 * db + t_chunk) + t_half) * 2u;
   }
+  const char* kt = reinterpret_cast<const char*>(sK + (wk >> 1) * kTileElems) + (wk & 1) * 32 * kTileD * 2;
+  const char* vt = kt + 2 * kTileElems * 2;
 
+  constexpr int kOpenStores = EXPORT ? 2 : 0;
+  float bias[16];
   ScoreMod<SCORE> sm;
+  int qb = 0, st = 0, g = 0, t = 0;   // the entry that is computed
   for (int it = 0; it < n_iter; ++it) {
     const int buf = it & 1;
-    const int qb = __builtin_amdgcn_readfirstlane(qb_cur);
-    const bool partial = __builtin_amdgcn_readfirstlane(st_cur) == 1 || (qb == nQ - 1 && ragged_q);
-    sm.init(a.score, a.sm_scale, hk * group + it / n_tiles, b);
-    const int qb_n2 = (it + 2 < n_iter) ? q_block_of(it + 2) : 0;
-    int st_nxt = 0;
-    if (it + 1 < n_iter) {
-      const int qbn = __builtin_amdgcn_readfirstlane(qb_nxt);
-      st_nxt = a.map.state[(size_t)qbn * a.map.nk + kb];
-      issue_tile(it + 1, qbn, buf ^ 1);
+    if (buf == 0) {   // an entry's first half: the entry that was copied ahead
+      if (it == 0 || g != g_at) sm.init(a.score, a.sm_scale, hk * group + g_at, b);
+      qb = qb_at;
+      st = st_at;
+      g = g_at;
+      t = t_at;
     }
+    const bool partial = __builtin_amdgcn_readfirstlane(st) == 1 || (qb == nQ - 1 && ragged_q);
     const int q0 = tile_base(qb, BQ, a.Sq);
+    const int cc = 2 * buf + wq;   // the wave's 32-row block of the q tile
     // (elements before this offset belong to the q tile before; a column of the kv tile before owns none)
     const int own = first_owned(qb, BQ, q0, 4 * hh, own_col);
-    // An additive bias: the values of a 32-row block are loaded a block ahead of their use (the first block's in front of
-    // its products).  Loaded where they are added, behind the products, the latency of every load showed: 1310 -> 456 us
-    // on B=4, H=16, S=1500 (dq, the same: 841 -> 400; forward 532 -> 166).
+    // An additive bias: a block's values are loaded behind the element-wise work of the block before and are there before
+    // the next rows' copies are issued (vector-memory operations complete in order: behind the copies the first use would
+    // wait for them too).
     const unsigned lane_off = (unsigned)(4 * hh) * (unsigned)a.Sk + (unsigned)k_idx;   // (of a bias or its gradient)
-    float bias_next[16];
-    auto load_bias = [&](int row0) {
+    auto load_bias = [&](const ScoreMod<SCORE>& of, int row0) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) bias_next[e] = sm.bias2_rows(row0 + acc_row(e, 0), lane_off);
+      for (int e = 0; e < 16; ++e) bias[e] = of.bias2_rows(row0 + acc_row(e, 0), lane_off);
     };
-    if (kBias) load_bias(q0);
-    // S and dP of a 32-row block (cc: block of the 128 rows).  kAhead: a block's products are issued while the block before
-    // goes through its element-wise work, which needs neither: the matrix pipe and the vector unit then work at the same
-    // time (one wave per SIMD: nothing else overlaps them; symmetric ALiBi closure, B=8, H=4, S=2048, forward and backward:
-    // 383.5 -> 378.8 us, two builds in turn).  With the code of a bias there are no registers for it.
-    constexpr bool kAhead = kNoBias;
-    auto products = [&](int cc, f32x16& s, f32x16& dp) {
-      const char* qt = reinterpret_cast<const char*>(sQ + (2 * buf + (cc >> 1)) * kTileElems) + (cc & 1) * 32 * kTileD * 2;
-      const char* dot = reinterpret_cast<const char*>(sDO + (2 * buf + (cc >> 1)) * kTileElems) + (cc & 1) * 32 * kTileD * 2;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        s[e] = 0.f;
-        dp[e] = 0.f;
-      }
-      bf16x8 qf[8], df[8];
-#pragma unroll
-      for (int ks = 0; ks < 8; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(qt + r_off[ks]);
-#pragma unroll
-      for (int ks = 0; ks < 8; ++ks) s = mfma32(qf[ks], kreg[ks], s);
-#pragma unroll
-      for (int ks = 0; ks < 8; ++ks) df[ks] = *reinterpret_cast<const bf16x8*>(dot + r_off[ks]);
-#pragma unroll
-      for (int ks = 0; ks < 8; ++ks) dp = mfma32(df[ks], vreg[ks], dp);
-    };
-    f32x16 s_acc, dp_acc, s_next, dp_next;
-    if (kAhead) products(0, s_acc, dp_acc);
-#pragma unroll
-    for (int cc = 0; cc < 4; ++cc) {
-      const int c = cc & 1;  // 32-row block inside the 64-row LDS tile cc >> 1
-      const char* qt = reinterpret_cast<const char*>(sQ + (2 * buf + (cc >> 1)) * kTileElems);
-      const char* dot = reinterpret_cast<const char*>(sDO + (2 * buf + (cc >> 1)) * kTileElems);
-      float bias[16];
-      if (kBias) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) bias[e] = bias_next[e];
-        if (cc < 3) load_bias(q0 + 32 * (cc + 1));
-      }
-      if (!kAhead) products(cc, s_acc, dp_acc);
-      // transposed fragments of this 32-row q block for the dv / dk products
-      s16x4 dolo[2][4], dohi[2][4], qlo[2][4], qhi[2][4];
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int db = 0; db < 4; ++db) {
-          const int off = (32 * c + 16 * u) * kTileD * 2;
-          dolo[u][db] = lds_read_tr16(reinterpret_cast<const bf16_t*>(dot + t_off[db][0] + off));
-          dohi[u][db] = lds_read_tr16(reinterpret_cast<const bf16_t*>(dot + t_off[db][1] + off));
-          qlo[u][db] = lds_read_tr16(reinterpret_cast<const bf16_t*>(qt + t_off[db][0] + off));
-          qhi[u][db] = lds_read_tr16(reinterpret_cast<const bf16_t*>(qt + t_off[db][1] + off));
-        }
-
-      bf16x8 pb[2], dsb[2];
-      // (DAB: the bias gradient, float32 [B, Hq, Sq, Sk], a row's 32 columns per store.  The block's 32 rows are a buffer of
-      // their own: a store at an offset beyond it is dropped, which is how an element that another work-group owns is
-      // left out; a branch around each of the 64 stores instead cuts the block into as many pieces for the scheduler:
-      // forward and backward of B=4, H=16, S=1500 1052 us, 1002 this way.)
-      __amdgpu_buffer_rsrc_t dab_block;
-      if (DAB)
-        dab_block = __builtin_amdgcn_make_buffer_rsrc(
-            a.dab + ((size_t)(b * a.Hq + hk * group + it / n_tiles) * a.Sq + (size_t)(q0 + 32 * cc)) * a.Sk, 0, 32 * a.Sk * 4, 0x00020000);
-      auto elementwise = [&](auto masked) {
-        constexpr bool MASKED = decltype(masked)::value;
-        if (kAhead && cc < 3) products(cc + 1, s_next, dp_next);
-        const bool has_doc = MASKED && (mk.flags & FLEXATTN_MASK_DOC) != 0;
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          const int r0 = 32 * cc + 8 * g4 + 4 * hh;  // the lane's q rows come in runs of 4
-          const f32x4 lse4 = *reinterpret_cast<const f32x4*>(sLse + buf * BQ + r0);
-          const f32x4 dl4 = *reinterpret_cast<const f32x4*>(sDl + buf * BQ + r0);
-          int di[4] = {0, 0, 0, 0};
-          if (MASKED && has_doc) {
-            const auto d4 = *reinterpret_cast<const i32x4_a4*>(mk.doc_q + q0 + r0);
-            di[0] = d4[0]; di[1] = d4[1]; di[2] = d4[2]; di[3] = d4[3];
-          }
-          float pv[4], dsv[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int e = 4 * g4 + u;
-            const int i = q0 + r0 + u;
-            const float tv = sm.to_log2(s_acc[e], i, k_idx);
-            float pe = fast_exp2(tv + (kBias ? bias[e] : kNoBias ? 0.f : sm.bias2(i, k_idx)) - lse4[u]);
-            float gl = pe * (dp_acc[e] - dl4[u]);   // the gradient of the logit itself: what an additive bias receives
-            float gd = gl * sm.dfactor(tv, s_acc[e], i, k_idx);
-            unsigned dab_off = 4u * lane_off;
-            if (MASKED) {
-              const bool owned = 32 * cc + 8 * g4 + u >= own;
-              const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j) & owned;
-              if (DAB) gl = keep ? gl : 0.f;
-              pe = keep ? pe : 0.f;
-              gd = keep ? gd : 0.f;
-              // (rows and columns of the tiles before: the work-groups of those store them)
-              dab_off = owned ? dab_off : ~0u;
-            }
-            if (DAB) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, gl), dab_block, (int)dab_off, (8 * g4 + u) * a.Sk * 4, 0);
-            pv[u] = pe;
-            dsv[u] = gd;
-          }
-          const bf16x2 p01 = pack_bf16(pv[0], pv[1]), p23 = pack_bf16(pv[2], pv[3]);
-          const bf16x2 d01 = pack_bf16(dsv[0], dsv[1]), d23 = pack_bf16(dsv[2], dsv[3]);
-          const int o = 4 * (g4 & 1);
-          pb[g4 >> 1][o] = p01[0]; pb[g4 >> 1][o + 1] = p01[1]; pb[g4 >> 1][o + 2] = p23[0]; pb[g4 >> 1][o + 3] = p23[1];
-          dsb[g4 >> 1][o] = d01[0]; dsb[g4 >> 1][o + 1] = d01[1]; dsb[g4 >> 1][o + 2] = d23[0]; dsb[g4 >> 1][o + 3] = d23[1];
-        }
-        if (kAhead && cc < 3) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one of the next block's MFMAs,
-            __builtin_amdgcn_sched_group_barrier(0x002, 10, 0);  // ten vector instructions of this one
-          }
-        }
-      };
-      if (partial) {
-        elementwise(std::true_type{});
-      } else {
-        elementwise(std::false_type{});
-      }
-      if constexpr (EXPORT) {
-        // block of (query head, kept tile pair): head a.ds_pairs + a.ds_col[kv tile] + place of the q tile in the kv
-        // tile's list; inside it wave w writes 1 KB per (32-row q block cc, 16-row half u), lane L its 8 values
-        char* blk = static_cast<char*>(a.ds) +
-                    ((size_t)(b * a.Hq + hk * group + it / n_tiles) * (size_t)a.ds_pairs + (size_t)a.ds_col[kb] +
-                     (size_t)(it % n_tiles)) * kDsBlockBytes + 8192 * w + 16 * (2 * l32 + hh);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) *reinterpret_cast<bf16x8*>(blk + 1024 * (2 * cc + u)) = dsb[u];
-      }
-
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-#pragma unroll
-        for (int db = 0; db < 4; ++db) {
-          dv_acc[db] = mfma32(join_tr(dolo[u][db], dohi[u][db]), pb[u], dv_acc[db]);
-          dk_acc[db] = mfma32(join_tr(qlo[u][db], qhi[u][db]), dsb[u], dk_acc[db]);
-        }
-      }
-      if (kAhead) {
-        s_acc = s_next;
-        dp_acc = dp_next;
-      }
+    if (kBias) {
+      if (it == 0) load_bias(sm, q0 + 32 * cc);
+      wait_vmem<kOpenStores>();
+    }
+    const bool more = it + 1 < n_iter;
+    if (more) {
+      if (buf == 1) advance();
+      issue_rows(buf ^ 1, buf ^ 1);
     }
 
-    qb_cur = qb_nxt; qb_nxt = qb_n2;
-    st_cur = st_nxt;
-    if (it + 1 < n_iter) store_rows(buf ^ 1);
-    wait_vmem_all();
+    const char* qt = reinterpret_cast<const char*>(sQ + 2 * buf * kTileElems) + wq * 32 * kTileD * 2;
+    const char* dot = qt + kTileElems * 2;
+    f32x16 s_acc, dp_acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      s_acc[e] = 0.f;
+      dp_acc[e] = 0.f;
+    }
+    // (operands are read four products ahead: left to itself the compiler reads each pair in front of its product and waits
+    // out the LDS latency 16 times)
+    bf16x8 fa[2][4], fb[2][4];
+    auto read_rows = [&](int stage) {   // stages 0, 1: Q and K, 2, 3: dO and V
+      const char* ra = stage < 2 ? qt : dot;
+      const char* rb = stage < 2 ? kt : vt;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        fa[stage & 1][i] = *reinterpret_cast<const bf16x8*>(ra + r_off[4 * (stage & 1) + i]);
+        fb[stage & 1][i] = *reinterpret_cast<const bf16x8*>(rb + r_off[4 * (stage & 1) + i]);
+      }
+    };
+    read_rows(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int stage = 0; stage < 4; ++stage) {
+      if (stage < 3) read_rows(stage + 1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (stage < 2) s_acc = mfma32(fa[stage & 1][i], fb[stage & 1][i], s_acc);
+        else dp_acc = mfma32(fa[stage & 1][i], fb[stage & 1][i], dp_acc);
+      }
+      if (stage < 3) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // an MFMA,
+          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);   // two LDS reads
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+
+    bf16x8 pb[2], dsb[2];
+    // (DAB: the bias gradient, float32 [B, Hq, Sq, Sk], a row's 32 columns per store.  The block's 32 rows are a buffer of
+    // their own: a store at an offset beyond it is dropped, which is how an element that another work-group owns is
+    // left out; a branch around each of the 16 stores instead cuts the block into as many pieces for the scheduler.)
+    __amdgpu_buffer_rsrc_t dab_block;
+    if (DAB)
+      dab_block = __builtin_amdgcn_make_buffer_rsrc(
+          a.dab + ((size_t)(b * a.Hq + hk * group + g) * a.Sq + (size_t)(q0 + 32 * cc)) * a.Sk, 0, 32 * a.Sk * 4, 0x00020000);
+    auto elementwise = [&](auto masked) {
+      constexpr bool MASKED = decltype(masked)::value;
+      const bool has_doc = MASKED && (mk.flags & FLEXATTN_MASK_DOC) != 0;
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const int r0 = 32 * cc + 8 * g4 + 4 * hh;  // the lane's q rows come in runs of 4
+        const f32x4 lse4 = *reinterpret_cast<const f32x4*>(sLse + r0);
+        const f32x4 dl4 = *reinterpret_cast<const f32x4*>(sDl + r0);
+        int di[4] = {0, 0, 0, 0};
+        if (MASKED && has_doc) {
+          const auto d4 = *reinterpret_cast<const i32x4_a4*>(mk.doc_q + q0 + r0);
+          di[0] = d4[0]; di[1] = d4[1]; di[2] = d4[2]; di[3] = d4[3];
+        }
+        float pv[4], dsv[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int e = 4 * g4 + u;
+          const int i = q0 + r0 + u;
+          const float tv = sm.to_log2(s_acc[e], i, k_idx);
+          float pe = fast_exp2(tv + (kBias ? bias[e] : kNoBias ? 0.f : sm.bias2(i, k_idx)) - lse4[u]);
+          float gl = pe * (dp_acc[e] - dl4[u]);   // the gradient of the logit itself: what an additive bias receives
+          float gd = gl * sm.dfactor(tv, s_acc[e], i, k_idx);
+          unsigned dab_off = 4u * lane_off;
+          if (MASKED) {
+            const bool owned = 32 * cc + 8 * g4 + u >= own;
+            const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j) & owned;
+            if (DAB) gl = keep ? gl : 0.f;
+            pe = keep ? pe : 0.f;
+            gd = keep ? gd : 0.f;
+            // (rows and columns of the tiles before: the work-groups of those store them)
+            dab_off = owned ? dab_off : ~0u;
+          }
+          if (DAB) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, gl), dab_block, (int)dab_off, (8 * g4 + u) * a.Sk * 4, 0);
+          pv[u] = pe;
+          dsv[u] = gd;
+        }
+        const bf16x2 p01 = pack_bf16(pv[0], pv[1]), p23 = pack_bf16(pv[2], pv[3]);
+        const bf16x2 d01 = pack_bf16(dsv[0], dsv[1]), d23 = pack_bf16(dsv[2], dsv[3]);
+        const int o = 4 * (g4 & 1);
+        pb[g4 >> 1][o] = p01[0]; pb[g4 >> 1][o + 1] = p01[1]; pb[g4 >> 1][o + 2] = p23[0]; pb[g4 >> 1][o + 3] = p23[1];
+        dsb[g4 >> 1][o] = d01[0]; dsb[g4 >> 1][o + 1] = d01[1]; dsb[g4 >> 1][o + 2] = d23[0]; dsb[g4 >> 1][o + 3] = d23[1];
+      }
+    };
+    if (partial) {
+      elementwise(std::true_type{});
+    } else {
+      elementwise(std::false_type{});
+    }
+    if (kBias && more) {
+      ScoreMod<SCORE> of;   // (the next block's head, which an entry's second half shares)
+      of.init(a.score, a.sm_scale, hk * group + g_at, b);
+      load_bias(of, tile_base(qb_at, BQ, a.Sq) + 64 * (buf ^ 1) + 32 * wq);
+    }
+    if constexpr (EXPORT) {
+      // block of (query head, kept tile pair): head a.ds_pairs + a.ds_col[kv tile] + place of the q tile in the kv
+      // tile's list; inside it kv block wk's 1 KB per (32-row q block cc, 16-row half u), lane L its 8 values
+      char* blk = static_cast<char*>(a.ds) +
+                  ((size_t)(b * a.Hq + hk * group + g) * (size_t)a.ds_pairs + (size_t)a.ds_col[kb] + (size_t)t) * kDsBlockBytes +
+                  8192 * wk + 16 * (2 * l32 + hh);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) *reinterpret_cast<bf16x8*>(blk + 1024 * (2 * cc + u)) = dsb[u];
+    }
+
+    // transposed fragments of the block's rows, dv^T += dO^T P, dk^T += Q^T dS
+    s16x4 tr[2][4][4];   // [16-row half][column block][dO low, dO high, Q low, Q high]
+    auto read_tr = [&](int u) {
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          tr[u][db][i] = lds_read_tr16(reinterpret_cast<const bf16_t*>((i < 2 ? dot : qt) + t_off[db][i & 1] + 16 * u * kTileD * 2));
+    };
+    read_tr(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (u == 0) read_tr(1);
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+        dv_acc[db] = mfma32(join_tr(tr[u][db][0], tr[u][db][1]), pb[u], dv_acc[db]);
+        dk_acc[db] = mfma32(join_tr(tr[u][db][2], tr[u][db][3]), dsb[u], dk_acc[db]);
+      }
+      if (u == 0) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+
+    if (more) store_rows(buf ^ 1);
+    // (the copies are there; what was issued behind them, the next bias values and the stores of dS, may stay open)
+    wait_vmem<kOpenStores + (kBias ? 16 : 0)>();
     __syncthreads();
   }
+  wait_vmem_all();
 
-  if (!own_col) return;
-  bf16_t* dKg = static_cast<bf16_t*>(a.dk) + kv_off;
-  bf16_t* dVg = static_cast<bf16_t*>(a.dv) + kv_off;
+  // the two waves of a kv block add up: one finishes dk, the other dv
+  {
+    float* ex = reinterpret_cast<float*>(smem_raw) + (size_t)w * 64 * 64;   // 16 KB per wave
+    auto put = [&](const f32x16 (&x)[4]) {
 #pragma unroll
-  for (int db = 0; db < 4; ++db) {
+      for (int db = 0; db < 4; ++db)
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      bf16x2 lo = pack_bf16(dk_acc[db][4 * g], dk_acc[db][4 * g + 1]);
-      bf16x2 hi = pack_bf16(dk_acc[db][4 * g + 2], dk_acc[db][4 * g + 3]);
-      bf16x4 out = {lo[0], lo[1], hi[0], hi[1]};
-      *reinterpret_cast<bf16x4*>(dKg + (size_t)kv_local * D + 32 * db + 8 * g + 4 * hh) = out;
-      lo = pack_bf16(dv_acc[db][4 * g], dv_acc[db][4 * g + 1]);
-      hi = pack_bf16(dv_acc[db][4 * g + 2], dv_acc[db][4 * g + 3]);
-      bf16x4 out2 = {lo[0], lo[1], hi[0], hi[1]};
-      *reinterpret_cast<bf16x4*>(dVg + (size_t)kv_local * D + 32 * db + 8 * g + 4 * hh) = out2;
-    }
+        for (int g4 = 0; g4 < 4; ++g4)
+          *reinterpret_cast<f32x4*>(ex + ((4 * db + g4) * 64 + lane) * 4) =
+              f32x4{x[db][4 * g4], x[db][4 * g4 + 1], x[db][4 * g4 + 2], x[db][4 * g4 + 3]};
+    };
+    if (wq == 0) put(dv_acc); else put(dk_acc);
+    __syncthreads();
+    const float* other = reinterpret_cast<const float*>(smem_raw) + (size_t)(w ^ 4) * 64 * 64;
+    auto finish = [&](const f32x16 (&x)[4], bf16_t* out) {
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const f32x4 y = *reinterpret_cast<const f32x4*>(other + ((4 * db + g4) * 64 + lane) * 4);
+          const bf16x2 lo = pack_bf16(x[db][4 * g4] + y[0], x[db][4 * g4 + 1] + y[1]);
+          const bf16x2 hi = pack_bf16(x[db][4 * g4 + 2] + y[2], x[db][4 * g4 + 3] + y[3]);
+          const bf16x4 o = {lo[0], lo[1], hi[0], hi[1]};
+          if (own_col) *reinterpret_cast<bf16x4*>(out + (size_t)kv_local * D + 32 * db + 8 * g4 + 4 * hh) = o;
+        }
+    };
+    if (wq == 0) finish(dk_acc, static_cast<bf16_t*>(a.dk) + kv_off); else finish(dv_acc, static_cast<bf16_t*>(a.dv) + kv_off);
   }
 }
 
@@ -1190,10 +1225,10 @@ static int launch_dkv_on(const BwdArgs& a, hipStream_t stream) {
   using namespace dkv_cfg;
   auto kern = bwd_dkv_bf16_d128_kernel<SCORE, EXPORT, AB, DAB>;
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, LOOP_LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dkv): %s", hipGetErrorString(attr));
   const int n_wg = a.B * a.Hkv * a.map.nk;
-  hipLaunchKernelGGL(kern, dim3(n_wg), dim3(256), LDS_BYTES, stream, a);
+  hipLaunchKernelGGL(kern, dim3(n_wg), dim3(512), LOOP_LDS_BYTES, stream, a);
   return check_launch("flexattn_bwd_dkv bf16");
 }
 template <int SCORE>

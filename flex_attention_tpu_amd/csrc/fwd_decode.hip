@@ -52,10 +52,6 @@ __device__ __forceinline__ void decode_copy(const char* g, unsigned dst, const u
                  : "memory", "m0", "vcc");
   }
 }
-template <int N>
-__device__ __forceinline__ void wait_vmem() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 
 // NR: blocks of 32 query rows (1 or 2).
 template <int D, int NR>

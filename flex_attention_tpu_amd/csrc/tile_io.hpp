@@ -77,5 +77,14 @@ struct TileLoader {
 // Waits until every outstanding vector-memory operation of this wave (including LDS-direct loads)
 // has completed.
 __device__ __forceinline__ void wait_vmem_all() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+// The same for all but this wave's N latest operations (they complete in the order they were issued).  The fences keep the
+// compiler from moving a load or store over the wait; the builtin, not asm, tells it what it need not wait for again.
+template <int N>
+__device__ __forceinline__ void wait_vmem() {
+  static_assert(N >= 0 && N < 64, "six bits");
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+  asm volatile("" ::: "memory");
+}
 
 }  // namespace fa
