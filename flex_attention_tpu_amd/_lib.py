@@ -156,6 +156,8 @@ EXPORTS = (
     "flexattn_bwd_ds_bytes",
     "flexattn_bwd_dq",
     "flexattn_bwd_dkv",
+    "flexattn_bwd_dab_pays",
+    "flexattn_bwd_dab",
     "flexattn_bwd",
     "flexattn_custom_tag",
 )
@@ -185,9 +187,11 @@ def _bind(lib: C.CDLL) -> C.CDLL:
     lib.flexattn_bwd_ds_bytes.restype = C.c_int64
     lib.flexattn_bwd_dkv.argtypes = [C.POINTER(BwdParamsC), C.c_void_p]
     lib.flexattn_bwd.argtypes = [C.POINTER(BwdParamsC), C.POINTER(BwdParamsC), C.c_void_p]
+    lib.flexattn_bwd_dab_pays.argtypes = [C.POINTER(BwdParamsC)]
+    lib.flexattn_bwd_dab.argtypes = [C.POINTER(BwdParamsC), C.c_void_p]
     lib.flexattn_takes_head_dim_64.argtypes = [C.c_int32, C.c_float, C.c_int32, C.c_int32]
     for name in ("flexattn_takes_head_dim_64", "flexattn_tile_shape", "flexattn_build_block_mask", "flexattn_build_block_mask_ragged", "flexattn_build_ds_index", "flexattn_fwd",
-                 "flexattn_fwd_noalloc", "flexattn_fwd_decode", "flexattn_bwd_delta", "flexattn_bwd_dq", "flexattn_bwd_dkv", "flexattn_bwd"):
+                 "flexattn_fwd_noalloc", "flexattn_fwd_decode", "flexattn_bwd_delta", "flexattn_bwd_dq", "flexattn_bwd_dkv", "flexattn_bwd_dab_pays", "flexattn_bwd_dab", "flexattn_bwd"):
         getattr(lib, name).restype = C.c_int
     return lib
 

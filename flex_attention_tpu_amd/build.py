@@ -23,6 +23,7 @@ SOURCES = [
     "bwd_dq_bf16.hip",
     "bwd_dkv_bf16.hip",
     "bwd_dq_ds.hip",
+    "bwd_dab_bf16.hip",
 ]
 
 # instruction streams generated before compiling: (generator script, output it writes next to itself)

@@ -571,4 +571,33 @@ int flexattn_bwd_dkv(const flexattn_bwd_params* p, void* stream) {
   return launch_dkv(p, a, s);
 }
 
+// The arguments of a bias gradient summed over the pairs that share it, from the dk/dv pass's parameter block.
+static int to_dab_args(const flexattn_bwd_params* p, BwdArgs* a) {
+  if (p == nullptr) return set_error(FLEXATTN_EINVAL, "params is NULL");
+  flexattn_bwd_params own = *p;
+  own.ds = nullptr;    // (neither read nor written; the dk/dv pass's check of dab is of its full-size gradient)
+  own.dab = nullptr;
+  if (own.ab.ptr == nullptr) return set_error(FLEXATTN_EINVAL, "flexattn_bwd_dab: no additive bias");
+  if (own.o != nullptr) return set_error(FLEXATTN_EINVAL, "flexattn_bwd_dab takes delta, not o");
+  const int rc = to_bwd_args(&own, FLEXATTN_PASS_DKV, a);
+  if (rc != FLEXATTN_OK) return rc;
+  a->dab = p->dab;
+  return FLEXATTN_OK;
+}
+
+int flexattn_bwd_dab_pays(const flexattn_bwd_params* p) {
+  BwdArgs a;
+  return to_dab_args(p, &a) == FLEXATTN_OK && p->dtype == FLEXATTN_BF16 && p->D == 128 && bwd_dab_bf16_pays(a);
+}
+
+int flexattn_bwd_dab(const flexattn_bwd_params* p, void* stream) {
+  BwdArgs a;
+  const int rc = to_dab_args(p, &a);
+  if (rc != FLEXATTN_OK) return rc;
+  if (a.dab == nullptr) return set_error(FLEXATTN_EINVAL, "flexattn_bwd_dab: dab is NULL");
+  if (p->dtype != FLEXATTN_BF16 || p->D != 128 || p->score.kind != FLEXATTN_SCORE_NONE)
+    return set_error(FLEXATTN_ENOTSUP, "flexattn_bwd_dab: bf16, head dim 128, no score function");
+  return bwd_dab_bf16(a, static_cast<hipStream_t>(stream));
+}
+
 }  // extern "C"

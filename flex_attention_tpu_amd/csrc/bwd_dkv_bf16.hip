@@ -104,8 +104,8 @@ __global__ __launch_bounds__(512, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
   const int nQ = a.map.nq;
   const int n_wg = a.B * a.Hkv * nKb;
   const int wg = xcd_remap(blockIdx.x, n_wg);
-  const int bhk = wg / nKb;
-  const int kb = wg % nKb;  // low kv tiles have the most q tiles under causal masks: they go first
+  int bhk, kb;  // (low kv tiles have the most q tiles under causal masks: they go first)
+  block_item(wg, a.B, a.Hkv, nKb, kBias && a.score.ab_sb_rows == 0, bhk, kb);
   const int b = bhk / a.Hkv;
   const MaskArgs mk = mask_of_batch(a.mask, b, a.Sq, a.Sk);
   const int hk = bhk % a.Hkv;

@@ -577,6 +577,20 @@ __device__ __forceinline__ int xcd_remap(int wg, int n_wg) {
   return (wg % kXcd) * (n_wg / kXcd) + wg / kXcd;
 }
 
+// (batch, head) pair and block of a work-group of the compiled-loop kernels.  A bias that the batch shares: the batch entries of
+// one (head, block) stand next to each other, so that they walk the same part of the bias at the same time and all but the first
+// find it in the XCD's L2 (B=4, H=16, S=1500, forward and backward: 801 -> 769 us).
+__device__ __forceinline__ void block_item(int wg, int B, int H, int n_blocks, bool batch_shares, int& bh, int& block) {
+  if (batch_shares) {
+    const int r = wg / B, h = r / n_blocks;
+    bh = (wg - r * B) * H + h;
+    block = r - h * n_blocks;
+  } else {
+    bh = wg / n_blocks;
+    block = wg - bh * n_blocks;
+  }
+}
+
 // Static schedule of a generated-stream kernel when it runs one work-group per CU (256 CUs = 8 XCDs x
 // 32, consecutive work-group ids go round-robin to the XCDs).  Every XCD takes a contiguous share
 // of the (batch, kv head) pairs; its 32 work-groups walk through the share's heads together, so

@@ -78,8 +78,9 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
   const int nK = a.map.nk;
   const int n_wg = a.B * a.Hq * nQ;
   const int wg = xcd_remap(blockIdx.x, n_wg);
-  const int bh = wg / nQ;
-  const int qb = nQ - 1 - (wg % nQ);  // longest rows first under causal masks
+  int bh, qb;
+  block_item(wg, a.B, a.Hq, nQ, SCORE == kScoreBiasOnly && a.score.ab_sb_rows == 0, bh, qb);
+  qb = nQ - 1 - qb;  // longest rows first under causal masks
   const int b = bh / a.Hq;
   const MaskArgs mk = mask_of_batch(a.mask, b, a.Sq, a.Sk);
   const int h = bh % a.Hq;

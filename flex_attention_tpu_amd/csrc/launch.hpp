@@ -34,6 +34,10 @@ int bwd_dkv_bf16_d256(const BwdArgs& a, hipStream_t stream);
 // factor 4; the kernel with a compiled main loop exports dS complete)
 bool bwd_dkv_bf16_d128_on_stream(int kind, int flags, int nq, bool has_ab, int Hq, int Hkv);
 void bwd_dkv_bf16_d128_tile(int* bq, int* bk);
+// the gradient of a bias that several (batch, head) pairs share, in the bias's own shape; whether it is expected to beat the
+// full-size gradient of the dk/dv pass and a sum over it
+bool bwd_dab_bf16_pays(const BwdArgs& a);
+int bwd_dab_bf16(const BwdArgs& a, hipStream_t stream);
 // dq = out_scale dS K from the dS blocks that the dk/dv stream kernels wrote to a.ds (a.map: row lists at the
 // dk/dv tiles)
 int bwd_dq_from_ds(const BwdArgs& a, int D, float out_scale, hipStream_t stream);

@@ -57,7 +57,7 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
         if Sk_p != Sk or Sq_p != Sq or D != D_user or return_ds:
             return None
         return {"params": p, "lib": lib, "finish": lambda: (dk, dv), "keep": (q, k, v, do, l, m, di, ab_keep, bm)}
-    dab = None
+    dab, shared = None, False
     with on_device(q.device):
         if return_ds:
             if _wide_ds and D == 256:   # (flex_attention's own backward: head dimension 256 hands dS over too)
@@ -65,20 +65,26 @@ def flash_attention_bwd_dkv(k, v, q, ab, segment_ids, l, m, di, do, *, block_b=N
             p.ds_index.pairs = 1   # (asks whether the kernels of the call exchange at all, before the index is built)
             if lib.flexattn_bwd_ds_bytes(C.byref(p)) > 0 and bm.ds_index_at_hand():
                 if _dab and D == 128:   # (flex_attention's own backward: the bias gradient next to the dS it comes from.  It is
-                    # needed with and without the hand-over, dS only with it: dS is what gives way where both do not fit)
-                    dab = alloc_dab(spec, B, Hq, Sq_p, Sk_p, q.device)
+                    # needed with and without the hand-over, dS only with it: dS is what gives way where both do not fit.
+                    # A bias that several pairs share gets its sum from a pass of its own where that pays: B=4, H=16, S=1500
+                    # with one bias for the batch writes 144 MB that way instead of writing 576 MB and reading them back.)
+                    shared = bool(lib.flexattn_bwd_dab_pays(C.byref(p)))
+                    dab = alloc_dab(spec, *(ab.shape[:2] if shared else (B, Hq)), Sq_p, Sk_p, q.device)
                 p.ds_index = bm.ds_index_c()
                 need = lib.flexattn_bwd_ds_bytes(C.byref(p))
                 buf = alloc_ds(need, q.device)
                 if buf is not None:
                     ds = DsBlocks(buf, (B, Hq, Sq_p, Sk_p), index=bm.ds_index(), compiled_loop=bool(compiled_loop))
                     p.ds, p.ds_bytes = buf.data_ptr(), need
-                    if dab is not None:
+                    if dab is not None and not shared:
                         p.dab = dab.data_ptr()
             if ds is None:
                 p.ds_index = _lib.DsIndexC()
                 dab = None
         _lib.check(lib.flexattn_bwd_dkv(C.byref(p), stream_of(q)), lib)
+        if dab is not None and shared:
+            p.dab = dab.data_ptr()
+            _lib.check(lib.flexattn_bwd_dab(C.byref(p), stream_of(q)), lib)
     if Sk_p != Sk or D != D_user:
         dk, dv = dk[:, :, :Sk, :D_user].contiguous(), dv[:, :, :Sk, :D_user].contiguous()
     if _dab:

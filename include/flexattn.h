@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define FLEXATTN_VERSION 104 /* major*10000 + minor*100 + patch */
+#define FLEXATTN_VERSION 105 /* major*10000 + minor*100 + patch */
 
 /* status codes */
 #define FLEXATTN_OK 0
@@ -292,6 +292,16 @@ int flexattn_bwd_dq(const flexattn_bwd_params* p, void* stream);
 /* dk/dv backward.  Replaces the pallas_call in flash_attention_bwd_dkv
  * (flex_attention_dkv_kernel.py:158-172; mask-aware twin flash_attention_dkv_bwd.py:164-178). */
 int flexattn_bwd_dkv(const flexattn_bwd_params* p, void* stream);
+
+/* Gradient of an additive bias that several (batch, head) pairs share (a stride of p->ab is 0), in the bias's own shape:
+ * p->dab is float32 with the strides of p->ab, every element the sum over its pairs.  p is the parameter block of the
+ * dk/dv pass (delta given, not o; dk, dv are not written, ds is not looked at).  bf16, head dimension 128, no score
+ * function.  Only the tiles the block map visits are written: clear the buffer first.  The full-size gradient that
+ * flexattn_bwd_dq and flexattn_bwd_dkv return costs B Hq Sq Sk floats of memory written, and read again by the caller's
+ * sum; flexattn_bwd_dab_pays says 1 for requests where this call is expected to be the faster way (it looks at shapes,
+ * score and the bias's strides), 0 for others and those it does not take. */
+int flexattn_bwd_dab_pays(const flexattn_bwd_params* p);
+int flexattn_bwd_dab(const flexattn_bwd_params* p, void* stream);
 
 /* The whole backward from one call: delta (when the dq block names `o` and `delta_out`), the dq pass of `dq` and the
  * dk/dv pass of `dkv` (the two blocks describe the same problem, each with the block map of its pass; no dS hand-over),
