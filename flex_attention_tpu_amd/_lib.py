@@ -209,6 +209,25 @@ def load() -> C.CDLL:
     return _lib
 
 
+_host = None
+
+
+def load_host():
+    """The C++ side of the prepared calls (csrc/host_path.cpp), bound to libflexattn.so; raises ImportError if it has not
+    been built."""
+    global _host
+    if _host is None:
+        if not os.path.exists(os.path.join(_PKG_DIR, "_host.so")):
+            raise ImportError(f"{_PKG_DIR}/_host.so is missing: build it with `python -m flex_attention_tpu_amd.build`")
+        import torch  # noqa: F401  (its libraries come first)
+        from . import _host as mod
+        lib = load()
+        mod.bind(*(C.cast(getattr(lib, "flexattn_" + n), C.c_void_p).value
+                   for n in ("fwd", "bwd", "bwd_dq", "bwd_dkv", "bwd_delta", "last_error_string")))
+        _host = mod
+    return _host
+
+
 def load_for(score_code=None, mask_code=None) -> C.CDLL:
     """The library whose kernels contain the given compiled closures (compiler.CustomCode objects, or None):
     libflexattn.so when there is none, else the functor library of the pair, compiled with hipcc at first

@@ -3,9 +3,9 @@ dimension that needs no padding): what their parameter blocks hold besides point
 alone and is assembled once per combination.
 
 Small problems are bound by the host's path to a launch: forward and backward of B=1, H=4, S=512, D=64 in float32 keep
-the GPU busy for 83 us and took the host 221 us, 154 us this way (the autograd thread runs Python from cold caches, at
-about half the speed; bf16, B=1, H=8, S=1024: 223 -> 153 us).  A prepared call checks its tensors as every other call does, takes the
-template, writes its pointers into a copy of its own and launches: nothing of a call's tensors is kept.
+the GPU busy for 83 us and took the host 221 us, 154 us this way.  A prepared call checks its tensors as every other call does, takes the
+template, writes its pointers into a copy of its own and launches: nothing of a call's tensors is kept.  `attend` is the same
+with the autograd function, the allocations and the launches in C++ (csrc/host_path.cpp): 81 us, the kernels' own time.
 """
 from __future__ import annotations
 
@@ -58,6 +58,44 @@ def _plan(key, q, k, spec, sm_scale, cls, passes):
     for bm in maps:   # (a map built on another stream: this one waits for it)
         bm.wait_ready(q.device)
     return plan.templates, maps
+
+
+_attend_plans = LRU(64)   # (shapes, dtype, device, mask, scale, blocks) -> (C++ plan, weak references to its block maps), or False
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def ordinary(q, k, v) -> bool:
+    """Whether a call is one that the C++ autograd function serves exactly as the Python one does: plain contiguous tensors
+    outside function transforms, forward-mode differentiation, tracing and compilation, and modes that watch Python's calls."""
+    return (not torch.compiler.is_compiling() and type(q) in _PLAIN and type(k) in _PLAIN and type(v) in _PLAIN and q.is_contiguous() and k.is_contiguous() and v.is_contiguous()
+            and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and torch._C._get_tracing_state() is None)
+
+
+def attend(q, k, v, spec: MaskSpec, sm_scale, block_q, block_k, prepared):
+    """o of a differentiable call without score function, bias and segment ids on `ordinary` tensors, or None where the call is not
+    a prepared one.  ``prepared(q, k, v, spec)``: whether its shapes, mask and scale are (asked once per combination; it
+    raises for what the entry points refuse)."""
+    if q.dtype != k.dtype or q.dtype != v.dtype or k.shape != v.shape or q.device != k.device or q.device != v.device:
+        return None   # (the general path says what is wrong)
+    key = (q.shape, k.shape, q.dtype, q.device, spec, sm_scale, block_q, block_k)
+    plan = _attend_plans.get(key)
+    if plan is False:
+        return None
+    maps = [ref() for ref in plan[1]] if plan is not None else (None,)
+    if None in maps:
+        if not prepared(q, k, v, spec):
+            _attend_plans.put(key, False)
+            return None
+        parts = [_template(cls, pass_id, q, k, spec, sm_scale) for cls, pass_id in
+                 ((_lib.FwdParamsC, _lib.PASS_FWD), (_lib.BwdParamsC, _lib.PASS_DQ), (_lib.BwdParamsC, _lib.PASS_DKV))]
+        maps = [bm for _, bm in parts]
+        plan = (_lib.load_host().Plan(*(t for t, _ in parts)), tuple(weakref.ref(bm) for bm in maps))
+        _attend_plans.put(key, plan)
+    for bm in maps:   # (a map built on another stream: this one waits for it; the backward runs on this one too)
+        bm.wait_ready(q.device)
+    return _lib.load_host().attend(q, k, v, plan[0], maps[0].host_map(), maps[1].host_map(), maps[2].host_map())
 
 
 def takes(q, k, spec: MaskSpec, sm_scale, *passes: int) -> bool:

@@ -83,6 +83,14 @@ class BlockMap:
         self.ready = None      # event recorded behind it
         self._ds_index = None  # (col, rank, pairs) of the dS exchange buffer, built at first use
         self._partial_share = None
+        self._host_map = None  # the C++ side's view of the arrays
+
+    def host_map(self):
+        """The map as the C++ path of the prepared calls takes it (holds the arrays, not this object)."""
+        if self._host_map is None:
+            self._host_map = _lib.load_host().Map(self.state, self.kv_cnt, self.kv_idx, self.q_cnt, self.q_idx, self.nq, self.nk,
+                                                  self.block_q, self.block_k)
+        return self._host_map
 
     def _tensors(self):
         t = [self.state, self.kv_cnt, self.kv_idx, self.q_cnt, self.q_idx]

@@ -11,6 +11,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 BUILD_DIR = os.path.join(CSRC, "_build")
 LIB_PATH = os.path.join(PKG_DIR, "libflexattn.so")
+HOST_PATH = os.path.join(PKG_DIR, "_host.so")
 
 SOURCES = [
     "api.hip",
@@ -98,5 +99,28 @@ def build_library(force: bool = True, jobs: int = 8, out_path: str = LIB_PATH, b
     return out_path
 
 
+def build_host(force: bool = True) -> str:
+    """Compiles the C++ side of the prepared calls (csrc/host_path.cpp) against the installed torch into the package."""
+    src = os.path.join(CSRC, "host_path.cpp")
+    if not force and os.path.exists(HOST_PATH) and all(
+            os.path.getmtime(d) <= os.path.getmtime(HOST_PATH) for d in (src, os.path.join(INCLUDE, "flexattn.h"))):
+        return HOST_PATH
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    tmp = f"{HOST_PATH}.{os.getpid()}.tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-DTORCH_EXTENSION_NAME=_host", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
+           *(f"-I{d}" for d in cpp_extension.include_paths("cuda")), f"-I{sysconfig.get_paths()['include']}", src, "-o", tmp,
+           *(f"-L{d}" for d in cpp_extension.library_paths("cuda")), "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed for host_path.cpp:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, HOST_PATH)
+    return HOST_PATH
+
+
 if __name__ == "__main__":
     print(build_library(force="--incremental" not in sys.argv))
+    print(build_host(force="--incremental" not in sys.argv))

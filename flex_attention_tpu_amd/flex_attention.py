@@ -178,5 +178,18 @@ def flex_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, score_fn: 
     else:
         mask_fn, block_mask_fn = mask_fns if mask_fns is not None else (None, None)
     score_fn, mask_fn, block_mask_fn = tagged_closures(score_fn, mask_fn, block_mask_fn, block_q, block_k)
+    if score_fn is None and ab is None and segment_ids is None and _plans.ordinary(q, k, v):
+        spec = spec_of(mask_fn, block_mask_fn)
+        if causal:
+            spec = spec.combine(_CAUSAL)
+
+        def prepared(q, k, v, spec):
+            B, Hq, Hkv, Sq, Sk, D = check_qkv(q, k, v)
+            check_blocks(Sq, Sk, block_q=block_q, block_k_major=block_k, block_k=block_k)
+            return (_plans.takes(q, k, spec, sm_scale, _lib.PASS_FWD, _lib.PASS_DQ, _lib.PASS_DKV) and
+                    not (q.dtype is torch.bfloat16 and _hands_ds_over(q, k, None, None, sm_scale, None, mask_fn, block_mask_fn, False)))
+        o = _plans.attend(q, k, v, spec, float(sm_scale), block_q, block_k, prepared)
+        if o is not None:
+            return o
     opts = (score_fn, mask_fn, block_mask_fn, segment_ids, bool(causal), float(sm_scale), int(block_q), int(block_k))
     return _FlexAttention.apply(q, k, v, ab, opts)

@@ -1,0 +1,168 @@
+"""The prepared calls' autograd function in C++ against the Python one that every other call takes: the same kernels on the same
+arguments, so the same bits, for each set of wanted gradients, under the hooks and modes that watch an autograd function, and
+where the call is handed to the Python one."""
+import math
+import threading
+
+import pytest
+import torch
+
+from oracle import mha_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def inputs(B=2, Hq=4, Hkv=2, Sq=300, Sk=300, D=128, dtype=torch.bfloat16, seed=0):
+    return [t.cuda() for t in O.make_inputs(B, Hq, Hkv, Sq, Sk, D, dtype=dtype, seed=seed)]
+
+
+def masks_of(causal):
+    from flex_attention_tpu_amd import masks
+    return masks.make_causal_mask_fns(128, 128) if causal else None
+
+
+def python_path(q, k, v, pair, sc, causal=False):
+    import sys
+    fa = sys.modules["flex_attention_tpu_amd.flex_attention"]
+    mf, bf = pair or (None, None)
+    return fa._FlexAttention.apply(q, k, v, None, (None, mf, bf, None, causal, sc, 128, 128))
+
+
+def taken(q, k, v, pair, sc, **kw):
+    """flex_attention's result, and whether the C++ function made it."""
+    import flex_attention_tpu_amd as F
+    o = F.flex_attention(q, k, v, None, pair, sm_scale=sc, **kw)
+    return o, o.grad_fn is not None and "_FlexAttentionBackward" not in type(o.grad_fn).__name__
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.bfloat16, 64), (torch.float32, 64), (torch.float32, 128)])
+@pytest.mark.parametrize("Sq,Sk,causal", [(128, 128, False), (300, 300, True), (257, 640, False)])
+@pytest.mark.parametrize("wanted", ["qkv", "q", "k", "v", "kv"])
+def test_same_bits_as_the_python_function(wanted, Sq, Sk, causal, dtype, D):
+    q, k, v, do = inputs(Sq=Sq, Sk=Sk, D=D, dtype=dtype)
+    sc, pair = 1 / math.sqrt(D), masks_of(causal)
+    leaves = [t for n, t in zip("qkv", (q, k, v)) if n in wanted]
+    for t in leaves:
+        t.requires_grad_(True)
+    o, native = taken(q, k, v, pair, sc)
+    assert native
+    want = python_path(q, k, v, pair, sc)
+    assert torch.equal(o, want)
+    for a, b in zip(torch.autograd.grad(o, leaves, do), torch.autograd.grad(want, leaves, do)):
+        assert torch.equal(a, b)
+    with torch.no_grad():
+        assert torch.equal(taken(q, k, v, pair, sc)[0], want)
+
+
+def test_views_hooks_and_repeated_backward():
+    sc, pair = 1 / math.sqrt(128), masks_of(True)
+    q, k, v, do = inputs()
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    want = torch.autograd.grad(python_path(q, k, v, pair, sc), (q, k, v), do)
+
+    def check(o, do=do, **kw):
+        got = torch.autograd.grad(o, (q, k, v), do, **kw)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    o, native = taken(q, k, v, pair, sc)
+    assert native
+    check(o, retain_graph=True)
+    check(o, do=do.transpose(1, 2).contiguous().transpose(1, 2))   # (a gradient of other strides; frees the graph)
+    with pytest.raises(RuntimeError, match="backward through the graph a second time"):
+        torch.autograd.grad(o, (q, k, v), do)
+    with torch.autograd.graph.save_on_cpu():
+        o, native = taken(q, k, v, pair, sc)
+    assert native
+    check(o)
+    o = torch.utils.checkpoint.checkpoint(lambda *a: taken(*a, pair, sc)[0], q, k, v, use_reentrant=False)
+    check(o)
+    # operands at an address that is no multiple of 16 bytes
+    off = [torch.cat([t.detach().new_zeros(1), t.detach().flatten()])[1:].view(t.shape).requires_grad_(True) for t in (q, k, v)]
+    o, native = taken(*off, pair, sc)
+    assert native and all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(o, off, do), want))
+    # an operand that changes before the backward
+    x = q.detach().clone().requires_grad_(True)
+    y = x * 1.0
+    o, _ = taken(y, k, v, pair, sc)
+    with torch.no_grad():
+        y.add_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(o, x, do)
+
+
+def test_calls_that_stay_with_the_python_function():
+    import flex_attention_tpu_amd as F
+    sc = 1 / math.sqrt(128)
+    q, k, v, do = inputs()
+    q.requires_grad_(True)
+    strided = q.detach().transpose(1, 2).contiguous().transpose(1, 2).requires_grad_(True)
+    o, native = taken(strided, k, v, None, sc)
+    assert not native and torch.equal(o, taken(q, k, v, None, sc)[0])
+    with torch.autograd.forward_ad.dual_level():
+        assert not taken(q, k, v, None, sc)[1]
+    for bad in ((q[0], k, v), (q, k[:, :, :-1], v), (q, k.float(), v), (q, k, v.cpu()), (q[:, :3].contiguous(), k, v)):
+        for call in (lambda: F.flex_attention(*bad, sm_scale=sc), lambda: python_path(*bad, None, sc)):
+            with pytest.raises(ValueError):
+                call()
+
+
+def test_streams_and_threads():
+    sc, pair = 1 / math.sqrt(128), masks_of(True)
+    want, errors = {}, []
+    sets = [inputs(seed=s) for s in range(4)]
+    for n, (q, k, v, do) in enumerate(sets):
+        for t in (q, k, v):
+            t.requires_grad_(True)
+        want[n] = torch.autograd.grad(python_path(q, k, v, pair, sc), (q, k, v), do)
+    torch.cuda.synchronize()
+
+    def work(n):
+        try:
+            q, k, v, do = sets[n]
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                for _ in range(10):
+                    o, native = taken(q, k, v, pair, sc)
+                    got = torch.autograd.grad(o, (q, k, v), do)
+                    assert native
+            stream.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(got, want[n]))
+        except BaseException as e:
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(n,)) for n in range(len(sets))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+
+
+def test_captured_and_replayed():
+    from flex_attention_tpu_amd import _plans, block_mask
+    sc, pair = 1 / math.sqrt(64), masks_of(True)
+    q, k, v, do = inputs(Sq=384, Sk=384, D=64, dtype=torch.float32)
+    for t in (q, k, v):
+        t.requires_grad_(True)
+
+    def step():
+        o, native = taken(q, k, v, pair, sc)
+        assert native
+        return (o, *torch.autograd.grad(o, (q, k, v), do))
+    step()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    block_mask._map_cache.clear()   # (the captured call builds its maps, which the graph's memory then holds)
+    _plans._attend_plans.clear()
+    with torch.cuda.graph(graph, stream=side):
+        got = step()
+    block_mask._map_cache.clear()
+    _plans._attend_plans.clear()
+    for seed in (1, 2, 3):
+        for t, n in zip((q, k, v, do), inputs(Sq=384, Sk=384, D=64, dtype=torch.float32, seed=seed)):
+            t.data.copy_(n)
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(got, step()):
+            assert torch.equal(a, b)
