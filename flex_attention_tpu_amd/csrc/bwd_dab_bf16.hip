@@ -73,17 +73,17 @@ __global__ __launch_bounds__(512, 1) void bwd_dab_bf16_kernel(BwdArgs a, int n_b
   ScoreMod<kScoreBiasOnly> sm;
   // the tile's bias, shared by the pairs: element e of block c is row qw + 32 c + acc_row(e, hh), key kw + l32
   // (qw, kw: first row and key of the wave's part)
-  f32x16 bias[2], acc[2];
+  f32x16 acc[2];
+  float bias[2][16];
   auto load_bias = [&](const Tile& x) {
     sm.init(a.score, a.sm_scale, x.h0, x.b0);
     const unsigned lane_off = (unsigned)(4 * hh) * (unsigned)a.Sk + (unsigned)(x.k0 + 32 * (w & 3) + l32);
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
+    for (int c = 0; c < 2; ++c) {
+      sm.bias_rows(bias[c], x.q0 + 64 * (w >> 2) + 32 * c, lane_off);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        bias[c][e] = sm.bias2_rows(x.q0 + 64 * (w >> 2) + 32 * c + acc_row(e, 0), lane_off);
-        acc[c][e] = 0.f;
-      }
+      for (int e = 0; e < 16; ++e) acc[c][e] = 0.f;
+    }
   };
 
   TileLoader<8> loader;
@@ -109,10 +109,10 @@ __global__ __launch_bounds__(512, 1) void bwd_dab_bf16_kernel(BwdArgs a, int n_b
     if (tid < T) {
       int b, h;
       pair_of(x, p, b, h);
-      const size_t row = (size_t)(b * a.Hq + h) * a.Sq + (size_t)(x.q0 + tid);
-      l_st = a.l[row];
-      m_st = a.m[row];
-      dl_st = a.delta[row];
+      const size_t row = (size_t)(b * a.Hq + h) * a.Sq + (size_t)x.q0;
+      l_st = (a.l + row)[tid];
+      m_st = (a.m + row)[tid];
+      dl_st = (a.delta + row)[tid];
     }
   };
   auto store_rows = [&](int buf) {
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dab_bf16_kernel(BwdArgs a, int n_b
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const int e = 4 * g + u;
-            const float pe = fast_exp2(sm.to_log2(s[c][e], 0, 0) + bias[c][e] - lse4[u]);
+            const float pe = fast_exp2(__builtin_fmaf(bias[c][e], kLog2e, sm.to_log2(s[c][e], 0, 0)) - lse4[u]);
             float gl = pe * (dp[c][e] - dl4[u]);
             if (MASKED) gl = keep_elem(mk, qw + r0 + u, kw + l32, di[u], doc_j) ? gl : 0.f;
             acc[c][e] += gl;

@@ -140,6 +140,8 @@ __global__ __launch_bounds__(512, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
   const bool ragged_q = nQ * BQ != a.Sq;   // (the last q tile then shares rows with the one before)
   const int n_iter = 2 * n_tiles * group;
 
+  // (dS block of the list's first entry, for query head 0: read here, for a load in the loop would wait for the copies before it)
+  const int ds_first = EXPORT ? __builtin_amdgcn_readfirstlane(a.ds_col[kb]) : 0;
   TileLoader<8> loader;
   loader.init(w, lane);
   // Iteration `it` covers rows 64 (it & 1) .. of list entry t of query head hk group + g, it = 2 (g n_tiles + t) + (it & 1).
@@ -152,14 +154,18 @@ __global__ __launch_bounds__(512, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
     qb_next = n_tiles > 1 ? tile_idx[1] : qb_at;
   }
   float l_st = 0.f, m_st = 0.f, dl_st = 0.f;
-  auto issue_rows = [&](int half, int buf) {
-    const size_t rbase = ((size_t)(b * a.Hq + hk * group + g_at) * a.Sq + (size_t)(tile_base(qb_at, BQ, a.Sq) + half * HQ));
-    loader.load(static_cast<const bf16_t*>(a.q) + rbase * D, sQ + 2 * buf * kTileElems);
-    loader.load(static_cast<const bf16_t*>(a.dout) + rbase * D, sQ + (2 * buf + 1) * kTileElems);
+  size_t rbase = 0;   // first row of the rows that are copied next
+  auto copy_of = [&](int n, int buf) {   // one of the wave's four pieces of them: Q, Q, dO, dO
+    loader.load_block(static_cast<const bf16_t*>(n < 2 ? a.q : a.dout) + rbase * D, sQ + (2 * buf + (n >> 1)) * kTileElems, n & 1);
+  };
+  auto locate_rows = [&](int half) {
+    rbase = ((size_t)(b * a.Hq + hk * group + g_at) * a.Sq + (size_t)(tile_base(qb_at, BQ, a.Sq) + half * HQ));
     if (tid < HQ) {
-      l_st = a.l[rbase + tid];
-      m_st = a.m[rbase + tid];
-      dl_st = a.delta[rbase + tid];
+      unsigned at = 4u * (unsigned)tid;   // (opaque: three addresses per thread, kept through the loop, would spill)
+      asm volatile("" : "+v"(at));
+      l_st = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.l + rbase) + at);
+      m_st = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.m + rbase) + at);
+      dl_st = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.delta + rbase) + at);
     }
   };
   auto store_rows = [&](int buf) {
@@ -183,7 +189,9 @@ __global__ __launch_bounds__(512, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
       loader.load(static_cast<const bf16_t*>(a.k) + kv_off + half * kTileElems, sK + half * kTileElems);
       loader.load(static_cast<const bf16_t*>(a.v) + kv_off + half * kTileElems, sK + (2 + half) * kTileElems);
     }
-    issue_rows(0, 0);
+    locate_rows(0);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) copy_of(n, 0);
     store_rows(0);
   }
   wait_vmem_all();
@@ -227,18 +235,14 @@ __global__ __launch_bounds__(512, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
     // the next rows' copies are issued (vector-memory operations complete in order: behind the copies the first use would
     // wait for them too).
     const unsigned lane_off = (unsigned)(4 * hh) * (unsigned)a.Sk + (unsigned)k_idx;   // (of a bias or its gradient)
-    auto load_bias = [&](const ScoreMod<SCORE>& of, int row0) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) bias[e] = of.bias2_rows(row0 + acc_row(e, 0), lane_off);
-    };
     if (kBias) {
-      if (it == 0) load_bias(sm, q0 + 32 * cc);
+      if (it == 0) sm.bias_rows(bias, q0 + 32 * cc, lane_off);
       wait_vmem<kOpenStores>();
     }
     const bool more = it + 1 < n_iter;
     if (more) {
       if (buf == 1) advance();
-      issue_rows(buf ^ 1, buf ^ 1);
+      locate_rows(buf ^ 1);
     }
 
     const char* qt = reinterpret_cast<const char*>(sQ + 2 * buf * kTileElems) + wq * 32 * kTileD * 2;
@@ -279,6 +283,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
         }
       }
       __builtin_amdgcn_sched_barrier(0);
+      if (more) copy_of(stage, buf ^ 1);   // (under the products: in front of them, each copy holds the wave for some 50 cycles)
     }
 
     bf16x8 pb[2], dsb[2];
@@ -308,7 +313,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
           const int e = 4 * g4 + u;
           const int i = q0 + r0 + u;
           const float tv = sm.to_log2(s_acc[e], i, k_idx);
-          float pe = fast_exp2(tv + (kBias ? bias[e] : kNoBias ? 0.f : sm.bias2(i, k_idx)) - lse4[u]);
+          float pe = fast_exp2((kBias ? __builtin_fmaf(bias[e], kLog2e, tv) : kNoBias ? tv : tv + sm.bias2(i, k_idx)) - lse4[u]);
           float gl = pe * (dp_acc[e] - dl4[u]);   // the gradient of the logit itself: what an additive bias receives
           float gd = gl * sm.dfactor(tv, s_acc[e], i, k_idx);
           unsigned dab_off = 4u * lane_off;
@@ -340,13 +345,13 @@ __global__ __launch_bounds__(512, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
     if (kBias && more) {
       ScoreMod<SCORE> of;   // (the next block's head, which an entry's second half shares)
       of.init(a.score, a.sm_scale, hk * group + g_at, b);
-      load_bias(of, tile_base(qb_at, BQ, a.Sq) + 64 * (buf ^ 1) + 32 * wq);
+      of.bias_rows(bias, tile_base(qb_at, BQ, a.Sq) + 64 * (buf ^ 1) + 32 * wq, lane_off);
     }
     if constexpr (EXPORT) {
       // block of (query head, kept tile pair): head a.ds_pairs + a.ds_col[kv tile] + place of the q tile in the kv
       // tile's list; inside it kv block wk's 1 KB per (32-row q block cc, 16-row half u), lane L its 8 values
       char* blk = static_cast<char*>(a.ds) +
-                  ((size_t)(b * a.Hq + hk * group + g) * (size_t)a.ds_pairs + (size_t)a.ds_col[kb] + (size_t)t) * kDsBlockBytes +
+                  ((size_t)(b * a.Hq + hk * group + g) * (size_t)a.ds_pairs + (size_t)(ds_first + t)) * kDsBlockBytes +
                   8192 * wk + 16 * (2 * l32 + hh);
 #pragma unroll
       for (int u = 0; u < 2; ++u) *reinterpret_cast<bf16x8*>(blk + 1024 * (2 * cc + u)) = dsb[u];
@@ -418,32 +423,39 @@ __global__ __launch_bounds__(512, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
   }
 }
 
-// Head dimension 128 NP, NP >= 2: compiled C++ path.  A row of Q or dO is NP panels of 128 columns, each panel of a
-// 64-row tile one LDS tile (tile_io.hpp) at [buffer][panel]; a loop iteration covers 64 q rows (half an entry of the
-// kv tile's list: the two buffers of Q and dO panels then take the LDS the 128-row steps take at head dim 128), the
-// contractions of S and dP run over the panels, dk^T and dv^T have four accumulators per panel.
+// Head dimension 256: compiled C++ path.  One work-group = 4 waves = 64 kv rows, half a tile of the block map; a loop iteration
+// covers 64 q rows, half an entry of the tile's list, as one LDS tile (tile_io.hpp) per 128-column panel at [buffer][panel].
+// Wave w has kv rows 32 (w & 1) and, of the iteration, q rows 32 (w >> 1) for S and dP, over all 256 columns; P and dS go to the
+// other wave of the kv rows through LDS, and each of the two adds the products of both q blocks to dk and dv in columns
+// 128 (w >> 1): 128 accumulator registers and 128 of K and V, which leaves room to read operands ahead.
+// BOUND: one wave a SIMD: an iteration is 64 MFMAs (2048 cycles) among some 700 instructions, copies into LDS of 64 KB and two
+// barriers, about 6400 cycles.  The form before this one had 128 kv rows a work-group and all columns in each wave: 256
+// accumulators beside K and V left 128 registers for everything else, operands were read in front of each product and the
+// reloads of spilled registers, like the row values and the dS index read in the loop, waited for the copies in flight: dk/dv of
+// B=4, H=16, S=4096, causal, 1776 -> 1520-1610 us, and twice the work-groups where few fill the chip.
 // EXPORT: the pass also writes its bf16 dS, as bwd_dkv_bf16_d128_kernel does: at two panels the dq pass that recomputes S
 // and dP costs three products of a 256-deep contraction, from dS one (B=4, H=16, S=4096, causal, forward and backward: 3.61
 // -> 3.08 ms).
-template <int SCORE, int NP, bool EXPORT, bool AB>
+template <int SCORE, bool EXPORT, bool AB>
 __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
   using namespace dkv_cfg;
   constexpr bool kNoBias = SCORE == FLEXATTN_SCORE_NONE || !AB;   // (a bias without a score function: kScoreBiasOnly)
-  constexpr int D = 128 * NP;
+  constexpr int NP = 2, D = 128 * NP;
   constexpr int HQ = 64;                  // q rows per iteration
   constexpr int kPanel = kTileElems * 2;  // bytes
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
   bf16_t* sQ = reinterpret_cast<bf16_t*>(smem_raw);
   bf16_t* sDO = sQ + 2 * NP * kTileElems;
-  float* sLse = reinterpret_cast<float*>(sDO + 2 * NP * kTileElems);
+  char* sX = reinterpret_cast<char*>(sDO + 2 * NP * kTileElems);   // P and dS of the four waves, 4 KB each
+  float* sLse = reinterpret_cast<float*>(sX + 4 * 4096);
   float* sDl = sLse + 2 * HQ;
 
   const int nKb = a.map.nk;
   const int nQ = a.map.nq;
-  const int n_wg = a.B * a.Hkv * nKb;
+  const int n_wg = a.B * a.Hkv * nKb * 2;
   const int wg = xcd_remap(blockIdx.x, n_wg);
-  const int bhk = wg / nKb;
-  const int kb = wg % nKb;
+  const int bhk = wg / (2 * nKb);
+  const int kb = (wg - bhk * 2 * nKb) >> 1, kx = wg & 1;   // tile of the block map and half of it
   const int b = bhk / a.Hkv;
   const MaskArgs mk = mask_of_batch(a.mask, b, a.Sq, a.Sk);
   const int hk = bhk % a.Hkv;
@@ -451,19 +463,18 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
 
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = w & 1, wc = w >> 1;   // the wave's kv rows; its q rows in S and dP, its columns in dk and dv
   const int lane = tid & 63;
   const int l32 = lane & 31;
   const int hh = lane >> 5;
 
-  const int kv_local = w * 32 + l32;
+  const int kv_local = 64 * kx + 32 * wr + l32;   // in the tile
   const int k0 = tile_base(kb, BNK, a.Sk);
   const int k_idx = k0 + kv_local;
   const bool own_col = k_idx >= kb * BNK;   // (else a row of the kv tile before)
   const size_t kv_off = ((size_t)bhk * a.Sk + (size_t)k0) * D;
   const bf16_t* Kg = static_cast<const bf16_t*>(a.k) + kv_off;
   const bf16_t* Vg = static_cast<const bf16_t*>(a.v) + kv_off;
-  const bf16_t* Qall = static_cast<const bf16_t*>(a.q);
-  const bf16_t* dOall = static_cast<const bf16_t*>(a.dout);
 
   bf16x8 kreg[8 * NP], vreg[8 * NP];
 #pragma unroll
@@ -474,9 +485,9 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
   int doc_j = 0;
   if (mk.flags & FLEXATTN_MASK_DOC) doc_j = mk.doc_k[k_idx];
 
-  f32x16 dk_acc[4 * NP], dv_acc[4 * NP];
+  f32x16 dk_acc[4], dv_acc[4];
 #pragma unroll
-  for (int i = 0; i < 4 * NP; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       dk_acc[i][e] = 0.f;
@@ -488,39 +499,56 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
   const bool ragged_q = nQ * BQ != a.Sq;   // (the last q tile then shares rows with the one before)
   const int n_iter = 2 * n_tiles * group;
 
-  // Iteration `it` covers rows 64 (it & 1) .. of q tile tile_idx[(it / 2) % n_tiles] of query head
-  // hk*group + (it / 2) / n_tiles.  Its q block index is fetched two iterations ahead, its state one ahead.
-  auto q_block_of = [&](int it) { return tile_idx[(it >> 1) % n_tiles]; };
-  int qb_cur = 0, qb_nxt = 0, st_cur = 0;
-  if (n_iter > 0) qb_cur = q_block_of(0);
-  if (n_iter > 1) qb_nxt = q_block_of(1);
-  if (n_iter > 0) st_cur = a.map.state[(size_t)qb_cur * a.map.nk + kb];
-
+  // (as in bwd_dkv_bf16_d128_kernel)
+  const int ds_first = EXPORT ? __builtin_amdgcn_readfirstlane(a.ds_col[kb]) : 0;
   TileLoader<4, D> loader;
   loader.init(w, lane);
-  float lse_st = 0.f, dl_st = 0.f;
-  auto issue_tile = [&](int it, int qb, int buf) {
-    const int g = (it >> 1) / n_tiles;
-    const size_t rbase = ((size_t)(b * a.Hq + hk * group + g) * a.Sq + (size_t)tile_base(qb, BQ, a.Sq) + (size_t)(it & 1) * HQ);
-#pragma unroll
-    for (int pn = 0; pn < NP; ++pn) {
-      loader.load(Qall + rbase * D + 128 * pn, sQ + (buf * NP + pn) * kTileElems);
-      loader.load(dOall + rbase * D + 128 * pn, sDO + (buf * NP + pn) * kTileElems);
-    }
+  // Iteration `it` covers rows 64 (it & 1) .. of a list entry of query head hk group + g.  The list is walked from its end:
+  // under causal masks the lists of a head's kv tiles share their ends, and its work-groups then read the same rows at the same
+  // time.  `at` names the entry that is copied next; its q block index and state are fetched an entry ahead.
+  int g_at = 0, t_at = n_tiles - 1;
+  int qb_at = 0, st_at = 0, qb_next = 0;
+  if (n_iter > 0) {
+    qb_at = __builtin_amdgcn_readfirstlane(tile_idx[t_at]);
+    st_at = a.map.state[(size_t)qb_at * nKb + kb];
+    qb_next = tile_idx[n_tiles > 1 ? t_at - 1 : t_at];
+  }
+  float l_st = 0.f, m_st = 0.f, dl_st = 0.f;
+  size_t rbase = 0;   // first row of the rows that are copied next
+  auto copy_of = [&](int n, int buf) {   // one of the wave's 16 KB-sized pieces of them: n = 8 panel + 4 (0: Q, 1: dO) + block
+    const int pn = n >> 3;
+    if (n & 4) loader.load_block(static_cast<const bf16_t*>(a.dout) + rbase * D + 128 * pn, sDO + (buf * NP + pn) * kTileElems, n & 3);
+    else loader.load_block(static_cast<const bf16_t*>(a.q) + rbase * D + 128 * pn, sQ + (buf * NP + pn) * kTileElems, n & 3);
+  };
+  auto locate_rows = [&](int half) {
+    rbase = ((size_t)(b * a.Hq + hk * group + g_at) * a.Sq + (size_t)(tile_base(qb_at, BQ, a.Sq) + half * HQ));
     if (tid < HQ) {
-      const float l_i = a.l[rbase + tid], m_i = a.m[rbase + tid];
-      lse_st = (l_i > 0.f) ? __builtin_fmaf(m_i, kLog2e, log2f(l_i)) : __builtin_huge_valf();
-      dl_st = a.delta[rbase + tid];
+      unsigned at = 4u * (unsigned)tid;   // (opaque: three addresses per thread, kept through the loop, would spill)
+      asm volatile("" : "+v"(at));
+      l_st = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.l + rbase) + at);
+      m_st = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.m + rbase) + at);
+      dl_st = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.delta + rbase) + at);
     }
   };
   auto store_rows = [&](int buf) {
-    if (tid < HQ) {
-      sLse[buf * HQ + tid] = lse_st;
+    if (tid < HQ) {   // (the loads' values are first touched here: touched where they are issued, every iteration waits for its copies there)
+      sLse[buf * HQ + tid] = (l_st > 0.f) ? __builtin_fmaf(m_st, kLog2e, log2f(l_st)) : __builtin_huge_valf();
       sDl[buf * HQ + tid] = dl_st;
     }
   };
+  auto advance = [&]() {   // `at` to the next entry
+    if (--t_at < 0) {
+      t_at = n_tiles - 1;
+      ++g_at;
+    }
+    qb_at = __builtin_amdgcn_readfirstlane(qb_next);
+    st_at = a.map.state[(size_t)qb_at * nKb + kb];
+    qb_next = tile_idx[t_at > 0 ? t_at - 1 : n_tiles - 1];
+  };
   if (n_iter > 0) {
-    issue_tile(0, __builtin_amdgcn_readfirstlane(qb_cur), 0);
+    locate_rows(0);
+#pragma unroll
+    for (int n = 0; n < 8 * NP; ++n) copy_of(n, 0);
     store_rows(0);
   }
   wait_vmem_all();
@@ -541,168 +569,222 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_bf16_wide_kernel(BwdArgs a) {
   }
 
   ScoreMod<SCORE> sm;
+  int qb = 0, st = 0, g = 0, t = 0;   // the entry that is computed
   for (int it = 0; it < n_iter; ++it) {
     const int buf = it & 1;
-    const int qb = __builtin_amdgcn_readfirstlane(qb_cur);
-    const bool partial = __builtin_amdgcn_readfirstlane(st_cur) == 1 || (qb == nQ - 1 && ragged_q);
-    sm.init(a.score, a.sm_scale, hk * group + (it >> 1) / n_tiles, b);
-    const int qb_n2 = (it + 2 < n_iter) ? q_block_of(it + 2) : 0;
-    int st_nxt = 0;
-    if (it + 1 < n_iter) {
-      const int qbn = __builtin_amdgcn_readfirstlane(qb_nxt);
-      st_nxt = a.map.state[(size_t)qbn * a.map.nk + kb];
-      issue_tile(it + 1, qbn, buf ^ 1);
+    if (buf == 0) {   // an entry's first half: the entry that was copied ahead
+      if (it == 0 || g != g_at) sm.init(a.score, a.sm_scale, hk * group + g_at, b);
+      qb = qb_at;
+      st = st_at;
+      g = g_at;
+      t = t_at;
     }
-    const int q0 = tile_base(qb, BQ, a.Sq) + (it & 1) * HQ;
+    const bool partial = __builtin_amdgcn_readfirstlane(st) == 1 || (qb == nQ - 1 && ragged_q);
+    const int q0 = tile_base(qb, BQ, a.Sq);
+    const int cc = 2 * buf + wc;   // the wave's 32-row block of the q tile
     // (elements before this offset belong to the q tile before; a column of the kv tile before owns none)
     const int own = first_owned(qb, BQ, q0, 4 * hh, own_col);
+    const bool more = it + 1 < n_iter;
+    if (more) {
+      if (buf == 1) advance();
+      locate_rows(buf ^ 1);
+    }
     const char* qt = reinterpret_cast<const char*>(sQ + buf * NP * kTileElems);
     const char* dot = reinterpret_cast<const char*>(sDO + buf * NP * kTileElems);
-#pragma unroll 1   // (rolled: unrolled, the second block's operand loads are hoisted over the first block's and 72 registers spill; 2.72 -> 2.01 ms on B=4, H=16, S=4096)
-    for (int c = 0; c < 2; ++c) {   // 32-row blocks of the 64 rows
-      f32x16 s_acc, dp_acc;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        s_acc[e] = 0.f;
-        dp_acc[e] = 0.f;
-      }
-#pragma unroll
-      for (int pn = 0; pn < NP; ++pn) {
-        bf16x8 qf[8];
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(qt + pn * kPanel + r_off[ks] + c * 32 * kTileD * 2);
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) s_acc = mfma32(qf[ks], kreg[8 * pn + ks], s_acc);
-      }
-#pragma unroll
-      for (int pn = 0; pn < NP; ++pn) {
-        bf16x8 df[8];
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) df[ks] = *reinterpret_cast<const bf16x8*>(dot + pn * kPanel + r_off[ks] + c * 32 * kTileD * 2);
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) dp_acc = mfma32(df[ks], vreg[8 * pn + ks], dp_acc);
-      }
 
-      bf16x8 pb[2], dsb[2];
-      auto elementwise = [&](auto masked) {
-        constexpr bool MASKED = decltype(masked)::value;
-        const bool has_doc = MASKED && (mk.flags & FLEXATTN_MASK_DOC) != 0;
+    f32x16 s_acc, dp_acc;
 #pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          const int r0 = 32 * c + 8 * g4 + 4 * hh;  // the lane's q rows come in runs of 4
-          const f32x4 lse4 = *reinterpret_cast<const f32x4*>(sLse + buf * HQ + r0);
-          const f32x4 dl4 = *reinterpret_cast<const f32x4*>(sDl + buf * HQ + r0);
-          int di[4] = {0, 0, 0, 0};
-          if (MASKED && has_doc) {
-            const auto d4 = *reinterpret_cast<const i32x4_a4*>(mk.doc_q + q0 + r0);
-            di[0] = d4[0]; di[1] = d4[1]; di[2] = d4[2]; di[3] = d4[3];
-          }
-          float pv[4], dsv[4];
+    for (int e = 0; e < 16; ++e) {
+      s_acc[e] = 0.f;
+      dp_acc[e] = 0.f;
+    }
+    // (operands are read four products ahead: left to itself the compiler waits out the LDS latency in front of each)
+    bf16x8 rf[2][4];
+    auto read_rows = [&](int stage) {   // four k-steps each: those of Q, panel by panel, then those of dO
+      const int at = stage % (2 * NP);
+      const char* rows = (stage < 2 * NP ? qt : dot) + (at >> 1) * kPanel + wc * 32 * kTileD * 2;
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int e = 4 * g4 + u;
-            const int i = q0 + r0 + u;
-            const float tv = sm.to_log2(s_acc[e], i, k_idx);
-            float pe = fast_exp2(tv + (kNoBias ? 0.f : sm.bias2(i, k_idx)) - lse4[u]);
-            float gd = pe * (dp_acc[e] - dl4[u]) * sm.dfactor(tv, s_acc[e], i, k_idx);
-            if (MASKED) {
-              const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j) & (8 * g4 + u >= own - 32 * c);
-              pe = keep ? pe : 0.f;
-              gd = keep ? gd : 0.f;
-            }
-            pv[u] = pe;
-            dsv[u] = gd;
-          }
-          const bf16x2 p01 = pack_bf16(pv[0], pv[1]), p23 = pack_bf16(pv[2], pv[3]);
-          const bf16x2 d01 = pack_bf16(dsv[0], dsv[1]), d23 = pack_bf16(dsv[2], dsv[3]);
-          const int o = 4 * (g4 & 1);
-          pb[g4 >> 1][o] = p01[0]; pb[g4 >> 1][o + 1] = p01[1]; pb[g4 >> 1][o + 2] = p23[0]; pb[g4 >> 1][o + 3] = p23[1];
-          dsb[g4 >> 1][o] = d01[0]; dsb[g4 >> 1][o + 1] = d01[1]; dsb[g4 >> 1][o + 2] = d23[0]; dsb[g4 >> 1][o + 3] = d23[1];
-        }
-      };
-      if (partial) {
-        elementwise(std::true_type{});
-      } else {
-        elementwise(std::false_type{});
+      for (int i = 0; i < 4; ++i) rf[stage & 1][i] = *reinterpret_cast<const bf16x8*>(rows + r_off[4 * (at & 1) + i]);
+    };
+    read_rows(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int stage = 0; stage < 4 * NP; ++stage) {
+      if (stage < 4 * NP - 1) read_rows(stage + 1);
+      const int at = 4 * (stage % (2 * NP));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (stage < 2 * NP) s_acc = mfma32(rf[stage & 1][i], kreg[at + i], s_acc);
+        else dp_acc = mfma32(rf[stage & 1][i], vreg[at + i], dp_acc);
       }
-      if constexpr (EXPORT) {
-        // (the block layout of bwd_dkv_bf16_d128_kernel's export; 32-row block 2 (it & 1) + c of the q tile)
-        char* blk = static_cast<char*>(a.ds) +
-                    ((size_t)(b * a.Hq + hk * group + (it >> 1) / n_tiles) * (size_t)a.ds_pairs + (size_t)a.ds_col[kb] +
-                     (size_t)((it >> 1) % n_tiles)) * kDsBlockBytes + 8192 * w + 16 * (2 * l32 + hh);
+      if (stage < 4 * NP - 1) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) *reinterpret_cast<bf16x8*>(blk + 1024 * (4 * (it & 1) + 2 * c + u)) = dsb[u];
-      }
-
-      // dv^T += dO^T P, dk^T += Q^T dS, a panel at a time (the transposed fragments of one panel are live at once)
-#pragma unroll
-      for (int pn = 0; pn < NP; ++pn) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int off = (32 * c + 16 * u) * kTileD * 2 + pn * kPanel;
-          s16x4 dolo[4], dohi[4], qlo[4], qhi[4];
-#pragma unroll
-          for (int db = 0; db < 4; ++db) {
-            dolo[db] = lds_read_tr16(reinterpret_cast<const bf16_t*>(dot + t_off[db][0] + off));
-            dohi[db] = lds_read_tr16(reinterpret_cast<const bf16_t*>(dot + t_off[db][1] + off));
-            qlo[db] = lds_read_tr16(reinterpret_cast<const bf16_t*>(qt + t_off[db][0] + off));
-            qhi[db] = lds_read_tr16(reinterpret_cast<const bf16_t*>(qt + t_off[db][1] + off));
-          }
-#pragma unroll
-          for (int db = 0; db < 4; ++db) {
-            dv_acc[4 * pn + db] = mfma32(join_tr(dolo[db], dohi[db]), pb[u], dv_acc[4 * pn + db]);
-            dk_acc[4 * pn + db] = mfma32(join_tr(qlo[db], qhi[db]), dsb[u], dk_acc[4 * pn + db]);
-          }
-          __builtin_amdgcn_sched_barrier(0);   // (keeps the next group's fragments out of this one's registers)
+        for (int i = 0; i < 4; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // an MFMA,
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // an LDS read
         }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) {   // (under the products: in front of them, each copy holds the wave for some 50 cycles)
+        copy_of(2 * stage, buf ^ 1);
+        copy_of(2 * stage + 1, buf ^ 1);
       }
     }
 
-    qb_cur = qb_nxt; qb_nxt = qb_n2;
-    st_cur = st_nxt;
-    if (it + 1 < n_iter) store_rows(buf ^ 1);
-    wait_vmem_all();
+    // dv^T += dO^T P, dk^T += Q^T dS in the wave's columns, over the q rows of both waves: groups of 16 rows, this wave's own
+    // first; the next group's transposed fragments are read under this one's products
+    s16x4 tr[2][4][4];   // [group & 1][column block][dO low, dO high, Q low, Q high]
+    auto read_tr = [&](int ga) {
+      const int off = (32 * (wc ^ (ga >> 1)) + 16 * (ga & 1)) * kTileD * 2 + wc * kPanel;
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          tr[ga & 1][db][i] = lds_read_tr16(reinterpret_cast<const bf16_t*>((i < 2 ? dot : qt) + t_off[db][i & 1] + off));
+    };
+    read_tr(0);   // (in front of the element-wise work, which hides their latency)
+    __builtin_amdgcn_sched_barrier(0);
+    bf16x8 pb[2], dsb[2];
+    auto elementwise = [&](auto masked) {
+      constexpr bool MASKED = decltype(masked)::value;
+      const bool has_doc = MASKED && (mk.flags & FLEXATTN_MASK_DOC) != 0;
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const int r0 = 32 * cc + 8 * g4 + 4 * hh;  // the lane's q rows come in runs of 4 (64 buf + ..: the buffer's row values)
+        const f32x4 lse4 = *reinterpret_cast<const f32x4*>(sLse + r0);
+        const f32x4 dl4 = *reinterpret_cast<const f32x4*>(sDl + r0);
+        int di[4] = {0, 0, 0, 0};
+        if (MASKED && has_doc) {
+          const auto d4 = *reinterpret_cast<const i32x4_a4*>(mk.doc_q + q0 + r0);
+          di[0] = d4[0]; di[1] = d4[1]; di[2] = d4[2]; di[3] = d4[3];
+        }
+        float pv[4], dsv[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int e = 4 * g4 + u;
+          const int i = q0 + r0 + u;
+          const float tv = sm.to_log2(s_acc[e], i, k_idx);
+          float pe = fast_exp2(tv + (kNoBias ? 0.f : sm.bias2(i, k_idx)) - lse4[u]);
+          float gd = pe * (dp_acc[e] - dl4[u]) * sm.dfactor(tv, s_acc[e], i, k_idx);
+          if (MASKED) {
+            const bool keep = keep_elem(mk, i, k_idx, di[u], doc_j) & (32 * cc + 8 * g4 + u >= own);
+            pe = keep ? pe : 0.f;
+            gd = keep ? gd : 0.f;
+          }
+          pv[u] = pe;
+          dsv[u] = gd;
+        }
+        const bf16x2 p01 = pack_bf16(pv[0], pv[1]), p23 = pack_bf16(pv[2], pv[3]);
+        const bf16x2 d01 = pack_bf16(dsv[0], dsv[1]), d23 = pack_bf16(dsv[2], dsv[3]);
+        const int o = 4 * (g4 & 1);
+        pb[g4 >> 1][o] = p01[0]; pb[g4 >> 1][o + 1] = p01[1]; pb[g4 >> 1][o + 2] = p23[0]; pb[g4 >> 1][o + 3] = p23[1];
+        dsb[g4 >> 1][o] = d01[0]; dsb[g4 >> 1][o + 1] = d01[1]; dsb[g4 >> 1][o + 2] = d23[0]; dsb[g4 >> 1][o + 3] = d23[1];
+      }
+    };
+    if (partial) {
+      elementwise(std::true_type{});
+    } else {
+      elementwise(std::false_type{});
+    }
+    // P and dS to the other wave of these kv rows
+    {
+      char* mine = sX + w * 4096 + 16 * lane;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        *reinterpret_cast<bf16x8*>(mine + 1024 * u) = pb[u];
+        *reinterpret_cast<bf16x8*>(mine + 2048 + 1024 * u) = dsb[u];
+      }
+    }
+    if constexpr (EXPORT) {
+      // (the block layout of bwd_dkv_bf16_d128_kernel's export)
+      char* blk = static_cast<char*>(a.ds) +
+                  ((size_t)(b * a.Hq + hk * group + g) * (size_t)a.ds_pairs + (size_t)(ds_first + t)) * kDsBlockBytes +
+                  8192 * (2 * kx + wr) + 16 * (2 * l32 + hh);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) *reinterpret_cast<bf16x8*>(blk + 1024 * (2 * cc + u)) = dsb[u];
+    }
+
+    auto products = [&](int ga, bf16x8 p, bf16x8 ds) {
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+        dv_acc[db] = mfma32(join_tr(tr[ga & 1][db][0], tr[ga & 1][db][1]), p, dv_acc[db]);
+        dk_acc[db] = mfma32(join_tr(tr[ga & 1][db][2], tr[ga & 1][db][3]), ds, dk_acc[db]);
+      }
+    };
+    auto interleave = [&]() {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    read_tr(1);
+    products(0, pb[0], dsb[0]);
+    interleave();
+    read_tr(2);
+    products(1, pb[1], dsb[1]);
+    interleave();
+    // (the other wave's P and dS are there; copies and stores stay open over this barrier)
+    __syncthreads();
+    {
+      const char* other = sX + (w ^ 2) * 4096 + 16 * lane;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        pb[u] = *reinterpret_cast<const bf16x8*>(other + 1024 * u);
+        dsb[u] = *reinterpret_cast<const bf16x8*>(other + 2048 + 1024 * u);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    read_tr(3);
+    products(2, pb[0], dsb[0]);
+    interleave();
+    products(3, pb[1], dsb[1]);
+
+    if (more) store_rows(buf ^ 1);
+    wait_vmem<EXPORT ? 2 : 0>();   // (the copies are there; the stores of dS behind them may stay open)
     __syncthreads();
   }
 
   if (!own_col) return;
-  bf16_t* dKg = static_cast<bf16_t*>(a.dk) + kv_off;
-  bf16_t* dVg = static_cast<bf16_t*>(a.dv) + kv_off;
+  bf16_t* dKg = static_cast<bf16_t*>(a.dk) + kv_off + (size_t)kv_local * D + 128 * wc;
+  bf16_t* dVg = static_cast<bf16_t*>(a.dv) + kv_off + (size_t)kv_local * D + 128 * wc;
 #pragma unroll
-  for (int db = 0; db < 4 * NP; ++db) {
+  for (int db = 0; db < 4; ++db) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      bf16x2 lo = pack_bf16(dk_acc[db][4 * g], dk_acc[db][4 * g + 1]);
-      bf16x2 hi = pack_bf16(dk_acc[db][4 * g + 2], dk_acc[db][4 * g + 3]);
-      bf16x4 out = {lo[0], lo[1], hi[0], hi[1]};
-      *reinterpret_cast<bf16x4*>(dKg + (size_t)kv_local * D + 32 * db + 8 * g + 4 * hh) = out;
-      lo = pack_bf16(dv_acc[db][4 * g], dv_acc[db][4 * g + 1]);
-      hi = pack_bf16(dv_acc[db][4 * g + 2], dv_acc[db][4 * g + 3]);
-      bf16x4 out2 = {lo[0], lo[1], hi[0], hi[1]};
-      *reinterpret_cast<bf16x4*>(dVg + (size_t)kv_local * D + 32 * db + 8 * g + 4 * hh) = out2;
+    for (int g4 = 0; g4 < 4; ++g4) {
+      bf16x2 lo = pack_bf16(dk_acc[db][4 * g4], dk_acc[db][4 * g4 + 1]);
+      bf16x2 hi = pack_bf16(dk_acc[db][4 * g4 + 2], dk_acc[db][4 * g4 + 3]);
+      const bf16x4 out = {lo[0], lo[1], hi[0], hi[1]};
+      *reinterpret_cast<bf16x4*>(dKg + 32 * db + 8 * g4 + 4 * hh) = out;
+      lo = pack_bf16(dv_acc[db][4 * g4], dv_acc[db][4 * g4 + 1]);
+      hi = pack_bf16(dv_acc[db][4 * g4 + 2], dv_acc[db][4 * g4 + 3]);
+      const bf16x4 out2 = {lo[0], lo[1], hi[0], hi[1]};
+      *reinterpret_cast<bf16x4*>(dVg + 32 * db + 8 * g4 + 4 * hh) = out2;
     }
   }
 }
 
-template <int SCORE, int NP, bool EXPORT, bool AB = true>
+template <int SCORE, bool EXPORT, bool AB = true>
 static int launch_dkv_wide_on(const BwdArgs& a, hipStream_t stream) {
   if constexpr (AB && splits_bias(SCORE))
-    if (a.score.ab == nullptr) return launch_dkv_wide_on<SCORE, NP, EXPORT, false>(a, stream);
+    if (a.score.ab == nullptr) return launch_dkv_wide_on<SCORE, EXPORT, false>(a, stream);
   if constexpr (SCORE == FLEXATTN_SCORE_NONE)
-    if (a.score.ab != nullptr) return launch_dkv_wide_on<kScoreBiasOnly, NP, EXPORT>(a, stream);
+    if (a.score.ab != nullptr) return launch_dkv_wide_on<kScoreBiasOnly, EXPORT>(a, stream);
   using namespace dkv_cfg;
-  constexpr int kLds = 4 * NP * kTileElems * 2 + 4 * 64 * 4;   // (Q, dO) x 2 buffers x NP panels; lse, delta x 2 buffers
-  auto kern = bwd_dkv_bf16_wide_kernel<SCORE, NP, EXPORT, AB>;
+  constexpr int kLds = 8 * kTileElems * 2 + 4 * 4096 + 4 * 64 * 4;   // (Q, dO) x 2 buffers x 2 panels; P, dS; lse, delta x 2 buffers
+  auto kern = bwd_dkv_bf16_wide_kernel<SCORE, EXPORT, AB>;
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dkv): %s", hipGetErrorString(attr));
-  const int n_wg = a.B * a.Hkv * a.map.nk;
+  const int n_wg = a.B * a.Hkv * a.map.nk * 2;
   hipLaunchKernelGGL(kern, dim3(n_wg), dim3(256), kLds, stream, a);
   return check_launch("flexattn_bwd_dkv bf16");
 }
-template <int SCORE, int NP>
+template <int SCORE>
 static int launch_dkv_wide(const BwdArgs& a, hipStream_t stream) {
-  return a.ds != nullptr ? launch_dkv_wide_on<SCORE, NP, true>(a, stream) : launch_dkv_wide_on<SCORE, NP, false>(a, stream);
+  return a.ds != nullptr ? launch_dkv_wide_on<SCORE, true>(a, stream) : launch_dkv_wide_on<SCORE, false>(a, stream);
 }
 
 #ifndef FLEXATTN_CUSTOM_ONLY
@@ -1322,13 +1404,13 @@ int bwd_dkv_bf16_d64(const BwdArgs& a, hipStream_t stream) {
 // Head dim 256: the kernel with a compiled main loop (two 128-column panels per row), every score kind.
 int bwd_dkv_bf16_d256(const BwdArgs& a, hipStream_t stream) {
   switch (a.score.kind) {
-    case FLEXATTN_SCORE_NONE: return launch_dkv_wide<FLEXATTN_SCORE_NONE, 2>(a, stream);
+    case FLEXATTN_SCORE_NONE: return launch_dkv_wide<FLEXATTN_SCORE_NONE>(a, stream);
 #ifdef FLEXATTN_CUSTOM_ONLY
-    case FLEXATTN_SCORE_CUSTOM: return launch_dkv_wide<FLEXATTN_SCORE_CUSTOM, 2>(a, stream);
+    case FLEXATTN_SCORE_CUSTOM: return launch_dkv_wide<FLEXATTN_SCORE_CUSTOM>(a, stream);
 #else
-    case FLEXATTN_SCORE_ALIBI: return launch_dkv_wide<FLEXATTN_SCORE_ALIBI, 2>(a, stream);
-    case FLEXATTN_SCORE_SOFTCAP: return launch_dkv_wide<FLEXATTN_SCORE_SOFTCAP, 2>(a, stream);
-    case FLEXATTN_SCORE_ALIBI_TILE: return launch_dkv_wide<FLEXATTN_SCORE_ALIBI_TILE, 2>(a, stream);
+    case FLEXATTN_SCORE_ALIBI: return launch_dkv_wide<FLEXATTN_SCORE_ALIBI>(a, stream);
+    case FLEXATTN_SCORE_SOFTCAP: return launch_dkv_wide<FLEXATTN_SCORE_SOFTCAP>(a, stream);
+    case FLEXATTN_SCORE_ALIBI_TILE: return launch_dkv_wide<FLEXATTN_SCORE_ALIBI_TILE>(a, stream);
 #endif
   }
   return set_error(FLEXATTN_ENOTSUP, "score kind %d is not in this library", a.score.kind);

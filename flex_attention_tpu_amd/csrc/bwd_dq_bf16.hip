@@ -189,10 +189,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
     for (int c = 0; c < 2; ++c) {
       // (an additive bias: loaded in front of the products, which hide the latency)
       f32x4 bias_pre[4];
-      if (kBias) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g) bias_pre[g] = sm.bias2x4(q_idx, kv0 + 32 * c + 8 * g + 4 * hh);
-      }
+      if (kBias) sm.bias_keys(bias_pre, q_idx, kv0 + 32 * c + 4 * hh);
       // ---- S^T and dP^T for kv rows [32c, 32c+32) ----
       f32x16 s_acc, dp_acc;
 #pragma unroll
@@ -248,7 +245,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void bwd_dq_bf16_kernel(BwdAr
           for (int u = 0; u < 4; ++u) {
             const int e = 4 * g + u;
             const float tv = sm.to_log2(s_acc[e], q_idx, j0 + u);
-            const float pe = fast_exp2(tv + bias[u] - lse2);
+            const float pe = fast_exp2((kBias ? __builtin_fmaf(bias[u], kLog2e, tv) : tv + bias[u]) - lse2);
             float gl = pe * (dp_acc[e] - delta);
             float gd = gl * sm.dfactor(tv, s_acc[e], q_idx, j0 + u);
             if (MASKED) {   // (selected, not multiplied: a score function may return anything at a dropped element)

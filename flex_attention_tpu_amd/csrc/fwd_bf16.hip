@@ -213,11 +213,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
     // (an additive bias: the tile's 32 values per lane are loaded in front of the products, which hide the latency)
     constexpr bool kBias = NP == 1 && SCORE == kScoreBiasOnly;
     f32x4 bias_pre[8];
-    if (kBias) {
-      const int kv0_b = tile_base(kb, BN, a.Sk);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) bias_pre[i] = sm.bias2x4(q_idx, kv0_b + 32 * (i >> 2) + 8 * (i & 3) + 4 * hh);
-    }
+    if (kBias) sm.bias_keys(bias_pre, q_idx, tile_base(kb, BN, a.Sk) + 4 * hh);
     read_k(0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -243,11 +239,16 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
     }
     if (kEarlyV) read_v(1);
 
+    // (the bias is there; the eight copies issued behind it may stay open)
+    if (kBias) {
+      if (prefetch) wait_vmem<8>(); else wait_vmem<0>();
+    }
     // ---- score mod, mask, online softmax ----
     // For the plain score the running maximum is kept on the raw dot products and the scale is
     // folded into the exponent (one FMA per element); score mods go through the log2-domain logit.
     const int kv0 = tile_base(kb, BN, a.Sk);
     constexpr bool kPlain = (SCORE == FLEXATTN_SCORE_NONE);
+    auto with_bias = [](float t, float x) { return kBias ? __builtin_fmaf(x, kLog2e, t) : t + x; };
     float m_tile = kNegInf;
     if (!partial) {
 #pragma unroll
@@ -260,7 +261,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const int e = 4 * g + u;
-            if (!kPlain) s_acc[c][e] = sm.to_log2(s_acc[c][e], q_idx, j0 + u) + bias[u];
+            if (!kPlain) s_acc[c][e] = with_bias(sm.to_log2(s_acc[c][e], q_idx, j0 + u), bias[u]);
             m_tile = fmaxf(m_tile, s_acc[c][e]);
           }
         }
@@ -285,7 +286,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const int e = 4 * g + u;
-            float tv = kPlain ? s_acc[c][e] : sm.to_log2(s_acc[c][e], q_idx, j0 + u) + bias[u];
+            float tv = kPlain ? s_acc[c][e] : with_bias(sm.to_log2(s_acc[c][e], q_idx, j0 + u), bias[u]);
             tv = keep_elem(mk, q_idx, j0 + u, doc_i, dj[u]) ? tv : kNegInf;
             s_acc[c][e] = tv;
             m_tile = fmaxf(m_tile, tv);
