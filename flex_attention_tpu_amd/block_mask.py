@@ -20,6 +20,8 @@ from .masks import DocIds, MaskSpec
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
+_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", torch.cuda.is_current_stream_capturing)   # (no Python around the query)
+
 
 def raw_stream(device) -> int:
     """Handle of the current stream of `device` (the lookup that builds no Stream object where torch has one: the
@@ -101,8 +103,12 @@ class BlockMap:
     def wait_ready(self, device) -> None:
         """Makes the current stream wait for the builder kernel if that ran on another stream, and tells the
         caching allocator that the map is in use on this stream too (a map evicted from the cache must not be
-        handed out again while a kernel on this stream still walks it)."""
-        if self.ready is None or raw_stream(device) == self.built_on:
+        handed out again while a kernel on this stream still walks it).  A call that is being captured keeps the map: the graph
+        holds its addresses, whatever the cache drops."""
+        stream = raw_stream(device)
+        if stream != 0 and _capturing():   # (the default stream is never captured: the usual case asks nothing)
+            _captured_maps.put(id(self), self)
+        if self.ready is None or stream == self.built_on:
             return
         cur = torch.cuda.current_stream(device)
         if cur.cuda_stream != self.built_on:
@@ -159,6 +165,7 @@ class BlockMap:
 MAP_CACHE_SIZE = 64
 DOC_CACHE_SIZE = 64
 _doc_cache = LRU(DOC_CACHE_SIZE)   # (DocIds, device) -> int32 device array
+_captured_maps = LRU(256)   # maps that captured calls read, by identity: as long-lived as the graphs of the last 256 of them
 _map_cache = LRU(MAP_CACHE_SIZE)   # (spec, Sq, Sk, block_q, block_k, device) -> BlockMap
 
 
@@ -265,7 +272,9 @@ def build_block_map(spec: MaskSpec, Sq: int, Sk: int, block_q: int, block_k: int
         bm.built_on = stream
         bm.ready = torch.cuda.Event()
         bm.ready.record(torch.cuda.current_stream(device))
-    if cache:
+    if _capturing():
+        _captured_maps.put(id(bm), bm)   # (built when the graph is replayed, not before: no map for other calls)
+    elif cache:
         _map_cache.put(key, bm)
     return bm
 
