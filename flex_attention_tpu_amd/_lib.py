@@ -149,6 +149,8 @@ EXPORTS = (
     "flexattn_build_block_mask_ragged",
     "flexattn_build_ds_index",
     "flexattn_fwd",
+    "flexattn_fwd_work_bytes",
+    "flexattn_fwd_work",
     "flexattn_fwd_noalloc",
     "flexattn_fwd_decode_bytes",
     "flexattn_fwd_decode",
@@ -177,6 +179,9 @@ def _bind(lib: C.CDLL) -> C.CDLL:
     lib.flexattn_build_block_mask_ragged.argtypes = lib.flexattn_build_block_mask.argtypes
     lib.flexattn_build_ds_index.argtypes = [C.POINTER(BlockMapC), C.c_void_p, C.c_void_p, C.c_void_p]
     lib.flexattn_fwd.argtypes = [C.POINTER(FwdParamsC), C.c_void_p]
+    lib.flexattn_fwd_work_bytes.argtypes = [C.POINTER(FwdParamsC)]
+    lib.flexattn_fwd_work_bytes.restype = C.c_int64
+    lib.flexattn_fwd_work.argtypes = [C.POINTER(FwdParamsC), C.c_void_p, C.c_int64, C.c_void_p]
     lib.flexattn_fwd_noalloc.argtypes = [C.POINTER(FwdParamsC), C.c_void_p]
     lib.flexattn_fwd_decode_bytes.argtypes = [C.POINTER(FwdParamsC)]
     lib.flexattn_fwd_decode_bytes.restype = C.c_int64
@@ -190,7 +195,7 @@ def _bind(lib: C.CDLL) -> C.CDLL:
     lib.flexattn_bwd_dab_pays.argtypes = [C.POINTER(BwdParamsC)]
     lib.flexattn_bwd_dab.argtypes = [C.POINTER(BwdParamsC), C.c_void_p]
     lib.flexattn_takes_head_dim_64.argtypes = [C.c_int32, C.c_float, C.c_int32, C.c_int32]
-    for name in ("flexattn_takes_head_dim_64", "flexattn_tile_shape", "flexattn_build_block_mask", "flexattn_build_block_mask_ragged", "flexattn_build_ds_index", "flexattn_fwd",
+    for name in ("flexattn_takes_head_dim_64", "flexattn_tile_shape", "flexattn_build_block_mask", "flexattn_build_block_mask_ragged", "flexattn_build_ds_index", "flexattn_fwd", "flexattn_fwd_work",
                  "flexattn_fwd_noalloc", "flexattn_fwd_decode", "flexattn_bwd_delta", "flexattn_bwd_dq", "flexattn_bwd_dkv", "flexattn_bwd_dab_pays", "flexattn_bwd_dab", "flexattn_bwd"):
         getattr(lib, name).restype = C.c_int
     return lib
@@ -223,7 +228,7 @@ def load_host():
         from . import _host as mod
         lib = load()
         mod.bind(*(C.cast(getattr(lib, "flexattn_" + n), C.c_void_p).value
-                   for n in ("fwd", "bwd", "bwd_dq", "bwd_dkv", "bwd_delta", "last_error_string")))
+                   for n in ("fwd_work", "fwd_work_bytes", "bwd", "bwd_dq", "bwd_dkv", "bwd_delta", "last_error_string")))
         _host = mod
     return _host
 

@@ -29,10 +29,11 @@ _BWD_POINTERS = struct.Struct("10P")    # q, k, v, dout, l, m, delta, dq, dk, dv
 class _Plan:
     """Parameter templates (bytes) of one combination and weak references to the block maps they point at: the maps
     belong to their own bounded cache, and a plan whose map has been dropped there is made again."""
-    __slots__ = ("templates", "maps")
+    __slots__ = ("templates", "maps", "work_bytes")
 
     def __init__(self, templates, maps):
         self.templates, self.maps = templates, tuple(weakref.ref(bm) for bm in maps)
+        self.work_bytes = None   # (of the forward, asked at first use)
 
 
 def _template(cls, pass_id, q, k, spec, sm_scale):
@@ -48,7 +49,7 @@ def _template(cls, pass_id, q, k, spec, sm_scale):
 
 
 def _plan(key, q, k, spec, sm_scale, cls, passes):
-    """(templates, block maps) of a combination; the caller holds the maps until its launch is out."""
+    """(plan, block maps) of a combination; the caller holds the maps until its launch is out."""
     plan = _plans.get(key)
     maps = [ref() for ref in plan.maps] if plan is not None else (None,)
     if None in maps:
@@ -57,7 +58,7 @@ def _plan(key, q, k, spec, sm_scale, cls, passes):
         _plans.put(key, plan)
     for bm in maps:   # (a map built on another stream: this one waits for it)
         bm.wait_ready(q.device)
-    return plan.templates, maps
+    return plan, maps
 
 
 _attend_plans = LRU(64)   # (shapes, dtype, device, mask, scale, blocks) -> (C++ plan, weak references to its block maps), or False
@@ -65,9 +66,11 @@ _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def ordinary(q, k, v) -> bool:
-    """Whether a call is one that the C++ autograd function serves exactly as the Python one does: plain contiguous tensors
-    outside function transforms, forward-mode differentiation, tracing and compilation, and modes that watch Python's calls."""
-    return (not torch.compiler.is_compiling() and type(q) in _PLAIN and type(k) in _PLAIN and type(v) in _PLAIN and q.is_contiguous() and k.is_contiguous() and v.is_contiguous()
+    """Whether a call is one that the C++ autograd function serves exactly as the Python one does: plain contiguous tensors of
+    lengths and head dimensions that it may take, outside function transforms, forward-mode differentiation, tracing and compilation, and modes that watch Python's calls."""
+    if type(q) not in _PLAIN or q.ndim != 4 or q.shape[2] < 128 or q.shape[3] > 128:
+        return False   # (decoding, and head dimension 256, whose backward hands dS over)
+    return (not torch.compiler.is_compiling() and type(k) in _PLAIN and type(v) in _PLAIN and q.is_contiguous() and k.is_contiguous() and v.is_contiguous()
             and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
             and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
             and torch._C._get_tracing_state() is None)
@@ -110,37 +113,45 @@ def takes(q, k, spec: MaskSpec, sm_scale, *passes: int) -> bool:
     return all([call_head_dim(p, D, q.dtype, sm_scale, None, None, spec, Sq, Sk) == D for p in passes])
 
 
-def forward(q, k, v, spec: MaskSpec, sm_scale, save_residuals):
-    """(o, l, m), or o, of a call that `takes` accepts."""
-    templates, maps = _plan((0, q.shape, k.shape, q.dtype, q.device, spec, sm_scale), q, k, spec, sm_scale, _lib.FwdParamsC, (_lib.PASS_FWD,))
+def forward(q, k, v, spec: MaskSpec, sm_scale, save_residuals, with_work=False):
+    """(o, l, m), or o, of a call that `takes` accepts.  ``with_work``: through flexattn_fwd_work, which cuts the lists of small
+    grids (flex_attention's own forward)."""
+    plan, maps = _plan((0, q.shape, k.shape, q.dtype, q.device, spec, sm_scale), q, k, spec, sm_scale, _lib.FwdParamsC, (_lib.PASS_FWD,))
     qp, kp, vp = q.data_ptr(), k.data_ptr(), v.data_ptr()
     if (qp | kp | vp) % 16:
-        return forward(aligned(q), aligned(k), aligned(v), spec, sm_scale, save_residuals)
+        return forward(aligned(q), aligned(k), aligned(v), spec, sm_scale, save_residuals, with_work)
     o = torch.empty_like(q)
     l = m = None
     if save_residuals:
         l = torch.empty(q.shape[:3], dtype=torch.float32, device=q.device)
         m = torch.empty_like(l)
-    p = _lib.FwdParamsC.from_buffer_copy(templates[0])
+    p = _lib.FwdParamsC.from_buffer_copy(plan.templates[0])
     _FWD_POINTERS.pack_into(p, 0, qp, kp, vp, o.data_ptr(),
                             l.data_ptr() if save_residuals else 0, m.data_ptr() if save_residuals else 0)
     lib = _lib.load()
     with on_device(q.device):
-        _lib.check(lib.flexattn_fwd(C.byref(p), stream_of(q)), lib)
+        if with_work:
+            if plan.work_bytes is None:
+                plan.work_bytes = lib.flexattn_fwd_work_bytes(C.byref(p))
+            need = plan.work_bytes
+            work = torch.empty(need, dtype=torch.uint8, device=q.device) if need > 0 else None
+            _lib.check(lib.flexattn_fwd_work(C.byref(p), work.data_ptr() if need > 0 else None, need, stream_of(q)), lib)
+        else:
+            _lib.check(lib.flexattn_fwd(C.byref(p), stream_of(q)), lib)
     return (o, l, m) if save_residuals else o
 
 
 def backward(q, k, v, l, m, o, do, spec: MaskSpec, sm_scale):
     """(dq, dk, dv) of a call that `takes` accepts: delta, the dq and the dk/dv pass (flexattn_bwd)."""
-    templates, maps = _plan((1, q.shape, k.shape, q.dtype, q.device, spec, sm_scale), q, k, spec, sm_scale, _lib.BwdParamsC,
+    plan, maps = _plan((1, q.shape, k.shape, q.dtype, q.device, spec, sm_scale), q, k, spec, sm_scale, _lib.BwdParamsC,
                             (_lib.PASS_DQ, _lib.PASS_DKV))
     head = (q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(), l.data_ptr(), m.data_ptr())
     op = o.data_ptr()
     if (head[0] | head[1] | head[2] | head[3] | op) % 16:
         return backward(aligned(q), aligned(k), aligned(v), l, m, aligned(o), aligned(do), spec, sm_scale)
     dq, dk, dv, delta = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v), torch.empty_like(l)
-    pq = _lib.BwdParamsC.from_buffer_copy(templates[0])
-    pkv = _lib.BwdParamsC.from_buffer_copy(templates[1])
+    pq = _lib.BwdParamsC.from_buffer_copy(plan.templates[0])
+    pkv = _lib.BwdParamsC.from_buffer_copy(plan.templates[1])
     d = delta.data_ptr()
     _BWD_POINTERS.pack_into(pq, 0, *head, 0, dq.data_ptr(), 0, 0)
     _BWD_POINTERS.pack_into(pkv, 0, *head, d, 0, dk.data_ptr(), dv.data_ptr())

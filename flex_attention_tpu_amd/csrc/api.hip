@@ -304,7 +304,23 @@ static int delta_first(BwdArgs* a, int D, int dtype, hipStream_t s) {
   return rc;
 }
 
-static int fwd_with_map(const flexattn_fwd_params* p, const flexattn_block_map& map, hipStream_t s) {
+// What the kernels see of a checked forward request.
+static FwdArgs fwd_args(const flexattn_fwd_params* p, const flexattn_block_map& map) {
+  const int Sq = p->Sq - (p->pad & 0xffff), Sk = p->Sk - (p->pad >> 16);   // the tensors' lengths
+  FwdArgs a;
+  a.q = p->q; a.k = p->k; a.v = p->v; a.o = p->o; a.l = p->l; a.m = p->m;
+  a.B = p->B; a.Hq = p->Hq; a.Hkv = p->Hkv; a.Sq = Sq; a.Sk = Sk;
+  a.sm_scale = p->sm_scale;
+  a.flags = p->flags;
+  a.score = to_args(p->score, p->ab, Sk);
+  a.mask = to_args(p->mask);
+  a.map = row_view(map);
+  return a;
+}
+
+// (with_work: the caller has brought flexattn_fwd_work_bytes bytes, or there is nothing to bring)
+static int fwd_with_map(const flexattn_fwd_params* p, const flexattn_block_map& map, hipStream_t s, bool with_work = false,
+                        void* work = nullptr) {
   if (!p->q || !p->k || !p->v || !p->o) return set_error(FLEXATTN_EINVAL, "q, k, v or o is NULL");
   if ((p->l == nullptr) != (p->m == nullptr)) return set_error(FLEXATTN_EINVAL, "l and m must both be given or both NULL");
   const int Sq = p->Sq - (p->pad & 0xffff), Sk = p->Sk - (p->pad >> 16);   // the tensors' lengths
@@ -317,14 +333,8 @@ static int fwd_with_map(const flexattn_fwd_params* p, const flexattn_block_map& 
   if ((rc = check_mask(p->mask)) != FLEXATTN_OK) return rc;
   if ((rc = check_doc_batches(p->mask, p->B)) != FLEXATTN_OK) return rc;
   if ((rc = check_bias(p->ab, p->B, p->Hq, Sq, Sk)) != FLEXATTN_OK) return rc;
-  FwdArgs a;
-  a.q = p->q; a.k = p->k; a.v = p->v; a.o = p->o; a.l = p->l; a.m = p->m;
-  a.B = p->B; a.Hq = p->Hq; a.Hkv = p->Hkv; a.Sq = Sq; a.Sk = Sk;
-  a.sm_scale = p->sm_scale;
-  a.flags = p->flags;
-  a.score = to_args(p->score, p->ab, Sk);
-  a.mask = to_args(p->mask);
-  a.map = row_view(map);
+  const FwdArgs a = fwd_args(p, map);
+  if (with_work && p->dtype == FLEXATTN_BF16) return fwd_bf16_with_work(a, p->D, work, s);
   if (p->dtype == FLEXATTN_BF16) return p->D == 256 ? fwd_bf16_d256(a, s) : p->D == 64 ? fwd_bf16_d64(a, s) : fwd_bf16_d128(a, s);
   return (a.flags & FLEXATTN_FLAG_COMPILED_LOOP) ? fwd_f32(a, p->D, s) : fwd_f32_mfma(a, p->D, s);
 }
@@ -432,6 +442,20 @@ int flexattn_build_ds_index(const flexattn_block_map* map, int32_t* col, int32_t
 int flexattn_fwd(const flexattn_fwd_params* p, void* stream) {
   if (p == nullptr) return set_error(FLEXATTN_EINVAL, "params is NULL");
   return fwd_with_map(p, p->map, static_cast<hipStream_t>(stream));
+}
+
+int64_t flexattn_fwd_work_bytes(const flexattn_fwd_params* p) {
+  if (p == nullptr || p->dtype != FLEXATTN_BF16 || p->B <= 0 || p->Hq <= 0 || p->map.nq <= 0 || p->map.nk <= 0 || p->Sk <= (p->pad >> 16)) return 0;
+  return fwd_bf16_work_bytes(fwd_args(p, p->map), p->D);
+}
+
+int flexattn_fwd_work(const flexattn_fwd_params* p, void* work, int64_t work_bytes, void* stream) {
+  if (p == nullptr) return set_error(FLEXATTN_EINVAL, "params is NULL");
+  const int64_t need = flexattn_fwd_work_bytes(p);
+  if (need > 0 && (work == nullptr || work_bytes < need))
+    return set_error(FLEXATTN_EINVAL, "work holds %lld bytes, the request needs %lld", (long long)(work ? work_bytes : 0), (long long)need);
+  if (reinterpret_cast<uintptr_t>(work) & 15) return set_error(FLEXATTN_EINVAL, "work's address is no multiple of 16 bytes");
+  return fwd_with_map(p, p->map, static_cast<hipStream_t>(stream), true, need > 0 ? work : nullptr);
 }
 
 int flexattn_fwd_noalloc(const flexattn_fwd_params* p, void* stream) {

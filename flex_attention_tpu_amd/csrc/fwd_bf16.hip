@@ -66,8 +66,11 @@ struct FwdPinned {
 // Head dimension 128 NP: a row of K or V is NP panels of 128 columns, each panel of a 64-row tile one LDS tile
 // (tile_io.hpp) at [buffer][panel]; the contraction of S runs over the panels, O^T has four accumulators per panel.
 // AB: the call may have an additive bias (false: splits_bias() kinds without one).
-template <int SCORE, int NP, bool AB>
-__global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs a) {
+// SPLIT: each q tile's list is cut into `parts` runs of equal length, a work-group each; what a work-group leaves is its float32
+// sums, relative to its own maximum, which fwd_merge_kernel puts together.  For grids that leave CUs idle: a tile's list is a serial
+// chain (see fwd_split_parts).
+template <int SCORE, int NP, bool AB, bool SPLIT>
+__global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs a, float* work, int parts) {
   using namespace fwd_cfg;
   constexpr int D = 128 * NP;
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
@@ -76,8 +79,9 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
 
   const int nQ = a.map.nq;
   const int nK = a.map.nk;
-  const int n_wg = a.B * a.Hq * nQ;
-  const int wg = xcd_remap(blockIdx.x, n_wg);
+  const int n_wg = a.B * a.Hq * nQ * (SPLIT ? parts : 1);
+  const int wg_all = xcd_remap(blockIdx.x, n_wg);
+  const int wg = SPLIT ? wg_all / parts : wg_all, part = SPLIT ? wg_all - wg * parts : 0;
   int bh, qb;
   block_item(wg, a.B, a.Hq, nQ, SCORE == kScoreBiasOnly && a.score.ab_sb_rows == 0, bh, qb);
   qb = nQ - 1 - qb;  // longest rows first under causal masks
@@ -110,8 +114,10 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
   for (int ks = 0; ks < 8 * NP; ++ks)
     qreg[ks] = *reinterpret_cast<const bf16x8*>(Qg + (size_t)q_local * D + ks * 16 + hh * 8);
 
-  const int n_tiles = a.map.cnt[qb];
-  const int* tile_idx = a.map.idx + (size_t)qb * nK;
+  const int n_list = a.map.cnt[qb];
+  const int first = SPLIT ? n_list * part / parts : 0;   // (at most 2^12 tiles by 2^4 parts)
+  const int n_tiles = (SPLIT ? n_list * (part + 1) / parts : n_list) - first;
+  const int* tile_idx = a.map.idx + (size_t)qb * nK + first;
   const uint8_t* tile_state = a.map.state + (size_t)qb * nK;
 
   int doc_i = 0;
@@ -367,6 +373,22 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
   const float l_tot = half_sum(l_run);
   const float inv = (l_tot > 0.f) ? 1.0f / l_tot : 0.f;
   if (q_idx < qb * BM) return;   // (a row of the q tile before)
+  if constexpr (SPLIT) {
+    const size_t rows = (size_t)a.B * a.Hq * a.Sq, r = (size_t)bh * a.Sq + q_idx;
+    float* out = work + ((size_t)part * rows + r) * D;
+#pragma unroll
+    for (int db = 0; db < 4 * NP; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4*>(out + 32 * db + 8 * g + 4 * hh) =
+            f32x4{o_acc[db][4 * g], o_acc[db][4 * g + 1], o_acc[db][4 * g + 2], o_acc[db][4 * g + 3]};
+    if (hh == 0) {   // (behind the parts' rows: (maximum in the log2 domain, sum) per part and row)
+      float* ml = work + (size_t)parts * rows * D + ((size_t)part * rows + r) * 2;
+      ml[0] = SCORE == FLEXATTN_SCORE_NONE ? m_run * sm.c2 : m_run;
+      ml[1] = l_tot;
+    }
+    return;
+  }
 #pragma unroll
   for (int db = 0; db < 4 * NP; ++db) {
 #pragma unroll
@@ -384,18 +406,55 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
   }
 }
 
-template <int SCORE, int NP = 1, bool AB = true>
-static int launch_fwd(const FwdArgs& a, hipStream_t stream) {
+// The parts of a split list into one row: D / 4 threads per row.
+template <int D>
+__global__ __launch_bounds__(256) void fwd_merge_kernel(const float* work, int parts, long long rows, bf16_t* o, float* l, float* m) {
+  constexpr int TPR = D / 4;
+  const long long r = (long long)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+  if (r >= rows) return;
+  const int c = 4 * (threadIdx.x % TPR);
+  const float* ml = work + (size_t)parts * rows * D;
+  float m_all = kNegInf;
+  for (int p = 0; p < parts; ++p) m_all = fmaxf(m_all, ml[((size_t)p * rows + r) * 2]);
+  const float m_safe = m_all == kNegInf ? 0.f : m_all;
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+  float l_all = 0.f;
+  for (int p = 0; p < parts; ++p) {
+    const float f = fast_exp2(ml[((size_t)p * rows + r) * 2] - m_safe);   // (0 for a part that kept nothing)
+    l_all = __builtin_fmaf(ml[((size_t)p * rows + r) * 2 + 1], f, l_all);
+    const f32x4 x = *reinterpret_cast<const f32x4*>(work + ((size_t)p * rows + r) * D + c);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] = __builtin_fmaf(x[i], f, sum[i]);
+  }
+  const float inv = l_all > 0.f ? 1.0f / l_all : 0.f;
+  const bf16x2 lo = pack_bf16(sum[0] * inv, sum[1] * inv), hi = pack_bf16(sum[2] * inv, sum[3] * inv);
+  *reinterpret_cast<bf16x4*>(o + (size_t)r * D + c) = bf16x4{lo[0], lo[1], hi[0], hi[1]};
+  if (l != nullptr && c == 0) {
+    l[r] = l_all;
+    m[r] = m_all * kLn2;   // natural units
+  }
+}
+
+template <int SCORE, int NP = 1, bool AB = true, bool SPLIT = false>
+static int launch_fwd(const FwdArgs& a, hipStream_t stream, float* work = nullptr, int parts = 1) {
   using namespace fwd_cfg;
   if constexpr (AB && splits_bias(SCORE))
-    if (a.score.ab == nullptr) return launch_fwd<SCORE, NP, false>(a, stream);
-  auto kern = fwd_bf16_kernel<SCORE, NP, AB>;
+    if (a.score.ab == nullptr) return launch_fwd<SCORE, NP, false, SPLIT>(a, stream, work, parts);
+  if constexpr (!SPLIT && SCORE == FLEXATTN_SCORE_NONE)
+    if (parts > 1) return launch_fwd<SCORE, NP, AB, true>(a, stream, work, parts);
+  auto kern = fwd_bf16_kernel<SCORE, NP, AB, SPLIT>;
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, NP * LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(fwd): %s", hipGetErrorString(attr));
-  const int n_wg = a.B * a.Hq * a.map.nq;
-  hipLaunchKernelGGL(kern, dim3(n_wg), dim3(256), NP * LDS_BYTES, stream, a);
-  return check_launch("flexattn_fwd bf16");
+  const int n_wg = a.B * a.Hq * a.map.nq * parts;
+  hipLaunchKernelGGL(kern, dim3(n_wg), dim3(256), NP * LDS_BYTES, stream, a, work, parts);
+  const int rc = check_launch("flexattn_fwd bf16");
+  if (!SPLIT || rc != FLEXATTN_OK) return rc;
+  constexpr int kRows = 256 / (128 * NP / 4);
+  const long long rows = (long long)a.B * a.Hq * a.Sq;
+  hipLaunchKernelGGL((fwd_merge_kernel<128 * NP>), dim3((unsigned)((rows + kRows - 1) / kRows)), dim3(256), 0, stream, work, parts, rows,
+                     static_cast<bf16_t*>(a.o), a.l, a.m);
+  return check_launch("flexattn_fwd merge");
 }
 
 #ifndef FLEXATTN_CUSTOM_ONLY
@@ -954,6 +1013,36 @@ static int launch_fwd_plain(const FwdArgs& a, hipStream_t stream) {
 }
 
 #endif  // FLEXATTN_CUSTOM_ONLY
+
+// Parts that the lists of a plain call are cut into where its q tiles leave CUs idle: as many as fill the CUs' places for
+// work-groups (two at head dimension 128, one at 256), of at least four kv tiles each.  A part costs its float32 sums
+// written and read; B=1, H=8, S=1024, D=128, causal, forward: 34.3 -> 26.1 us
+// with the other kernel, B=2, H=1, S=5888 118.7 -> 54.2, B=1, H=1, S=16384 299 -> 137.
+static int split_parts(long long tiles, int nk, int D) {
+  const long long fill = (D == 128 && nk >= 64 ? 512 : 256) / tiles;
+  const int most = nk / 8 < 16 ? nk / 8 : 16;
+  return fill < 2 || most < 2 ? 1 : fill < most ? (int)fill : most;
+}
+static bool small_plain(const FwdArgs& a, int D) {
+  return (D == 128 || D == 256) && a.score.kind == FLEXATTN_SCORE_NONE && a.score.ab == nullptr && a.flags == 0;
+}
+int64_t fwd_bf16_work_bytes(const FwdArgs& a, int D) {
+  if (!small_plain(a, D)) return 0;
+  const int parts = split_parts((long long)a.B * a.Hq * a.map.nq, a.map.nk, D);
+  return parts < 2 ? 0 : (int64_t)parts * a.B * a.Hq * a.Sq * (D + 2) * 4;
+}
+// The forward of a caller that has brought such memory.  Up to 256 q tiles the compiled loop, two work-groups of 128 rows a CU,
+// is the faster kernel of head dimension 128 in one part too: the stream's work-groups take 256 rows (B=1, S=1024, causal, H=8
+// 34.5 against 28.0 us, H=32 39.2 / 30.3, H=64, 512 tiles, 41.3 / 45.3).
+int fwd_bf16_with_work(const FwdArgs& a, int D, void* work, hipStream_t stream) {
+  const long long tiles = (long long)a.B * a.Hq * a.map.nq;
+  if (small_plain(a, D) && tiles <= 256) {
+    const int parts = work != nullptr ? split_parts(tiles, a.map.nk, D) : 1;
+    return D == 128 ? launch_fwd<FLEXATTN_SCORE_NONE>(a, stream, static_cast<float*>(work), parts)
+                    : launch_fwd<FLEXATTN_SCORE_NONE, 2>(a, stream, static_cast<float*>(work), parts);
+  }
+  return D == 256 ? fwd_bf16_d256(a, stream) : D == 64 ? fwd_bf16_d64(a, stream) : fwd_bf16_d128(a, stream);
+}
 
 int fwd_bf16_d128(const FwdArgs& a, hipStream_t stream) {
 #ifdef FLEXATTN_CUSTOM_ONLY

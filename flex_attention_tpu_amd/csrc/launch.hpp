@@ -18,6 +18,9 @@ int fwd_bf16_d64(const FwdArgs& a, hipStream_t stream);    // (same tiles as hea
 bool fwd_bf16_d64_ok(float sm_scale, int nk);
 int fwd_bf16_d256(const FwdArgs& a, hipStream_t stream);   // (same tiles as head dim 128)
 void fwd_bf16_d128_tile(int* bq, int* bk);
+// the forward with scratch memory for split lists (0 bytes: nothing to split)
+int64_t fwd_bf16_work_bytes(const FwdArgs& a, int D);
+int fwd_bf16_with_work(const FwdArgs& a, int D, void* work, hipStream_t stream);
 // few query rows against long keys, plain scores, no mask (head dim 64 or 128)
 bool fwd_decode_ok(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D);
 int64_t fwd_decode_bytes(int B, int Hq, int Hkv, int Sq, int Sk, int D);

@@ -107,7 +107,7 @@ class _FlexAttention(torch.autograd.Function):
         score_fn, mask_fn, block_mask_fn, segment_ids, causal, sm_scale, block_q, block_k = opts
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
         o, l, m = _flex_attention_impl(q, k, v, ab, segment_ids, True, causal, sm_scale, 1, block_q, block_k, block_k,
-                                       False, block_mask_fn, mask_fn, score_fn)
+                                       False, block_mask_fn, mask_fn, score_fn, _with_work=q.shape[-1] == 256)
         ctx.save_for_backward(q, k, v, o, l, m, *([ab] if ab is not None else []))
         ctx.opts = opts
         return o
@@ -188,7 +188,8 @@ def flex_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, score_fn: 
             check_blocks(Sq, Sk, block_q=block_q, block_k_major=block_k, block_k=block_k)
             return (_plans.takes(q, k, spec, sm_scale, _lib.PASS_FWD, _lib.PASS_DQ, _lib.PASS_DKV) and
                     not (q.dtype is torch.bfloat16 and _hands_ds_over(q, k, None, None, sm_scale, None, mask_fn, block_mask_fn, False)))
-        o = _plans.attend(q, k, v, spec, float(sm_scale), block_q, block_k, prepared)
+        # (what _plans.takes never takes goes on at once: those calls pay for no further look)
+        o = _plans.attend(q, k, v, spec, float(sm_scale), block_q, block_k, prepared) if spec.doc_ids is None and spec.custom is None else None
         if o is not None:
             return o
     opts = (score_fn, mask_fn, block_mask_fn, segment_ids, bool(causal), float(sm_scale), int(block_q), int(block_k))

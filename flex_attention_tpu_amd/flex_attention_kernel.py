@@ -56,7 +56,7 @@ def _decode(q, k, v, mask_fn, block_mask_fn, save_residuals, sm_scale):
 
 
 def _flex_attention_impl(q, k, v, ab, segment_ids, save_residuals, causal, sm_scale, block_b, block_q,
-                         block_k_major, block_k, debug, block_mask_fn, mask_fn, score_fn, *, compiled_loop=False):
+                         block_k_major, block_k, debug, block_mask_fn, mask_fn, score_fn, *, compiled_loop=False, _with_work=False):
     """Returns ``o`` (q.dtype) or ``(o, l, m)`` with float32 ``l, m`` of shape [B, H, Sq].
 
     Semantics (flex_attention_kernel.py:248-319): S = score_mod(sm_scale * q k^T) + ab; masked
@@ -80,7 +80,7 @@ def _flex_attention_impl(q, k, v, ab, segment_ids, save_residuals, causal, sm_sc
         if causal:
             spec = spec.combine(_CAUSAL)
         if _plans.takes(q, k, spec, sm_scale, _lib.PASS_FWD):
-            return _plans.forward(q, k, v, spec, float(sm_scale), save_residuals)
+            return _plans.forward(q, k, v, spec, float(sm_scale), save_residuals, _with_work)
     # (lengths below one tile: the tensors are zero-padded to it, a document id of their own drops the padded keys
     # and the padded query rows are cut off again)
     Sq_p, Sk_p = padded_len(Sq), padded_len(Sk)

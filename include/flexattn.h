@@ -239,6 +239,13 @@ int flexattn_build_block_mask_ragged(const flexattn_mask_spec* mask, int32_t Sq,
 /* Forward.  Replaces the pallas_call in _flex_attention_impl (flex_attention_kernel.py:173-187). */
 int flexattn_fwd(const flexattn_fwd_params* p, void* stream);
 
+/* The same for a caller that brings scratch device memory: `work`, 16-byte aligned, of flexattn_fwd_work_bytes bytes, which may be
+ * 0.  Where the q tiles of a plain call (bf16, head dimension 128 or 256, flags 0) leave CUs idle, their lists are cut into parts
+ * whose float32 sums lie there and a second launch puts together; such a call may also run another kernel than flexattn_fwd's
+ * (results agree to the rounding of their sums).  The bytes depend on shapes, dtype, score, bias and flags. */
+int64_t flexattn_fwd_work_bytes(const flexattn_fwd_params* p);
+int flexattn_fwd_work(const flexattn_fwd_params* p, void* work, int64_t work_bytes, void* stream);
+
 /* Forward without any allocation.  No counterpart in the reference; for callers that cannot allocate
  * device memory around the call: code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc.  Same request and same results as flexattn_fwd, except that p->map is ignored: the block map of
