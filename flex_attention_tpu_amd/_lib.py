@@ -228,7 +228,7 @@ def load_host():
         from . import _host as mod
         lib = load()
         mod.bind(*(C.cast(getattr(lib, "flexattn_" + n), C.c_void_p).value
-                   for n in ("fwd_work", "fwd_work_bytes", "bwd", "bwd_dq", "bwd_dkv", "bwd_delta", "last_error_string")))
+                   for n in ("fwd", "fwd_work", "fwd_work_bytes", "bwd", "bwd_dq", "bwd_dkv", "bwd_delta", "last_error_string")))
         _host = mod
     return _host
 

@@ -114,8 +114,8 @@ def takes(q, k, spec: MaskSpec, sm_scale, *passes: int) -> bool:
 
 
 def forward(q, k, v, spec: MaskSpec, sm_scale, save_residuals, with_work=False):
-    """(o, l, m), or o, of a call that `takes` accepts.  ``with_work``: through flexattn_fwd_work, which cuts the lists of small
-    grids (flex_attention's own forward)."""
+    """(o, l, m), or o, of a call that `takes` accepts.  ``with_work``: through flexattn_fwd_work where that cuts
+    the lists of a small grid (flex_attention's own forward)."""
     plan, maps = _plan((0, q.shape, k.shape, q.dtype, q.device, spec, sm_scale), q, k, spec, sm_scale, _lib.FwdParamsC, (_lib.PASS_FWD,))
     qp, kp, vp = q.data_ptr(), k.data_ptr(), v.data_ptr()
     if (qp | kp | vp) % 16:
@@ -130,12 +130,11 @@ def forward(q, k, v, spec: MaskSpec, sm_scale, save_residuals, with_work=False):
                             l.data_ptr() if save_residuals else 0, m.data_ptr() if save_residuals else 0)
     lib = _lib.load()
     with on_device(q.device):
-        if with_work:
-            if plan.work_bytes is None:
-                plan.work_bytes = lib.flexattn_fwd_work_bytes(C.byref(p))
-            need = plan.work_bytes
-            work = torch.empty(need, dtype=torch.uint8, device=q.device) if need > 0 else None
-            _lib.check(lib.flexattn_fwd_work(C.byref(p), work.data_ptr() if need > 0 else None, need, stream_of(q)), lib)
+        if with_work and plan.work_bytes is None:
+            plan.work_bytes = lib.flexattn_fwd_work_bytes(C.byref(p))
+        if with_work and plan.work_bytes > 0:
+            work = torch.empty(plan.work_bytes, dtype=torch.uint8, device=q.device)
+            _lib.check(lib.flexattn_fwd_work(C.byref(p), work.data_ptr(), plan.work_bytes, stream_of(q)), lib)
         else:
             _lib.check(lib.flexattn_fwd(C.byref(p), stream_of(q)), lib)
     return (o, l, m) if save_residuals else o

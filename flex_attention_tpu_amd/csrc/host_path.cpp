@@ -15,7 +15,8 @@
 namespace {
 
 struct Entries {   // of libflexattn.so, which Python has loaded
-  decltype(&flexattn_fwd_work) fwd;
+  decltype(&flexattn_fwd) fwd;
+  decltype(&flexattn_fwd_work) fwd_work;
   decltype(&flexattn_fwd_work_bytes) fwd_bytes;
   decltype(&flexattn_bwd) bwd;
   decltype(&flexattn_bwd_dq) bwd_dq;
@@ -82,9 +83,13 @@ at::Tensor forward_pass(const Call& call, const at::Tensor& q_, const at::Tensor
     p.l = l->data_ptr<float>();
     p.m = m->data_ptr<float>();
   }
-  const int64_t bytes = lib.fwd_bytes(&p);   // (small grids: sums of the parts that lists are cut into; freed in the stream's order)
-  const at::Tensor work = bytes > 0 ? at::empty({bytes}, q.options().dtype(at::kByte)) : at::Tensor();
-  check(lib.fwd(&p, bytes > 0 ? work.data_ptr() : nullptr, bytes, stream_of(q)));
+  const int64_t bytes = lib.fwd_bytes(&p);
+  if (bytes > 0) {   // (a small grid: sums of the parts that lists are cut into; freed in the stream's order)
+    const at::Tensor work = at::empty({bytes}, q.options().dtype(at::kByte));
+    check(lib.fwd_work(&p, work.data_ptr(), bytes, stream_of(q)));
+  } else {
+    check(lib.fwd(&p, stream_of(q)));
+  }
   return o;
 }
 
@@ -183,8 +188,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
         Plan{block_of<flexattn_fwd_params>(fwd), block_of<flexattn_bwd_params>(dq), block_of<flexattn_bwd_params>(dkv)});
   }));
   mod.def("attend", &attend, py::call_guard<py::gil_scoped_release>());
-  mod.def("bind", [](uintptr_t fwd, uintptr_t fwd_bytes, uintptr_t bwd, uintptr_t bwd_dq, uintptr_t bwd_dkv, uintptr_t bwd_delta, uintptr_t error) {
+  mod.def("bind", [](uintptr_t fwd, uintptr_t fwd_work, uintptr_t fwd_bytes, uintptr_t bwd, uintptr_t bwd_dq, uintptr_t bwd_dkv, uintptr_t bwd_delta, uintptr_t error) {
     lib.fwd = reinterpret_cast<decltype(lib.fwd)>(fwd);
+    lib.fwd_work = reinterpret_cast<decltype(lib.fwd_work)>(fwd_work);
     lib.fwd_bytes = reinterpret_cast<decltype(lib.fwd_bytes)>(fwd_bytes);
     lib.bwd = reinterpret_cast<decltype(lib.bwd)>(bwd);
     lib.bwd_dq = reinterpret_cast<decltype(lib.bwd_dq)>(bwd_dq);

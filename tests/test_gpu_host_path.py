@@ -1,5 +1,5 @@
 """The prepared calls' autograd function in C++ against the Python one that every other call takes: the same kernels on the same
-arguments, so the same bits (bf16 at head dimension 128: the forward of a small grid takes another kernel and cuts its lists, see
+arguments, so the same bits (bf16 at head dimension 128: the forward of a small grid may take another kernel and cut its lists, see
 flexattn_fwd_work; its results agree within twice the bounds of helpers.assert_close), for each set of wanted gradients, under the hooks
 and modes that watch an autograd function, and where the call is handed to the Python one."""
 import math
