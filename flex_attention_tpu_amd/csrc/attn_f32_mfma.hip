@@ -7,7 +7,10 @@
 // their partial results through LDS at the end.  NW = 4 (one wave per SIMD) in general; head dim 64 on a grid
 // that leaves CUs idle takes NW = 8: the two waves of a SIMD hide each other's operand loads, which nothing
 // prefetches (208 registers per lane at head dim 64 allow two waves; head dim 128 needs 304).  Operands go from global memory (L2-resident at these sizes) straight
-// into MFMA operand registers: no LDS staging, no barriers in the main loop.
+// into MFMA operand registers: no LDS staging, no barriers in the main loop.  What a unit may or may not have (a bias, a mask, the
+// bias's gradient) is tested once per unit: a test at each of a lane's 16 elements cuts the unit into as many pieces for the
+// scheduler, and the row values that an element loads are then waited for one by one (B=1, H=8, S=2048, D=128, per launch:
+// forward 651 -> 214 us, dq 525 -> 447, dk/dv 809 -> 390; B=2, H=16, S=2048, D=64, causal: 548 -> 329, 482 -> 450, 900 -> 620).
 //
 // MFMA operand layout (32x32x2 fp32): lane L supplies A[L % 32][L / 32] and B[L / 32][L % 32] (one float
 // each) and holds C[8 (i / 4) + 4 (L / 32) + i % 4][L % 32] in accumulator element i.  A contraction over
@@ -121,16 +124,21 @@ __global__ __launch_bounds__(64 * NW) void fwd_f32_mfma_kernel(FwdArgs a) {
       float x[16];
       float m_blk = kNegInf;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int j = j0 + acc_row(i, half);
-        float v = sm.to_log2(s[i], q_idx, j) + sm.bias2(q_idx, j);
-        if (partial) {
-          const int doc_j = has_doc ? mk.doc_k[j] : 0;
-          if (!keep_elem(mk, q_idx, j, doc_i, doc_j) || j < j_first) v = kNegInf;
-        }
-        x[i] = v;
-        m_blk = fmaxf(m_blk, v);
+      for (int i = 0; i < 16; ++i) x[i] = sm.to_log2(s[i], q_idx, j0 + acc_row(i, half));
+      if (sm.has_bias()) {   // (tests per unit, not per element: see the file's head)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[i] += sm.bias2(q_idx, j0 + acc_row(i, half));
       }
+      if (partial) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int j = j0 + acc_row(i, half);
+          const int doc_j = has_doc ? mk.doc_k[j] : 0;
+          if (!keep_elem(mk, q_idx, j, doc_i, doc_j) || j < j_first) x[i] = kNegInf;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) m_blk = fmaxf(m_blk, x[i]);
       m_blk = half_max(m_blk);
       const float m_new = fmaxf(m_run, m_blk);
       const float m_safe = (m_new == kNegInf) ? 0.f : m_new;
@@ -268,21 +276,41 @@ __global__ __launch_bounds__(64 * NW) void bwd_dq_f32_mfma_kernel(BwdArgs a) {
       const int j0 = min(j_first, a.Sk - 32);
       const f32x16 s = dot_block<D>(Kg + (size_t)(j0 + l32) * D, qf, half);
       const f32x16 dp = dot_block<D>(Vg + (size_t)(j0 + l32) * D, dof, half);
-      float ds[16];
+      if (D != 64) __builtin_amdgcn_sched_barrier(0);
+      float ds[16], x[16], gl[16];
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const int j = j0 + acc_row(i, half);
-        const float tv = sm.to_log2(s[i], q_idx, j);   // (the score function's value: what its derivative is taken from)
-        float x = tv + sm.bias2(q_idx, j);
-        if (partial) {
-          const int doc_j = has_doc ? mk.doc_k[j] : 0;
-          if (!keep_elem(mk, q_idx, j, doc_i, doc_j) || j < j_first) x = kNegInf;
-        }
-        const float pe = exp2f(x - lse2);
-        const float gl = (x == kNegInf) ? 0.f : pe * (dp[i] - dl);   // gradient with respect to the logit (the bias's share)
-        if (a.dab != nullptr && j >= j_first && q_idx >= ob * BO) a.dab[row * (size_t)a.Sk + j] = gl;
-        ds[i] = (x == kNegInf) ? 0.f : gl * sm.dfactor(tv, s[i], q_idx, j);
+        ds[i] = sm.to_log2(s[i], q_idx, j0 + acc_row(i, half));   // (the score function's value: what its derivative is taken from)
+        x[i] = ds[i];
       }
+      if (sm.has_bias()) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[i] += sm.bias2(q_idx, j0 + acc_row(i, half));
+      }
+      if (partial) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int j = j0 + acc_row(i, half);
+          const int doc_j = has_doc ? mk.doc_k[j] : 0;
+          if (!keep_elem(mk, q_idx, j, doc_i, doc_j) || j < j_first) x[i] = kNegInf;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float pe = exp2f(x[i] - lse2);
+        gl[i] = (x[i] == kNegInf) ? 0.f : pe * (dp[i] - dl);   // gradient with respect to the logit (the bias's share)
+        ds[i] = (x[i] == kNegInf) ? 0.f : gl[i] * sm.dfactor(ds[i], s[i], q_idx, j0 + acc_row(i, half));
+      }
+      if (a.dab != nullptr) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int j = j0 + acc_row(i, half);
+          if (j >= j_first && q_idx >= ob * BO) a.dab[row * (size_t)a.Sk + j] = gl[i];
+        }
+      }
+      // (head dimension 128: the operands of the sum are not fetched over the element-wise work; B=1, H=8, S=2048: 487 -> 447 us,
+      // at 64 442 -> 486)
+      if (D != 64) __builtin_amdgcn_sched_barrier(0);
       accumulate_rows<D>(acc, Kg + (size_t)j0 * D, ds, l32, half);
     }
   }
@@ -338,23 +366,53 @@ __global__ __launch_bounds__(64 * NW) void bwd_dkv_f32_mfma_kernel(BwdArgs a) {
     const bool partial = state[(size_t)qb * a.map.nk + kb] == 1 || i_first + 32 > a.Sq;
     if (i_first < a.Sq) {
       const int i0 = min(i_first, a.Sq - 32);
+      // (the unit's row values: on their way while the products run; at head dimension 64 behind the products, for the 48
+      // registers would cost a wavefront per SIMD: B=2, H=16, S=2048, causal, 1043 us in front, 965 behind)
+      f32x4 l4[4], m4[4], d4[4];
+      auto load_row_values = [&]() {
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const size_t r = head_row + i0 + 8 * g4 + 4 * half;
+          l4[g4] = *reinterpret_cast<const f32x4_a4*>(a.l + r);
+          m4[g4] = *reinterpret_cast<const f32x4_a4*>(a.m + r);
+          d4[g4] = *reinterpret_cast<const f32x4_a4*>(a.delta + r);
+        }
+      };
+      if (D != 64) load_row_values();
       const f32x16 s = dot_block<D>(Qg + (size_t)(i0 + l32) * D, kf, half);
       const f32x16 dp = dot_block<D>(dOg + (size_t)(i0 + l32) * D, vf, half);
-      float pv[16], ds[16];
+      if (D == 64) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_row_values();
+      }
+      float pv[16], ds[16], x[16];
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int i = i0 + acc_row(e, half);
-        const float tv = sm.to_log2(s[e], i, k_idx);
-        float x = tv + sm.bias2(i, k_idx);
-        if (partial) {
-          const int doc_i = has_doc ? mk.doc_q[i] : 0;
-          if (!keep_elem(mk, i, k_idx, doc_i, doc_j) || i < i_first) x = kNegInf;
-        }
-        const float pe = exp2f(x - lse2_from(a.l[head_row + i], a.m[head_row + i]));
-        pv[e] = pe;
-        ds[e] = (x == kNegInf) ? 0.f : pe * (dp[e] - a.delta[head_row + i]) * sm.dfactor(tv, s[e], i, k_idx);
+        ds[e] = sm.to_log2(s[e], i0 + acc_row(e, half), k_idx);
+        x[e] = ds[e];
       }
+      if (sm.has_bias()) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) x[e] += sm.bias2(i0 + acc_row(e, half), k_idx);
+      }
+      if (partial) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int i = i0 + acc_row(e, half);
+          const int doc_i = has_doc ? mk.doc_q[i] : 0;
+          if (!keep_elem(mk, i, k_idx, doc_i, doc_j) || i < i_first) x[e] = kNegInf;
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float pe = exp2f(x[e] - lse2_from(l4[e >> 2][e & 3], m4[e >> 2][e & 3]));
+        pv[e] = pe;
+        ds[e] = (x[e] == kNegInf) ? 0.f : pe * (dp[e] - d4[e >> 2][e & 3]) * sm.dfactor(ds[e], s[e], i0 + acc_row(e, half), k_idx);
+      }
+      // (head dimension 64: the operands of the sums are not fetched over the element-wise work, whose registers they would take: 965 -> 620)
+      if (D == 64) __builtin_amdgcn_sched_barrier(0);
       accumulate_rows<D>(dv_acc, dOg + (size_t)i0 * D, pv, l32, half);
+      if (D == 64) __builtin_amdgcn_sched_barrier(0);
       accumulate_rows<D>(dk_acc, Qg + (size_t)i0 * D, ds, l32, half);
     }
   }
