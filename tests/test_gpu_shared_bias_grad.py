@@ -15,8 +15,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("kind", ["plain", "causal", "window", "ids per entry", "bf16 bias"])
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,ab_shape", [
-    (2, 32, 32, 129, 257, 128, "1h"), (3, 22, 11, 255, 383, 64, "1h"), (2, 32, 32, 256, 256, 128, "1h"),
-    (22, 3, 1, 321, 130, 128, "b1"), (2, 2, 2, 1500, 1411, 96, "11"), (1, 2, 1, 1408, 1536, 128, "11")])
+    (2, 34, 34, 129, 257, 128, "1h"), (3, 34, 17, 255, 383, 64, "1h"), (2, 50, 50, 256, 256, 128, "1h"),
+    (34, 3, 1, 321, 130, 128, "b1"), (2, 2, 2, 1800, 1700, 96, "11"), (1, 2, 1, 1792, 1920, 128, "11")])
 def test_shared_bias_gradient(B, Hq, Hkv, Sq, Sk, D, ab_shape, kind, monkeypatch):
     import flex_attention_tpu_amd as F
     from flex_attention_tpu_amd import _lib, masks
