@@ -48,6 +48,12 @@ def _template(cls, pass_id, q, k, spec, sm_scale):
     return bytes(p), bm
 
 
+def _keep(plans, key, plan, maps):
+    """Adds a plan to its cache, unless it refers to a map that a captured call has built: only that call's graph fills it."""
+    if not any(bm.captured for bm in maps):
+        plans.put(key, plan)
+
+
 def _plan(key, q, k, spec, sm_scale, cls, passes):
     """(plan, block maps) of a combination; the caller holds the maps until its launch is out."""
     plan = _plans.get(key)
@@ -55,7 +61,7 @@ def _plan(key, q, k, spec, sm_scale, cls, passes):
     if None in maps:
         templates, maps = zip(*(_template(cls, pass_id, q, k, spec, sm_scale) for pass_id in passes))
         plan = _Plan(templates, maps)
-        _plans.put(key, plan)
+        _keep(_plans, key, plan, maps)
     for bm in maps:   # (a map built on another stream: this one waits for it)
         bm.wait_ready(q.device)
     return plan, maps
@@ -95,7 +101,7 @@ def attend(q, k, v, spec: MaskSpec, sm_scale, block_q, block_k, prepared):
                  ((_lib.FwdParamsC, _lib.PASS_FWD), (_lib.BwdParamsC, _lib.PASS_DQ), (_lib.BwdParamsC, _lib.PASS_DKV))]
         maps = [bm for _, bm in parts]
         plan = (_lib.load_host().Plan(*(t for t, _ in parts)), tuple(weakref.ref(bm) for bm in maps))
-        _attend_plans.put(key, plan)
+        _keep(_attend_plans, key, plan, maps)
     for bm in maps:   # (a map built on another stream: this one waits for it; the backward runs on this one too)
         bm.wait_ready(q.device)
     return _lib.load_host().attend(q, k, v, plan[0], maps[0].host_map(), maps[1].host_map(), maps[2].host_map())

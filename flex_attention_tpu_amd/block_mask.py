@@ -83,6 +83,7 @@ class BlockMap:
         self.q_idx = torch.empty(self.nk, self.nq, dtype=torch.int32, device=device)
         self.built_on = None   # stream the builder kernel was launched on
         self.ready = None      # event recorded behind it
+        self.captured = False  # built by a call that was being captured: filled when the graph is replayed, and for that graph alone
         self._ds_index = None  # (col, rank, pairs) of the dS exchange buffer, built at first use
         self._partial_share = None
         self._host_map = None  # the C++ side's view of the arrays
@@ -273,7 +274,8 @@ def build_block_map(spec: MaskSpec, Sq: int, Sk: int, block_q: int, block_k: int
         bm.ready = torch.cuda.Event()
         bm.ready.record(torch.cuda.current_stream(device))
     if _capturing():
-        _captured_maps.put(id(bm), bm)   # (built when the graph is replayed, not before: no map for other calls)
+        bm.captured = True   # (no map for other calls: it enters no cache, and no plan that one keeps refers to it)
+        _captured_maps.put(id(bm), bm)
     elif cache:
         _map_cache.put(key, bm)
     return bm
