@@ -148,6 +148,8 @@ EXPORTS = (
     "flexattn_build_block_mask",
     "flexattn_build_block_mask_ragged",
     "flexattn_build_ds_index",
+    "flexattn_capture_token",
+    "flexattn_captures_ended",
     "flexattn_fwd",
     "flexattn_fwd_work_bytes",
     "flexattn_fwd_work",
@@ -178,6 +180,10 @@ def _bind(lib: C.CDLL) -> C.CDLL:
         C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
     lib.flexattn_build_block_mask_ragged.argtypes = lib.flexattn_build_block_mask.argtypes
     lib.flexattn_build_ds_index.argtypes = [C.POINTER(BlockMapC), C.c_void_p, C.c_void_p, C.c_void_p]
+    lib.flexattn_capture_token.argtypes = [C.c_void_p]
+    lib.flexattn_capture_token.restype = C.c_int64
+    lib.flexattn_captures_ended.argtypes = [C.POINTER(C.c_int64), C.c_int32]
+    lib.flexattn_captures_ended.restype = C.c_int32
     lib.flexattn_fwd.argtypes = [C.POINTER(FwdParamsC), C.c_void_p]
     lib.flexattn_fwd_work_bytes.argtypes = [C.POINTER(FwdParamsC)]
     lib.flexattn_fwd_work_bytes.restype = C.c_int64

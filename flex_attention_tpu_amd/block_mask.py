@@ -32,6 +32,45 @@ def raw_stream(device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def capturing(device) -> bool:
+    """Whether the current stream of `device` is being captured into a graph."""
+    if device.index is None or device.index == torch.cuda.current_device():
+        return _capturing()
+    with torch.cuda.device(device):
+        return _capturing()
+
+
+class _Capture:
+    """What the calls of one capture read: the graph holds the addresses, whatever the caches drop.  `maps`: those it has built."""
+    __slots__ = ("things", "maps")
+
+    def __init__(self):
+        self.things, self.maps = {}, {}
+
+
+_captures = {}   # token of a capture -> _Capture; from its first call here until its graph is gone
+
+
+def captured_by(stream: int) -> _Capture:
+    """The capture that `stream` is part of."""
+    release_ended()
+    token = _lib.load().flexattn_capture_token(stream)
+    if token <= 0:
+        raise RuntimeError(f"the capture of stream {stream:#x}: {_lib.load().flexattn_last_error_string()}")
+    return _captures.setdefault(token, _Capture())
+
+
+def release_ended() -> None:
+    """Drops what graphs that are gone have read."""
+    tokens = (C.c_int64 * 16)()
+    while True:
+        n = _lib.load().flexattn_captures_ended(tokens, 16)
+        for token in tokens[:n]:
+            _captures.pop(token, None)
+        if n < 16:
+            return
+
+
 class LRU:
     """Small least-recently-used cache: holds at most ``maxsize`` entries (each may pin device
     tensors), so a training loop with a new document layout every batch does not grow it."""
@@ -104,11 +143,10 @@ class BlockMap:
     def wait_ready(self, device) -> None:
         """Makes the current stream wait for the builder kernel if that ran on another stream, and tells the
         caching allocator that the map is in use on this stream too (a map evicted from the cache must not be
-        handed out again while a kernel on this stream still walks it).  A call that is being captured keeps the map: the graph
-        holds its addresses, whatever the cache drops."""
+        handed out again while a kernel on this stream still walks it).  The graph of a call that is being captured keeps the map."""
         stream = raw_stream(device)
-        if stream != 0 and _capturing():   # (the default stream is never captured: the usual case asks nothing)
-            _captured_maps.put(id(self), self)
+        if stream != 0 and capturing(device):   # (the default stream is never captured: the usual case asks nothing)
+            captured_by(stream).things[id(self)] = self
         if self.ready is None or stream == self.built_on:
             return
         cur = torch.cuda.current_stream(device)
@@ -166,7 +204,6 @@ class BlockMap:
 MAP_CACHE_SIZE = 64
 DOC_CACHE_SIZE = 64
 _doc_cache = LRU(DOC_CACHE_SIZE)   # (DocIds, device) -> int32 device array
-_captured_maps = LRU(256)   # maps that captured calls read, by identity: as long-lived as the graphs of the last 256 of them
 _map_cache = LRU(MAP_CACHE_SIZE)   # (spec, Sq, Sk, block_q, block_k, device) -> BlockMap
 
 
@@ -262,6 +299,13 @@ def build_block_map(spec: MaskSpec, Sq: int, Sk: int, block_q: int, block_k: int
         if hit is not None:
             hit.wait_ready(device)
             return hit
+    capture = captured_by(raw_stream(device)) if capturing(device) else None
+    if capture is None:
+        release_ended()
+    elif cache and key in capture.maps:
+        hit = capture.maps[key]
+        hit.wait_ready(device)
+        return hit
     lib = _lib.load_for(score_code if spec.custom is not None else None, spec.custom)
     bm = BlockMap(spec, Sq, Sk, block_q, block_k, device)
     mc = mask_spec_c(spec, Sq, Sk, device)
@@ -273,9 +317,11 @@ def build_block_map(spec: MaskSpec, Sq: int, Sk: int, block_q: int, block_k: int
         bm.built_on = stream
         bm.ready = torch.cuda.Event()
         bm.ready.record(torch.cuda.current_stream(device))
-    if _capturing():
-        bm.captured = True   # (no map for other calls: it enters no cache, and no plan that one keeps refers to it)
-        _captured_maps.put(id(bm), bm)
+    if capture is not None:
+        bm.captured = True   # (no map for calls outside: it enters none of their caches, and no plan that one keeps refers to it)
+        capture.things[id(bm)] = bm
+        if cache:
+            capture.maps[key] = bm
     elif cache:
         _map_cache.put(key, bm)
     return bm

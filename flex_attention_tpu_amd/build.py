@@ -16,6 +16,7 @@ HOST_PATH = os.path.join(PKG_DIR, "_host.so")
 SOURCES = [
     "api.hip",
     "block_mask.hip",
+    "capture.hip",
     "delta.hip",
     "attn_f32.hip",
     "attn_f32_mfma.hip",

@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define FLEXATTN_VERSION 105 /* major*10000 + minor*100 + patch */
+#define FLEXATTN_VERSION 106 /* major*10000 + minor*100 + patch */
 
 /* status codes */
 #define FLEXATTN_OK 0
@@ -235,6 +235,13 @@ int flexattn_build_block_mask_ragged(const flexattn_mask_spec* mask, int32_t Sq,
                                      int32_t block_q, int32_t block_k, uint8_t* state,
                                      int32_t* kv_cnt, int32_t* kv_idx, int32_t* q_cnt, int32_t* q_idx,
                                      void* stream);
+
+/* Captured streams.  A graph holds the addresses of what its calls read (block maps, document ids, slopes): these have to live as
+ * long as it.  flexattn_capture_token: a positive number that names the capture `stream` is part of, the same for all its calls and
+ * never used again; 0 when the stream is not being captured.  flexattn_captures_ended: fetches up to n tokens of captures whose graph,
+ * and every executable made of it, has been destroyed, and returns how many; each is told once. */
+int64_t flexattn_capture_token(void* stream);
+int32_t flexattn_captures_ended(int64_t* tokens, int32_t n);
 
 /* Forward.  Replaces the pallas_call in _flex_attention_impl (flex_attention_kernel.py:173-187). */
 int flexattn_fwd(const flexattn_fwd_params* p, void* stream);

@@ -182,7 +182,9 @@ def test_captured_and_replayed():
 
 @pytest.mark.parametrize("known", [False, True])
 def test_a_captured_call_keeps_its_maps(known):
-    """The graph holds the maps' addresses: they outlive the caches, and a map that only a replay builds serves no other call."""
+    """The graph holds the maps' addresses: they live as long as the graph, whatever the caches drop, and a map that only a replay
+    builds serves no call outside."""
+    import gc
     import weakref
 
     from flex_attention_tpu_amd import _plans, block_mask
@@ -198,19 +200,76 @@ def test_a_captured_call_keeps_its_maps(known):
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     torch.cuda.synchronize()
-    before = set(block_mask._captured_maps._d)
+    gc.collect()
+    before = set(block_mask._captures)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=side):
         o, _ = taken(q, k, v, pair, sc)
         dq, = torch.autograd.grad(o, q, do)
-    used = [weakref.ref(m) for i, m in block_mask._captured_maps._d.items() if i not in before]
-    assert used and (known or not any(m is r() for m in block_mask._map_cache._d.values() for r in used))
+    capture, = set(block_mask._captures) - before
+    maps = list(block_mask._captures[capture].things.values())
+    used = [weakref.ref(m) for m in maps]
+    assert used and all(m.captured is not known and any(m is c for c in block_mask._map_cache._d.values()) is known for m in maps)
+    del maps
     o1, _ = taken(q, k, v, pair, sc)   # (in front of the first replay: on maps of its own)
     dq1, = torch.autograd.grad(o1, q, do)
     block_mask._map_cache.clear()
-    assert all(r() is not None for r in used)
-    graph.replay()
-    torch.cuda.synchronize()
-    assert torch.equal(o, o1) and torch.equal(dq, dq1)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, o1) and torch.equal(dq, dq1)
+        block_mask.release_ended()
+        gc.collect()
+        assert all(r() is not None for r in used)
     o2, _ = taken(q, k, v, pair, sc)
     assert torch.equal(o, o2) and torch.equal(dq, torch.autograd.grad(o2, q, do)[0])
+    block_mask._map_cache.clear()
+    del graph
+    gc.collect()
+    block_mask.release_ended()
+    assert capture not in block_mask._captures and all(r() is None for r in used)
+
+
+def test_names_of_captures():
+    """One name per capture, the same on its forked streams; told as ended when the graph has been dropped or reset, not before."""
+    import ctypes as C
+    import gc
+
+    from flex_attention_tpu_amd import _lib, block_mask
+    lib, x = _lib.load(), torch.zeros(8, device="cuda")
+
+    def name():
+        return lib.flexattn_capture_token(torch.cuda.current_stream().cuda_stream)
+
+    def ended():
+        out = (C.c_int64 * 4)()
+        return sorted(out[:lib.flexattn_captures_ended(out, 4)])
+    gc.collect()
+    block_mask.release_ended()
+    side, fork = torch.cuda.Stream(), torch.cuda.Stream()
+    assert name() == 0
+    with torch.cuda.stream(side):
+        assert name() == 0
+    graphs, names = [], []
+    for _ in range(3):
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1], stream=side):
+            names.append(name())
+            x.add_(1)
+            fork.wait_stream(side)
+            with torch.cuda.stream(fork):
+                assert name() == names[-1]
+                x.add_(1)
+            side.wait_stream(fork)
+            assert name() == names[-1]
+        graphs[-1].replay()
+        torch.cuda.synchronize()
+    assert len(set(names)) == 3 and min(names) > 0 and ended() == [] and x[0] == 6
+    graphs[1].reset()
+    assert ended() == [names[1]]
+    graphs[0].replay()
+    torch.cuda.synchronize()
+    assert ended() == [] and x[0] == 8
+    del graphs
+    gc.collect()
+    assert ended() == sorted((names[0], names[2]))
