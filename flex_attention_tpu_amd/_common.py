@@ -10,7 +10,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .block_mask import LRU, BlockMap, build_block_map, mask_spec_c, raw_stream, spec_of
+from .block_mask import LRU, BlockMap, build_block_map, keep_for_graph, mask_spec_c, raw_stream, spec_of
 from .masks import DocIds, MaskSpec
 from .scores import ScoreSpec
 
@@ -345,6 +345,7 @@ def score_spec_c(score_fn: Optional[Callable], Hq: int, device, mod_q: int, mod_
         if t is None:
             t = torch.tensor(slopes, dtype=torch.float32, device=device)
             _slopes_cache.put(key, t)
+        keep_for_graph(device, t)
         slopes_ptr = t.data_ptr()
     return _lib.ScoreSpecC(spec.kind, spec.cap, spec.slope, int(mod_q), int(mod_k), 0, slopes_ptr)
 

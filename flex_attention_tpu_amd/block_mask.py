@@ -60,6 +60,14 @@ def captured_by(stream: int) -> _Capture:
     return _captures.setdefault(token, _Capture())
 
 
+def keep_for_graph(device, *things) -> int:
+    """Keeps what a call reads for the graph that the call may be captured into; returns the current stream of `device`."""
+    stream = raw_stream(device)
+    if stream != 0 and capturing(device):   # (the default stream is never captured: the usual case asks nothing)
+        captured_by(stream).things.update((id(t), t) for t in things)
+    return stream
+
+
 def release_ended() -> None:
     """Drops what graphs that are gone have read."""
     tokens = (C.c_int64 * 16)()
@@ -144,9 +152,7 @@ class BlockMap:
         """Makes the current stream wait for the builder kernel if that ran on another stream, and tells the
         caching allocator that the map is in use on this stream too (a map evicted from the cache must not be
         handed out again while a kernel on this stream still walks it).  The graph of a call that is being captured keeps the map."""
-        stream = raw_stream(device)
-        if stream != 0 and capturing(device):   # (the default stream is never captured: the usual case asks nothing)
-            captured_by(stream).things[id(self)] = self
+        stream = keep_for_graph(device, self)
         if self.ready is None or stream == self.built_on:
             return
         cur = torch.cuda.current_stream(device)
@@ -269,6 +275,7 @@ def mask_spec_c(spec: MaskSpec, Sq: int, Sk: int, device) -> _lib.MaskSpecC:
         cur = torch.cuda.current_stream(device)
         tq.record_stream(cur)   # (cached arrays may be evicted while a kernel on this stream still reads them)
         tk.record_stream(cur)
+        keep_for_graph(device, tq, tk)
         doc_q, doc_k = tq.data_ptr(), tk.data_ptr()
         # sorted ids (the usual case: documents packed one after the other): the interval of the other side's
         # positions with a position's id, from which the kernels mask partial tiles without comparing ids
@@ -276,9 +283,11 @@ def mask_spec_c(spec: MaskSpec, Sq: int, Sk: int, device) -> _lib.MaskSpecC:
             rq, rk = doc_ranges_on(ids_q, ids_k, device), doc_ranges_on(ids_k, ids_q, device)
             if rq is not None:
                 rq.record_stream(cur)
+                keep_for_graph(device, rq)
                 range_q = rq.data_ptr()
             if rk is not None:
                 rk.record_stream(cur)
+                keep_for_graph(device, rk)
                 range_k = rk.data_ptr()
         doc_batches = batches
     return _lib.MaskSpecC(spec.flags, spec.window, spec.stride, doc_batches, doc_q, doc_k, range_q, range_k)

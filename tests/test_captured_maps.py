@@ -121,3 +121,37 @@ def test_one_capture_builds_a_map_once(gpu):
             if call is attend:
                 first = len(gpu.built)
         assert before < first and len(gpu.built) <= first + 1   # (general: a map at blocks of its own)
+
+
+def test_a_graph_s_ids_and_slopes_live_as_long_as_it(gpu, monkeypatch):
+    """The other arrays that parameter blocks point at and that bounded caches hold: document ids, their ranges, position-bias
+    slopes."""
+    from flex_attention_tpu_amd import _common
+    from flex_attention_tpu_amd.masks import DocIds
+    from flex_attention_tpu_amd.scores import make_alibi_global_score_fn
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda self, stream: None)
+    caches = [(block_mask, "_doc_cache"), (block_mask, "_range_cache"), (block_mask, "_rows_cache"), (_common, "_slopes_cache")]
+    for module, name in caches:
+        monkeypatch.setattr(module, name, block_mask.LRU(64))
+    cpu = torch.device("cpu")
+    shared, entries = torch.arange(256) // 100, torch.stack([torch.arange(256) // n for n in (60, 90)])
+    specs = [MaskSpec(_lib.MASK_DOC, doc_ids=DocIds(ids.numpy())) for ids in (shared, entries)]
+
+    def call():
+        for spec in specs:
+            block_mask.mask_spec_c(spec, 256, 256, cpu)
+        _common.score_spec_c(make_alibi_global_score_fn(4), 4, cpu, 128, 128)
+    call()   # (a captured call copies nothing to the device: the arrays are an eager call's)
+    gpu.capture = 1
+    call()
+    gpu.capture = 0
+    arrays = [weakref.ref(t) for module, name in caches for t in getattr(module, name)._d.values() if isinstance(t, torch.Tensor)]
+    assert len(arrays) >= 4
+    for module, name in caches:
+        getattr(module, name).clear()
+    gc.collect()
+    assert all(ref() is not None for ref in arrays)
+    gpu.ended = [1]
+    block_mask.release_ended()
+    gc.collect()
+    assert all(ref() is None for ref in arrays)

@@ -230,6 +230,38 @@ def test_a_captured_call_keeps_its_maps(known):
     assert capture not in block_mask._captures and all(r() is None for r in used)
 
 
+def test_a_captured_call_keeps_its_ids_and_slopes():
+    """The caches of document ids and position-bias slopes drop the arrays that a captured call reads, and their memory goes to other
+    tensors: the replays still read them."""
+    import gc
+
+    import flex_attention_tpu_amd as F
+    from flex_attention_tpu_amd import _common, block_mask, masks, scores
+    pair, sfn, sc = masks.make_jagged_mask_fns(128, 128, [150, 250, 112]), scores.make_alibi_global_score_fn(4), 1 / math.sqrt(128)
+    q, k, v, do = inputs(Sq=512, Sk=512)
+    q.requires_grad_(True)
+
+    def step():
+        o = F.flex_attention(q, k, v, sfn, pair, sm_scale=sc)
+        return o.detach(), torch.autograd.grad(o, q, do)[0]
+    want = step()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        got = step()
+    for cache in (block_mask._map_cache, block_mask._doc_cache, block_mask._range_cache, _common._slopes_cache):
+        cache.clear()
+    gc.collect()
+    others = [torch.full((n,), -1, dtype=torch.int32, device="cuda") for n in (4, 16, 64, 256, 512, 1024) for _ in range(64)]
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert all(int(t.max()) == -1 for t in others)
+
+
 def test_names_of_captures():
     """One name per capture, the same on its forked streams; told as ended when the graph has been dropped or reset, not before."""
     import ctypes as C
