@@ -7,7 +7,9 @@ fallback implementation.
 from __future__ import annotations
 
 import ctypes as C
+import importlib
 import os
+import warnings
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "libflexattn.so")
@@ -220,23 +222,28 @@ def load() -> C.CDLL:
     return _lib
 
 
-_host = None
+_host = None   # the module, or False where it cannot be had
 
 
 def load_host():
-    """The C++ side of the prepared calls (csrc/host_path.cpp), bound to libflexattn.so; raises ImportError if it has not
-    been built."""
+    """The C++ side of the prepared calls (csrc/host_path.cpp), bound to libflexattn.so.  None, with a warning, where it has not been
+    built or was built for another Python or torch: those calls then take the Python autograd function, which runs the same
+    kernels at a higher cost on the host."""
     global _host
     if _host is None:
-        if not os.path.exists(os.path.join(_PKG_DIR, "_host.so")):
-            raise ImportError(f"{_PKG_DIR}/_host.so is missing: build it with `python -m flex_attention_tpu_amd.build`")
-        import torch  # noqa: F401  (its libraries come first)
-        from . import _host as mod
-        lib = load()
-        mod.bind(*(C.cast(getattr(lib, "flexattn_" + n), C.c_void_p).value
-                   for n in ("fwd", "fwd_work", "fwd_work_bytes", "bwd", "bwd_dq", "bwd_dkv", "bwd_delta", "last_error_string")))
-        _host = mod
-    return _host
+        try:
+            import torch  # noqa: F401  (its libraries come first)
+            mod = importlib.import_module("._host", __package__)
+        except ImportError as e:
+            warnings.warn(f"small calls are slower than they could be, their C++ side is not to be had ({e}): build it with "
+                          "`python -m flex_attention_tpu_amd.build`", RuntimeWarning, stacklevel=2)
+            _host = False
+        else:
+            lib = load()
+            mod.bind(*(C.cast(getattr(lib, "flexattn_" + n), C.c_void_p).value
+                       for n in ("fwd", "fwd_work", "fwd_work_bytes", "bwd", "bwd_dq", "bwd_dkv", "bwd_delta", "last_error_string")))
+            _host = mod
+    return _host or None
 
 
 def load_for(score_code=None, mask_code=None) -> C.CDLL:

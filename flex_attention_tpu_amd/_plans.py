@@ -84,10 +84,13 @@ def ordinary(q, k, v) -> bool:
 
 def attend(q, k, v, spec: MaskSpec, sm_scale, block_q, block_k, prepared):
     """o of a differentiable call without score function, bias and segment ids on `ordinary` tensors, or None where the call is not
-    a prepared one.  ``prepared(q, k, v, spec)``: whether its shapes, mask and scale are (asked once per combination; it
+    a prepared one or there is no C++ side.  ``prepared(q, k, v, spec)``: whether its shapes, mask and scale are (asked once per combination; it
     raises for what the entry points refuse)."""
     if q.dtype != k.dtype or q.dtype != v.dtype or k.shape != v.shape or q.device != k.device or q.device != v.device:
         return None   # (the general path says what is wrong)
+    host = _lib.load_host()
+    if host is None:
+        return None
     key = (q.shape, k.shape, q.dtype, q.device, spec, sm_scale, block_q, block_k)
     plan = _attend_plans.get(key)
     if plan is False:
@@ -100,11 +103,11 @@ def attend(q, k, v, spec: MaskSpec, sm_scale, block_q, block_k, prepared):
         parts = [_template(cls, pass_id, q, k, spec, sm_scale) for cls, pass_id in
                  ((_lib.FwdParamsC, _lib.PASS_FWD), (_lib.BwdParamsC, _lib.PASS_DQ), (_lib.BwdParamsC, _lib.PASS_DKV))]
         maps = [bm for _, bm in parts]
-        plan = (_lib.load_host().Plan(*(t for t, _ in parts)), tuple(weakref.ref(bm) for bm in maps))
+        plan = (host.Plan(*(t for t, _ in parts)), tuple(weakref.ref(bm) for bm in maps))
         _keep(_attend_plans, key, plan, maps)
     for bm in maps:   # (a map built on another stream: this one waits for it; the backward runs on this one too)
         bm.wait_ready(q.device)
-    return _lib.load_host().attend(q, k, v, plan[0], maps[0].host_map(), maps[1].host_map(), maps[2].host_map())
+    return host.attend(q, k, v, plan[0], maps[0].host_map(), maps[1].host_map(), maps[2].host_map())
 
 
 def takes(q, k, spec: MaskSpec, sm_scale, *passes: int) -> bool:

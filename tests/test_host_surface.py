@@ -291,3 +291,28 @@ def test_no_compute_path_without_the_library(monkeypatch, tmp_path):
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("why", ["not built", "built for another torch"])
+def test_prepared_calls_without_their_cpp_side(monkeypatch, why):
+    """Without the C++ autograd function a prepared call goes to the Python one: a warning, once, and no error."""
+    import sys
+    import warnings
+
+    from flex_attention_tpu_amd import _plans
+
+    def refuse(name, package=None):
+        assert name == "._host"
+        raise ModuleNotFoundError("No module named '_host'") if why == "not built" else ImportError("undefined symbol: _ZN3c10")
+    monkeypatch.setattr(_lib, "_host", None)
+    monkeypatch.delitem(sys.modules, "flex_attention_tpu_amd._host", raising=False)
+    monkeypatch.setattr("importlib.import_module", refuse)
+    q, k, v = (torch.empty(1, 2, 256, 128, dtype=torch.bfloat16) for _ in range(3))
+
+    def never(*a):
+        raise AssertionError("no combination is looked at that nothing will serve")
+    with pytest.warns(RuntimeWarning, match="flex_attention_tpu_amd.build"):
+        assert _plans.attend(q, k, v, masks.MaskSpec(), 0.1, 128, 128, never) is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _plans.attend(q, k, v, masks.MaskSpec(), 0.1, 128, 128, never) is None
