@@ -247,11 +247,13 @@ __global__ __launch_bounds__(512, 1) void bwd_dab_bf16_kernel(BwdArgs a, int n_b
   }
 }
 
-// Planes of the bias gradient, and the pairs that share each.
-static void dab_planes(const BwdArgs& a, int* n_b, int* n_h, long long* planes) {
+// Planes of the bias gradient, the pairs that share each, and the tiles that the kernel walks; -1: more than its int counters and their
+// steps of a work-group hold.
+static long long dab_tiles(const BwdArgs& a, int* n_b, int* n_h) {
   *n_b = a.score.ab_sb_rows == 0 ? a.B : 1;
   *n_h = a.score.ab_sh_rows == 0 ? a.Hq : 1;
-  *planes = (long long)a.B * a.Hq / (*n_b * *n_h);
+  const long long planes = (long long)a.B * a.Hq / ((long long)*n_b * *n_h), per_plane = (long long)a.map.nq * a.map.nk;
+  return (double)planes * (double)per_plane > (double)((1ll << 31) - 512) ? -1 : planes * per_plane;
 }
 
 // From 200 tiles on: fewer leave CUs idle, and the full-size gradient and its sum are small then.  Forward and backward, full-size
@@ -259,21 +261,17 @@ static void dab_planes(const BwdArgs& a, int* n_b, int* n_h, long long* planes) 
 // 200 (B=2, H=8, S=640) 96.7 / 90.8, 256 (B=4, H=16, S=512) 106 / 103.
 bool bwd_dab_bf16_pays(const BwdArgs& a) {
   int n_b, n_h;
-  long long planes;
-  dab_planes(a, &n_b, &n_h, &planes);
-  const long long n_wg = planes * a.map.nq * a.map.nk;
-  return a.score.kind == FLEXATTN_SCORE_NONE && n_b * n_h > 1 && n_wg >= 200 && n_wg < (1ll << 31);
+  return a.score.kind == FLEXATTN_SCORE_NONE && dab_tiles(a, &n_b, &n_h) >= 200 && n_b * n_h > 1;
 }
 
 int bwd_dab_bf16(const BwdArgs& a, hipStream_t stream) {
   using namespace dab_cfg;
   int n_b, n_h;
-  long long planes;
-  dab_planes(a, &n_b, &n_h, &planes);
+  const long long tiles = dab_tiles(a, &n_b, &n_h);
+  if (tiles < 0) return set_error(FLEXATTN_ENOTSUP, "flexattn_bwd_dab: more than 2^31 - 512 tiles of the bias");
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(bwd_dab_bf16_kernel),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
   if (attr != hipSuccess) return set_error(FLEXATTN_ELAUNCH, "hipFuncSetAttribute(dab): %s", hipGetErrorString(attr));
-  const long long tiles = planes * a.map.nq * a.map.nk;
   const unsigned grid = tiles < 256 ? (unsigned)((tiles + 7) / 8 * 8) : 256u;   // one work-group per CU, the same number per XCD
   hipLaunchKernelGGL(bwd_dab_bf16_kernel, dim3(grid), dim3(512), LDS_BYTES, stream, a, n_b, n_h);
   return check_launch("flexattn_bwd_dab bf16");

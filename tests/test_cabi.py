@@ -188,3 +188,16 @@ def test_the_wide_ds_flag_belongs_to_one_kind_of_backward(lib):
         bq, bk = _lib.tile_shape(which, dtype, D)
         p.map = _lib.BlockMapC(base, base, base, base, base, 256 // bq, 256 // bk, bq, bk)
         assert fn(C.byref(p), None) == _lib.EINVAL and b"unknown flags" in lib.flexattn_last_error_string(), (D, dtype)
+
+
+def test_shared_bias_gradient_refuses_more_tiles_than_it_counts(lib):
+    """flexattn_bwd_dab walks the bias's tiles with 32-bit counters: a request of more is refused before any launch, and
+    flexattn_bwd_dab_pays does not advise it."""
+    base = C.addressof(C.create_string_buffer(64))
+    for Hq, Sq, Sk, shared in ((4, 1 << 22, 1 << 23, False), (2, 1 << 22, 1 << 30, True), (2, 1 << 30, 1 << 30, True)):
+        p = _lib.BwdParamsC(q=base, k=base, v=base, dout=base, l=base, m=base, delta=base, dk=base, dv=base, dab=base, B=2, Hq=Hq, Hkv=Hq,
+                            Sq=Sq, Sk=Sk, D=128, dtype=_lib.BF16, sm_scale=1.0)
+        p.map = _lib.BlockMapC(base, base, base, base, base, Sq // 128, Sk // 128, 128, 128)
+        p.ab = _lib.BiasC(base, 0, 0 if shared else Sq * Sk, _lib.F32, 0)
+        assert lib.flexattn_bwd_dab_pays(C.byref(p)) == 0
+        assert lib.flexattn_bwd_dab(C.byref(p), None) == _lib.ENOTSUP and b"tiles" in lib.flexattn_last_error_string()
