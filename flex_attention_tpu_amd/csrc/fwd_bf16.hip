@@ -68,7 +68,7 @@ struct FwdPinned {
 // AB: the call may have an additive bias (false: splits_bias() kinds without one).
 // SPLIT: each q tile's list is cut into `parts` runs of equal length, a work-group each; what a work-group leaves is its float32
 // sums, relative to its own maximum, which fwd_merge_kernel puts together.  For grids that leave CUs idle: a tile's list is a serial
-// chain (see fwd_split_parts).
+// chain (see split_parts).  A part may be empty: a list can be shorter than the parts are many.
 template <int SCORE, int NP, bool AB, bool SPLIT>
 __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs a, float* work, int parts) {
   using namespace fwd_cfg;
@@ -115,7 +115,7 @@ __global__ __launch_bounds__(256, NP == 1 ? 2 : 1) void fwd_bf16_kernel(FwdArgs 
     qreg[ks] = *reinterpret_cast<const bf16x8*>(Qg + (size_t)q_local * D + ks * 16 + hh * 8);
 
   const int n_list = a.map.cnt[qb];
-  const int first = SPLIT ? n_list * part / parts : 0;   // (at most 2^12 tiles by 2^4 parts)
+  const int first = SPLIT ? n_list * part / parts : 0;   // (at most 2^25 tiles, of a 32-bit length, by 2^4 parts)
   const int n_tiles = (SPLIT ? n_list * (part + 1) / parts : n_list) - first;
   const int* tile_idx = a.map.idx + (size_t)qb * nK + first;
   const uint8_t* tile_state = a.map.state + (size_t)qb * nK;
@@ -1015,32 +1015,38 @@ static int launch_fwd_plain(const FwdArgs& a, hipStream_t stream) {
 #endif  // FLEXATTN_CUSTOM_ONLY
 
 // Parts that the lists of a plain call are cut into where its q tiles leave CUs idle: as many as fill the CUs' places for
-// work-groups (two at head dimension 128, one at 256), of at least four kv tiles each.  A part costs its float32 sums
-// written and read; B=1, H=8, S=1024, D=128, causal, forward: 34.3 -> 26.1 us
-// with the other kernel, B=2, H=1, S=5888 118.7 -> 54.2, B=1, H=1, S=16384 299 -> 137.
-static int split_parts(long long tiles, int nk, int D) {
-  const long long fill = (D == 128 && nk >= 64 ? 512 : 256) / tiles;
-  const int most = nk / 8 < 16 ? nk / 8 : 16;
-  return fill < 2 || most < 2 ? 1 : fill < most ? (int)fill : most;
-}
-static bool small_plain(const FwdArgs& a, int D) {
-  return (D == 128 || D == 256) && a.score.kind == FLEXATTN_SCORE_NONE && a.score.ab == nullptr && a.flags == 0;
+// work-groups, of at least eight kv tiles of a full list each.  A part costs its float32 sums written and read; B=1, H=8, S=1024,
+// D=128, causal, forward: 34.3 -> 26.1 us with the other kernel, B=2, H=1, S=5888 118.7 -> 54.2, B=1, H=1, S=16384 299 -> 137.
+// A cut has to shorten the longest list by four tiles, or the sums cost more than it saves: the lists of a causal window are short
+// whatever the length (D=256, H=1, S=8192, whole / four parts: window 64 22.5 / 28.8 us, 128 26.9 / 28.3, 200 33.9 / 31.3, 300
+// 36.6 / 31.1; window 200, S=16384, two parts: 34.7 / 35.2).
+// Places: two a CU at head dimension 128 from 64 kv tiles on, else one.  (Two below that as well gain on most grids, not on all: H=3,
+// S=3968, causal, 53.0 -> 41.9 us, H=8, S=2048, causal, 38.4 -> 34.2, without a mask 38.3 -> 39.4.)
+static int split_parts(const FwdArgs& a, int D) {
+  using namespace fwd_cfg;
+  const long long tiles = (long long)a.B * a.Hq * a.map.nq;
+  if (!((D == 128 || D == 256) && a.score.kind == FLEXATTN_SCORE_NONE && a.score.ab == nullptr && a.flags == 0) || tiles > 256) return 1;
+  const long long nk = a.map.nk;
+  long long parts = (D == 128 && nk >= 64 ? 512 : 256) / tiles;
+  if (parts > nk / 8) parts = nk / 8;
+  if (parts > 16) parts = 16;
+  long long longest = nk;
+  if ((a.mask.flags & FLEXATTN_MASK_CAUSAL) && (a.mask.flags & FLEXATTN_MASK_WINDOW)) {   // (keys i - window + 1 .. i of a tile's rows i)
+    const long long list = ((long long)BM + a.mask.window - 2) / BN + 2;
+    if (list < longest) longest = list;
+  }
+  return parts < 2 || longest - (longest + parts - 1) / parts < 4 ? 1 : (int)parts;
 }
 int64_t fwd_bf16_work_bytes(const FwdArgs& a, int D) {
-  if (!small_plain(a, D)) return 0;
-  const int parts = split_parts((long long)a.B * a.Hq * a.map.nq, a.map.nk, D);
+  const int parts = split_parts(a, D);
   return parts < 2 ? 0 : (int64_t)parts * a.B * a.Hq * a.Sq * (D + 2) * 4;
 }
-// The forward of a caller that has brought such memory.  Up to 256 q tiles the compiled loop, two work-groups of 128 rows a CU,
-// is the faster kernel of head dimension 128 in one part too: the stream's work-groups take 256 rows (B=1, S=1024, causal, H=8
-// 34.5 against 28.0 us, H=32 39.2 / 30.3, H=64, 512 tiles, 41.3 / 45.3).
+// The forward of a caller that has brought such memory, or for which there is none to bring.
 int fwd_bf16_with_work(const FwdArgs& a, int D, void* work, hipStream_t stream) {
-  const long long tiles = (long long)a.B * a.Hq * a.map.nq;
-  if (small_plain(a, D) && tiles <= 256) {
-    const int parts = work != nullptr ? split_parts(tiles, a.map.nk, D) : 1;
+  const int parts = work != nullptr ? split_parts(a, D) : 1;
+  if (parts > 1)
     return D == 128 ? launch_fwd<FLEXATTN_SCORE_NONE>(a, stream, static_cast<float*>(work), parts)
                     : launch_fwd<FLEXATTN_SCORE_NONE, 2>(a, stream, static_cast<float*>(work), parts);
-  }
   return D == 256 ? fwd_bf16_d256(a, stream) : D == 64 ? fwd_bf16_d64(a, stream) : fwd_bf16_d128(a, stream);
 }
 

@@ -247,9 +247,10 @@ int32_t flexattn_captures_ended(int64_t* tokens, int32_t n);
 int flexattn_fwd(const flexattn_fwd_params* p, void* stream);
 
 /* The same for a caller that brings scratch device memory: `work`, 16-byte aligned, of flexattn_fwd_work_bytes bytes, which may be
- * 0.  Where the q tiles of a plain call (bf16, head dimension 128 or 256, flags 0) leave CUs idle, their lists are cut into parts
- * whose float32 sums lie there and a second launch puts together; such a call may also run another kernel than flexattn_fwd's
- * (results agree to the rounding of their sums).  The bytes depend on shapes, dtype, score, bias and flags. */
+ * 0: the call is then flexattn_fwd's.  Where the q tiles of a plain call (bf16, head dimension 128 or 256, flags 0) leave CUs idle,
+ * their lists are cut into parts whose float32 sums lie there and a second launch puts together; head dimension 128 runs
+ * another kernel for that than flexattn_fwd does (results agree to the rounding of their sums).  The bytes depend on shapes, dtype,
+ * score, mask, bias and flags. */
 int64_t flexattn_fwd_work_bytes(const flexattn_fwd_params* p);
 int flexattn_fwd_work(const flexattn_fwd_params* p, void* work, int64_t work_bytes, void* stream);
 

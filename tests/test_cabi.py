@@ -201,3 +201,23 @@ def test_shared_bias_gradient_refuses_more_tiles_than_it_counts(lib):
         p.ab = _lib.BiasC(base, 0, 0 if shared else Sq * Sk, _lib.F32, 0)
         assert lib.flexattn_bwd_dab_pays(C.byref(p)) == 0
         assert lib.flexattn_bwd_dab(C.byref(p), None) == _lib.ENOTSUP and b"tiles" in lib.flexattn_last_error_string()
+
+
+def test_work_of_a_split_forward_follows_the_lists(lib):
+    """Lists are cut where a cut shortens the longest by four tiles or more: a narrow causal window's are short whatever the length
+    (D=256, H=1, S=8192: window 64 22.5 us whole, 28.8 in four parts; 128 26.9 / 28.3; 200 33.9 / 31.3)."""
+    C_, W, S2 = _lib.MASK_CAUSAL, _lib.MASK_WINDOW, _lib.MASK_S2
+
+    def parts(S, flags=0, window=0, Hq=1, D=256, stride=0):
+        p = _lib.FwdParamsC(B=1, Hq=Hq, Hkv=Hq, Sq=S, Sk=S, D=D, dtype=_lib.BF16, sm_scale=1.0)
+        p.map = _lib.BlockMapC(None, None, None, None, None, S // 128, S // 64, 128, 64)
+        p.mask = _lib.MaskSpecC(flags, window, stride, 0, None, None, None, None)
+        bytes_, part = lib.flexattn_fwd_work_bytes(C.byref(p)), Hq * S * (D + 2) * 4
+        assert bytes_ % part == 0
+        return bytes_ // part
+    assert [parts(8192, C_ | W, w) for w in (1, 64, 128, 200, 300, 1025, 1 << 30)] == [0, 0, 0, 4, 4, 4, 4]
+    assert [parts(16384, C_ | W, w) for w in (64, 200, 300)] == [0, 0, 2]
+    assert parts(8192) == parts(8192, C_) == 4
+    assert parts(8192, W, 64) == 4              # (every key behind a query as well: full lists)
+    assert parts(8192, S2, 64, stride=8) == 4
+    assert [parts(S, C_) for S in (512, 896, 1024, 2048, 32768)] == [0, 0, 2, 4, 0]

@@ -62,3 +62,23 @@ def test_bytes_and_refusals():
             _lib.check(lib.flexattn_fwd_work(C.byref(p), ptr, n, None), lib)
     p.score.kind = _lib.SCORE_SOFTCAP
     assert lib.flexattn_fwd_work_bytes(C.byref(p)) == 0
+
+
+@pytest.mark.parametrize("B,Hq,S,D", [(1, 16, 128, 128), (1, 8, 640, 128), (1, 2, 128, 256), (1, 2, 256, 64)])
+def test_nothing_to_cut(B, Hq, S, D):
+    """Where there is no memory to bring, flexattn_fwd_work is flexattn_fwd: the same bits."""
+    from flex_attention_tpu_amd import _lib
+    from flex_attention_tpu_amd.block_mask import build_block_map
+    from flex_attention_tpu_amd.masks import MaskSpec
+    lib = _lib.load()
+    q, k, v, _ = (t.cuda() for t in O.make_inputs(B, Hq, Hq, S, S, D, dtype=torch.bfloat16, seed=D))
+    bm = build_block_map(MaskSpec(), S, S, *_lib.tile_shape(_lib.PASS_FWD, _lib.BF16, D), q.device)
+    got = [[torch.empty_like(q), *torch.empty(2, B, Hq, S, device="cuda")] for _ in range(2)]
+    for o, l, m in got:
+        p = _lib.FwdParamsC(q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), o=o.data_ptr(), l=l.data_ptr(), m=m.data_ptr(), B=B, Hq=Hq,
+                            Hkv=Hq, Sq=S, Sk=S, D=D, dtype=_lib.BF16, sm_scale=D ** -0.5)
+        p.map = bm.as_c()
+        assert lib.flexattn_fwd_work_bytes(C.byref(p)) == 0
+        stream = torch.cuda.current_stream().cuda_stream
+        _lib.check(lib.flexattn_fwd_work(C.byref(p), None, 0, stream) if o is got[0][0] else lib.flexattn_fwd(C.byref(p), stream), lib)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
