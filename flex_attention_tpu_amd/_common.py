@@ -26,9 +26,8 @@ def dtype_code(t: torch.Tensor) -> int:
     raise NotImplementedError(f"dtype {t.dtype} is not supported (bfloat16 and float32 are)")
 
 
-def check_qkv(q, k, v, *others):
-    """Shape / layout checks in the spirit of the reference's rank asserts
-    (flex_attention_dq_bwd.py:161-164); returns (B, Hq, Hkv, Sq, Sk, D)."""
+def _refuse_operand(q, k, v, *others):
+    """Says what is wrong with the operands of a call that check_qkv refuses."""
     for name, t in (("q", q), ("k", k), ("v", v)) + tuple((f"arg{i}", o) for i, o in enumerate(others)):
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"{name} must be a torch.Tensor")
@@ -40,6 +39,14 @@ def check_qkv(q, k, v, *others):
             raise ValueError(f"{name} must be contiguous")
         if t.dtype != q.dtype:
             raise ValueError(f"{name} has dtype {t.dtype}, expected {q.dtype}")
+
+
+def check_qkv(q, k, v, *others):
+    """Shape / layout checks in the spirit of the reference's rank asserts
+    (flex_attention_dq_bwd.py:161-164); returns (B, Hq, Hkv, Sq, Sk, D)."""
+    for t in (q, k, v, *others):
+        if not (isinstance(t, torch.Tensor) and t.dim() == 4 and t.is_cuda and t.is_contiguous() and t.dtype is q.dtype):
+            _refuse_operand(q, k, v, *others)
     B, Hq, Sq, D = q.shape
     Bk, Hkv, Sk, Dk = k.shape
     if v.shape != k.shape:

@@ -71,12 +71,16 @@ _attend_plans = LRU(64)   # (shapes, dtype, device, mask, scale, blocks) -> (C++
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
+def long_and_narrow(q) -> bool:
+    """Whether a call's query is a plain contiguous tensor of a length and head dimension that the C++ autograd function takes: not
+    decoding, and not head dimension 256, whose backward hands dS over."""
+    return type(q) in _PLAIN and q.dim() == 4 and q.size(2) >= 128 and q.size(3) <= 128 and q.is_contiguous()
+
+
 def ordinary(q, k, v) -> bool:
-    """Whether a call is one that the C++ autograd function serves exactly as the Python one does: plain contiguous tensors of
-    lengths and head dimensions that it may take, outside function transforms, forward-mode differentiation, tracing and compilation, and modes that watch Python's calls."""
-    if type(q) not in _PLAIN or q.ndim != 4 or q.shape[2] < 128 or q.shape[3] > 128:
-        return False   # (decoding, and head dimension 256, whose backward hands dS over)
-    return (not torch.compiler.is_compiling() and type(k) in _PLAIN and type(v) in _PLAIN and q.is_contiguous() and k.is_contiguous() and v.is_contiguous()
+    """Whether a call whose query is `long_and_narrow` is one that the C++ autograd function serves exactly as the Python one does: plain
+    contiguous tensors, outside function transforms, forward-mode differentiation, tracing and compilation, and modes that watch Python's calls."""
+    return (type(k) in _PLAIN and type(v) in _PLAIN and k.is_contiguous() and v.is_contiguous() and not torch.compiler.is_compiling()
             and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
             and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
             and torch._C._get_tracing_state() is None)

@@ -60,12 +60,11 @@ def captured_by(stream: int) -> _Capture:
     return _captures.setdefault(token, _Capture())
 
 
-def keep_for_graph(device, *things) -> int:
-    """Keeps what a call reads for the graph that the call may be captured into; returns the current stream of `device`."""
+def keep_for_graph(device, *things) -> None:
+    """Keeps what a call reads for the graph that the call may be captured into."""
     stream = raw_stream(device)
     if stream != 0 and capturing(device):   # (the default stream is never captured: the usual case asks nothing)
         captured_by(stream).things.update((id(t), t) for t in things)
-    return stream
 
 
 def release_ended() -> None:
@@ -152,7 +151,9 @@ class BlockMap:
         """Makes the current stream wait for the builder kernel if that ran on another stream, and tells the
         caching allocator that the map is in use on this stream too (a map evicted from the cache must not be
         handed out again while a kernel on this stream still walks it).  The graph of a call that is being captured keeps the map."""
-        stream = keep_for_graph(device, self)
+        stream = raw_stream(device)
+        if stream != 0:   # (the default stream is never captured)
+            keep_for_graph(device, self)
         if self.ready is None or stream == self.built_on:
             return
         cur = torch.cuda.current_stream(device)
@@ -342,6 +343,9 @@ def create_block_mask(mask_fns, Sq: int, Sk: int, block_q: int, block_k: int, de
     return build_block_map(spec, Sq, Sk, block_q, block_k, device)
 
 
+_NO_MASK = MaskSpec()
+
+
 def spec_of(mask_fn: Optional[Callable], block_mask_fn: Optional[Callable]) -> MaskSpec:
     """MaskSpec carried by the closures: those of this package's factories, or of compiler.compile_mask_fn
     for arbitrary element predicates.  Untagged closures are rejected."""
@@ -354,10 +358,10 @@ def spec_of(mask_fn: Optional[Callable], block_mask_fn: Optional[Callable]) -> M
             raise NotImplementedError(
                 "mask_fn/block_mask_fn must come from flex_attention_tpu_amd.masks factories or from "
                 "flex_attention_tpu_amd.compiler.compile_mask_fn (which compiles a Python predicate into the kernels)")
-        if spec is not None and s != spec:
+        if spec is not None and s is not spec and s != spec:
             raise ValueError("mask_fn and block_mask_fn describe different masks")
         spec = s
-    return spec if spec is not None else MaskSpec()
+    return spec if spec is not None else _NO_MASK
 
 
 def host_block_map(block_mask_fn: Callable, nq: int, nk: int) -> torch.Tensor:

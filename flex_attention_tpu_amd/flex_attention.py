@@ -107,7 +107,7 @@ class _FlexAttention(torch.autograd.Function):
         score_fn, mask_fn, block_mask_fn, segment_ids, causal, sm_scale, block_q, block_k = opts
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
         o, l, m = _flex_attention_impl(q, k, v, ab, segment_ids, True, causal, sm_scale, 1, block_q, block_k, block_k,
-                                       False, block_mask_fn, mask_fn, score_fn, _with_work=q.shape[-1] == 256)
+                                       False, block_mask_fn, mask_fn, score_fn, _with_work=True)
         ctx.save_for_backward(q, k, v, o, l, m, *([ab] if ab is not None else []))
         ctx.opts = opts
         return o
@@ -178,19 +178,22 @@ def flex_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, score_fn: 
     else:
         mask_fn, block_mask_fn = mask_fns if mask_fns is not None else (None, None)
     score_fn, mask_fn, block_mask_fn = tagged_closures(score_fn, mask_fn, block_mask_fn, block_q, block_k)
-    if score_fn is None and ab is None and segment_ids is None and _plans.ordinary(q, k, v):
-        spec = spec_of(mask_fn, block_mask_fn)
-        if causal:
-            spec = spec.combine(_CAUSAL)
+    if score_fn is None and ab is None and segment_ids is None and _plans.long_and_narrow(q):
+        known = getattr(mask_fn if mask_fn is not None else block_mask_fn, "spec", None)
+        # (in the order of their cost: documents, compiled masks and windows pay for no further look)
+        if (known is None or (known.doc_ids is None and known.custom is None and
+                              not (q.dtype is torch.bfloat16 and q.size(3) > 64 and ds_exchange_pays(None, mask_fn)))) and _plans.ordinary(q, k, v):
+            spec = spec_of(mask_fn, block_mask_fn)
+            if causal:
+                spec = spec.combine(_CAUSAL)
 
-        def prepared(q, k, v, spec):
-            B, Hq, Hkv, Sq, Sk, D = check_qkv(q, k, v)
-            check_blocks(Sq, Sk, block_q=block_q, block_k_major=block_k, block_k=block_k)
-            return (_plans.takes(q, k, spec, sm_scale, _lib.PASS_FWD, _lib.PASS_DQ, _lib.PASS_DKV) and
-                    not (q.dtype is torch.bfloat16 and _hands_ds_over(q, k, None, None, sm_scale, None, mask_fn, block_mask_fn, False)))
-        # (what _plans.takes never takes goes on at once: those calls pay for no further look)
-        o = _plans.attend(q, k, v, spec, float(sm_scale), block_q, block_k, prepared) if spec.doc_ids is None and spec.custom is None else None
-        if o is not None:
-            return o
+            def prepared(q, k, v, spec):
+                B, Hq, Hkv, Sq, Sk, D = check_qkv(q, k, v)
+                check_blocks(Sq, Sk, block_q=block_q, block_k_major=block_k, block_k=block_k)
+                return (_plans.takes(q, k, spec, sm_scale, _lib.PASS_FWD, _lib.PASS_DQ, _lib.PASS_DKV) and
+                        not (q.dtype is torch.bfloat16 and _hands_ds_over(q, k, None, None, sm_scale, None, mask_fn, block_mask_fn, False)))
+            o = _plans.attend(q, k, v, spec, float(sm_scale), block_q, block_k, prepared)
+            if o is not None:
+                return o
     opts = (score_fn, mask_fn, block_mask_fn, segment_ids, bool(causal), float(sm_scale), int(block_q), int(block_k))
     return _FlexAttention.apply(q, k, v, ab, opts)

@@ -80,7 +80,7 @@ def _flex_attention_impl(q, k, v, ab, segment_ids, save_residuals, causal, sm_sc
         if causal:
             spec = spec.combine(_CAUSAL)
         if _plans.takes(q, k, spec, sm_scale, _lib.PASS_FWD):
-            return _plans.forward(q, k, v, spec, float(sm_scale), save_residuals, _with_work)
+            return _plans.forward(q, k, v, spec, float(sm_scale), save_residuals, _with_work and D == 256)
     # (lengths below one tile: the tensors are zero-padded to it, a document id of their own drops the padded keys
     # and the padded query rows are cut off again)
     Sq_p, Sk_p = padded_len(Sq), padded_len(Sk)
