@@ -1,27 +1,20 @@
 """The prepared calls' autograd function in C++ against the Python one that every other call takes: the same kernels on the same
-arguments, so the same bits (bf16 at head dimension 128: the forward of a small grid may take another kernel and cut its lists, see
-flexattn_fwd_work; its results agree within twice the bounds of helpers.assert_close), for each set of wanted gradients, under the hooks
-and modes that watch an autograd function, and where the call is handed to the Python one."""
+arguments, so the same bits, for each set of wanted gradients, under the hooks and modes that watch an autograd function, and where
+the call is handed to the Python one; where the forward's lists are cut (flexattn_fwd_work), against that forward and its backward."""
 import math
 import threading
 
 import pytest
 import torch
 
-from helpers import BF16_ABS, BF16_REL
+from helpers import assert_close, same_residual_grads
 from oracle import mha_oracle as O
 
 pytestmark = pytest.mark.gpu
 
 
 def agree(got, want):
-    for n, (a, b) in enumerate(zip(got, want)):
-        if a.dtype is torch.float32 or a.shape[-1] != 128:
-            assert torch.equal(a, b)
-        else:
-            # (each side is held to this bound against the oracle elsewhere: the two differ by at most twice it)
-            bound = 2 * torch.clamp(b.float().abs() * 2.0 ** -7, min=BF16_ABS)
-            assert O.rel_l2(a, b) <= BF16_REL and bool(((a.float() - b.float()).abs() <= bound).all()), n
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
 def inputs(B=2, Hq=4, Hkv=2, Sq=300, Sk=300, D=128, dtype=torch.bfloat16, seed=0):
@@ -62,6 +55,34 @@ def test_same_bits_as_the_python_function(wanted, Sq, Sk, causal, dtype, D):
     with torch.no_grad():
         assert torch.equal(taken(q, k, v, pair, sc)[0], o)
     agree((o, *torch.autograd.grad(o, leaves, do)), (want, *torch.autograd.grad(want, leaves, do)))
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,causal", [(1, 2, 1, 1024, 1024, True), (1, 2, 2, 1100, 1100, True), (2, 1, 1, 200, 1601, False)])
+def test_cut_lists(B, Hq, Hkv, Sq, Sk, causal):
+    """Small grids of long lists: the C++ forward brings the memory for the parts' sums, and its backward takes the residuals of
+    the merged rows."""
+    from flex_attention_tpu_amd import _lib, _plans
+    from flex_attention_tpu_amd.block_mask import spec_of
+    q, k, v, do = inputs(B, Hq, Hkv, Sq, Sk)
+    sc, pair = 1 / math.sqrt(128), masks_of(causal)
+    spec = spec_of(*(pair or (None, None)))
+    o, l, m = _plans.forward(q, k, v, spec, sc, True, with_work=True)
+    assert next(p for p in reversed(_plans._plans._d.values())).work_bytes >= 2 * q.numel() * 4   # (two parts or more)
+    whole, _, _ = _plans.forward(q, k, v, spec, sc, True)
+    assert not torch.equal(o, whole)
+    want = (o, *_plans.backward(q, k, v, l, m, o, do, spec, sc))
+    with torch.no_grad():
+        assert torch.equal(taken(q, k, v, pair, sc)[0], o)
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    for _ in range(2):
+        got, native = taken(q, k, v, pair, sc)
+        assert native
+        agree((got, *torch.autograd.grad(got, (q, k, v), do)), want)
+    cpu = [t.detach().cpu() for t in (q, k, v, do)]
+    assert_close("o", o, O.mha_reference(*cpu[:3], sm_scale=sc, causal=causal), torch.bfloat16)
+    for name, t, r in zip(("dq", "dk", "dv"), want[1:], same_residual_grads(*cpu, o, l, m, sm_scale=sc, causal=causal)):
+        assert_close(name, t, r, torch.bfloat16)
 
 
 def test_views_hooks_and_repeated_backward():
@@ -116,6 +137,9 @@ def test_calls_that_stay_with_the_python_function():
         for call in (lambda: F.flex_attention(*bad, sm_scale=sc), lambda: python_path(*bad, None, sc)):
             with pytest.raises(ValueError):
                 call()
+    for scale in (0.0, -1.0, math.inf, math.nan):   # (refused by the library, behind the C++ function)
+        with pytest.raises(ValueError, match="sm_scale"):
+            F.flex_attention(q, k, v, sm_scale=scale)
 
 
 def test_streams_and_threads():

@@ -3,6 +3,7 @@ bias broadcasts, masks whose tiles are partial or empty, documents per batch ent
 on the kernels' own forward.  Tolerances as in test_gpu_bias_grad: values are P (dP - delta) summed over the pairs, 1e-2 of a value
 where that exceeds 1."""
 import math
+import types
 
 import pytest
 import torch
@@ -28,10 +29,9 @@ def test_shared_bias_gradient(B, Hq, Hkv, Sq, Sk, D, ab_shape, kind, monkeypatch
         window = 100 + max(0, Sq - Sk)   # (every query keeps a key)
         pair, okw = masks.make_causal_sliding_window_mask_fns(128, 128, window), dict(mask=(j <= i) & (i - j < window))
     elif kind == "ids per entry":
-        if Sq != Sk:
-            pytest.skip("one id per position for both sides")
-        sid = torch.stack([torch.arange(Sq) * (2 + b) // Sq for b in range(B)])
-        okw = dict(segment_ids=sid)
+        ids = [torch.stack([torch.arange(S) * (2 + b) // S for b in range(B)]) for S in (Sq, Sk)]
+        sid = types.SimpleNamespace(q=ids[0], kv=ids[1])
+        okw = dict(mask=ids[0][:, :, None] == ids[1][:, None, :])
     ab = torch.randn(B if ab_shape[0] == "b" else 1, Hq if ab_shape[1] == "h" else 1, Sq, Sk, generator=torch.Generator().manual_seed(3))
     if kind == "bf16 bias":
         ab = ab.bfloat16()
