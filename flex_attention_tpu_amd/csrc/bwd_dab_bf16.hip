@@ -256,9 +256,15 @@ static long long dab_tiles(const BwdArgs& a, int* n_b, int* n_h) {
   return (double)planes * (double)per_plane > (double)((1ll << 31) - 512) ? -1 : planes * per_plane;
 }
 
-// From 200 tiles on: fewer leave CUs idle, and the full-size gradient and its sum are small then.  Forward and backward, full-size
-// against this pass: 50 tiles (B=4, H=2, S=640) 90.2 / 94.4 us, 128 (B=8, H=8, S=512) 103 / 109, (B=2, H=2, S=1024) 128 / 121,
-// 200 (B=2, H=8, S=640) 96.7 / 90.8, 256 (B=4, H=16, S=512) 106 / 103.
+// From 200 tiles on.  Kernel times of forward and backward, us, full-size gradient and its sum against this pass:
+//                              2 pairs a tile   8               32              64
+//    49 tiles (H=1, S=896)     112.6 / 108.6    119.5 / 131.0   148.5 / 210.6   267.8 / 368.2
+//   128 tiles (H=2, S=1024)    129.6 / 122.6    143.4 / 147.9   351.3 / 322.8   723.9 / 647.6
+//   196 tiles (H=1, S=1792)    204.7 / 189.2    219.7 / 216.4   555.8 / 443.1   1069  /  892
+//   256 tiles (H=4, S=1024)    137.6 / 126.8    174.7 / 164.9   731.8 / 580.3   1441  / 1161
+//   288 tiles (H=2, S=1536)    187.4 / 177.3    218.7 / 227.9   804.7 / 701.3   1509  / 1332
+// Fewer tiles leave CUs idle for as long as a tile's pairs take, one after the other.  The number of pairs moves the line little: it
+// lengthens that chain and the full-size gradient's bytes alike.  (288: a second round of the 256 work-groups with few tiles in it.)
 bool bwd_dab_bf16_pays(const BwdArgs& a) {
   int n_b, n_h;
   return a.score.kind == FLEXATTN_SCORE_NONE && dab_tiles(a, &n_b, &n_h) >= 200 && n_b * n_h > 1;

@@ -1,18 +1,17 @@
 // Flex-attention dk/dv backward, bf16, head dim 128, gfx950.
 //
-// One work-group = 4 waves = one 128-row KV tile of one (batch, kv head); each wave owns 32 kv
-// rows, whose K and V stay in registers as MFMA B operands.  Q / dO tiles of 128 rows stream
-// through double-buffered LDS (LDS-direct loads, swizzled unpadded tiles) together with their
-// lse and delta, for every query head of the KV group and every q tile the transposed block map
-// lists.  Per tile:
+// A work-group takes a KV tile of one (batch, kv head).  Q / dO rows stream through double-buffered LDS (LDS-direct loads,
+// swizzled unpadded tiles) together with their lse and delta, for every query head of the KV group and every q tile the
+// transposed block map lists.  Per tile:
 //   S = Q K^T,  dP = dO V^T   (lane owns a kv column, accumulator rows are q),
 //   P = exp2(S' - lse_q),  dS = P (dP - delta_q) f'(S),
 //   dv^T += dO^T P,  dk^T += Q^T dS   (dO^T, Q^T via transposing LDS reads).
 // Each dk/dv tile has exactly one writer, so the result is deterministic and needs no atomics.
 //
-// The plain score runs generated, hand-scheduled instruction streams (gen_dkv_tile.py ->
-// bwd_dkv_tile.inc) that software-pipeline MFMA, VALU and LDS work inside the wave with a fixed
-// register allocation; score modifications run the compiled C++ kernel.
+// The plain score, the soft-cap and the global position bias (one query head per kv head) run generated, hand-scheduled instruction
+// streams (gen_dkv_tile.py -> bwd_dkv_tile.inc) that software-pipeline MFMA, VALU and LDS work inside the wave with a fixed
+// register allocation: 4 waves, 32 of the 128 kv rows each, K and V in registers as MFMA B operands.  Everything else runs kernels
+// with a compiled loop: head dimension 128 with 8 waves and K and V in LDS, 256 with 4 waves on 64 kv rows (see there).
 #include <cstdlib>
 #include "fa_common.hpp"
 #include "launch.hpp"
@@ -429,7 +428,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dkv_bf16_d128_kernel(BwdArgs a) {
 // other wave of the kv rows through LDS, and each of the two adds the products of both q blocks to dk and dv in columns
 // 128 (w >> 1): 128 accumulator registers and 128 of K and V, which leaves room to read operands ahead.
 // BOUND: one wave a SIMD: an iteration is 64 MFMAs (2048 cycles) among some 700 instructions, copies into LDS of 64 KB and two
-// barriers, about 6400 cycles.  The form before this one had 128 kv rows a work-group and all columns in each wave: 256
+// barriers, 6280 cycles (with the export of dS).  The form before this one had 128 kv rows a work-group and all columns in each wave: 256
 // accumulators beside K and V left 128 registers for everything else, operands were read in front of each product and the
 // reloads of spilled registers, like the row values and the dS index read in the loop, waited for the copies in flight: dk/dv of
 // B=4, H=16, S=4096, causal, 1776 -> 1520-1610 us, and twice the work-groups where few fill the chip.

@@ -442,8 +442,8 @@ constexpr int kScoreBiasOnly = 100;
 // pointers and strides take registers through the loop, and kernels at the limit spill: symmetric ALiBi closure, B=8, H=4,
 // S=2048, 399 -> 375 us; tile-local ALiBi forward 28 spilled registers -> none).  Plain scores have no such
 // code at all, see kScoreBiasOnly.  The global position bias and the soft-cap keep one variant: at head dimension 128 they take
-// the generated streams where there is no bias (the position bias's dk/dv pass with grouped heads excepted); at 256 their
-// calls without a bias do carry the code of one (dk/dv: 60 and 45 spilled registers where plain scores have 12).
+// the generated streams where there is no bias, except the position bias's dk/dv pass with grouped heads, whose loop spills 17
+// registers; at 256 their calls without a bias carry the code of one, and nothing spills.
 constexpr bool splits_bias(int kind) { return kind == FLEXATTN_SCORE_CUSTOM || kind == FLEXATTN_SCORE_ALIBI_TILE; }
 
 template <int KIND>
