@@ -79,8 +79,8 @@ def long_and_narrow(q) -> bool:
 
 def ordinary(q, k, v) -> bool:
     """Whether a call whose query is `long_and_narrow` is one that the C++ autograd function serves exactly as the Python one does: plain
-    contiguous tensors, outside function transforms, forward-mode differentiation, tracing and compilation, and modes that watch Python's calls."""
-    return (type(k) in _PLAIN and type(v) in _PLAIN and k.is_contiguous() and v.is_contiguous() and not torch.compiler.is_compiling()
+    contiguous tensors, outside function transforms, forward-mode differentiation, tracing, and modes that watch Python's calls."""
+    return (type(k) in _PLAIN and type(v) in _PLAIN and k.is_contiguous() and v.is_contiguous()
             and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
             and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
             and torch._C._get_tracing_state() is None)

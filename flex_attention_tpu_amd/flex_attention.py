@@ -171,6 +171,9 @@ def flex_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, score_fn: 
     Gradients flow to q, k, v and ab (``torch.autograd.grad`` / ``.backward()``); higher-order
     differentiation is not supported, as in the reference (jax_exp.py:243-244).
     """
+    if torch.compiler.is_compiling():   # (torch.compile makes the call between its graphs: block maps, plans and launches are no part of one)
+        return torch.compiler.disable(_uncompiled)(q, k, v, score_fn, mask_fns, segment_ids=segment_ids, causal=causal, sm_scale=sm_scale,
+                                                   block_q=block_q, block_k=block_k, ab=ab)
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(q.shape[-1])
     if callable(mask_fns):   # (a bare mask function instead of a pair)
@@ -197,3 +200,7 @@ def flex_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, score_fn: 
                 return o
     opts = (score_fn, mask_fn, block_mask_fn, segment_ids, bool(causal), float(sm_scale), int(block_q), int(block_k))
     return _FlexAttention.apply(q, k, v, ab, opts)
+
+
+def _uncompiled(*args, **kwargs):
+    return flex_attention(*args, **kwargs)

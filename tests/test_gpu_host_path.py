@@ -142,6 +142,27 @@ def test_calls_that_stay_with_the_python_function():
             F.flex_attention(q, k, v, sm_scale=scale)
 
 
+@pytest.mark.parametrize("D,S,mask", [(128, 512, "causal"), (64, 300, "causal"), (128, 384, "window"), (256, 512, "causal"), (128, 512, "documents")])
+def test_under_compilation(D, S, mask):
+    """torch.compile makes the call between its graphs: its first call of a combination as well as later ones, with the same bits."""
+    import flex_attention_tpu_amd as F
+    from flex_attention_tpu_amd import block_mask, masks
+    pair = {"causal": lambda: masks_of(True), "window": lambda: masks.make_causal_sliding_window_mask_fns(128, 128, 100),
+            "documents": lambda: masks.make_jagged_mask_fns(128, 128, [200, S - 200])}[mask]()
+    q, k, v, do = inputs(Sq=S, Sk=S, D=D)
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    block_mask._map_cache.clear()
+    torch._dynamo.reset()
+    f = torch.compile(lambda q, k, v: 2 * F.flex_attention(q * 1, k, v, None, pair) + 0, backend="eager")
+    got = [torch.autograd.grad(f(q, k, v), (q, k, v), do) for _ in range(2)]
+    o = 2 * F.flex_attention(q * 1, k, v, None, pair) + 0
+    want = torch.autograd.grad(o, (q, k, v), do)
+    assert torch.equal(f(q, k, v), o)
+    for g in got:
+        agree(g, want)
+
+
 def test_streams_and_threads():
     sc, pair = 1 / math.sqrt(128), masks_of(True)
     want, errors = {}, []
