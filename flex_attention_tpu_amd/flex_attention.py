@@ -171,7 +171,7 @@ def flex_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, score_fn: 
     Gradients flow to q, k, v and ab (``torch.autograd.grad`` / ``.backward()``); higher-order
     differentiation is not supported, as in the reference (jax_exp.py:243-244).
     """
-    if torch.compiler.is_compiling():   # (torch.compile makes the call between its graphs: block maps, plans and launches are no part of one)
+    if torch.compiler.is_dynamo_compiling():   # (torch.compile makes the call between its graphs: block maps, plans and launches are no part of one)
         return torch.compiler.disable(_uncompiled)(q, k, v, score_fn, mask_fns, segment_ids=segment_ids, causal=causal, sm_scale=sm_scale,
                                                    block_q=block_q, block_k=block_k, ab=ab)
     if sm_scale is None:
